@@ -562,16 +562,17 @@ class HandoverEngine final : public Engine {
   int advance(uint64_t* next_count, uint32_t* fatal) override {
     int s = inner_->advance(next_count, fatal);
     if (s == kAdvanceHandover) {
-      PackedHandover h;
-      if (!inner_->handover(h)) throw std::runtime_error("ENGINE_HANDOVER");
-      const uint64_t cand = inner_->candidates, uniq = inner_->unique_candidates, launches_before = inner_->launches;
-      const double secs = inner_->kernel_seconds;
-      const uint64_t streamed = inner_->streamed_bytes;
-      std::unique_ptr<Engine> next(make_segmented_from_packed(g_, o_, state_space_bound(g_), h));
-      inner_ = std::move(next);
-      carried_ = {cand, uniq, launches_before, streamed, secs};
-      ++handovers_;
+      hand_over();
       s = inner_->advance(next_count, fatal);
+    }
+    mirror();
+    return s;
+  }
+  int run_to_end() override {
+    int s = inner_->run_to_end();
+    if (s == kAdvanceHandover) {
+      hand_over();
+      s = inner_->run_to_end();
     }
     mirror();
     return s;
@@ -613,6 +614,17 @@ class HandoverEngine final : public Engine {
     uint64_t candidates = 0, unique = 0, launches = 0, streamed = 0;
     double seconds = 0.0;
   };
+  void hand_over() {
+    PackedHandover h;
+    if (!inner_->handover(h)) throw std::runtime_error("ENGINE_HANDOVER");
+    const uint64_t cand = inner_->candidates, uniq = inner_->unique_candidates, launches_before = inner_->launches;
+    const double secs = inner_->kernel_seconds;
+    const uint64_t streamed = inner_->streamed_bytes;
+    std::unique_ptr<Engine> next(make_segmented_from_packed(g_, o_, state_space_bound(g_), h));
+    inner_ = std::move(next);
+    carried_ = {cand, uniq, launches_before, streamed, secs};
+    ++handovers_;
+  }
   // Counters of the sorted part of a handed-over run are added to the
   // segmented engine's.
   void mirror() {

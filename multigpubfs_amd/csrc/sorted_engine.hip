@@ -23,7 +23,15 @@ namespace mgbfs {
 
 namespace {
 
-constexpr uint32_t kPhaseCount = 4;  // expand, partition, unique, compact
+// Phases: expand, partition, unique, compact of the general path; layers run
+// ahead of the host (sorted_queue.hip) count as a whole.
+constexpr uint32_t kPhaseCount = 5;
+constexpr size_t kCtlOffset = 64;       // in control_: the queue's control ring, then sub-bucket totals
+constexpr uint32_t kQueueRing = 64;     // queued layers' control blocks and records
+constexpr uint32_t kQueueAhead = 3;     // layers queued beyond the one the host waits for
+constexpr uint32_t kBlockLayers = 126;  // layers per one-workgroup launch at most
+constexpr uint64_t kQueueRows = 1ull << 22;  // bank rows reserved for queued layers
+constexpr int kAheadNone = -1;          // run_ahead(): the next layer is one for the general path
 
 }  // namespace
 
@@ -40,6 +48,7 @@ class SortedEngine final : public Engine {
     for (auto& p : cev_)
       for (auto& e : p) MGBFS_HIP(hipEventCreate(&e));
     budget_ = vram_budget(o);
+    bound_ = state_space_bound(g);
     cap_limit_ = o.capacity ? o.capacity : ~0ull;
     flags_ = o.flags;
     // Stored-value layout and parent-edge tags.
@@ -51,11 +60,22 @@ class SortedEngine final : public Engine {
     // per CU, prefetching the next sub-bucket's bounds, measured slower
     // (127 and 122 vs 120 ms per S13 BFS).
     unique_grid_ = 1u << kMaxBucketBits;
-    control_.allocate(64);
+    control_.allocate(kCtlOffset + sizeof(QueueCtl) * kQueueRing + 4 * kQueueSub);
     fine_counts_.allocate(((1ull << kMaxBucketBits) + 1) * 4);
     for (int b = 0; b < 3; ++b) off_[b].allocate(((1ull << kMaxBucketBits) + 1) * 4);
-    MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_), 64, hipHostMallocDefault));
-    grow_bank(0, 1024);
+    // Pinned: the general path's readback words, then the layer records.
+    const size_t host_bytes = 64 + sizeof(LayerRecord) * (kBlockLayers + 1);
+    MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_), host_bytes, hipHostMallocDefault));
+    std::memset(host_, 0, host_bytes);
+    rec_ = reinterpret_cast<LayerRecord*>(host_ + 8);
+    int khz = 0;
+    MGBFS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
+    tick_seconds_ = khz > 0 ? 1e-3 / khz : 0.0;
+    // Test flags that force a mechanism of the general path keep to it.
+    general_only_ = flags_ & (MGBFS_FLAG_TEST_COARSE_BUCKETS | MGBFS_FLAG_TEST_TIGHT_SLABS |
+                              MGBFS_FLAG_TEST_WIDE_ROUTING | MGBFS_FLAG_TEST_SORTED_CAP);
+    update_bytes();
+    if (!grow_bank(0, 1024)) throw std::runtime_error("SORTED_VRAM_CAPACITY");
     reset();
   }
 
@@ -79,11 +99,9 @@ class SortedEngine final : public Engine {
     last_ratio_ = 0.0;
     for (int b = 0; b < 3; ++b) count_[b] = 0;
     count_[0] = 1;
-    nbo_[0] = 1u << kMaxBucketBits;
-    MGBFS_HIP(sorted_seed(start_key_, layout_, bank_[0].as<uint64_t>(), off_[0].as<uint32_t>(), kMaxBucketBits,
-                          stream_));
-    MGBFS_HIP(fill_u64(control_.as<uint64_t>(), 0ull, 8, stream_));
-    MGBFS_HIP(hipStreamSynchronize(stream_));
+    nbo_[0] = 1;  // the start bank has one fine bucket
+    block_rejected_ = 0;
+    start_bank();
     cpending_[0] = cpending_[1] = false;
     layers.assign(1, 1);
     candidates = unique_candidates = 0;
@@ -100,6 +118,30 @@ class SortedEngine final : public Engine {
   int advance(uint64_t* next_count, uint32_t* fatal) override {
     if (terminal) throw std::runtime_error("ENGINE_TERMINAL");
     MGBFS_HIP(hipSetDevice(device_));
+    const int s = run_ahead(1);
+    if (s == kAheadNone) return advance_general(next_count, fatal);
+    *next_count = s == MGBFS_LAYER ? layers.back() : 0;
+    return s;
+  }
+
+  int run_to_end() override {
+    int s = MGBFS_LAYER;
+    if (!terminal) MGBFS_HIP(hipSetDevice(device_));
+    while (!terminal) {
+      s = run_ahead(kBlockLayers);
+      if (s != kAheadNone) continue;
+      uint64_t nc;
+      uint32_t f;
+      s = advance_general(&nc, &f);
+      if (s == kAdvanceHandover) return s;
+    }
+    return s;
+  }
+
+ private:
+  // One layer with its geometry set by the host: every size, owner lanes
+  // above 2^10 sub-buckets, retries after overflows.
+  int advance_general(uint64_t* next_count, uint32_t* fatal) {
     const uint64_t F = count_[cur_];
     const uint32_t G = gens_.count;
     // Every parent yields at most G children, at most G-1 when it carries a
@@ -223,6 +265,7 @@ class SortedEngine final : public Engine {
     }
   }
 
+ public:
   // Another inverse-closed graph of the same degree reuses every bank and slab.
   void rebind(const Graph& g) override {
     if (g.elements != n_ || !g.packable() || !g.inverse_closed) throw std::runtime_error("ENGINE_REBIND_SHAPE");
@@ -267,8 +310,8 @@ class SortedEngine final : public Engine {
     for (int s = 0; s < 2; ++s) read_compact(s);
   }
 
-  double phase_seconds[kPhaseCount] = {0, 0, 0, 0};
-  uint64_t phase_bytes[kPhaseCount] = {0, 0, 0, 0};
+  double phase_seconds[kPhaseCount] = {};
+  uint64_t phase_bytes[kPhaseCount] = {};
   uint64_t retries = 0;
 
   void fill_phases(double* seconds, uint64_t* bytes, uint32_t n) const override {
@@ -279,6 +322,201 @@ class SortedEngine final : public Engine {
   }
 
  private:
+  // Bank rows for the one-workgroup and queued layers, so that they need no
+  // growth: as many as the state space has, at most kQueueRows.  Called with
+  // the start layer current, which is moved if bank 0 grows.  Without the
+  // memory for it (an eighth of the budget at most, so that larger layers
+  // find theirs) the layers take the general path.
+  void reserve_banks() {
+    const uint64_t rows = std::max<uint64_t>(
+        2 * kBlockParents, std::min({bound_ ? bound_ : kQueueRows, cap_limit_, kQueueRows}));
+    const bool have = bank_cap_[0] >= rows && bank_cap_[1] >= rows && bank_cap_[2] >= rows;
+    if (!have && 8 * (3 * rows + kQueueSub * static_cast<uint64_t>(kSlabStride) + kRouteDump) > budget_ / 8) return;
+    if (have) return;
+    const bool grown = grow_bank(0, rows);
+    start_bank();
+    if (grown && grow_bank(1, rows)) grow_bank(2, rows);
+  }
+  void start_bank() {
+    MGBFS_HIP(sorted_start(keymix(start_key_, layout_.km) << layout_.tagbits, bank_[0].as<uint64_t>(),
+                           off_[0].as<uint32_t>(), control_.as<uint64_t>(), stream_));
+  }
+  uint64_t bank_rows() const {
+    return std::min({bank_cap_[0], bank_cap_[1], bank_cap_[2], cap_limit_, static_cast<uint64_t>(0xfffffff0u)});
+  }
+
+  // Runs up to max_layers layers in the one-workgroup kernel or the queue,
+  // whichever the current layer's size asks for; kAheadNone when it is one
+  // for the general path (too large, or rejected on the device).
+  int run_ahead(uint32_t max_layers) {
+    if (general_only_) return kAheadNone;
+    if (layers.size() == 1) reserve_banks();
+    const uint64_t F = count_[cur_], rows = bank_rows();
+    const bool probe_prev = prev_ >= 0 && !layout_.prune;
+    const uint64_t Fp = prev_ >= 0 ? count_[prev_] : 0;
+    if (F <= kBlockParents && (!probe_prev || Fp <= kBlockParents) && rows >= 2 * kBlockParents &&
+        children_guess(F) <= kBlockChildren && block_rejected_ != layers.size()) {
+      const int s = run_block(max_layers, static_cast<uint32_t>(rows));
+      if (s != kAheadNone) return s;
+    }
+    if (F > rows || F * gens_.count > 0x7fffffffull) return kAheadNone;
+    return run_queue(max_layers, static_cast<uint32_t>(rows));
+  }
+
+  // Children expected of the current layer (see advance_general): the last
+  // masked layer's children per parent plus 10%, else every child.
+  uint64_t children_guess(uint64_t F) const {
+    const uint32_t G = gens_.count;
+    const bool masked = layout_.prune && layers.size() > 1;
+    const uint64_t most = F * (masked && G > 1 ? G - 1 : G);
+    if (!masked || last_ratio_ <= 0) return most;
+    return std::min<uint64_t>(most, static_cast<uint64_t>(static_cast<double>(F) * last_ratio_ * 1.1));
+  }
+
+  int run_block(uint32_t max_layers, uint32_t rows) {
+    BlockRun r{};
+    for (int b = 0; b < 3; ++b) {
+      r.bank[b] = bank_[b].as<uint64_t>();
+      r.off[b] = off_[b].as<uint32_t>();
+    }
+    r.L = layout_;
+    r.cur = static_cast<uint32_t>(cur_);
+    r.prev = prev_ >= 0 ? static_cast<uint32_t>(prev_) : 3u;
+    r.F = static_cast<uint32_t>(count_[cur_]);
+    r.prev_count = prev_ >= 0 ? static_cast<uint32_t>(std::min<uint64_t>(count_[prev_], ~0u)) : 0u;
+    r.depth = static_cast<uint32_t>(layers.size() - 1);
+    r.max_layers = std::min(max_layers, kBlockLayers);
+    r.rows = rows;
+    r.rec = rec_ + 1;
+    r.seq = seq_ + 1;
+    seq_ += kBlockLayers + 1;
+    MGBFS_HIP(sorted_block_run(r, gens_, stream_));
+    uint64_t first = 0;
+    for (uint32_t i = 0;; ++i) {
+      const LayerRecord& rec = await(rec_[1 + i], r.seq + i);
+      if (i == 0) first = rec.ticks;
+      const int s = take(rec, rec.ticks - first);
+      first = rec.ticks;
+      if (s != kTakeNext) {
+        if (i > 0 || rec.state == kLayerStop) {  // layers were accepted: the live banks have one fine bucket
+          nbo_[cur_] = 1;
+          if (prev_ >= 0) nbo_[prev_] = 1;
+        }
+        if (s == kTakeRejected) block_rejected_ = layers.size();
+        return finish(s, i);
+      }
+    }
+  }
+
+  // Queued layers: each is three launches whose geometry the layer before
+  // it left in ctl_; the host stays kQueueAhead layers ahead of the records.
+  int run_queue(uint32_t max_layers, uint32_t rows) {
+    const uint64_t F = count_[cur_];
+    const uint32_t G = gens_.count, kids = layout_.prune ? (G > 1 ? G - 1 : 1) : G;
+    const bool masked = layout_.prune && layers.size() > 1;
+    const uint64_t guess = children_guess(F);
+    if (guess > static_cast<uint64_t>(kQueueSub) * kQueueTarget) return kAheadNone;
+    if (!ensure_slabs(0, kQueueSub * static_cast<uint64_t>(kSlabStride) + kRouteDump)) return kAheadNone;
+    ensure_u32(scount_, kQueueSub);
+    QueueCtl first{};
+    first.F = static_cast<uint32_t>(F);
+    first.nsub = queue_sub_buckets(guess);
+    first.fb = queue_fine_bits(first.nsub, margin_);
+    first.nbo_cur = nbo_[cur_];
+    first.nbo_prev = prev_ >= 0 ? nbo_[prev_] : 1;
+    first.masked = masked;
+    first.range_inv = range_inverse(first.nsub);
+    const QueueRules rules{kids, G, layout_.prune, margin_, rows, kBlockChildren / 2};
+    QueueCtl* ctl = reinterpret_cast<QueueCtl*>(control_.as<char>() + kCtlOffset);
+    uint32_t* totals = reinterpret_cast<uint32_t*>(ctl + kQueueRing);
+    const uint64_t seq = seq_;
+    seq_ += kBlockLayers + 1;
+    MGBFS_HIP(sorted_queue_begin(ctl, first, scount_.as<uint32_t>(), rec_, seq, stream_));
+    int qcur = cur_, qprev = prev_;
+    uint32_t queued = 0;
+    const uint32_t most = std::min(max_layers, kBlockLayers);
+    uint64_t ticks = 0;
+    for (uint32_t got = 0;; ++got) {
+      for (; queued < most && queued <= got + kQueueAhead; ++queued) {
+        const int nxt = free_bank(qcur, qprev);
+        // Small tiles while the layer is too small to fill the CUs with full ones.
+        const bool large = static_cast<uint64_t>(count_[cur_]) * G > (1ull << 20);
+        const uint64_t* prev_bank = qprev >= 0 && !layout_.prune ? bank_[qprev].as<uint64_t>() : nullptr;
+        MGBFS_HIP(sorted_queue_expand(bank_[qcur].as<uint64_t>(), ctl + queued % kQueueRing, gens_, layout_,
+                                      scount_.as<uint32_t>(), sub_.as<uint64_t>(), large ? 8 : 4, 1024, stream_));
+        MGBFS_HIP(sorted_unique_queued(sub_.as<uint64_t>(), scount_.as<uint32_t>(), kQueueSub,
+                                       bank_[qcur].as<uint64_t>(), off_[qcur].as<uint32_t>(), prev_bank,
+                                       prev_bank ? off_[qprev].as<uint32_t>() : nullptr, fine_counts_.as<uint32_t>(),
+                                       totals, ctl + queued % kQueueRing, layout_.tagbits,
+                                       layout_.prune != 0, stream_));
+        MGBFS_HIP(sorted_queue_compact(sub_.as<uint64_t>(), fine_counts_.as<uint32_t>(), totals,
+                                       scount_.as<uint32_t>(), ctl + queued % kQueueRing,
+                                       ctl + (queued + 1) % kQueueRing, rules, bank_[nxt].as<uint64_t>(),
+                                       off_[nxt].as<uint32_t>(), rec_ + 1 + queued % kQueueRing, seq + 1 + queued,
+                                       stream_));
+        qprev = qcur;
+        qcur = nxt;
+      }
+      if (got == 0) ticks = await(rec_[0], seq).ticks;
+      const LayerRecord& rec = await(rec_[1 + got % kQueueRing], seq + 1 + got);
+      const int s = take(rec, rec.ticks - ticks);
+      ticks = rec.ticks;
+      if (s == kTakeNext && got + 1 < most) continue;
+      return finish(s, got);
+    }
+  }
+
+  enum Take { kTakeNext, kTakeStop, kTakeEmpty, kTakeRejected };
+  // A layer's record into the engine's state and counters.
+  int take(const LayerRecord& rec, uint64_t ticks) {
+    const double seconds = static_cast<double>(ticks) * tick_seconds_;
+    phase_seconds[4] += seconds;
+    kernel_seconds += seconds;
+    if (rec.state == kLayerRejected) return kTakeRejected;
+    const uint64_t F = count_[cur_];
+    const bool masked = layout_.prune && layers.size() > 1;
+    candidates += rec.cand;
+    unique_candidates += rec.unique;
+    last_ratio_ = masked ? static_cast<double>(rec.cand) / static_cast<double>(F) : 0.0;
+    const uint64_t bytes = 8 * F + 16 * rec.cand + 8 * F + 24 * rec.N;
+    phase_bytes[4] += bytes;
+    streamed_bytes += bytes;
+    ++launches;
+    if (rec.state == kLayerEmpty) return kTakeEmpty;
+    const int nxt = next_bank();
+    nbo_[nxt] = rec.nbo;
+    count_[nxt] = rec.N;
+    prev_ = cur_;
+    cur_ = nxt;
+    layers.push_back(rec.N);
+    return rec.state == kLayerStop ? kTakeStop : kTakeNext;
+  }
+  // Status of a finished run of layers, `accepted` of them before the last.
+  int finish(int s, uint32_t accepted) {
+    if (s == kTakeEmpty) {
+      terminal = true;
+      return MGBFS_COMPLETE;
+    }
+    if (s == kTakeRejected && accepted == 0) return kAheadNone;
+    return MGBFS_LAYER;  // a rejected layer after accepted ones is met again by the next call
+  }
+  // Waits for a record in pinned memory: 6 us after its kernel against 16
+  // for a copy and a stream wait.  The kernels always leave their records,
+  // so a long silence means a device error, which the stream wait reports.
+  const LayerRecord& await(const LayerRecord& rec, uint64_t seq) {
+    for (uint32_t spin = 0;; ++spin) {
+      if (__atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) == seq) return rec;
+      if (spin >= (1u << 20)) break;
+    }
+    MGBFS_HIP(hipStreamSynchronize(stream_));
+    if (__atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) != seq) throw std::runtime_error("SORTED_LAYER_RECORD");
+    return rec;
+  }
+  int free_bank(int cur, int prev) const {
+    for (int b = 0; b < 3; ++b)
+      if (b != cur && b != prev) return b;
+    return -1;
+  }
   uint32_t* error_word() { return reinterpret_cast<uint32_t*>(control_.as<uint64_t>() + 1); }
   // Back-edge masks of gens_ (tag bits 0..G-1; bit tagbits-1 is the in-bank
   // mark and bit tagbits-2 stays clear, so no entry is all ones), the
@@ -320,11 +558,7 @@ class SortedEngine final : public Engine {
   uint64_t routed(uint64_t entries) const {
     return (flags_ & MGBFS_FLAG_TEST_WIDE_ROUTING) ? ~0ull : entries;
   }
-  int next_bank() const {
-    for (int b = 0; b < 3; ++b)
-      if (b != cur_ && b != prev_) return b;
-    return -1;
-  }
+  int next_bank() const { return free_bank(cur_, prev_); }
   // Phase times (events on the engine stream) and modelled streaming bytes
   // (see the kernel file header).  Phase 2 is unique_diff alone; the fine
   // count scan is charged to phase 3 with the compaction it feeds.
@@ -409,6 +643,11 @@ class SortedEngine final : public Engine {
   uint32_t nbo_[3] = {0, 0, 0};  // fine buckets of each bank
   int cur_ = 0, prev_ = -1;
   uint64_t* host_ = nullptr;
+  LayerRecord* rec_ = nullptr;       // pinned, after host_'s words: begin record, then one per layer
+  uint64_t seq_ = 1, bound_ = 0;     // next unused record number; state-space bound (0 = unknown)
+  double tick_seconds_ = 0.0;        // one wall_clock64() tick
+  size_t block_rejected_ = 0;        // layers.size() when the one-workgroup kernel last refused a layer
+  bool general_only_ = false;
   hipEvent_t ev_[6] = {}, cev_[2][2] = {};
   bool cpending_[2] = {false, false};
   int cslot_ = 0;

@@ -386,3 +386,47 @@ def test_capacity_limit_stops_with_resource(backend):
         ref = O.packed_bfs(8)["layers"]
         sizes = e.layer_sizes()
         assert sizes == ref[:len(sizes)]
+
+
+def coxeter(n):
+    return [list(range(i)) + [i + 1, i] + list(range(i + 2, n)) for i in range(n - 1)]
+
+
+# run() lets the sorted backend run layers ahead of the host: small ones in
+# one workgroup, larger ones queued.  The sizes cross from one form to the
+# other and back (S_8: one workgroup and the queue around its 4,913-state
+# peak; S_10: the queue up to 316,158 states; ten generators; flag 8: three
+# banks without masks; degree 15 with repeated labels: no room for masks).
+RUN_AHEAD = {
+    "lrx3": (lambda: (O.lrx_generators(3), [0, 1, 2]), 0),
+    "lrx8": (lambda: (O.lrx_generators(8), list(range(8))), 0),
+    "lrx9": (lambda: (O.lrx_generators(9), list(range(9))), 0),
+    "lrx9_unmasked": (lambda: (O.lrx_generators(9), list(range(9))), 8),
+    "coxeter8": (lambda: (coxeter(8), list(range(8))), 0),
+    "coxeter8_unmasked": (lambda: (coxeter(8), list(range(8))), 8),
+    "labels15": (lambda: (O.lrx_generators(15), [0] * 6 + [1] * 9), 0),
+    "labels13": (lambda: (O.lrx_generators(13), [0] * 4 + [1] * 4 + [2] * 5), 0),
+}
+
+
+@pytest.mark.parametrize("name", list(RUN_AHEAD))
+def test_sorted_run_ahead_matches_oracle_and_layer_loop(name):
+    make, flags = RUN_AHEAD[name]
+    gens, start = make()
+    graph = GraphDefinition.permutation(gens, start)
+    ref = [sorted(O.pack(s) for s in layer) for layer in O.c_exact_layers(graph.to_dict(), math.factorial(10))]
+    sizes = [len(x) for x in ref]
+    with NativeEngine(graph, backend="sorted", flags=flags) as e:
+        for stop in (0, 1, len(sizes) // 2):  # from the start, after one layer, from the middle
+            e.reset()
+            for d in range(stop):
+                assert e.advance() == 0
+                assert sorted(e.layer_keys()) == ref[d + 1]
+            assert e.run() == 1
+            assert e.layer_sizes() == sizes
+            assert sorted(e.layer_keys()) == ref[-1]
+            prev = sorted(O.pack(r) for r in e.sample(1, 1 << 20))
+            assert prev == ref[-2]
+        e.reset()
+        assert e.run(max_layers=len(sizes) - 2) == 0
+        assert sorted(e.layer_keys()) == ref[-2]
