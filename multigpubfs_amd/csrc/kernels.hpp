@@ -41,66 +41,30 @@ struct SortedLayout {
   uint64_t tagmask;  // (1 << tagbits) - 1
 };
 
-// Layers run ahead of the host (sorted_queue.hip).  Geometry and counters
-// of one queued layer, written on the device by the layer before it.
-struct QueueCtl {
-  uint32_t F;         // parents; 0: the queue has stopped and the layer does nothing
-  uint32_t nsub, fb;  // sub-buckets (no owner lanes) and fine-bucket bits
-  uint32_t nbo_cur, nbo_prev;  // fine buckets of the current and previous bank
-  uint32_t masked;    // parents carry back-edge masks
-  uint64_t range_inv;  // range_inverse(nsub)
-  unsigned long long unique, cand;
-  uint32_t error, pad;
-};
-
+// Layers run ahead of the host (sorted_queue.hip).
 // What the host learns of a layer, in pinned memory; seq is written last.
 enum LayerState : uint32_t {
-  kLayerNext = 0,      // accepted, the next queued layer runs
-  kLayerStop = 1,      // accepted, the queue stops here
+  kLayerNext = 0,      // accepted, the next layer runs
+  kLayerStop = 1,      // accepted, no further layer runs
   kLayerEmpty = 2,     // no new states: the search is complete
-  kLayerRejected = 3,  // not accepted (an error bit, or too many rows): the host redoes it
+  kLayerRejected = 3,  // not accepted (an overflow, or too many rows): the host redoes it
 };
 struct LayerRecord {
-  uint64_t N, cand, unique, ticks;  // ticks: wall_clock64() when the layer was counted
-  uint32_t state, nbo;              // nbo: fine buckets of the bank written
+  uint64_t N, unique, ticks;  // ticks: wall_clock64() when the layer was counted
+  uint64_t children;          // block_run: generated for this layer; owner layers: from it
+  uint32_t state, pad;
   uint64_t seq;
-};
-
-// Rules of the queue, the same for every layer of a session.
-struct QueueRules {
-  uint32_t kids, kids_first;  // children per parent at most (later layers; the start layer)
-  uint32_t prune, margin;     // back-edge masks in use; fine-bucket margin
-  uint32_t rows;              // rows every bank holds (and the caller's layer capacity)
-  uint32_t low;               // stop once a layer is expected to have at most this many children
 };
 
 // One-workgroup layers: everything fits one LDS table.
 constexpr uint32_t kBlockSlots = 16384;
 constexpr uint32_t kBlockFill = 14336;     // entries accepted (plus one per lane in flight)
 constexpr uint32_t kBlockParents = 4096;   // parents of such a layer at most
-// A layer of more children than this is quicker in the queue: on S_8 and
-// S_10 LRX one workgroup takes 8 us for 1,200 children, 15 for 2,600, 24 for
-// 4,700 and 34 for 5,700 (10 generators: 44 for 12,000, 300 for 28,000, as
-// the table fills), a queued layer 19 to 23 us up to 60,000.
+// A layer of more children than this is quicker with one owner per
+// workgroup: on S_8 and S_10 LRX one workgroup takes 8 us for 1,200
+// children, 15 for 2,600, 24 for 4,700 and 34 for 5,700 (10 generators: 44
+// for 12,000, 300 for 28,000, as the table fills).
 constexpr uint32_t kBlockChildren = 4096;
-constexpr uint32_t kQueueSub = 1024;       // sub-buckets of a queued layer at most (one routing pass)
-
-// Sub-buckets of a queued layer of about `children` children: one per
-// kQueueFill while that gives at most one workgroup per CU (a sub-bucket's
-// latency falls with its size), then as full as the LDS table takes them.
-constexpr uint32_t kQueueFill = 1024;
-constexpr uint32_t kQueueTarget = 5000;
-__host__ __device__ inline uint32_t queue_sub_buckets(uint64_t children) {
-  const uint64_t spread = (children + kQueueFill - 1) / kQueueFill;
-  const uint64_t full = (children + kQueueTarget - 1) / kQueueTarget;
-  const uint64_t n = spread < 256 ? spread : (full > 256 ? full : 256);
-  return static_cast<uint32_t>(n ? n : 1);
-}
-__host__ __device__ inline uint32_t queue_fine_bits(uint32_t nsub, uint32_t margin) {
-  uint32_t k = 0;
-  while ((1u << k) < nsub) ++k;
-  return margin < kMaxBucketBits - k ? margin : kMaxBucketBits - k;
-}
 
 struct BlockRun {
   uint64_t* bank[3];
@@ -110,26 +74,71 @@ struct BlockRun {
   uint32_t F, prev_count, depth;
   uint32_t generators, max_layers;
   uint32_t rows;             // rows every bank holds (and the caller's layer capacity)
-  LayerRecord* rec;          // pinned, max_layers + 1 records: one per layer run
+  LayerRecord* rec;          // pinned: one record per layer run
   uint64_t seq;              // rec[i].seq = seq + i
 };
 
-hipError_t sorted_block_run(const BlockRun& run, const PackedGenerators& gens, hipStream_t stream);
+// Owner layers: `owners` sub-buckets (equal ranges of the top 32 bits), one
+// workgroup each; the layers' states and the candidates live in slabs of
+// kSlabStride entries per owner.
+constexpr uint32_t kOwnersMax = 1024;
+constexpr uint32_t kOwnersSmall = 256;
+constexpr uint32_t kOwnerMean = 4600;  // children per owner at most (a slab holds kUniqueCap)
+
+// Totals of one owner layer; zeroed two launches before its own.
+struct OwnerCtl {
+  unsigned long long counts;  // states of the layer, + children made from it << 32
+  unsigned long long unique;  // distinct children the layer was selected from
+  uint32_t error;             // the layer is not usable
+  uint32_t spill;             // the children made from it are incomplete (a slab was full)
+  uint32_t halt;              // no layer: an earlier one was the last
+  uint32_t imported;          // the session's first: goes on however few its children
+};
+
+struct OwnerRules {
+  uint32_t owners;
+  uint32_t rows;       // states a layer may have (bank rows, the caller's capacity)
+  uint32_t low, high;  // children outside [low, high] end the session
+};
+
+struct OwnerSlabs {
+  uint64_t* data;   // owners x kSlabStride entries
+  uint32_t* count;  // entries per owner
+};
+
+struct OwnerImport {
+  const uint64_t* cur;   // dense banks
+  const uint64_t* prev;  // null unless both retained layers are probed
+  uint32_t F, prev_count, masked;
+  OwnerSlabs own, own_prev, cand;
+  OwnerCtl* ctl;  // the imported layer's
+};
+
+struct OwnerLayer {
+  OwnerSlabs in, out;          // candidates of this layer; of the next one
+  OwnerSlabs cur, prev, next;  // retained layers (prev.data null: masked) and the new one
+  const OwnerCtl* before;
+  OwnerCtl *now, *after;
+  OwnerRules rules;
+  LayerRecord* rec;  // record of the layer before
+  uint64_t seq;
+};
+
 hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t* control, hipStream_t stream);
-hipError_t sorted_queue_begin(QueueCtl* ctl, const QueueCtl& first, uint32_t* scount, LayerRecord* rec, uint64_t seq,
-                              hipStream_t stream);
-// One queued layer: expand, unique, compact (geometry in ctl[0], the next
-// layer's written to *next).
-hipError_t sorted_queue_expand(const uint64_t* bank, QueueCtl* ctl, const PackedGenerators& gens,
-                               const SortedLayout& L, uint32_t* scount, uint64_t* out, uint32_t items, uint32_t grid,
-                               hipStream_t stream);
-hipError_t sorted_unique_queued(uint64_t* cand, const uint32_t* scount, uint32_t max_sub, const uint64_t* cur,
-                                const uint32_t* cur_off, const uint64_t* prev, const uint32_t* prev_off,
-                                uint32_t* fine_counts, uint32_t* totals, QueueCtl* ctl, uint32_t tagbits, bool merge,
-                                hipStream_t stream);
-hipError_t sorted_queue_compact(const uint64_t* cand, const uint32_t* fine_counts, const uint32_t* totals,
-                                uint32_t* scount, const QueueCtl* ctl, QueueCtl* next, const QueueRules& rules,
-                                uint64_t* bank, uint32_t* off, LayerRecord* rec, uint64_t seq, hipStream_t stream);
+hipError_t sorted_block_run(const BlockRun& run, const PackedGenerators& gens, hipStream_t stream);
+// Zeroes the owners' counts (`words` of them from `counts`) and the first
+// control blocks; ctl[0] becomes the imported layer's, of F states.
+hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream);
+hipError_t owner_import(const OwnerImport& im, const PackedGenerators& gens, const SortedLayout& L, uint32_t owners,
+                        hipStream_t stream);
+hipError_t owner_layer(const OwnerLayer& a, const PackedGenerators& gens, const SortedLayout& L, hipStream_t stream);
+// Reports the last layer queued (a layer launch reports the one before it).
+hipError_t owner_report(const OwnerCtl* ctl, const OwnerRules& rules, LayerRecord* rec, uint64_t seq,
+                        hipStream_t stream);
+// Owner slabs -> dense bank and offset table of `owners` fine buckets, for
+// the current layer and the one before.
+hipError_t owner_export(const OwnerSlabs& cur, uint64_t* bank, uint32_t* off, const OwnerSlabs& prev,
+                        uint64_t* prev_bank, uint32_t* prev_off, uint32_t owners, hipStream_t stream);
 
 uint64_t scan_workspace_words(uint64_t n);
 hipError_t exclusive_scan_u32(const uint32_t* in, uint64_t n, uint32_t* out, uint32_t* workspace,

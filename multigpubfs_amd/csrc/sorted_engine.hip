@@ -26,11 +26,12 @@ namespace {
 // Phases: expand, partition, unique, compact of the general path; layers run
 // ahead of the host (sorted_queue.hip) count as a whole.
 constexpr uint32_t kPhaseCount = 5;
-constexpr size_t kCtlOffset = 64;       // in control_: the queue's control ring, then sub-bucket totals
-constexpr uint32_t kQueueRing = 64;     // queued layers' control blocks and records
-constexpr uint32_t kQueueAhead = 3;     // layers queued beyond the one the host waits for
+constexpr size_t kCtlOffset = 64;       // in control_: the owner layers' control ring, then their slab counts
+constexpr uint32_t kOwnerRing = 64;     // owner layers' control blocks and records
+constexpr uint32_t kOwnerAhead = 3;     // layers queued beyond the one whose record the host waits for
+constexpr uint32_t kOwnerBuffers = 5;   // slab arrays: two of candidates, three of layers
 constexpr uint32_t kBlockLayers = 126;  // layers per one-workgroup launch at most
-constexpr uint64_t kQueueRows = 1ull << 22;  // bank rows reserved for queued layers
+constexpr uint64_t kAheadRows = 1ull << 22;  // bank rows reserved for layers run ahead
 constexpr int kAheadNone = -1;          // run_ahead(): the next layer is one for the general path
 
 }  // namespace
@@ -60,7 +61,7 @@ class SortedEngine final : public Engine {
     // per CU, prefetching the next sub-bucket's bounds, measured slower
     // (127 and 122 vs 120 ms per S13 BFS).
     unique_grid_ = 1u << kMaxBucketBits;
-    control_.allocate(kCtlOffset + sizeof(QueueCtl) * kQueueRing + 4 * kQueueSub);
+    control_.allocate(kCtlOffset + sizeof(OwnerCtl) * kOwnerRing + 4 * kOwnerBuffers * kOwnersMax);
     fine_counts_.allocate(((1ull << kMaxBucketBits) + 1) * 4);
     for (int b = 0; b < 3; ++b) off_[b].allocate(((1ull << kMaxBucketBits) + 1) * 4);
     // Pinned: the general path's readback words, then the layer records.
@@ -100,7 +101,7 @@ class SortedEngine final : public Engine {
     for (int b = 0; b < 3; ++b) count_[b] = 0;
     count_[0] = 1;
     nbo_[0] = 1;  // the start bank has one fine bucket
-    block_rejected_ = 0;
+    block_rejected_ = owner_rejected_ = 0;
     start_bank();
     cpending_[0] = cpending_[1] = false;
     layers.assign(1, 1);
@@ -322,21 +323,22 @@ class SortedEngine final : public Engine {
   }
 
  private:
-  // Bank rows for the one-workgroup and queued layers, so that they need no
-  // growth: as many as the state space has, at most kQueueRows.  Called with
-  // the start layer current, which is moved if bank 0 grows.  Without the
+  // Bank rows for the layers run ahead, so that they need no growth: as many
+  // as the state space has, at most kAheadRows.  Called with the start layer
+  // current, which is written again as bank 0 may have moved.  Without the
   // memory for it (an eighth of the budget at most, so that larger layers
   // find theirs) the layers take the general path.
   void reserve_banks() {
-    const uint64_t rows = std::max<uint64_t>(
-        2 * kBlockParents, std::min({bound_ ? bound_ : kQueueRows, cap_limit_, kQueueRows}));
-    const bool have = bank_cap_[0] >= rows && bank_cap_[1] >= rows && bank_cap_[2] >= rows;
-    if (!have && 8 * (3 * rows + kQueueSub * static_cast<uint64_t>(kSlabStride) + kRouteDump) > budget_ / 8) return;
-    if (have) return;
+    const uint64_t rows =
+        std::max<uint64_t>(2 * kBlockParents, std::min({bound_ ? bound_ : kAheadRows, cap_limit_, kAheadRows}));
+    if (bank_cap_[0] >= rows && bank_cap_[1] >= rows && bank_cap_[2] >= rows) return;
+    if (8 * (3 * rows + kOwnerBuffers * owner_entries(kOwnersSmall)) > budget_ / 8) return;
     const bool grown = grow_bank(0, rows);
     start_bank();
     if (grown && grow_bank(1, rows)) grow_bank(2, rows);
   }
+  // Entries of one slab array (with the routing dump area).
+  static constexpr uint64_t owner_entries(uint32_t owners) { return owners * static_cast<uint64_t>(kSlabStride) + kRouteDump; }
   void start_bank() {
     MGBFS_HIP(sorted_start(keymix(start_key_, layout_.km) << layout_.tagbits, bank_[0].as<uint64_t>(),
                            off_[0].as<uint32_t>(), control_.as<uint64_t>(), stream_));
@@ -345,9 +347,9 @@ class SortedEngine final : public Engine {
     return std::min({bank_cap_[0], bank_cap_[1], bank_cap_[2], cap_limit_, static_cast<uint64_t>(0xfffffff0u)});
   }
 
-  // Runs up to max_layers layers in the one-workgroup kernel or the queue,
-  // whichever the current layer's size asks for; kAheadNone when it is one
-  // for the general path (too large, or rejected on the device).
+  // Runs up to max_layers layers in the one-workgroup kernel or as owner
+  // layers, whichever the current layer's size asks for; kAheadNone when it
+  // is one for the general path (too large, or rejected on the device).
   int run_ahead(uint32_t max_layers) {
     if (general_only_) return kAheadNone;
     if (layers.size() == 1) reserve_banks();
@@ -359,8 +361,8 @@ class SortedEngine final : public Engine {
       const int s = run_block(max_layers, static_cast<uint32_t>(rows));
       if (s != kAheadNone) return s;
     }
-    if (F > rows || F * gens_.count > 0x7fffffffull) return kAheadNone;
-    return run_queue(max_layers, static_cast<uint32_t>(rows));
+    if (F > rows || F * gens_.count > 0x7fffffffull || owner_rejected_ == layers.size()) return kAheadNone;
+    return run_owner(max_layers, static_cast<uint32_t>(rows));
   }
 
   // Children expected of the current layer (see advance_general): the last
@@ -387,15 +389,15 @@ class SortedEngine final : public Engine {
     r.depth = static_cast<uint32_t>(layers.size() - 1);
     r.max_layers = std::min(max_layers, kBlockLayers);
     r.rows = rows;
-    r.rec = rec_ + 1;
-    r.seq = seq_ + 1;
-    seq_ += kBlockLayers + 1;
+    r.rec = rec_;
+    r.seq = seq_;
+    seq_ += kBlockLayers + 2;
     MGBFS_HIP(sorted_block_run(r, gens_, stream_));
     uint64_t first = 0;
     for (uint32_t i = 0;; ++i) {
-      const LayerRecord& rec = await(rec_[1 + i], r.seq + i);
+      const LayerRecord& rec = await(rec_[i], r.seq + i);
       if (i == 0) first = rec.ticks;
-      const int s = take(rec, rec.ticks - first);
+      const int s = take(rec, rec.children, rec.ticks - first);
       first = rec.ticks;
       if (s != kTakeNext) {
         if (i > 0 || rec.state == kLayerStop) {  // layers were accepted: the live banks have one fine bucket
@@ -408,83 +410,115 @@ class SortedEngine final : public Engine {
     }
   }
 
-  // Queued layers: each is three launches whose geometry the layer before
-  // it left in ctl_; the host stays kQueueAhead layers ahead of the records.
-  int run_queue(uint32_t max_layers, uint32_t rows) {
-    const uint64_t F = count_[cur_];
-    const uint32_t G = gens_.count, kids = layout_.prune ? (G > 1 ? G - 1 : 1) : G;
-    const bool masked = layout_.prune && layers.size() > 1;
-    const uint64_t guess = children_guess(F);
-    if (guess > static_cast<uint64_t>(kQueueSub) * kQueueTarget) return kAheadNone;
-    if (!ensure_slabs(0, kQueueSub * static_cast<uint64_t>(kSlabStride) + kRouteDump)) return kAheadNone;
-    ensure_u32(scount_, kQueueSub);
-    QueueCtl first{};
-    first.F = static_cast<uint32_t>(F);
-    first.nsub = queue_sub_buckets(guess);
-    first.fb = queue_fine_bits(first.nsub, margin_);
-    first.nbo_cur = nbo_[cur_];
-    first.nbo_prev = prev_ >= 0 ? nbo_[prev_] : 1;
-    first.masked = masked;
-    first.range_inv = range_inverse(first.nsub);
-    const QueueRules rules{kids, G, layout_.prune, margin_, rows, kBlockChildren / 2};
-    QueueCtl* ctl = reinterpret_cast<QueueCtl*>(control_.as<char>() + kCtlOffset);
-    uint32_t* totals = reinterpret_cast<uint32_t*>(ctl + kQueueRing);
+  // A session of owner layers: each is one launch, which also reports the
+  // layer before it; the host stays kOwnerAhead launches ahead.  256 owners
+  // (one workgroup per CU) while the children fit their slabs, else 1,024.
+  int run_owner(uint32_t max_layers, uint32_t rows) {
+    const uint64_t F = count_[cur_], guess = children_guess(F);
+    const uint32_t owners = guess <= kOwnersSmall * kOwnerMean / 2 ? kOwnersSmall : kOwnersMax;
+    if (guess > static_cast<uint64_t>(owners) * kOwnerMean) return kAheadNone;
+    const uint64_t entries = owner_entries(owners);
+    if (owner_.bytes() < kOwnerBuffers * entries * 8) {
+      if (kOwnerBuffers * entries * 8 > budget_ / 8 || !fits(kOwnerBuffers * entries * 8 - owner_.bytes()))
+        return kAheadNone;
+      MGBFS_HIP(hipStreamSynchronize(stream_));
+      owner_.release();
+      owner_.allocate(kOwnerBuffers * entries * 8);
+      update_bytes();
+    }
+    OwnerCtl* ctl = reinterpret_cast<OwnerCtl*>(control_.as<char>() + kCtlOffset);
+    uint32_t* counts = reinterpret_cast<uint32_t*>(ctl + kOwnerRing);
+    OwnerSlabs slab[kOwnerBuffers];  // candidates 0 and 1, layers 2 + bank index
+    for (uint32_t k = 0; k < kOwnerBuffers; ++k)
+      slab[k] = OwnerSlabs{owner_.as<uint64_t>() + k * entries, counts + k * kOwnersMax};
+    const bool probe_prev = prev_ >= 0 && !layout_.prune;
+    // 1,024 owners take 28 us where 256 take 18 (12,000 children, S_11 with
+    // ten generators), so a shrinking search changes over; a new session
+    // costs about 25 us.
+    const uint32_t low = owners == kOwnersSmall ? kBlockChildren / 2 : 512 * kOwnersSmall;
+    const OwnerRules rules{owners, rows, low, owners * kOwnerMean};
     const uint64_t seq = seq_;
-    seq_ += kBlockLayers + 1;
-    MGBFS_HIP(sorted_queue_begin(ctl, first, scount_.as<uint32_t>(), rec_, seq, stream_));
+    seq_ += kBlockLayers + 2;
+    MGBFS_HIP(owner_begin(counts, kOwnerBuffers * kOwnersMax, ctl, static_cast<uint32_t>(F), stream_));
+    OwnerImport im{};
+    im.cur = bank_[cur_].as<uint64_t>();
+    im.F = static_cast<uint32_t>(F);
+    im.own = slab[2 + cur_];
+    if (probe_prev) {
+      im.prev = bank_[prev_].as<uint64_t>();
+      im.prev_count = static_cast<uint32_t>(count_[prev_]);
+      im.own_prev = slab[2 + prev_];
+    }
+    im.masked = layout_.prune && layers.size() > 1;
+    im.cand = slab[0];
+    im.ctl = ctl;
+    MGBFS_HIP(owner_import(im, gens_, layout_, owners, stream_));
     int qcur = cur_, qprev = prev_;
-    uint32_t queued = 0;
     const uint32_t most = std::min(max_layers, kBlockLayers);
-    uint64_t ticks = 0;
-    for (uint32_t got = 0;; ++got) {
-      for (; queued < most && queued <= got + kQueueAhead; ++queued) {
+    uint32_t queued = 0, accepted = 0;
+    uint64_t ticks = 0, children = 0;
+    int s = kTakeNext;
+    // Record r is layer r's (0: the imported one), written by launch r + 1.
+    for (uint32_t r = 0;; ++r) {
+      for (; queued < most && queued <= r + kOwnerAhead; ++queued) {
         const int nxt = free_bank(qcur, qprev);
-        // Small tiles while the layer is too small to fill the CUs with full ones.
-        const bool large = static_cast<uint64_t>(count_[cur_]) * G > (1ull << 20);
-        const uint64_t* prev_bank = qprev >= 0 && !layout_.prune ? bank_[qprev].as<uint64_t>() : nullptr;
-        MGBFS_HIP(sorted_queue_expand(bank_[qcur].as<uint64_t>(), ctl + queued % kQueueRing, gens_, layout_,
-                                      scount_.as<uint32_t>(), sub_.as<uint64_t>(), large ? 8 : 4, 1024, stream_));
-        MGBFS_HIP(sorted_unique_queued(sub_.as<uint64_t>(), scount_.as<uint32_t>(), kQueueSub,
-                                       bank_[qcur].as<uint64_t>(), off_[qcur].as<uint32_t>(), prev_bank,
-                                       prev_bank ? off_[qprev].as<uint32_t>() : nullptr, fine_counts_.as<uint32_t>(),
-                                       totals, ctl + queued % kQueueRing, layout_.tagbits,
-                                       layout_.prune != 0, stream_));
-        MGBFS_HIP(sorted_queue_compact(sub_.as<uint64_t>(), fine_counts_.as<uint32_t>(), totals,
-                                       scount_.as<uint32_t>(), ctl + queued % kQueueRing,
-                                       ctl + (queued + 1) % kQueueRing, rules, bank_[nxt].as<uint64_t>(),
-                                       off_[nxt].as<uint32_t>(), rec_ + 1 + queued % kQueueRing, seq + 1 + queued,
-                                       stream_));
+        OwnerLayer a{};
+        a.in = slab[queued & 1u];
+        a.out = slab[(queued & 1u) ^ 1u];
+        a.cur = slab[2 + qcur];
+        if (qprev >= 0 && !layout_.prune) a.prev = slab[2 + qprev];
+        a.next = slab[2 + nxt];
+        a.before = ctl + queued % kOwnerRing;
+        a.now = ctl + (queued + 1) % kOwnerRing;
+        a.after = ctl + (queued + 2) % kOwnerRing;
+        a.rules = rules;
+        a.rec = rec_ + queued % kOwnerRing;
+        a.seq = seq + queued;
+        MGBFS_HIP(owner_layer(a, gens_, layout_, stream_));
         qprev = qcur;
         qcur = nxt;
+        if (queued + 1 == most)  // nothing follows the last layer to report it
+          MGBFS_HIP(owner_report(ctl + most % kOwnerRing, rules, rec_ + most % kOwnerRing, seq + most, stream_));
       }
-      if (got == 0) ticks = await(rec_[0], seq).ticks;
-      const LayerRecord& rec = await(rec_[1 + got % kQueueRing], seq + 1 + got);
-      const int s = take(rec, rec.ticks - ticks);
+      const LayerRecord& rec = await(rec_[r % kOwnerRing], seq + r);
+      if (r == 0) {
+        s = rec.state == kLayerNext ? kTakeNext : kTakeRejected;
+      } else {
+        s = take(rec, children, rec.ticks - ticks);
+        accepted += s == kTakeNext || s == kTakeStop;
+      }
       ticks = rec.ticks;
-      if (s == kTakeNext && got + 1 < most) continue;
-      return finish(s, got);
+      children = rec.children;
+      if (s != kTakeNext || r == most) break;
     }
+    if (accepted) {
+      MGBFS_HIP(owner_export(slab[2 + cur_], bank_[cur_].as<uint64_t>(), off_[cur_].as<uint32_t>(), slab[2 + prev_],
+                             bank_[prev_].as<uint64_t>(), off_[prev_].as<uint32_t>(), owners, stream_));
+      nbo_[cur_] = nbo_[prev_] = owners;
+    }
+    if (s == kTakeRejected) owner_rejected_ = layers.size();
+    return finish(s, accepted);
   }
 
   enum Take { kTakeNext, kTakeStop, kTakeEmpty, kTakeRejected };
-  // A layer's record into the engine's state and counters.
-  int take(const LayerRecord& rec, uint64_t ticks) {
+  // A layer's record into the engine's state and counters; C: children
+  // generated for it.
+  int take(const LayerRecord& rec, uint64_t C, uint64_t ticks) {
     const double seconds = static_cast<double>(ticks) * tick_seconds_;
     phase_seconds[4] += seconds;
     kernel_seconds += seconds;
     if (rec.state == kLayerRejected) return kTakeRejected;
     const uint64_t F = count_[cur_];
     const bool masked = layout_.prune && layers.size() > 1;
-    candidates += rec.cand;
+    candidates += C;
     unique_candidates += rec.unique;
-    last_ratio_ = masked ? static_cast<double>(rec.cand) / static_cast<double>(F) : 0.0;
-    const uint64_t bytes = 8 * F + 16 * rec.cand + 8 * F + 24 * rec.N;
+    last_ratio_ = masked ? static_cast<double>(C) / static_cast<double>(F) : 0.0;
+    const uint64_t bytes = 16 * F + 16 * C + 8 * rec.N;
     phase_bytes[4] += bytes;
     streamed_bytes += bytes;
     ++launches;
     if (rec.state == kLayerEmpty) return kTakeEmpty;
     const int nxt = next_bank();
-    nbo_[nxt] = rec.nbo;
     count_[nxt] = rec.N;
     prev_ = cur_;
     cur_ = nxt;
@@ -629,7 +663,7 @@ class SortedEngine final : public Engine {
   }
   void update_bytes() {
     device_bytes = control_.bytes() + fine_counts_.bytes() + lane_.bytes() + sub_.bytes() + lcount_.bytes() +
-                   scount_.bytes() + scan_ws_.bytes();
+                   scount_.bytes() + scan_ws_.bytes() + owner_.bytes();
     for (int b = 0; b < 3; ++b) device_bytes += bank_[b].bytes() + off_[b].bytes();
   }
 
@@ -643,10 +677,12 @@ class SortedEngine final : public Engine {
   uint32_t nbo_[3] = {0, 0, 0};  // fine buckets of each bank
   int cur_ = 0, prev_ = -1;
   uint64_t* host_ = nullptr;
-  LayerRecord* rec_ = nullptr;       // pinned, after host_'s words: begin record, then one per layer
+  DeviceBuffer owner_;               // owner layers' slab arrays
+  LayerRecord* rec_ = nullptr;       // pinned, after host_'s words
   uint64_t seq_ = 1, bound_ = 0;     // next unused record number; state-space bound (0 = unknown)
   double tick_seconds_ = 0.0;        // one wall_clock64() tick
   size_t block_rejected_ = 0;        // layers.size() when the one-workgroup kernel last refused a layer
+  size_t owner_rejected_ = 0;        // the same of the owner layers
   bool general_only_ = false;
   hipEvent_t ev_[6] = {}, cev_[2][2] = {};
   bool cpending_[2] = {false, false};

@@ -237,10 +237,6 @@ struct UniqueArgs {
   uint32_t merge;    // OR the back-edge masks of duplicates into the kept entry
   uint32_t fb, nbo_c, nbo_p, tagbits, buckets;  // buckets: sub-buckets of this layer
   uint64_t range_inv;                           // range_inverse(buckets)
-  // Queued layers: the geometry fields above come from *ctl, and each
-  // sub-bucket's survivor count goes to totals[].
-  QueueCtl* ctl;
-  uint32_t* totals;
 };
 
 // Bank entry h: if its state is in the table, set `mark` in that slot's
@@ -388,24 +384,10 @@ constexpr int kPairsPerThread = kUniqueSlots / 2 / kUniqueThreads;  // table slo
 // banks, marking matched slots -> the occupied, unmarked slots are the
 // survivors: count them per fine bucket, scan, and write them back into
 // the slab grouped by fine bucket.
-// kQueued: a layer queued ahead of the host (sorted_queue.hip), its geometry
-// read from the device; a stopped queue (no parents) does nothing.
-template <bool kPrev, bool kQueued>
+template <bool kPrev>
 __global__ __launch_bounds__(kUniqueThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void unique_diff_kernel(
     UniqueArgs a) {
   __shared__ UniqueLds u;
-  if constexpr (kQueued) {
-    QueueCtl* c = a.ctl;
-    if (c->F == 0) return;
-    a.buckets = c->nsub;
-    a.range_inv = c->range_inv;
-    a.fb = c->fb;
-    a.nbo_c = c->nbo_cur;
-    a.nbo_p = c->nbo_prev;
-    a.error = &c->error;
-    a.unique_total = &c->unique;
-    a.cand_total = &c->cand;
-  }
   const uint32_t fine_bits = a.fb, fine = 1u << fine_bits;
   const uint32_t nbo = a.buckets << fine_bits;  // fine buckets of the layer written
   // Fine bucket of a survivor of sub-bucket f, within f.  A layer whose
@@ -438,7 +420,6 @@ __global__ __launch_bounds__(kUniqueThreads) __attribute__((amdgpu_waves_per_eu(
       if (threadIdx.x == 0) atomicOr(a.error, kErrBucketCap);
       for (uint32_t i = threadIdx.x; i < fine; i += kUniqueThreads)
         a.fine_counts[(static_cast<uint64_t>(f) << fine_bits) + i] = 0;
-      if (kQueued && threadIdx.x == 0) a.totals[f] = 0;
       continue;
     }
     // Table sized to the bucket: slots = next_pow2(2c) (load factor <= 0.5),
@@ -566,7 +547,6 @@ __global__ __launch_bounds__(kUniqueThreads) __attribute__((amdgpu_waves_per_eu(
           u.fhist[base + j] = run;
           run += c;
         }
-      if (kQueued && threadIdx.x == kWave - 1) a.totals[f] = run;  // the last lane's end is the total
     }
     __syncthreads();
     // Survivors are written back in place at their fine bucket's first row
@@ -708,27 +688,12 @@ hipError_t sorted_unique_diff(uint64_t* cand, const uint32_t* scount, uint32_t n
   // G <= tagbits - 2), so the mark bit tagbits-1 is free and a marked entry
   // never equals the all-ones empty marker.
   UniqueArgs a{cand, scount, cur, cur_off, prev, prev_off, fine_counts, error, unique_total, cand_total, tagmask,
-               1ull << (tagbits - 1), merge ? 1u : 0u, fb, nbo_c, nbo_p, tagbits, nsub, range_inverse(nsub), nullptr,
-               nullptr};
+               1ull << (tagbits - 1), merge ? 1u : 0u, fb, nbo_c, nbo_p, tagbits, nsub, range_inverse(nsub)};
   const uint32_t grid = std::min<uint32_t>(nsub, grid_limit);
   if (prev)
-    hipLaunchKernelGGL((unique_diff_kernel<true, false>), dim3(grid), dim3(kUniqueThreads), 0, stream, a);
+    hipLaunchKernelGGL(unique_diff_kernel<true>, dim3(grid), dim3(kUniqueThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL((unique_diff_kernel<false, false>), dim3(grid), dim3(kUniqueThreads), 0, stream, a);
-  return hipGetLastError();
-}
-
-hipError_t sorted_unique_queued(uint64_t* cand, const uint32_t* scount, uint32_t max_sub, const uint64_t* cur,
-                                const uint32_t* cur_off, const uint64_t* prev, const uint32_t* prev_off,
-                                uint32_t* fine_counts, uint32_t* totals, QueueCtl* ctl, uint32_t tagbits, bool merge,
-                                hipStream_t stream) {
-  if (max_sub == 0 || !cur || !cur_off || !ctl || tagbits < 4 || tagbits > 60) return hipErrorInvalidValue;
-  UniqueArgs a{cand, scount, cur, cur_off, prev, prev_off, fine_counts, nullptr, nullptr, nullptr,
-               (1ull << tagbits) - 1, 1ull << (tagbits - 1), merge ? 1u : 0u, 0, 0, 0, tagbits, 0, 0, ctl, totals};
-  if (prev)
-    hipLaunchKernelGGL((unique_diff_kernel<true, true>), dim3(max_sub), dim3(kUniqueThreads), 0, stream, a);
-  else
-    hipLaunchKernelGGL((unique_diff_kernel<false, true>), dim3(max_sub), dim3(kUniqueThreads), 0, stream, a);
+    hipLaunchKernelGGL(unique_diff_kernel<false>, dim3(grid), dim3(kUniqueThreads), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -5,17 +5,21 @@
 // wait: 83 us per layer of S_8, of which the kernels' work is a few.  Two
 // forms take over the layers whose work is smaller than that:
 //
-//   block_run     : one workgroup runs layer after layer without leaving
-//       the kernel, current and next layer in one LDS table.
-//   queued layers : three launches per layer (expand, unique, compact),
-//       their geometry read from the device, so the host queues layers
-//       ahead and only follows the records they leave in pinned memory.
-//       A dependent launch costs 3 us here, a grid-wide barrier with 256
-//       workgroups 7 to 15 us, so separate launches beat a persistent grid.
+//   block_run    : one workgroup runs layer after layer without leaving the
+//       kernel, current and next layer in one LDS table.
+//   owner layers : one launch per layer.  Every workgroup owns a range of
+//       the stored values for the whole session: it selects its new states
+//       from the candidates sent to it, keeps them in its slab, and sends
+//       their children to their owners' slabs for the next launch.  The
+//       host queues layers ahead and follows the records they leave in
+//       pinned memory.  A dependent launch costs 3 us here, a grid-wide
+//       barrier with 256 workgroups 7 to 15 us, so the launches are the
+//       barriers.
 //
-// Both leave banks and offset tables as the general path does, and anything
-// unusual (an overflow, a layer above the banks) is rejected, not handled:
-// the layer's parents are intact and the general path redoes it.
+// A session of owner layers starts from the dense bank (import) and ends by
+// writing the last two layers back as banks (export).  Anything unusual (an
+// overflow, a layer above the banks) is rejected, not handled: the layer's
+// parents are intact and the general path redoes it.
 #include <algorithm>
 #include "common.hpp"
 #include "kernels.hpp"
@@ -183,11 +187,10 @@ __global__ __launch_bounds__(kBlockThreads) void block_run_kernel(BlockRun r, Ac
       }
       LayerRecord* o = rec + done;
       o->N = N;
-      o->cand = t.children;
+      o->children = t.children;
       o->unique = N + t.known;
       o->ticks = wall_clock64();
       o->state = state;
-      o->nbo = 1;
       if (state != kLayerNext) __threadfence_system();
       __hip_atomic_store(&o->seq, r.seq + done, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
@@ -206,157 +209,305 @@ __global__ void sorted_start_kernel(uint64_t stored, uint64_t* bank, uint32_t* o
   if (threadIdx.x < 8) control[threadIdx.x] = 0;
 }
 
-__global__ __launch_bounds__(kQueueSub) void queue_begin_kernel(QueueCtl* ctl, QueueCtl first, uint32_t* scount,
-                                                                 LayerRecord* rec, uint64_t seq) {
-  scount[threadIdx.x] = 0;
-  if (threadIdx.x == 0) {
-    *ctl = first;
-    rec->ticks = wall_clock64();
-    __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+// ------------------------------------------------------------ owner layers
+
+__global__ __launch_bounds__(kBlockThreads) void owner_begin_kernel(uint32_t* counts, uint32_t words, OwnerCtl* ctl,
+                                                                     uint32_t F) {
+  for (uint32_t i = threadIdx.x; i < words; i += kBlockThreads) counts[i] = 0;
+  if (threadIdx.x < 2) {
+    OwnerCtl c{};
+    c.counts = threadIdx.x == 0 ? F : 0u;
+    c.imported = threadIdx.x == 0;
+    ctl[threadIdx.x] = c;
   }
 }
 
-// Children of the current bank into sub-bucket slabs.  A tile holds ITEMS x
-// 512 child slots, generator-major over P parents (a multiple of 64, so a
-// wave's slots share their generator): four items per thread give a layer
-// of 50,000 states 37 workgroups or more instead of 12 with a full tile.
-template <typename Action, int ITEMS>
-__global__ __launch_bounds__(kRouteThreads) void queue_expand_kernel(const uint64_t* __restrict__ bank,
-                                                                     QueueCtl* ctl, Action act, SortedLayout L,
-                                                                     uint32_t* __restrict__ scount,
-                                                                     uint64_t* __restrict__ out) {
-  __shared__ TileLds t;
-  const uint32_t F = ctl->F, nsub = ctl->nsub, G = act.count();
-  const bool masked = ctl->masked != 0;
-  const uint32_t P = ITEMS * kRouteThreads / G / kWave * kWave;
-  const uint32_t tiles = (F + P - 1) / P;
-  if (blockIdx.x >= tiles) return;
-  clear_tile_counters(t);
-  __syncthreads();
-  const RunCursors runs{scount, 1, kUniqueCap, &ctl->error, kErrBucketCap};
-  auto slab_base = [=](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; };
-  auto bkt = [nsub](uint64_t h) { return range_index(h, nsub); };
+// How a finished layer leaves the session; every workgroup of the next
+// launch comes to the same answer from the same totals.
+__device__ __forceinline__ uint32_t owner_state(const OwnerCtl& c, const OwnerRules& rules) {
+  const uint32_t N = static_cast<uint32_t>(c.counts), children = static_cast<uint32_t>(c.counts >> 32);
+  if (c.error || N > rules.rows) return kLayerRejected;
+  if (N == 0) return kLayerEmpty;
+  const bool few = children < rules.low && !c.imported;
+  return c.spill || few || children > rules.high ? kLayerStop : kLayerNext;
+}
+
+__device__ __forceinline__ void owner_publish(const OwnerCtl& c, uint32_t state, LayerRecord* rec, uint64_t seq) {
+  rec->N = static_cast<uint32_t>(c.counts);
+  rec->children = c.counts >> 32;
+  rec->unique = c.unique;
+  rec->ticks = wall_clock64();
+  rec->state = state;
+  __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A routing tile holds kOwnerItems x 512 child slots, generator-major over P
+// parents (a multiple of 64, so the lanes of a wave share their generator).
+constexpr int kOwnerItems = 8;
+
+__device__ __forceinline__ uint32_t owner_tile_parents(uint32_t G) {
+  return kOwnerItems * kRouteThreads / G / kWave * kWave;
+}
+
+// Children of parents[0, count) (count <= owner_tile_parents) to the slabs
+// of their owners; returns this thread's number of children.  Called by the
+// whole workgroup with cleared tile counters.
+template <typename Action>
+__device__ __forceinline__ uint32_t owner_send(TileLds& t, const uint64_t* parents, uint32_t count, bool masked,
+                                               const Action& act, const SortedLayout& L, uint32_t owners,
+                                               const OwnerSlabs& out, uint32_t* spill) {
+  const uint32_t G = act.count();
+  const uint32_t P = (count + kWave - 1) / kWave * kWave;
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x)) / kWave;
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const uint32_t t0 = tile * P;
-    uint64_t v[ITEMS];
-    uint32_t gen[ITEMS];
-    uint32_t valid = 0;
+  uint64_t v[kOwnerItems];
+  uint32_t gen[kOwnerItems];
+  uint32_t valid = 0;
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const uint32_t s = (k * (kRouteThreads / kWave) + wave) * kWave;  // the wave's first slot
-      const uint32_t g = s / P, m = t0 + (s - g * P) + lane;
-      gen[k] = g;
-      const bool live = g < G && m < F;
-      valid |= live ? 1u << k : 0u;
-      v[k] = bank[m < F ? m : F - 1];
-    }
+  for (int k = 0; k < kOwnerItems; ++k) {
+    const uint32_t s = (k * (kRouteThreads / kWave) + wave) * kWave;  // the wave's first slot
+    const uint32_t g = s / P, m = s - g * P + lane;
+    const bool live = g < G && m < count;
+    gen[k] = g < G ? g : G;
+    v[k] = live ? parents[m] : 0;
+    valid |= live ? 1u << k : 0u;
+  }
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const uint32_t g = gen[k] < G ? gen[k] : 0u;
+  for (int k = 0; k < kOwnerItems; ++k) {
+    const uint32_t g = gen[k];
+    if (g < G) {  // uniform
       if (masked && ((v[k] >> g) & 1u)) valid &= ~(1u << k);  // tag bit g: leads back
       const uint64_t child = act.child(keyunmix(v[k] >> L.tagbits, L.km), g);
       v[k] = (keymix(child, L.km) << L.tagbits) | act.mask(g);
     }
-    route_regs(t, v, valid, bkt, runs, slab_base, out, kQueueSub * kSlabStride, [] {});
+  }
+  const RunCursors runs{out.count, 1, kUniqueCap, spill, 1u};
+  auto slab_base = [](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; };
+  auto bkt = [owners](uint64_t h) { return range_index(h, owners); };
+  route_regs(t, v, valid, bkt, runs, slab_base, out.data, owners * kSlabStride, [] {});
+  return __popc(valid);
+}
+
+// Dense banks -> owner slabs of the retained layer(s), and the children of
+// the current one.  Block ranges: tiles of the current bank, of the
+// previous one, then tiles of parents.
+template <typename Action>
+__global__ __launch_bounds__(kRouteThreads) void owner_import_kernel(OwnerImport im, Action act, SortedLayout L,
+                                                                     uint32_t owners, uint32_t cur_tiles,
+                                                                     uint32_t prev_tiles) {
+  __shared__ TileLds t;
+  clear_tile_counters(t);
+  __syncthreads();
+  constexpr uint32_t kCopy = kOwnerItems * kRouteThreads;
+  if (blockIdx.x < cur_tiles + prev_tiles) {
+    const bool first = blockIdx.x < cur_tiles;
+    const uint64_t* from = first ? im.cur : im.prev;
+    const uint32_t n = first ? im.F : im.prev_count;
+    const OwnerSlabs to = first ? im.own : im.own_prev;
+    const uint32_t t0 = (first ? blockIdx.x : blockIdx.x - cur_tiles) * kCopy;
+    uint64_t v[kOwnerItems];
+    uint32_t valid = 0;
+#pragma unroll
+    for (int k = 0; k < kOwnerItems; ++k) {
+      const uint32_t i = t0 + k * kRouteThreads + threadIdx.x;
+      v[k] = i < n ? from[i] : 0;
+      valid |= i < n ? 1u << k : 0u;
+    }
+    const RunCursors runs{to.count, 1, kUniqueCap, &im.ctl->error, kErrBucketCap};
+    auto slab_base = [](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; };
+    auto bkt = [owners](uint64_t h) { return range_index(h, owners); };
+    route_regs(t, v, valid, bkt, runs, slab_base, to.data, owners * kSlabStride, [] {});
+    return;
+  }
+  const uint32_t P = owner_tile_parents(act.count());
+  const uint32_t p0 = (blockIdx.x - cur_tiles - prev_tiles) * P;
+  uint32_t made = owner_send(t, im.cur + p0, min(P, im.F - p0), im.masked != 0, act, L, owners, im.cand, &im.ctl->spill);
+  made = wave_incl_scan(made);
+  if ((threadIdx.x & (kWave - 1)) == kWave - 1 && made)
+    atomicAdd(&im.ctl->counts, static_cast<unsigned long long>(made) << 32);
+}
+
+// Marks h's state in the table if it is there (see probe_value in
+// sorted_kernels.hip: each slot matches at most one retained state).
+__device__ __forceinline__ void owner_mark(uint64_t* table, uint32_t slot_mask, const SortedLayout& L, uint64_t mark,
+                                           uint64_t h) {
+  const uint64_t key = h | L.tagmask;
+  uint32_t slot = static_cast<uint32_t>(h >> L.tagbits) & slot_mask;
+  for (uint32_t probe = 0; probe <= slot_mask; ++probe) {
+    const uint64_t v = table[slot];
+    if (v == kEmpty) return;
+    if ((v | L.tagmask) == key) {
+      table[slot] = v | mark;
+      return;
+    }
+    slot = (slot + 1) & slot_mask;
   }
 }
 
-// One workgroup per sub-bucket: survivors (at the start of their slab, fine
-// bucket order) -> the next bank, whose offsets come from the survivor
-// totals of the sub-buckets before (at most 1,024, summed by every
-// workgroup) and the sub-bucket's own fine counts; three scan launches
-// saved.  Workgroup 0 sizes the next layer and reports this one.
-__global__ __launch_bounds__(kRouteThreads) void queue_compact_kernel(
-    const uint64_t* __restrict__ cand, const uint32_t* __restrict__ fine_counts, const uint32_t* __restrict__ totals,
-    uint32_t* __restrict__ scount, const QueueCtl* __restrict__ ctl, QueueCtl* __restrict__ next, QueueRules rules,
-    uint64_t* __restrict__ bank, uint32_t* __restrict__ off, LayerRecord* rec, uint64_t seq) {
-  __shared__ uint32_t sums[2][kRouteThreads / kWave];
-  const uint32_t f = blockIdx.x, F = ctl->F, nsub = ctl->nsub, fb = ctl->fb;
-  if (threadIdx.x == 0) scount[f] = 0;  // the next layer's cursors
-  if (F == 0) {
-    if (f == 0 && threadIdx.x == 0) next->F = 0;
+// One layer of one owner: its candidates into an LDS table (duplicates
+// merge), the retained layers' states mark theirs, the unmarked entries are
+// the owner's part of the new layer; then the children of those go out.
+// Small layers are bound by the chain of dependent steps (candidate load,
+// LDS rounds, slab write and re-read, cursor atomics, child stores; about
+// 12 us with the launch), large ones by the same VALU and LDS work as the
+// general path's kernels, without its 40 bytes a state of compaction and
+// bank reload.  The routing tile reuses the table's LDS (two workgroups per
+// CU).
+template <typename Action>
+__global__ __launch_bounds__(kRouteThreads) void owner_layer_kernel(OwnerLayer a, Action act, SortedLayout L) {
+  __shared__ alignas(16) char lds[sizeof(TileLds) > kUniqueSlots * 8 ? sizeof(TileLds) : kUniqueSlots * 8];
+  __shared__ uint32_t rows, occupied, made;
+  uint64_t* table = reinterpret_cast<uint64_t*>(lds);
+  const uint32_t f = blockIdx.x;
+  const OwnerCtl before = *a.before;
+  uint32_t c = a.in.count[f];
+  const uint32_t ncur = a.cur.count[f], nprev = a.prev.data ? a.prev.count[f] : 0u;
+  const uint32_t state = owner_state(before, a.rules);
+  const bool run = !before.halt && state == kLayerNext;
+  if (f == 0 && threadIdx.x == 0) {
+    if (!before.halt) owner_publish(before, state, a.rec, a.seq);
+    if (!run) a.now->halt = 1;
+    *a.after = OwnerCtl{};
+  }
+  if (!run) return;
+  const uint64_t base = static_cast<uint64_t>(f) * kSlabStride;
+  const uint64_t* cand = a.in.data + base;
+  const uint64_t* cur = a.cur.data + base;
+  uint64_t* next = a.next.data + base;
+  if (c > kUniqueCap) {  // the sender flagged it; this layer cannot be selected
+    if (threadIdx.x == 0) {
+      atomicOr(&a.now->error, kErrBucketCap);
+      a.next.count[f] = 0;
+    }
+    c = 0;
+  }
+  if (c == 0) {
+    __syncthreads();  // every thread has read the count
+    if (threadIdx.x == 0) {
+      a.in.count[f] = 0;
+      a.next.count[f] = 0;
+    }
     return;
   }
-  if (f >= nsub) return;
-  const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  uint32_t before = 0, all = 0;
+  // The first candidates and retained states are loaded before the table is
+  // cleared; later ones in chunks of kChunk per thread.
+  constexpr int kChunk = 4;
+  auto load = [&](uint64_t (&v)[kChunk], const uint64_t* from, uint32_t at, uint32_t n) {
 #pragma unroll
-  for (uint32_t j = threadIdx.x; j < kQueueSub; j += kRouteThreads) {
-    const uint32_t c = j < nsub ? totals[j] : 0u;
-    all += c;
-    before += j < f ? c : 0u;
-  }
-  before = wave_incl_scan(before);
-  all = wave_incl_scan(all);
-  if (lane == kWave - 1) {
-    sums[0][wave] = before;
-    sums[1][wave] = all;
+    for (int k = 0; k < kChunk; ++k) {
+      const uint32_t i = at + k * kRouteThreads + threadIdx.x;
+      v[k] = from[i < n ? i : 0u];
+    }
+  };
+  uint64_t v[kChunk], w[kChunk];
+  load(v, cand, 0, c);
+  load(w, cur, 0, ncur);
+  uint32_t slots = 64;
+  while (slots < 2 * c && slots < kUniqueSlots) slots <<= 1;
+  const uint32_t slot_mask = slots - 1;
+  for (uint32_t i = threadIdx.x; i < slots / 2; i += kRouteThreads)
+    reinterpret_cast<ulonglong2*>(table)[i] = make_ulonglong2(kEmpty, kEmpty);
+  if (threadIdx.x == 0) rows = occupied = made = 0;
+  __syncthreads();
+  const uint64_t mark = 1ull << (L.tagbits - 1);
+  for (uint32_t at = 0; at < c; at += kChunk * kRouteThreads) {
+    if (at) load(v, cand, at, c);
+#pragma unroll
+    for (int k = 0; k < kChunk; ++k)
+      if (at + k * kRouteThreads + threadIdx.x < c) block_insert(table, slot_mask, L, mark, L.prune != 0, v[k]);
   }
   __syncthreads();
-  before = all = 0;
+  for (uint32_t at = 0; at < ncur; at += kChunk * kRouteThreads) {
+    if (at) load(w, cur, at, ncur);
 #pragma unroll
-  for (uint32_t w = 0; w < kRouteThreads / kWave; ++w) {
-    before += sums[0][w];
-    all += sums[1][w];
+    for (int k = 0; k < kChunk; ++k)
+      if (at + k * kRouteThreads + threadIdx.x < ncur) owner_mark(table, slot_mask, L, mark, w[k]);
   }
-  const uint32_t error = ctl->error;
-  const bool reject = error != 0 || all > rules.rows;
-  if (!reject && all != 0) {
-    // Offsets of the fine buckets: wave 0 scans the counts, 64 at a time.
-    const uint32_t fine = 1u << fb;
-    if (wave == 0) {
-      uint32_t run = before;
-      for (uint32_t j = lane; j < ((fine + kWave - 1) & ~(kWave - 1u)); j += kWave) {
-        const uint32_t c = j < fine ? fine_counts[(f << fb) + j] : 0u;
-        const uint32_t incl = wave_incl_scan(c);
-        if (j < fine) off[(f << fb) + j] = run + incl - c;
-        run += __shfl(incl, kWave - 1, kWave);
-      }
-      if (f == nsub - 1 && lane == 0) off[nsub << fb] = all;
+  if (nprev) {
+    const uint64_t* prev = a.prev.data + base;
+    for (uint32_t at = 0; at < nprev; at += kChunk * kRouteThreads) {
+      load(w, prev, at, nprev);
+#pragma unroll
+      for (int k = 0; k < kChunk; ++k)
+        if (at + k * kRouteThreads + threadIdx.x < nprev) owner_mark(table, slot_mask, L, mark, w[k]);
     }
-    const uint32_t mine = totals[f];
-    const uint64_t* src = cand + static_cast<uint64_t>(f) * kSlabStride;
-    for (uint32_t i = threadIdx.x; i < mine; i += kRouteThreads) bank[before + i] = src[i];
   }
-  if (f != 0 || threadIdx.x != 0) return;
-  const uint64_t C = ctl->cand;
-  QueueCtl n{};
-  n.masked = rules.prune;
-  n.nbo_cur = nsub << fb;
-  n.nbo_prev = ctl->nbo_cur;
-  // Children of the next layer: this layer's children per parent plus 10%
-  // when parents carry masks (both layers then skip every back-edge).
-  const uint64_t most = static_cast<uint64_t>(all) * rules.kids;
-  uint64_t guess = most;
-  if (rules.prune && ctl->masked) {
-    const uint64_t g = static_cast<uint64_t>(static_cast<double>(all) * (static_cast<double>(C) / F) * 1.1);
-    guess = g < most ? g : most;
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  uint32_t occ = 0;
+  for (uint32_t i = threadIdx.x; i < slots / 2; i += kRouteThreads) {  // whole waves: slots / 2 is 32 or a multiple of 64
+    const ulonglong2 p = reinterpret_cast<const ulonglong2*>(table)[i];
+    const bool ox = p.x != kEmpty, oy = p.y != kEmpty;
+    const bool sx = ox && !(p.x & mark), sy = oy && !(p.y & mark);
+    occ += (ox ? 1u : 0u) + (oy ? 1u : 0u);
+    const uint64_t bx = __ballot(sx), by = __ballot(sy);
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&rows, static_cast<uint32_t>(__popcll(bx) + __popcll(by)));
+    at = __shfl(at, 0, kWave);
+    const uint64_t below = (1ull << lane) - 1;
+    if (sx) next[at + __popcll(bx & below)] = p.x;
+    if (sy) next[at + __popcll(bx) + __popcll(by & below)] = p.y;
   }
-  n.nsub = queue_sub_buckets(guess);
-  n.range_inv = range_inverse(n.nsub);
-  n.fb = queue_fine_bits(n.nsub, rules.margin);
-  uint32_t state = kLayerNext;
-  if (reject) state = kLayerRejected;
-  else if (all == 0) state = kLayerEmpty;
-  else if (guess <= rules.low || guess > kQueueSub * static_cast<uint64_t>(kQueueTarget)) state = kLayerStop;
-  n.F = state == kLayerNext ? all : 0u;
-  *next = n;
-  rec->N = all;
-  rec->cand = C;
-  rec->unique = ctl->unique;
-  rec->ticks = wall_clock64();
-  rec->state = state;
-  rec->nbo = nsub << fb;
-  __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  occ = wave_incl_scan(occ);
+  if (lane == kWave - 1 && occ) atomicAdd(&occupied, occ);
+  __syncthreads();
+  const uint32_t N = rows;
+  TileLds& t = *reinterpret_cast<TileLds*>(lds);
+  clear_tile_counters(t);
+  __syncthreads();
+  uint32_t mine = 0;
+  const uint32_t P = owner_tile_parents(act.count());
+  for (uint32_t p0 = 0; p0 < N; p0 += P)
+    mine += owner_send(t, next + p0, min(P, N - p0), L.prune != 0, act, L, a.rules.owners, a.out, &a.now->spill);
+  mine = wave_incl_scan(mine);
+  if (lane == kWave - 1 && mine) atomicAdd(&made, mine);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a.in.count[f] = 0;
+    a.next.count[f] = N;
+    atomicAdd(&a.now->counts, static_cast<unsigned long long>(N) | (static_cast<unsigned long long>(made) << 32));
+    atomicAdd(&a.now->unique, static_cast<unsigned long long>(occupied));
+  }
+}
+
+__global__ void owner_report_kernel(const OwnerCtl* ctl, OwnerRules rules, LayerRecord* rec, uint64_t seq) {
+  if (threadIdx.x != 0 || ctl->halt) return;
+  owner_publish(*ctl, owner_state(*ctl, rules), rec, seq);
+}
+
+// Blocks [0, owners) write the current layer's bank, the others the
+// previous one's; every block sums the counts of the owners before its own.
+__global__ __launch_bounds__(kRouteThreads) void owner_export_kernel(OwnerSlabs cur, uint64_t* bank, uint32_t* off,
+                                                                     OwnerSlabs prev, uint64_t* prev_bank,
+                                                                     uint32_t* prev_off, uint32_t owners) {
+  __shared__ uint32_t sums[kRouteThreads / kWave];
+  const bool second = blockIdx.x >= owners;
+  const uint32_t f = second ? blockIdx.x - owners : blockIdx.x;
+  const OwnerSlabs s = second ? prev : cur;
+  uint64_t* to = second ? prev_bank : bank;
+  uint32_t* offsets = second ? prev_off : off;
+  uint32_t before = 0;
+  for (uint32_t j = threadIdx.x; j < f; j += kRouteThreads) before += s.count[j];
+  before = wave_incl_scan(before);
+  if ((threadIdx.x & (kWave - 1)) == kWave - 1) sums[threadIdx.x / kWave] = before;
+  __syncthreads();
+  before = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kRouteThreads / kWave; ++w) before += sums[w];
+  const uint32_t n = s.count[f];
+  if (threadIdx.x == 0) {
+    offsets[f] = before;
+    if (f + 1 == owners) offsets[owners] = before + n;
+  }
+  const uint64_t* from = s.data + static_cast<uint64_t>(f) * kSlabStride;
+  for (uint32_t i = threadIdx.x; i < n; i += kRouteThreads) to[before + i] = from[i];
 }
 
 }  // namespace
 
 hipError_t sorted_block_run(const BlockRun& run, const PackedGenerators& gens, hipStream_t stream) {
   if (run.cur > 2 || run.prev > kNoBank || run.prev == run.cur || run.F == 0 || run.max_layers == 0 || !run.rec ||
-      run.F + (run.prev < kNoBank && !run.L.prune ? run.prev_count : 0u) > kBlockFill / 2)
+      run.F > kBlockParents || (run.prev < kNoBank && !run.L.prune && run.prev_count > kBlockParents))
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(block_run_kernel<NibbleAction>, dim3(1), dim3(kBlockThreads), 0, stream, run, NibbleAction{gens});
   return hipGetLastError();
@@ -367,33 +518,42 @@ hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t
   return hipGetLastError();
 }
 
-hipError_t sorted_queue_begin(QueueCtl* ctl, const QueueCtl& first, uint32_t* scount, LayerRecord* rec, uint64_t seq,
-                              hipStream_t stream) {
-  hipLaunchKernelGGL(queue_begin_kernel, dim3(1), dim3(kQueueSub), 0, stream, ctl, first, scount, rec, seq);
+hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream) {
+  hipLaunchKernelGGL(owner_begin_kernel, dim3(1), dim3(kBlockThreads), 0, stream, counts, words, ctl, F);
   return hipGetLastError();
 }
 
-hipError_t sorted_queue_expand(const uint64_t* bank, QueueCtl* ctl, const PackedGenerators& gens,
-                               const SortedLayout& L, uint32_t* scount, uint64_t* out, uint32_t items, uint32_t grid,
-                               hipStream_t stream) {
-  if (grid == 0 || gens.count == 0 || gens.count > kMaxGenerators) return hipErrorInvalidValue;
-  const NibbleAction act{gens};
-  if (items == 4)
-    hipLaunchKernelGGL((queue_expand_kernel<NibbleAction, 4>), dim3(grid), dim3(kRouteThreads), 0, stream, bank, ctl,
-                       act, L, scount, out);
-  else if (items == 8)
-    hipLaunchKernelGGL((queue_expand_kernel<NibbleAction, 8>), dim3(grid), dim3(kRouteThreads), 0, stream, bank, ctl,
-                       act, L, scount, out);
-  else
+hipError_t owner_import(const OwnerImport& im, const PackedGenerators& gens, const SortedLayout& L, uint32_t owners,
+                        hipStream_t stream) {
+  if (!im.cur || im.F == 0 || owners == 0 || owners > kOwnersMax || gens.count == 0 || gens.count > kMaxGenerators)
     return hipErrorInvalidValue;
+  const uint32_t copy = kOwnerItems * kRouteThreads;
+  const uint32_t cur_tiles = (im.F + copy - 1) / copy;
+  const uint32_t prev_tiles = im.prev ? (im.prev_count + copy - 1) / copy : 0u;
+  const uint32_t P = kOwnerItems * kRouteThreads / gens.count / kWave * kWave;
+  const uint32_t tiles = cur_tiles + prev_tiles + (im.F + P - 1) / P;
+  hipLaunchKernelGGL(owner_import_kernel<NibbleAction>, dim3(tiles), dim3(kRouteThreads), 0, stream, im,
+                     NibbleAction{gens}, L, owners, cur_tiles, prev_tiles);
   return hipGetLastError();
 }
 
-hipError_t sorted_queue_compact(const uint64_t* cand, const uint32_t* fine_counts, const uint32_t* totals,
-                                uint32_t* scount, const QueueCtl* ctl, QueueCtl* next, const QueueRules& rules,
-                                uint64_t* bank, uint32_t* off, LayerRecord* rec, uint64_t seq, hipStream_t stream) {
-  hipLaunchKernelGGL(queue_compact_kernel, dim3(kQueueSub), dim3(kRouteThreads), 0, stream, cand, fine_counts, totals,
-                     scount, ctl, next, rules, bank, off, rec, seq);
+hipError_t owner_layer(const OwnerLayer& a, const PackedGenerators& gens, const SortedLayout& L, hipStream_t stream) {
+  if (a.rules.owners == 0 || a.rules.owners > kOwnersMax) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(owner_layer_kernel<NibbleAction>, dim3(a.rules.owners), dim3(kRouteThreads), 0, stream, a,
+                     NibbleAction{gens}, L);
+  return hipGetLastError();
+}
+
+hipError_t owner_report(const OwnerCtl* ctl, const OwnerRules& rules, LayerRecord* rec, uint64_t seq,
+                        hipStream_t stream) {
+  hipLaunchKernelGGL(owner_report_kernel, dim3(1), dim3(64), 0, stream, ctl, rules, rec, seq);
+  return hipGetLastError();
+}
+
+hipError_t owner_export(const OwnerSlabs& cur, uint64_t* bank, uint32_t* off, const OwnerSlabs& prev,
+                        uint64_t* prev_bank, uint32_t* prev_off, uint32_t owners, hipStream_t stream) {
+  hipLaunchKernelGGL(owner_export_kernel, dim3(2 * owners), dim3(kRouteThreads), 0, stream, cur, bank, off, prev,
+                     prev_bank, prev_off, owners);
   return hipGetLastError();
 }
 
