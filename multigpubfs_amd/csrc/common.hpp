@@ -267,19 +267,30 @@ __host__ __device__ __forceinline__ uint32_t range_start(uint32_t f, uint32_t n,
   return static_cast<uint32_t>(x);
 }
 
+//
+// m2 != 0 adds a second round: keys whose fields are not a permutation's
+// (matrices, few labels) are not spread evenly by one product.
 __host__ __device__ __forceinline__ uint64_t keymix(uint64_t x, const KeyMix& k) {
   x = (x * k.m1) & k.mask;
   x ^= x >> k.shift;
+  if (k.m2) {
+    x = (x * k.m2) & k.mask;
+    x ^= x >> k.shift;
+  }
   return x;
 }
 
 __host__ __device__ __forceinline__ uint64_t keyunmix(uint64_t x, const KeyMix& k) {
+  if (k.m2) {
+    x ^= x >> k.shift;
+    x = (x * k.i2) & k.mask;
+  }
   x ^= x >> k.shift;
   x = (x * k.i1) & k.mask;
   return x;
 }
 
-__host__ inline KeyMix make_keymix(uint32_t bits) {
+__host__ inline KeyMix make_keymix(uint32_t bits, bool second = false) {
   KeyMix k;
   k.bits = bits;
   k.shift = bits / 2 + 1;
@@ -287,7 +298,8 @@ __host__ inline KeyMix make_keymix(uint32_t bits) {
   // 2^64 / golden ratio, rounded to odd.
   k.m1 = 0x9e3779b97f4a7c15ull & k.mask;
   k.i1 = inverse_odd(0x9e3779b97f4a7c15ull) & k.mask;
-  k.m2 = k.i2 = 0;
+  k.m2 = second ? 0xd6e8feb86659fd93ull & k.mask : 0;
+  k.i2 = second ? inverse_odd(0xd6e8feb86659fd93ull) & k.mask : 0;
   return k;
 }
 

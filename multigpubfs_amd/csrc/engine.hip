@@ -10,6 +10,7 @@
 #include <memory>
 #include "engine.hpp"
 #include "kernels.hpp"
+#include "wide.hpp"
 
 namespace mgbfs {
 
@@ -647,6 +648,119 @@ class HandoverEngine final : public Engine {
   uint32_t handovers_ = 0;
 };
 
+// The segmented backend on graphs whose states are one packed word
+// (wide.hpp): layers run in the sorted backend's banks, and a layer beyond
+// its memory or limits goes on in the segmented tables.  What it reports is
+// the segmented backend's: name, history, row width, counters.
+class PackedSegmentedEngine final : public Engine {
+ public:
+  PackedSegmentedEngine(const Graph& g, const mgbfs_engine_options& o, const WideCode& code) : g_(g), o_(o), code_(code) {
+    inner_.reset(make_sorted_engine(g, o, &code_));
+    packed_ = true;
+    backend = MGBFS_BACKEND_SEGMENTED;
+    history_layers = 3;
+    state_bytes = generic_state_bytes(g);
+    mirror();
+  }
+  int advance(uint64_t* next_count, uint32_t* fatal) override {
+    int s = inner_->advance(next_count, fatal);
+    if (s == kAdvanceHandover) {
+      go_on_segmented();
+      s = inner_->advance(next_count, fatal);
+    }
+    complete_ = s == MGBFS_COMPLETE;
+    mirror();
+    return s;
+  }
+  int run_to_end() override {
+    int s = inner_->run_to_end();
+    if (s == kAdvanceHandover) {
+      go_on_segmented();
+      s = inner_->run_to_end();
+    }
+    complete_ = s == MGBFS_COMPLETE;
+    mirror();
+    return s;
+  }
+  void reset() override {
+    if (packed_) {
+      inner_->reset();
+    } else {
+      inner_.reset();
+      inner_.reset(make_sorted_engine(g_, o_, &code_));
+      packed_ = true;
+      seconds_ = 0.0;
+      launches_ = streamed_ = 0;
+    }
+    complete_ = false;
+    mirror();
+  }
+  void layer_keys(std::vector<uint64_t>& out) override {
+    if (!packed_) return inner_->layer_keys(out);
+    // As the segmented backend packs rows: the low nibbles of 16 entries.
+    std::vector<int64_t> rows;
+    uint64_t n = 0;
+    inner_->sample(0, layers.back(), rows, n);
+    out.assign(n, 0);
+    for (uint64_t r = 0; r < n; ++r)
+      for (uint32_t e = 0; e < g_.elements && e < 16; ++e)
+        out[r] |= (static_cast<uint64_t>(rows[r * g_.elements + e]) & 15u) << (4 * e);
+  }
+  void sample(uint32_t which, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) override {
+    inner_->sample(which, limit, rows, count);
+  }
+  const char* name() const override { return "SEGMENTED_OPEN_ADDRESSING_THREE_BANK"; }
+  uint64_t retry_count() const override { return packed_ ? 0 : inner_->retry_count(); }
+  void settle() override {
+    inner_->settle();
+    mirror();
+  }
+
+ private:
+  void go_on_segmented() {
+    PackedHandover h;
+    if (!inner_->handover(h)) throw std::runtime_error("ENGINE_HANDOVER");
+    seconds_ = inner_->kernel_seconds;
+    launches_ = inner_->launches;
+    streamed_ = inner_->streamed_bytes;
+    std::unique_ptr<Engine> next(make_segmented_from_packed(g_, o_, state_space_bound(g_), h));
+    inner_ = std::move(next);
+    packed_ = false;
+  }
+  // Every layer but the current one has been expanded, the last one too
+  // once the search is complete.
+  void mirror() {
+    layers = inner_->layers;
+    uint64_t total = 0;
+    for (uint64_t n : layers) total += n;
+    candidates = (total - (complete_ ? 0 : layers.back())) * g_.generators;
+    unique_candidates = total - 1;
+    device_bytes = inner_->device_bytes;
+    kernel_seconds = inner_->kernel_seconds + seconds_;
+    launches = inner_->launches + launches_;
+    streamed_bytes = inner_->streamed_bytes + streamed_;
+    terminal = inner_->terminal;
+  }
+  Graph g_;
+  mgbfs_engine_options o_;
+  WideCode code_;
+  std::unique_ptr<Engine> inner_;
+  bool packed_ = false, complete_ = false;
+  double seconds_ = 0.0;  // of the packed part of a run that went on segmented
+  uint64_t launches_ = 0, streamed_ = 0;
+};
+
+// Packed layers take the run unless the caller bounds rows (whose stops are
+// the tables'), forces a table mechanism, or leaves too little memory for
+// the packed layers' fixed buffers.
+static bool packed_segmented(const Graph& g, const mgbfs_engine_options& o, WideCode& code) {
+  if (!g.inverse_closed || o.capacity ||
+      (o.flags & (MGBFS_FLAG_TEST_COLLIDE_HASH | MGBFS_FLAG_TEST_TINY_SEGMENTS)) || !make_wide(g, code, 60))
+    return false;
+  MGBFS_HIP(hipSetDevice(o.device));
+  return vram_budget(o) >= (1ull << 30);
+}
+
 // Planned bytes per state of the widest layer on the sorted backend: three
 // banks grown by a quarter, plus per child (G-1 with back-edge masks, else
 // G) a sub-bucket slab entry (8 B at the mean fill of 5000 of 5120) and an
@@ -734,8 +848,11 @@ static Engine* create(const Graph& g, const mgbfs_engine_options& o) {
       return make_bitmap_engine(g, o);
     case MGBFS_BACKEND_SORTED:
       return new HandoverEngine(g, o);
-    case MGBFS_BACKEND_SEGMENTED:
+    case MGBFS_BACKEND_SEGMENTED: {
+      WideCode code;
+      if (packed_segmented(g, o, code)) return new PackedSegmentedEngine(g, o, code);
       return make_segmented_engine(g, o, state_space_bound(g));
+    }
     default:
       return make_generic_engine(g, o, state_space_bound(g));
   }

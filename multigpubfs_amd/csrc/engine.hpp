@@ -127,7 +127,9 @@ class Engine {
 constexpr int kAdvanceHandover = 3;
 
 Engine* make_bitmap_engine(const Graph& g, const mgbfs_engine_options& o);
-Engine* make_sorted_engine(const Graph& g, const mgbfs_engine_options& o);
+struct WideCode;
+// wide: packed code of a graph outside the nibble encoding (null: none).
+Engine* make_sorted_engine(const Graph& g, const mgbfs_engine_options& o, const WideCode* wide = nullptr);
 Engine* make_generic_engine(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound);
 Engine* make_segmented_engine(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound);
 // Layers d-1 and d of a sorted-backend run, handed to the segmented backend
@@ -140,6 +142,7 @@ struct PackedHandover {
   uint64_t cur_count = 0;
   KeyMix km{};
   uint32_t tagbits = 0;
+  const WideCode* wide = nullptr;  // null: nibble keys
   std::vector<uint64_t> layers;
 };
 Engine* make_segmented_from_packed(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound,

@@ -33,12 +33,26 @@ constexpr uint32_t kSlabStride = 5120;    // entries between sub-bucket slab sta
 // keymix on b = max(32, 4n) bits (at least 32, so keymix's mask leaves the
 // low word whole) and tagbits = 64 - b.
 inline uint32_t sorted_key_bits(uint32_t degree) { return degree >= 8 ? 4 * degree : 32u; }
+// Dump-area index for 32-bit destination indexing, or ~0 when the output
+// (entries, plus the dump area) does not fit 32-bit indices.
+inline uint32_t route_dump_index(uint64_t out_entries, uint64_t dump) {
+  return out_entries + dump < ~0u ? static_cast<uint32_t>(out_entries) : ~0u;
+}
 
 struct SortedLayout {
   KeyMix km;
   uint32_t tagbits;  // 64 - sorted_key_bits(n)
   uint32_t prune;    // back-edge masks in use: tag bit i = skip generator i
   uint64_t tagmask;  // (1 << tagbits) - 1
+};
+
+// How a layer's children are made: nibble-packed permutations (generators by
+// value) or wide keys (wide.hpp; the table in device memory).
+struct WideTable;
+struct ActionRef {
+  const PackedGenerators* nibble;
+  const WideTable* wide;  // device; null: nibble
+  uint32_t count;         // generators
 };
 
 // Layers run ahead of the host (sorted_queue.hip).
@@ -125,13 +139,13 @@ struct OwnerLayer {
 };
 
 hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t* control, hipStream_t stream);
-hipError_t sorted_block_run(const BlockRun& run, const PackedGenerators& gens, hipStream_t stream);
+hipError_t sorted_block_run(const BlockRun& run, const ActionRef& act, hipStream_t stream);
 // Zeroes the owners' counts (`words` of them from `counts`) and the first
 // control blocks; ctl[0] becomes the imported layer's, of F states.
 hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream);
-hipError_t owner_import(const OwnerImport& im, const PackedGenerators& gens, const SortedLayout& L, uint32_t owners,
+hipError_t owner_import(const OwnerImport& im, const ActionRef& act, const SortedLayout& L, uint32_t owners,
                         hipStream_t stream);
-hipError_t owner_layer(const OwnerLayer& a, const PackedGenerators& gens, const SortedLayout& L, hipStream_t stream);
+hipError_t owner_layer(const OwnerLayer& a, const ActionRef& act, const SortedLayout& L, hipStream_t stream);
 // Reports the last layer queued (a layer launch reports the one before it).
 hipError_t owner_report(const OwnerCtl* ctl, const OwnerRules& rules, LayerRecord* rec, uint64_t seq,
                         hipStream_t stream);
@@ -160,6 +174,11 @@ hipError_t sorted_expand_route(const uint64_t* bank, uint64_t F, const PackedGen
                                uint32_t stride,
                                uint32_t err_bit, uint32_t* cursors, uint32_t* error, uint64_t* out,
                                uint64_t out_entries, hipStream_t stream);
+// The same for wide keys: `act` has its table in device memory.
+hipError_t sorted_expand_route_wide(const uint64_t* bank, uint64_t F, const ActionRef& act, const SortedLayout& L,
+                                    bool masked, uint32_t nsub, uint32_t K2, uint32_t NB, uint32_t P, uint32_t cap,
+                                    uint32_t stride, uint32_t err_bit, uint32_t* cursors, uint32_t* error,
+                                    uint64_t* out, uint64_t out_entries, hipStream_t stream);
 // Lane slabs (lcount per slab, capacity and stride lcap) -> sub-bucket
 // slabs of kUniqueCap entries, kSlabStride apart (scount per sub-bucket,
 // zeroed by the caller).

@@ -56,8 +56,11 @@ hipError_t segmented_expand(const SegBatch<S>& b, hipStream_t stream);
 template <typename S>
 hipError_t segmented_seed(const SegBanks<S>& banks, uint32_t bank, uint32_t first, uint32_t count, uint32_t elements,
                           const SegSegment& seg, uint32_t bits, uint32_t* fill, uint32_t* error, hipStream_t stream);
-// Sorted-backend bank values -> nibble rows of a u8 SoA arena.
+// Sorted-backend bank values -> rows of a SoA arena (entries of `bits` bits,
+// label indices when `labels`, a device table, is given).
+template <typename S>
 hipError_t segmented_adopt_packed(const uint64_t* values, uint64_t count, const KeyMix& km, uint32_t tagbits,
-                                  uint32_t degree, uint8_t* arena, uint64_t stride, hipStream_t stream);
+                                  uint32_t elements, uint32_t bits, const int64_t* labels, S* arena, uint64_t stride,
+                                  hipStream_t stream);
 
 }  // namespace mgbfs

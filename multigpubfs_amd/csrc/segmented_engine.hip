@@ -21,6 +21,7 @@
 #include "engine.hpp"
 #include "kernels.hpp"
 #include "segmented.hpp"
+#include "wide.hpp"
 
 namespace mgbfs {
 
@@ -119,25 +120,30 @@ class SegmentedEngine final : public Engine {
     reset_counters();
   }
 
-  // Continues a BFS whose layers d-1 (prev) and d (cur) are nibble-packed
-  // states in sorted-backend banks (the sorted backend's hand-over when a
-  // layer exceeds its limits); `table` is the layer table so far.
-  void adopt_packed(const uint64_t* prev_vals, uint64_t prev_count, const uint64_t* cur_vals, uint64_t cur_count,
-                    const KeyMix& km, uint32_t tagbits, const std::vector<uint64_t>& table) {
+  // Continues a BFS whose layers d-1 (prev) and d (cur) are packed states in
+  // sorted-backend banks (the sorted backend's hand-over when a layer
+  // exceeds its limits).
+  void adopt_packed(const PackedHandover& h) {
     static_assert(sizeof(S) == 1 || sizeof(S) == 8, "state width");
-    if (!closed_ || sizeof(S) != 1) throw std::runtime_error("SEGMENTED_ADOPT_SHAPE");
+    if (!closed_ || (!h.wide && sizeof(S) != 1)) throw std::runtime_error("SEGMENTED_ADOPT_SHAPE");
+    const uint64_t prev_count = h.prev_count, cur_count = h.cur_count;
+    DeviceBuffer labels;
+    if (h.wide && !h.wide->labels.empty()) {
+      labels.allocate(h.wide->labels.size() * 8);
+      MGBFS_HIP(hipMemcpy(labels.as<void>(), h.wide->labels.data(), h.wide->labels.size() * 8, hipMemcpyHostToDevice));
+    }
     MGBFS_HIP(hipSetDevice(device_));
     for (auto& b : banks_) {
       b.segs.clear();
       b.used = 0;
     }
     const int pb = prev_count ? 0 : -1, cb = 1;
-    if (prev_count) adopt_bank(0, prev_vals, prev_count, km, tagbits);
-    adopt_bank(1, cur_vals, cur_count, km, tagbits);
+    if (prev_count) adopt_bank(0, h.prev, prev_count, h, labels);
+    adopt_bank(1, h.cur, cur_count, h, labels);
     prev_ = pb;
     cur_ = cb;
     count_ = cur_count;
-    layers = table;
+    layers = h.layers;
     reset_counters();
   }
 
@@ -373,11 +379,11 @@ class SegmentedEngine final : public Engine {
     seed_rows(b, 0, bank.used);
     return true;
   }
-  void adopt_bank(int b, const uint64_t* vals, uint64_t count, const KeyMix& km, uint32_t tagbits) {
+  void adopt_bank(int b, const uint64_t* vals, uint64_t count, const PackedHandover& h, const DeviceBuffer& labels) {
     if (!ensure_arena(b, count)) throw std::runtime_error("SEGMENTED_ADOPT_CAPACITY");
-    MGBFS_HIP(segmented_adopt_packed(vals, count, km, tagbits, elements_,
-                                     reinterpret_cast<uint8_t*>(banks_[b].arena.template as<S>()), banks_[b].capacity,
-                                     stream_));
+    MGBFS_HIP(segmented_adopt_packed<S>(vals, count, h.km, h.tagbits, elements_, h.wide ? h.wide->table.bits : 4,
+                                        labels.bytes() ? labels.as<int64_t>() : nullptr,
+                                        banks_[b].arena.template as<S>(), banks_[b].capacity, stream_));
     banks_[b].used = static_cast<uint32_t>(count);
     if (!add_segment(b, count)) throw std::runtime_error("SEGMENTED_ADOPT_CAPACITY");
     seed_rows(b, 0, static_cast<uint32_t>(count));
@@ -449,29 +455,26 @@ class SegmentedEngine final : public Engine {
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
 };
 
+static bool narrow_rows(const Graph& g) { return generic_state_bytes(g) == 1; }
+
 Engine* make_segmented_engine(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound) {
-  const bool narrow = g.kind == 0 && std::all_of(g.start.begin(), g.start.end(), [](int64_t v) { return v >= 0 && v <= 255; });
-  Engine* e = narrow ? static_cast<Engine*>(new SegmentedEngine<uint8_t>(g, o, state_bound))
-                     : static_cast<Engine*>(new SegmentedEngine<int64_t>(g, o, state_bound));
-  try {
-    e->reset();
-  } catch (...) {
-    delete e;
-    throw;
-  }
-  return e;
+  std::unique_ptr<Engine> e;
+  if (narrow_rows(g)) e.reset(new SegmentedEngine<uint8_t>(g, o, state_bound));
+  else e.reset(new SegmentedEngine<int64_t>(g, o, state_bound));
+  e->reset();
+  return e.release();
 }
 
 Engine* make_segmented_from_packed(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound,
                                    const PackedHandover& h) {
-  auto* e = new SegmentedEngine<uint8_t>(g, o, state_bound);
-  try {
-    e->adopt_packed(h.prev, h.prev_count, h.cur, h.cur_count, h.km, h.tagbits, h.layers);
-  } catch (...) {
-    delete e;
-    throw;
+  if (!h.wide || narrow_rows(g)) {
+    auto e = std::make_unique<SegmentedEngine<uint8_t>>(g, o, state_bound);
+    e->adopt_packed(h);
+    return e.release();
   }
-  return e;
+  auto e = std::make_unique<SegmentedEngine<int64_t>>(g, o, state_bound);
+  e->adopt_packed(h);
+  return e.release();
 }
 
 }  // namespace mgbfs

@@ -216,14 +216,19 @@ __global__ __launch_bounds__(kSegThreads) void segmented_seed_kernel(SegBanks<S>
   }
 }
 
-// Sorted-backend bank values (mix(key) << tagbits | tag) -> nibble rows of
-// a u8 SoA arena.
+// Sorted-backend bank values (mix(key) << tagbits | tag) -> rows of a SoA
+// arena: entry e is `bits` bits of the key, a label index when labels is set.
+template <typename S>
 __global__ void segmented_adopt_packed_kernel(const uint64_t* values, uint64_t count, KeyMix km, uint32_t tagbits,
-                                              uint32_t degree, uint8_t* arena, uint64_t stride) {
+                                              uint32_t elements, uint32_t bits, const int64_t* labels, S* arena,
+                                              uint64_t stride) {
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < count;
        i += static_cast<uint64_t>(blockDim.x) * gridDim.x) {
     const uint64_t key = keyunmix(values[i] >> tagbits, km);
-    for (uint32_t e = 0; e < degree; ++e) arena[static_cast<uint64_t>(e) * stride + i] = static_cast<uint8_t>((key >> (4 * e)) & 15u);
+    for (uint32_t e = 0; e < elements; ++e) {
+      const uint64_t v = (key >> (bits * e)) & ((1ull << bits) - 1);
+      arena[static_cast<uint64_t>(e) * stride + i] = static_cast<S>(labels ? labels[v] : static_cast<int64_t>(v));
+    }
   }
 }
 
@@ -257,14 +262,20 @@ hipError_t segmented_seed(const SegBanks<S>& banks, uint32_t bank, uint32_t firs
   return hipGetLastError();
 }
 
+template <typename S>
 hipError_t segmented_adopt_packed(const uint64_t* values, uint64_t count, const KeyMix& km, uint32_t tagbits,
-                                  uint32_t degree, uint8_t* arena, uint64_t stride, hipStream_t stream) {
+                                  uint32_t elements, uint32_t bits, const int64_t* labels, S* arena, uint64_t stride,
+                                  hipStream_t stream) {
   if (count == 0) return hipSuccess;
-  hipLaunchKernelGGL(segmented_adopt_packed_kernel, dim3(seg_grid(count)), dim3(kSegThreads), 0, stream, values, count,
-                     km, tagbits, degree, arena, stride);
+  hipLaunchKernelGGL(segmented_adopt_packed_kernel<S>, dim3(seg_grid(count)), dim3(kSegThreads), 0, stream, values,
+                     count, km, tagbits, elements, bits, labels, arena, stride);
   return hipGetLastError();
 }
 
+template hipError_t segmented_adopt_packed<uint8_t>(const uint64_t*, uint64_t, const KeyMix&, uint32_t, uint32_t,
+                                                    uint32_t, const int64_t*, uint8_t*, uint64_t, hipStream_t);
+template hipError_t segmented_adopt_packed<int64_t>(const uint64_t*, uint64_t, const KeyMix&, uint32_t, uint32_t,
+                                                    uint32_t, const int64_t*, int64_t*, uint64_t, hipStream_t);
 template hipError_t segmented_expand<uint8_t>(const SegBatch<uint8_t>&, hipStream_t);
 template hipError_t segmented_expand<int64_t>(const SegBatch<int64_t>&, hipStream_t);
 template hipError_t segmented_seed<uint8_t>(const SegBanks<uint8_t>&, uint32_t, uint32_t, uint32_t, uint32_t,

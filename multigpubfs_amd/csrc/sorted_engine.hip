@@ -15,9 +15,11 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include "engine.hpp"
 #include "kernels.hpp"
 #include "sorted_plan.hpp"
+#include "wide.hpp"
 
 namespace mgbfs {
 
@@ -38,7 +40,9 @@ constexpr int kAheadNone = -1;          // run_ahead(): the next layer is one fo
 
 class SortedEngine final : public Engine {
  public:
-  SortedEngine(const Graph& g, const mgbfs_engine_options& o) : gens_(g.packed_generators()), n_(g.elements) {
+  // wide: the graph's packed code when it is outside the nibble encoding.
+  SortedEngine(const Graph& g, const mgbfs_engine_options& o, const WideCode* wide) : n_(g.elements) {
+    if (wide) wide_ = std::make_unique<WideCode>(*wide);
     device_ = o.device;
     backend = MGBFS_BACKEND_SORTED;
     history_layers = 3;
@@ -53,8 +57,9 @@ class SortedEngine final : public Engine {
     cap_limit_ = o.capacity ? o.capacity : ~0ull;
     flags_ = o.flags;
     // Stored-value layout and parent-edge tags.
-    layout_.km = make_keymix(sorted_key_bits(n_));
-    layout_.tagbits = 64 - sorted_key_bits(n_);
+    const uint32_t key_bits = wide_ ? std::max(32u, wide_->key_bits()) : sorted_key_bits(n_);
+    layout_.km = make_keymix(key_bits, wide_ != nullptr);
+    layout_.tagbits = 64 - key_bits;
     layout_.tagmask = layout_.tagbits ? ((1ull << layout_.tagbits) - 1) : 0;
     set_generators(g);
     // One workgroup per sub-bucket: persistent grids of 2 or 8 workgroups
@@ -161,7 +166,7 @@ class SortedEngine final : public Engine {
     if (masked && last_ratio_ > 0)
       Cest = std::min<uint64_t>(Cest, static_cast<uint64_t>(static_cast<double>(F) * last_ratio_ * 1.1) + 4096);
     const uint64_t kMaxSub = 1ull << kMaxBucketBits;
-    uint64_t want = sub_buckets_for(Cest);
+    uint64_t want = sub_buckets_for(Cest, wide_ ? kTargetBucketWide : kTargetBucket);
     // Test hook: start eight times coarse so large layers exercise the
     // bucket-overflow retry path.
     if ((flags_ & MGBFS_FLAG_TEST_COARSE_BUCKETS) && want >= 8) want >>= 3;
@@ -171,9 +176,7 @@ class SortedEngine final : public Engine {
       const uint32_t K2 = geo.K2, nsub = geo.nsub, NB1 = geo.NB1, P = geo.P, lcap = geo.lcap;
       const uint64_t lslabs = geo.lslabs, lane_entries = geo.lane_entries, sub_entries = geo.sub_entries;
       if (!ensure_slabs(lane_entries + kRouteDump, sub_entries + kRouteDump)) {
-        *fatal = kErrFutureCap;
-        terminal = true;
-        return MGBFS_RESOURCE;
+        return out_of_room(fatal, kErrFutureCap);
       }
       ensure_u32(lcount_, lslabs);
       ensure_u32(scount_, nsub);
@@ -184,11 +187,17 @@ class SortedEngine final : public Engine {
                            lcount_.as<uint32_t>(), K2 ? lslabs : 0, stream_));
       MGBFS_HIP(hipEventRecord(ev_[0], stream_));
       uint64_t* sub = sub_.as<uint64_t>();
-      MGBFS_HIP(sorted_expand_route(bank_[cur_].as<uint64_t>(), F, gens_, layout_, masked, nsub, K2, NB1, P, lcap,
-                                    K2 ? lcap : kSlabStride, K2 ? kErrLaneSlab : kErrBucketCap,
-                                    K2 ? lcount_.as<uint32_t>() : scount_.as<uint32_t>(), error_word(),
-                                    K2 ? lane_.as<uint64_t>() : sub, routed(K2 ? lane_entries : sub_entries),
-                                    stream_));
+      const uint32_t stride = K2 ? lcap : kSlabStride, full = K2 ? kErrLaneSlab : kErrBucketCap;
+      uint32_t* cursors = K2 ? lcount_.as<uint32_t>() : scount_.as<uint32_t>();
+      uint64_t* routed_to = K2 ? lane_.as<uint64_t>() : sub;
+      const uint64_t routed_entries = routed(K2 ? lane_entries : sub_entries);
+      if (wide_)
+        MGBFS_HIP(sorted_expand_route_wide(bank_[cur_].as<uint64_t>(), F, action(), layout_, masked, nsub, K2, NB1, P,
+                                           lcap, stride, full, cursors, error_word(), routed_to, routed_entries,
+                                           stream_));
+      else
+        MGBFS_HIP(sorted_expand_route(bank_[cur_].as<uint64_t>(), F, gens_, layout_, masked, nsub, K2, NB1, P, lcap,
+                                      stride, full, cursors, error_word(), routed_to, routed_entries, stream_));
       MGBFS_HIP(hipEventRecord(ev_[1], stream_));
       if (K2)
         MGBFS_HIP(sorted_partition(lane_.as<uint64_t>(), lcount_.as<uint32_t>(), lcap, P, nsub, K2,
@@ -233,11 +242,7 @@ class SortedEngine final : public Engine {
           continue;
         }
       }
-      if (err) {
-        *fatal = err;
-        terminal = true;
-        return MGBFS_RESOURCE;
-      }
+      if (err) return out_of_room(fatal, err);
       candidates += C;
       last_ratio_ = masked ? static_cast<double>(C) / static_cast<double>(F) : 0.0;
       unique_candidates += host_[0];
@@ -246,11 +251,7 @@ class SortedEngine final : public Engine {
         terminal = true;
         return MGBFS_COMPLETE;
       }
-      if (N > cap_limit_ || !grow_bank(nxt, N)) {
-        *fatal = kErrFutureCap;
-        terminal = true;
-        return MGBFS_RESOURCE;
-      }
+      if (N > cap_limit_ || !grow_bank(nxt, N)) return out_of_room(fatal, kErrFutureCap);
       if (N > early_rows) compact(sub, nsub, fb, nxt);
       phase_bytes[3] += 16 * N;
       streamed_bytes += 16 * N;
@@ -269,8 +270,7 @@ class SortedEngine final : public Engine {
  public:
   // Another inverse-closed graph of the same degree reuses every bank and slab.
   void rebind(const Graph& g) override {
-    if (g.elements != n_ || !g.packable() || !g.inverse_closed) throw std::runtime_error("ENGINE_REBIND_SHAPE");
-    gens_ = g.packed_generators();
+    if (wide_ || g.elements != n_ || !g.packable() || !g.inverse_closed) throw std::runtime_error("ENGINE_REBIND_SHAPE");
     set_generators(g);
     reset();
   }
@@ -280,7 +280,9 @@ class SortedEngine final : public Engine {
     settle();
     lane_.release();
     sub_.release();
+    owner_.release();
     lane_cap_ = sub_cap_ = 0;
+    h.wide = wide_.get();
     h.cur = bank_[cur_].as<uint64_t>();
     h.cur_count = count_[cur_];
     h.prev = prev_ >= 0 ? bank_[prev_].as<uint64_t>() : nullptr;
@@ -300,7 +302,8 @@ class SortedEngine final : public Engine {
     else if (prev_ >= 0) read_bank(prev_, std::min(limit, count_[prev_]), keys);
     rows.resize(keys.size() * n_);
     for (size_t k = 0; k < keys.size(); ++k)
-      for (uint32_t i = 0; i < n_; ++i) rows[k * n_ + i] = static_cast<int64_t>((keys[k] >> (4u * i)) & 15u);
+      for (uint32_t i = 0; i < n_; ++i)
+        rows[k * n_ + i] = wide_ ? wide_->value(keys[k], i) : static_cast<int64_t>((keys[k] >> (4u * i)) & 15u);
     count = keys.size();
   }
 
@@ -392,7 +395,7 @@ class SortedEngine final : public Engine {
     r.rec = rec_;
     r.seq = seq_;
     seq_ += kBlockLayers + 2;
-    MGBFS_HIP(sorted_block_run(r, gens_, stream_));
+    MGBFS_HIP(sorted_block_run(r, action(), stream_));
     uint64_t first = 0;
     for (uint32_t i = 0;; ++i) {
       const LayerRecord& rec = await(rec_[i], r.seq + i);
@@ -452,7 +455,7 @@ class SortedEngine final : public Engine {
     im.masked = layout_.prune && layers.size() > 1;
     im.cand = slab[0];
     im.ctl = ctl;
-    MGBFS_HIP(owner_import(im, gens_, layout_, owners, stream_));
+    MGBFS_HIP(owner_import(im, action(), layout_, owners, stream_));
     int qcur = cur_, qprev = prev_;
     const uint32_t most = std::min(max_layers, kBlockLayers);
     uint32_t queued = 0, accepted = 0;
@@ -474,7 +477,7 @@ class SortedEngine final : public Engine {
         a.rules = rules;
         a.rec = rec_ + queued % kOwnerRing;
         a.seq = seq + queued;
-        MGBFS_HIP(owner_layer(a, gens_, layout_, stream_));
+        MGBFS_HIP(owner_layer(a, action(), layout_, stream_));
         qprev = qcur;
         qcur = nxt;
         if (queued + 1 == most)  // nothing follows the last layer to report it
@@ -556,13 +559,38 @@ class SortedEngine final : public Engine {
   // mark and bit tagbits-2 stays clear, so no entry is all ones), the
   // fine-bucket margin and the start state.
   void set_generators(const Graph& g) {
-    if (!fill_back_edge_masks(gens_)) throw std::runtime_error("SORTED_REQUIRES_INVERSE_CLOSED");
-    layout_.prune = gens_.count + 2 <= layout_.tagbits && !(flags_ & MGBFS_FLAG_TEST_NO_PRUNE);
+    bool pairs;  // every generator has its inverse in the set
+    if (wide_) {
+      std::memset(&gens_, 0, sizeof(gens_));
+      gens_.count = g.generators;
+      pairs = wide_->paired;
+    } else {
+      gens_ = g.packed_generators();
+      pairs = fill_back_edge_masks(gens_);
+      if (!pairs) throw std::runtime_error("SORTED_REQUIRES_INVERSE_CLOSED");
+    }
+    layout_.prune = pairs && gens_.count + 2 <= layout_.tagbits && !(flags_ & MGBFS_FLAG_TEST_NO_PRUNE);
     if (!layout_.prune)
-      for (uint32_t a = 0; a < gens_.count; ++a) gens_.child_mask[a] = 0;
+      for (uint32_t a = 0; a < gens_.count; ++a) {
+        gens_.child_mask[a] = 0;
+        if (wide_) wide_->table.child_mask[a] = 0;
+      }
     history_layers = layout_.prune ? 2 : 3;
     margin_ = fine_margin(gens_.count);
-    start_key_ = g.start_key();
+    start_key_ = wide_ ? wide_->start_key : g.start_key();
+    if (wide_) {
+      wide_dev_.allocate(sizeof(WideTable));
+      MGBFS_HIP(hipMemcpy(wide_dev_.as<void>(), &wide_->table, sizeof(WideTable), hipMemcpyHostToDevice));
+    }
+  }
+  ActionRef action() const { return ActionRef{&gens_, wide_ ? wide_dev_.as<WideTable>() : nullptr, gens_.count}; }
+  // A layer this engine has no room or geometry for.  Wide keys go on in the
+  // segmented backend, which made this engine.
+  int out_of_room(uint32_t* fatal, uint32_t bits) {
+    if (wide_) return kAdvanceHandover;
+    *fatal = bits;
+    terminal = true;
+    return MGBFS_RESOURCE;
   }
   // Compactions run unwaited; each is bracketed by one of two event pairs,
   // read (and charged to phase 3) when the pair is reused or on settle().
@@ -663,11 +691,13 @@ class SortedEngine final : public Engine {
   }
   void update_bytes() {
     device_bytes = control_.bytes() + fine_counts_.bytes() + lane_.bytes() + sub_.bytes() + lcount_.bytes() +
-                   scount_.bytes() + scan_ws_.bytes() + owner_.bytes();
+                   scount_.bytes() + scan_ws_.bytes() + owner_.bytes() + wide_dev_.bytes();
     for (int b = 0; b < 3; ++b) device_bytes += bank_[b].bytes() + off_[b].bytes();
   }
 
-  PackedGenerators gens_;
+  PackedGenerators gens_;            // wide keys: only the count and empty masks
+  std::unique_ptr<WideCode> wide_;   // set: keys are wide, their table in wide_dev_
+  DeviceBuffer wide_dev_;
   SortedLayout layout_{};
   uint32_t n_, margin_ = 0, flags_ = 0, unique_grid_ = 2048, slack_ = 1;
   double last_ratio_ = 0.0;  // children per parent of the last masked layer
@@ -689,6 +719,8 @@ class SortedEngine final : public Engine {
   int cslot_ = 0;
 };
 
-Engine* make_sorted_engine(const Graph& g, const mgbfs_engine_options& o) { return new SortedEngine(g, o); }
+Engine* make_sorted_engine(const Graph& g, const mgbfs_engine_options& o, const WideCode* wide) {
+  return new SortedEngine(g, o, wide);
+}
 
 }  // namespace mgbfs

@@ -621,11 +621,7 @@ hipError_t sorted_seed(uint64_t start_key, const SortedLayout& L, uint64_t* bank
   return hipGetLastError();
 }
 
-// Dump-area index for 32-bit destination indexing, or kWideOut when the
-// output (entries, plus kTile dump entries) does not fit 32-bit indices.
-static uint32_t dump_index(uint64_t out_entries) {
-  return out_entries + kTile < kWideOut ? static_cast<uint32_t>(out_entries) : kWideOut;
-}
+static uint32_t dump_index(uint64_t out_entries) { return route_dump_index(out_entries, kTile); }
 
 template <int G, bool MASKED>
 static hipError_t expand_route_g(const uint64_t* bank, uint64_t F, const PackedGenerators& gens, const SortedLayout& L,

@@ -18,6 +18,10 @@ inline uint32_t ceil_log2(uint64_t x) {
 // workgroup's fixed work (bounds, table clear, fine-count scan); the cap is
 // kUniqueCap = 5120 and counts stay within a few percent of the mean.
 constexpr uint64_t kTargetBucket = 5000;
+// Wide keys are spread like random placement (two mixer rounds), so exact
+// counts stay within sqrt(mean) of it: 4500 leaves nine deviations below the
+// cap where 5000 leaves two.
+constexpr uint64_t kTargetBucketWide = 4500;
 constexpr uint32_t kLaneParts = 32;  // slabs per owner lane (cursor contention / P)
 
 // Slab capacity for `mean` expected entries: mean + slack * (mean / 4 +
@@ -33,9 +37,9 @@ inline uint32_t slab_capacity(double mean, uint32_t slack) {
 
 // Sub-buckets wanted for an estimated candidate count: any count, not a
 // power of two, so the mean fill stays near kTargetBucket on every layer.
-inline uint64_t sub_buckets_for(uint64_t Cest) {
+inline uint64_t sub_buckets_for(uint64_t Cest, uint64_t target = kTargetBucket) {
   const uint64_t kMaxSub = 1ull << kMaxBucketBits;
-  return std::min<uint64_t>(kMaxSub, Cest <= kTargetBucket ? 1 : (Cest + kTargetBucket - 1) / kTargetBucket);
+  return std::min<uint64_t>(kMaxSub, Cest <= target ? 1 : (Cest + target - 1) / target);
 }
 
 // Fine-bucket bits beyond the layer's sub-bucket bits for G generators.

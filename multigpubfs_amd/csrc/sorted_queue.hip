@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "sorted_device.hpp"
+#include "wide.hpp"
 
 namespace mgbfs {
 
@@ -40,6 +41,19 @@ struct NibbleAction {
     return apply_groups(key, gens, static_cast<int>(g));
   }
   __device__ __forceinline__ uint32_t mask(uint32_t g) const { return gens.child_mask[g]; }
+};
+
+// Wide keys: the table through the constant address space, so that a
+// generator index that is uniform in the wave reads it with scalar loads.
+struct WideAction {
+  const WideTable* table;
+  uint32_t generators;
+  using ConstTable = const __attribute__((address_space(4))) WideTable*;
+  __device__ __forceinline__ uint32_t count() const { return generators; }
+  __device__ __forceinline__ uint64_t child(uint64_t key, uint32_t g) const {
+    return wide_child((ConstTable)table, key, g);
+  }
+  __device__ __forceinline__ uint32_t mask(uint32_t g) const { return ((ConstTable)table)->child_mask[g]; }
 };
 
 struct BlockLds {
@@ -241,30 +255,30 @@ __device__ __forceinline__ void owner_publish(const OwnerCtl& c, uint32_t state,
   __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// A routing tile holds kOwnerItems x 512 child slots, generator-major over P
+// A routing tile holds kSendItems x 512 child slots, generator-major over P
 // parents (a multiple of 64, so the lanes of a wave share their generator).
-constexpr int kOwnerItems = 8;
+constexpr int kSendItems = 8;
 
-__device__ __forceinline__ uint32_t owner_tile_parents(uint32_t G) {
-  return kOwnerItems * kRouteThreads / G / kWave * kWave;
+__device__ __forceinline__ uint32_t tile_parents(uint32_t G) {
+  return kSendItems * kRouteThreads / G / kWave * kWave;
 }
 
-// Children of parents[0, count) (count <= owner_tile_parents) to the slabs
-// of their owners; returns this thread's number of children.  Called by the
-// whole workgroup with cleared tile counters.
-template <typename Action>
-__device__ __forceinline__ uint32_t owner_send(TileLds& t, const uint64_t* parents, uint32_t count, bool masked,
-                                               const Action& act, const SortedLayout& L, uint32_t owners,
-                                               const OwnerSlabs& out, uint32_t* spill) {
+// Children of parents[0, count) (count <= tile_parents) routed into the
+// slabs of their buckets; returns this thread's number of children.  Called
+// by the whole workgroup with cleared tile counters.
+template <typename Action, typename BucketFn, typename BaseFn>
+__device__ __forceinline__ uint32_t send_tile(TileLds& t, const uint64_t* parents, uint32_t count, bool masked,
+                                              const Action& act, const SortedLayout& L, BucketFn bkt,
+                                              const RunCursors& runs, BaseFn slab_base, uint64_t* out, uint32_t dump) {
   const uint32_t G = act.count();
   const uint32_t P = (count + kWave - 1) / kWave * kWave;
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x)) / kWave;
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  uint64_t v[kOwnerItems];
-  uint32_t gen[kOwnerItems];
+  uint64_t v[kSendItems];
+  uint32_t gen[kSendItems];
   uint32_t valid = 0;
 #pragma unroll
-  for (int k = 0; k < kOwnerItems; ++k) {
+  for (int k = 0; k < kSendItems; ++k) {
     const uint32_t s = (k * (kRouteThreads / kWave) + wave) * kWave;  // the wave's first slot
     const uint32_t g = s / P, m = s - g * P + lane;
     const bool live = g < G && m < count;
@@ -273,7 +287,7 @@ __device__ __forceinline__ uint32_t owner_send(TileLds& t, const uint64_t* paren
     valid |= live ? 1u << k : 0u;
   }
 #pragma unroll
-  for (int k = 0; k < kOwnerItems; ++k) {
+  for (int k = 0; k < kSendItems; ++k) {
     const uint32_t g = gen[k];
     if (g < G) {  // uniform
       if (masked && ((v[k] >> g) & 1u)) valid &= ~(1u << k);  // tag bit g: leads back
@@ -281,11 +295,46 @@ __device__ __forceinline__ uint32_t owner_send(TileLds& t, const uint64_t* paren
       v[k] = (keymix(child, L.km) << L.tagbits) | act.mask(g);
     }
   }
-  const RunCursors runs{out.count, 1, kUniqueCap, spill, 1u};
-  auto slab_base = [](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; };
-  auto bkt = [owners](uint64_t h) { return range_index(h, owners); };
-  route_regs(t, v, valid, bkt, runs, slab_base, out.data, owners * kSlabStride, [] {});
+  route_regs(t, v, valid, bkt, runs, slab_base, out, dump, [] {});
   return __popc(valid);
+}
+
+// The same to the owners' slabs.
+template <typename Action>
+__device__ __forceinline__ uint32_t owner_send(TileLds& t, const uint64_t* parents, uint32_t count, bool masked,
+                                               const Action& act, const SortedLayout& L, uint32_t owners,
+                                               const OwnerSlabs& out, uint32_t* spill) {
+  return send_tile(
+      t, parents, count, masked, act, L, [owners](uint64_t h) { return range_index(h, owners); },
+      RunCursors{out.count, 1, kUniqueCap, spill, 1u},
+      [](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; }, out.data, owners * kSlabStride);
+}
+
+// The general path's expansion (expand_scatter_kernel) for wide keys: tiles
+// of contiguous parents dealt to blocks round-robin, children to the lane
+// slabs.  One instantiation serves every generator count: 4,096 child slots
+// per tile instead of 8,192 children, at 90 registers.
+template <typename Action>
+__global__ __launch_bounds__(kRouteThreads) void expand_wide_kernel(const uint64_t* __restrict__ bank, uint64_t F,
+                                                                    Action act, SortedLayout L, bool masked,
+                                                                    uint32_t nsub, uint32_t K2, uint32_t NB, uint32_t P,
+                                                                    uint32_t cap, uint32_t stride, uint32_t err_bit,
+                                                                    uint32_t* __restrict__ cursors,
+                                                                    uint32_t* __restrict__ error,
+                                                                    uint64_t* __restrict__ out, uint32_t dump) {
+  __shared__ TileLds t;
+  clear_tile_counters(t);
+  __syncthreads();
+  const uint32_t part = blockIdx.x % P;
+  const uint64_t parents = tile_parents(act.count()), tiles = (F + parents - 1) / parents;
+  for (uint64_t tile = blockIdx.x; tile < tiles; tile += NB) {
+    const uint64_t p0 = tile * parents;
+    const uint32_t n = static_cast<uint32_t>(F - p0 < parents ? F - p0 : parents);
+    send_tile(
+        t, bank + p0, n, masked, act, L, [nsub, K2](uint64_t h) { return range_index(h, nsub) >> K2; },
+        RunCursors{cursors + part, P, cap, error, err_bit},
+        [=](uint32_t b) { return (static_cast<uint64_t>(b) * P + part) * stride; }, out, dump);
+  }
 }
 
 // Dense banks -> owner slabs of the retained layer(s), and the children of
@@ -298,17 +347,17 @@ __global__ __launch_bounds__(kRouteThreads) void owner_import_kernel(OwnerImport
   __shared__ TileLds t;
   clear_tile_counters(t);
   __syncthreads();
-  constexpr uint32_t kCopy = kOwnerItems * kRouteThreads;
+  constexpr uint32_t kCopy = kSendItems * kRouteThreads;
   if (blockIdx.x < cur_tiles + prev_tiles) {
     const bool first = blockIdx.x < cur_tiles;
     const uint64_t* from = first ? im.cur : im.prev;
     const uint32_t n = first ? im.F : im.prev_count;
     const OwnerSlabs to = first ? im.own : im.own_prev;
     const uint32_t t0 = (first ? blockIdx.x : blockIdx.x - cur_tiles) * kCopy;
-    uint64_t v[kOwnerItems];
+    uint64_t v[kSendItems];
     uint32_t valid = 0;
 #pragma unroll
-    for (int k = 0; k < kOwnerItems; ++k) {
+    for (int k = 0; k < kSendItems; ++k) {
       const uint32_t i = t0 + k * kRouteThreads + threadIdx.x;
       v[k] = i < n ? from[i] : 0;
       valid |= i < n ? 1u << k : 0u;
@@ -319,7 +368,7 @@ __global__ __launch_bounds__(kRouteThreads) void owner_import_kernel(OwnerImport
     route_regs(t, v, valid, bkt, runs, slab_base, to.data, owners * kSlabStride, [] {});
     return;
   }
-  const uint32_t P = owner_tile_parents(act.count());
+  const uint32_t P = tile_parents(act.count());
   const uint32_t p0 = (blockIdx.x - cur_tiles - prev_tiles) * P;
   uint32_t made = owner_send(t, im.cur + p0, min(P, im.F - p0), im.masked != 0, act, L, owners, im.cand, &im.ctl->spill);
   made = wave_incl_scan(made);
@@ -456,7 +505,7 @@ __global__ __launch_bounds__(kRouteThreads) void owner_layer_kernel(OwnerLayer a
   clear_tile_counters(t);
   __syncthreads();
   uint32_t mine = 0;
-  const uint32_t P = owner_tile_parents(act.count());
+  const uint32_t P = tile_parents(act.count());
   for (uint32_t p0 = 0; p0 < N; p0 += P)
     mine += owner_send(t, next + p0, min(P, N - p0), L.prune != 0, act, L, a.rules.owners, a.out, &a.now->spill);
   mine = wave_incl_scan(mine);
@@ -505,12 +554,22 @@ __global__ __launch_bounds__(kRouteThreads) void owner_export_kernel(OwnerSlabs 
 
 }  // namespace
 
-hipError_t sorted_block_run(const BlockRun& run, const PackedGenerators& gens, hipStream_t stream) {
+// Calls f with the action the reference stands for.
+template <typename F>
+static hipError_t with_action(const ActionRef& act, F f) {
+  if (act.count == 0 || act.count > kMaxGenerators || (!act.wide && !act.nibble)) return hipErrorInvalidValue;
+  if (act.wide) f(WideAction{act.wide, act.count});
+  else f(NibbleAction{*act.nibble});
+  return hipGetLastError();
+}
+
+hipError_t sorted_block_run(const BlockRun& run, const ActionRef& act, hipStream_t stream) {
   if (run.cur > 2 || run.prev > kNoBank || run.prev == run.cur || run.F == 0 || run.max_layers == 0 || !run.rec ||
       run.F > kBlockParents || (run.prev < kNoBank && !run.L.prune && run.prev_count > kBlockParents))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(block_run_kernel<NibbleAction>, dim3(1), dim3(kBlockThreads), 0, stream, run, NibbleAction{gens});
-  return hipGetLastError();
+  return with_action(act, [&](auto a) {
+    hipLaunchKernelGGL(block_run_kernel<decltype(a)>, dim3(1), dim3(kBlockThreads), 0, stream, run, a);
+  });
 }
 
 hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t* control, hipStream_t stream) {
@@ -523,24 +582,38 @@ hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t
   return hipGetLastError();
 }
 
-hipError_t owner_import(const OwnerImport& im, const PackedGenerators& gens, const SortedLayout& L, uint32_t owners,
+hipError_t owner_import(const OwnerImport& im, const ActionRef& act, const SortedLayout& L, uint32_t owners,
                         hipStream_t stream) {
-  if (!im.cur || im.F == 0 || owners == 0 || owners > kOwnersMax || gens.count == 0 || gens.count > kMaxGenerators)
+  if (!im.cur || im.F == 0 || owners == 0 || owners > kOwnersMax || act.count == 0 || act.count > kMaxGenerators)
     return hipErrorInvalidValue;
-  const uint32_t copy = kOwnerItems * kRouteThreads;
+  const uint32_t copy = kSendItems * kRouteThreads;
   const uint32_t cur_tiles = (im.F + copy - 1) / copy;
   const uint32_t prev_tiles = im.prev ? (im.prev_count + copy - 1) / copy : 0u;
-  const uint32_t P = kOwnerItems * kRouteThreads / gens.count / kWave * kWave;
+  const uint32_t P = kSendItems * kRouteThreads / act.count / kWave * kWave;
   const uint32_t tiles = cur_tiles + prev_tiles + (im.F + P - 1) / P;
-  hipLaunchKernelGGL(owner_import_kernel<NibbleAction>, dim3(tiles), dim3(kRouteThreads), 0, stream, im,
-                     NibbleAction{gens}, L, owners, cur_tiles, prev_tiles);
-  return hipGetLastError();
+  return with_action(act, [&](auto a) {
+    hipLaunchKernelGGL(owner_import_kernel<decltype(a)>, dim3(tiles), dim3(kRouteThreads), 0, stream, im, a, L, owners,
+                       cur_tiles, prev_tiles);
+  });
 }
 
-hipError_t owner_layer(const OwnerLayer& a, const PackedGenerators& gens, const SortedLayout& L, hipStream_t stream) {
+hipError_t owner_layer(const OwnerLayer& a, const ActionRef& act, const SortedLayout& L, hipStream_t stream) {
   if (a.rules.owners == 0 || a.rules.owners > kOwnersMax) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(owner_layer_kernel<NibbleAction>, dim3(a.rules.owners), dim3(kRouteThreads), 0, stream, a,
-                     NibbleAction{gens}, L);
+  return with_action(act, [&](auto x) {
+    hipLaunchKernelGGL(owner_layer_kernel<decltype(x)>, dim3(a.rules.owners), dim3(kRouteThreads), 0, stream, a, x, L);
+  });
+}
+
+hipError_t sorted_expand_route_wide(const uint64_t* bank, uint64_t F, const ActionRef& act, const SortedLayout& L,
+                                    bool masked, uint32_t nsub, uint32_t K2, uint32_t NB, uint32_t P, uint32_t cap,
+                                    uint32_t stride, uint32_t err_bit, uint32_t* cursors, uint32_t* error,
+                                    uint64_t* out, uint64_t out_entries, hipStream_t stream) {
+  if (F == 0 || nsub == 0 || K2 > kMaxPassBits || (nsub & ((1u << K2) - 1u)) || (nsub >> K2) > (1u << kMaxPassBits) ||
+      NB == 0 || P == 0 || cap == 0 || stride < cap || !act.wide || act.count == 0 || act.count > kMaxGenerators)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(expand_wide_kernel<WideAction>, dim3(NB), dim3(kRouteThreads), 0, stream, bank, F,
+                     WideAction{act.wide, act.count}, L, masked, nsub, K2, NB, P, cap, stride, err_bit, cursors, error,
+                     out, route_dump_index(out_entries, kTile));
   return hipGetLastError();
 }
 

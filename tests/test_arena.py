@@ -45,3 +45,17 @@ def test_back_edge_masks_cover_repeated_generators(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "backedge ok" in out.stdout
+
+
+def test_wide_keys_match_plain_actions(tmp_path):
+    """Packed keys of wide permutations and small matrices
+    (multigpubfs_amd/csrc/wide.hpp) against the plain actions."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not installed")
+    exe = tmp_path / "wide_check"
+    subprocess.run([hipcc, "-std=c++17", "-O1", "-I", str(ROOT / "multigpubfs_amd" / "csrc"),
+                    str(ROOT / "tests" / "native" / "wide_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "wide keys ok" in out.stdout

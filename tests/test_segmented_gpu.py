@@ -176,3 +176,91 @@ def test_reset_repeats_and_segmented_memory_backend_through_cli(tmp_path):
     assert report["layer_sizes"] == first and report["backend"] == NAME
     report = run_graph(lrx(8), tmp_path / "out8", device=0, memory_backend="segmented_hash")
     assert report["layer_sizes"] == O.packed_bfs(8)["layers"] and report["backend"] == NAME
+
+
+# Graphs whose states fit one packed word run in the sorted backend's banks
+# (wide keys): few labels over many positions, and modular matrices.
+def closed(gens):
+    out = list(gens)
+    for g in gens:
+        q = [0] * len(g)
+        for i, v in enumerate(g):
+            q[v] = i
+        if q not in out:
+            out.append(q)
+    return out
+
+
+def random_closed(n, k, seed):
+    rng = random.Random(seed)
+    gens = []
+    for _ in range(k):
+        g = list(range(n))
+        rng.shuffle(g)
+        gens.append(g)
+    return closed(gens)
+
+
+def unitriangular(m):
+    x, y = [1, 1, 0, 0, 1, 0, 0, 0, 1], [1, 0, 0, 0, 1, 1, 0, 0, 1]
+    xi, yi = [1, m - 1, 0, 0, 1, 0, 0, 0, 1], [1, 0, 0, 0, 1, m - 1, 0, 0, 1]
+    return GraphDefinition.matrix(3, 3, [(g, m) for g in (x, y, xi, yi)], [1, 0, 0, 0, 1, 0, 0, 0, 1])
+
+
+def vectors(p):
+    return GraphDefinition.matrix(2, 1, [(g, p) for g in ([1, 1, 0, 1], [1, 0, 1, 1], [1, p - 1, 0, 1], [1, 0, p - 1, 1])],
+                                  [1, 0])
+
+
+WIDE = {
+    "sl2_31": lambda: sl2(31),
+    "vectors_257": lambda: vectors(257),
+    "unitriangular_11": lambda: unitriangular(11),
+    "units_4099": lambda: GraphDefinition.matrix(1, 1, [([2], 4099), ([2050], 4099)], [1]),
+    "ring18": lambda: GraphDefinition.permutation(O.lrx_generators(18), [0] * 12 + [1] * 6),
+    "three_labels17": lambda: GraphDefinition.permutation(O.lrx_generators(17), [-5] * 14 + [70000] * 2 + [9]),
+    "random24": lambda: GraphDefinition.permutation(random_closed(24, 2, 3), [0] * 20 + [1] * 4),
+    "eight_generators20": lambda: GraphDefinition.permutation(random_closed(20, 4, 5), [2] * 16 + [3] * 3 + [250]),
+}
+
+
+@pytest.mark.parametrize("flags", [0, 8, 1 | 4, 32])
+@pytest.mark.parametrize("name", list(WIDE))
+def test_wide_keys_layer_sets(name, flags):
+    g = WIDE[name]()
+    want = oracle_layers(g, 1 << 20)
+    with NativeEngine(g, backend="segmented", flags=flags) as e:
+        assert e.backend_name == NAME
+        if len(want) < 200:
+            sizes, rows = layers_of(e)
+            assert rows == want
+        e.reset()
+        assert e.run() == 1
+        sizes = e.layer_sizes()
+        info = e.info()
+        assert sizes == [len(x) for x in want]
+        assert sorted(map(tuple, e.sample(0, 1 << 20))) == want[-1]
+        assert sorted(map(tuple, e.sample(1, 1 << 20))) == want[-2]
+    assert info["backend"] == 3 and info["history_layers"] == 3
+    assert info["candidates"] == sum(sizes) * g.generator_count and info["unique_candidates"] == sum(sizes) - 1
+
+
+@pytest.mark.parametrize("name", ["sl2_101", "ring22"])
+def test_wide_keys_hand_over_to_segmented_tables(name):
+    # The lowered limit (2^18 children) sends the widest layers on to the
+    # segmented tables: int64 rows, and byte rows with their labels.
+    g = sl2(101) if name == "sl2_101" else GraphDefinition.permutation(O.lrx_generators(22), [7] * 11 + [200] * 11)
+    with NativeEngine(g, backend="segmented") as e:
+        assert e.run() == 1
+        want, last = e.layer_sizes(), sorted(map(tuple, e.sample(0, 1000)))
+    assert sum(want) == (101 * (101 ** 2 - 1) if name == "sl2_101" else math.comb(22, 11))
+    with NativeEngine(g, backend="segmented", flags=128) as e:  # the tables alone
+        assert e.run() == 1
+        assert e.layer_sizes() == want and sorted(map(tuple, e.sample(0, 1000))) == last
+    if name == "sl2_101":
+        with NativeEngine(g, backend="segmented", flags=SORTED_CAP) as e:
+            for _ in range(2):
+                assert e.run() == 1 and e.backend_name == NAME
+                assert e.layer_sizes() == want and sorted(map(tuple, e.sample(0, 1000))) == last
+                assert e.info()["candidates"] == 4 * sum(want)
+                e.reset()
