@@ -16,15 +16,27 @@ namespace mgbfs {
 
 constexpr int kBitmapThreads = 256;
 constexpr int kChildrenPerThread = 24;
+// Workgroups a layer is spread over before its threads take a second parent
+// (8 per CU are resident): a thread's parents go one after another, so 12
+// of them on every layer left S_10's (at most 233,633 parents, 76
+// workgroups) at 51 us each.
+constexpr uint32_t kSpreadBlocks = 2048;
 
+// Parents per thread at most, and for a layer of `count` parents.
 template <int G>
 constexpr int bitmap_items() { return (kChildrenPerThread / G) > 0 ? (kChildrenPerThread / G) : 1; }
+template <int G>
+__host__ __device__ inline uint32_t bitmap_layer_items(uint64_t count) {
+  const uint64_t per = static_cast<uint64_t>(kSpreadBlocks) * kBitmapThreads;
+  const uint64_t items = (count + per - 1) / per;
+  return static_cast<uint32_t>(items < 1 ? 1 : (items > bitmap_items<G>() ? bitmap_items<G>() : items));
+}
 
-// One tile of kBitmapThreads x kItems parents (tile index `tile_index`).
+// One tile of kBitmapThreads x items parents (tile index `tile_index`).
 template <int G>
 __device__ __forceinline__ void bitmap_tile(
-    uint64_t tile_index, const uint64_t* __restrict__ frontier, uint64_t count, const PackedGenerators& gens,
-    uint32_t* __restrict__ bitmap, uint64_t bitmap_bits, uint64_t* __restrict__ next,
+    uint64_t tile_index, uint32_t items, const uint64_t* __restrict__ frontier, uint64_t count,
+    const PackedGenerators& gens, uint32_t* __restrict__ bitmap, uint64_t bitmap_bits, uint64_t* __restrict__ next,
     unsigned long long* __restrict__ next_count, uint64_t count_base, uint64_t next_cap,
     uint32_t* __restrict__ error) {
   constexpr int kItems = bitmap_items<G>();
@@ -32,13 +44,13 @@ __device__ __forceinline__ void bitmap_tile(
   __shared__ uint32_t wave_sums[kBitmapThreads / kWave];
   __shared__ unsigned long long wg_base;
   const uint32_t n = gens.degree;
-  const uint64_t tile = tile_index * kBitmapThreads * kItems;
+  const uint64_t tile = tile_index * kBitmapThreads * items;
   uint32_t newmask = 0;
   uint32_t errbits = 0;
 
   // Phase 1: claim.  Children are not kept; the few new ones are recomputed
   // from the LDS copy of the parent when they are written.
-  for (int it = 0; it < kItems; ++it) {
+  for (uint32_t it = 0; it < items; ++it) {
     const uint64_t p = tile + static_cast<uint64_t>(it) * kBitmapThreads + threadIdx.x;
     const bool valid = p < count;
     const uint64_t key = valid ? frontier[p] : 0;
@@ -121,36 +133,31 @@ __device__ __forceinline__ void bitmap_tile(
 
 template <int G>
 __global__ __launch_bounds__(kBitmapThreads) void bitmap_expand_kernel(
-    const uint64_t* __restrict__ frontier, uint64_t count, PackedGenerators gens,
+    const uint64_t* __restrict__ frontier, uint64_t count, uint32_t items, PackedGenerators gens,
     uint32_t* __restrict__ bitmap, uint64_t bitmap_bits, uint64_t* __restrict__ next,
     unsigned long long* __restrict__ next_count, uint64_t count_base, uint64_t next_cap,
     uint32_t* __restrict__ error) {
-  bitmap_tile<G>(blockIdx.x, frontier, count, gens, bitmap, bitmap_bits, next, next_count, count_base, next_cap,
+  bitmap_tile<G>(blockIdx.x, items, frontier, count, gens, bitmap, bitmap_bits, next, next_count, count_base, next_cap,
                  error);
 }
 
 // A layer whose size is read from the device, so layers can be queued
-// without the host reading each size: marks[0] and marks[1] are the layer
-// counter before and after the previous layer was produced, so the frontier
-// holds marks[1] - marks[0] states and the children are counted from
-// marks[1].  A fixed grid walks the tiles.
+// without the host reading each size: counts[0] is this layer's size and
+// counts[1], zero before, receives the next one's.  A fixed grid walks the
+// tiles.
 template <int G>
-__global__ __launch_bounds__(kBitmapThreads) void bitmap_expand_marked_kernel(
-    const uint64_t* __restrict__ frontier, const unsigned long long* __restrict__ marks, PackedGenerators gens,
-    uint32_t* __restrict__ bitmap, uint64_t bitmap_bits, uint64_t* __restrict__ next,
-    unsigned long long* __restrict__ next_count, uint64_t next_cap, uint32_t* __restrict__ error) {
-  const uint64_t base = marks[1], count = base - marks[0];
-  const uint64_t per_block = static_cast<uint64_t>(kBitmapThreads) * bitmap_items<G>();
+__global__ __launch_bounds__(kBitmapThreads) void bitmap_expand_queued_kernel(
+    const uint64_t* __restrict__ frontier, unsigned long long* __restrict__ counts, PackedGenerators gens,
+    uint32_t* __restrict__ bitmap, uint64_t bitmap_bits, uint64_t* __restrict__ next, uint64_t next_cap,
+    uint32_t* __restrict__ error) {
+  const uint64_t count = counts[0];
+  const uint32_t items = bitmap_layer_items<G>(count);
+  const uint64_t per_block = static_cast<uint64_t>(kBitmapThreads) * items;
   const uint64_t tiles = (count + per_block - 1) / per_block;
   for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-    bitmap_tile<G>(t, frontier, count, gens, bitmap, bitmap_bits, next, next_count, base, next_cap, error);
+    bitmap_tile<G>(t, items, frontier, count, gens, bitmap, bitmap_bits, next, counts + 1, 0, next_cap, error);
     __syncthreads();  // the tile's shared arrays are reused by the next one
   }
-}
-
-// mark = the layer counter once the layers before it on the stream are done.
-__global__ void bitmap_mark_kernel(const unsigned long long* __restrict__ counter, unsigned long long* __restrict__ mark) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *mark = *counter;
 }
 
 __global__ void bitmap_seed_kernel(uint32_t degree, uint64_t start_key, uint32_t* bitmap, uint64_t bitmap_bits,
@@ -170,13 +177,13 @@ template <int G>
 static hipError_t launch_expand(const uint64_t* frontier, uint64_t count, const PackedGenerators& gens,
                                 uint32_t* bitmap, uint64_t bits, uint64_t* next, unsigned long long* next_count,
                                 uint64_t count_base, uint64_t next_cap, uint32_t* error, hipStream_t stream) {
-  constexpr int kItems = bitmap_items<G>();
-  const uint64_t per_block = static_cast<uint64_t>(kBitmapThreads) * kItems;
+  const uint32_t items = bitmap_layer_items<G>(count);
+  const uint64_t per_block = static_cast<uint64_t>(kBitmapThreads) * items;
   const uint64_t blocks = (count + per_block - 1) / per_block;
   if (blocks == 0) return hipSuccess;
   if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
   hipLaunchKernelGGL(bitmap_expand_kernel<G>, dim3(static_cast<uint32_t>(blocks)), dim3(kBitmapThreads), 0, stream,
-                     frontier, count, gens, bitmap, bits, next, next_count, count_base, next_cap, error);
+                     frontier, count, items, gens, bitmap, bits, next, next_count, count_base, next_cap, error);
   return hipGetLastError();
 }
 
@@ -196,16 +203,14 @@ hipError_t bitmap_expand(const uint64_t* frontier, uint64_t count, const PackedG
   }
 }
 
-hipError_t bitmap_expand_marked(const uint64_t* frontier, const unsigned long long* marks,
-                                const PackedGenerators& gens, uint32_t* bitmap, uint64_t bitmap_bits, uint64_t* next,
-                                unsigned long long* next_count, uint64_t next_cap, uint32_t* error, uint32_t grid,
-                                hipStream_t stream) {
-  if (grid == 0) return hipErrorInvalidValue;
+hipError_t bitmap_expand_queued(const uint64_t* frontier, unsigned long long* counts, const PackedGenerators& gens,
+                                uint32_t* bitmap, uint64_t bitmap_bits, uint64_t* next, uint64_t next_cap,
+                                uint32_t* error, hipStream_t stream) {
   switch (gens.count) {
-#define MGBFS_G(k)                                                                                             \
-  case k:                                                                                                      \
-    hipLaunchKernelGGL(bitmap_expand_marked_kernel<k>, dim3(grid), dim3(kBitmapThreads), 0, stream, frontier,   \
-                       marks, gens, bitmap, bitmap_bits, next, next_count, next_cap, error);                    \
+#define MGBFS_G(k)                                                                                              \
+  case k:                                                                                                       \
+    hipLaunchKernelGGL(bitmap_expand_queued_kernel<k>, dim3(kSpreadBlocks), dim3(kBitmapThreads), 0, stream,    \
+                       frontier, counts, gens, bitmap, bitmap_bits, next, next_cap, error);                     \
     break;
     MGBFS_G(1) MGBFS_G(2) MGBFS_G(3) MGBFS_G(4) MGBFS_G(5) MGBFS_G(6) MGBFS_G(7) MGBFS_G(8)
     MGBFS_G(9) MGBFS_G(10) MGBFS_G(11) MGBFS_G(12) MGBFS_G(13) MGBFS_G(14) MGBFS_G(15) MGBFS_G(16)
@@ -213,11 +218,6 @@ hipError_t bitmap_expand_marked(const uint64_t* frontier, const unsigned long lo
     default:
       return hipErrorInvalidValue;
   }
-  return hipGetLastError();
-}
-
-hipError_t bitmap_mark(const unsigned long long* counter, unsigned long long* mark, hipStream_t stream) {
-  hipLaunchKernelGGL(bitmap_mark_kernel, dim3(1), dim3(64), 0, stream, counter, mark);
   return hipGetLastError();
 }
 

@@ -247,22 +247,21 @@ class BitmapEngine final : public Engine {
     stash_count_ = 0;  // no layer here is chunked
     int status = MGBFS_LAYER;
     while (!terminal) {
-      host_marks_[0] = counter_base_ - count_;
-      host_marks_[1] = counter_base_;
-      MGBFS_HIP(hipMemcpyAsync(marks_.as<uint64_t>(), host_marks_, 16, hipMemcpyHostToDevice, stream_));
+      // counts[i] is the size of the batch's layer i (0: the current one).
+      std::memset(host_marks_, 0, (kAhead + 1) * 8);
+      host_marks_[0] = count_;
+      auto* counts = reinterpret_cast<unsigned long long*>(marks_.as<uint64_t>());
+      MGBFS_HIP(hipMemcpyAsync(counts, host_marks_, (kAhead + 1) * 8, hipMemcpyHostToDevice, stream_));
       MGBFS_HIP(hipEventRecord(ev0_, stream_));
-      auto* marks = reinterpret_cast<unsigned long long*>(marks_.as<uint64_t>());
-      auto* counter = reinterpret_cast<unsigned long long*>(control_.as<uint64_t>());
       for (uint32_t i = 0; i < kAhead; ++i) {
         const bool even = (i & 1u) == 0;
         uint64_t* src = (even ? front_ : next_).as<uint64_t>();
         uint64_t* dst = (even ? next_ : front_).as<uint64_t>();
-        MGBFS_HIP(bitmap_expand_marked(src, marks + i, gens_, bitmap_.as<uint32_t>(), domain_, dst, counter,
-                                       remaining, error_word(), kAheadGrid, stream_));
-        MGBFS_HIP(bitmap_mark(counter, marks + i + 2, stream_));
+        MGBFS_HIP(bitmap_expand_queued(src, counts + i, gens_, bitmap_.as<uint32_t>(), domain_, dst, remaining,
+                                       error_word(), stream_));
       }
       MGBFS_HIP(hipEventRecord(ev1_, stream_));
-      MGBFS_HIP(hipMemcpyAsync(host_marks_, marks, (kAhead + 2) * 8, hipMemcpyDeviceToHost, stream_));
+      MGBFS_HIP(hipMemcpyAsync(host_marks_, counts, (kAhead + 1) * 8, hipMemcpyDeviceToHost, stream_));
       read_control();  // queued behind the layers: one wait for all of them
       float ms = 0.f;
       MGBFS_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
@@ -275,12 +274,10 @@ class BitmapEngine final : public Engine {
         batch_failed_ = true;
         return MGBFS_RESOURCE;
       }
-      // Layer i + 1 of the batch holds marks[i + 2] - marks[i + 1] states;
-      // the batch ends at the first empty one.
+      // The batch ends at the first empty layer.
       uint32_t produced = 0;
       for (uint32_t i = 0; i < kAhead; ++i) {
-        const uint64_t parents = host_marks_[i + 1] - host_marks_[i];
-        const uint64_t kids = host_marks_[i + 2] - host_marks_[i + 1];
+        const uint64_t parents = host_marks_[i], kids = host_marks_[i + 1];
         ++launches;
         candidates += parents * gens_.count;
         streamed_bytes += 8 * parents + 8 * kids;
@@ -300,7 +297,6 @@ class BitmapEngine final : public Engine {
         std::swap(front_, next_);
         std::swap(front_cap_, next_cap_);
       }
-      counter_base_ = host_marks_[produced + 1];
       if (!terminal) status = MGBFS_LAYER;
     }
     return status;
@@ -408,11 +404,10 @@ class BitmapEngine final : public Engine {
   // Rows of the previous layer kept across an advance (the states.json
   // previous-layer sample holds at most 1000 rows).
   static constexpr uint64_t kStashRows = 1000;
-  // Layers queued per host wait by run_to_end, the fixed grid of those
-  // layers, and the largest unreached state count it runs with (two
-  // frontier buffers of that many states: 2 GiB).
+  // Layers queued per host wait by run_to_end, and the largest unreached
+  // state count it runs with (two frontier buffers of that many states:
+  // 2 GiB).
   static constexpr uint32_t kAhead = 16;
-  static constexpr uint32_t kAheadGrid = 2048;
   static constexpr uint64_t kAheadStates = 1ull << 27;
   PackedGenerators gens_;
   uint32_t n_;

@@ -430,3 +430,17 @@ def test_sorted_run_ahead_matches_oracle_and_layer_loop(name):
         e.reset()
         assert e.run(max_layers=len(sizes) - 2) == 0
         assert sorted(e.layer_keys()) == ref[-2]
+
+
+@pytest.mark.parametrize("generators", ["lrx", "directed", "coxeter"])
+def test_bitmap_run_to_end_at_every_tile_depth(generators):
+    # Queued layers give a thread one parent up to 524,288 parents per layer
+    # and more beyond, up to what its generator count allows (S_11's widest
+    # LRX layer: 3,049,721; coxeter: two items at most).
+    n = 10 if generators == "coxeter" else 11
+    gens = {"lrx": O.lrx_generators(n), "coxeter": coxeter(n),
+            "directed": [O.lrx_generators(n)[0], O.lrx_generators(n)[2]]}[generators]
+    ref = O.packed_bfs(n, gens)["layers"]
+    with NativeEngine(GraphDefinition.permutation(gens, list(range(n))), backend="permutation_bitmap") as e:
+        assert e.run() == 1
+        assert e.layer_sizes() == ref
