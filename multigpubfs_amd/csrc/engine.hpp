@@ -154,7 +154,12 @@ uint64_t vram_budget(const mgbfs_engine_options& o);
 uint64_t state_space_bound(const Graph& g);
 // Index of each generator's inverse in the set (-1 when absent).
 std::vector<int> inverse_index(const PackedGenerators& gens);
+// Generic backend on graphs whose states are one packed word
+// (generic_packed.hip).
+Engine* make_generic_packed_engine(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound,
+                                   const WideCode& code);
 // Generic backend sizing (generic_engine.hip).
+constexpr uint32_t kGenericMaxArena = 0x7ffffffeu;  // rows
 uint64_t generic_plan_bytes(uint32_t elements, uint64_t capacity, uint32_t state_bytes, uint64_t* slots_out);
 uint32_t generic_state_bytes(const Graph& g);
 uint64_t generic_capacity(const Graph& g, uint64_t budget, uint64_t state_bound);

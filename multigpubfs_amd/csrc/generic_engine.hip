@@ -9,6 +9,7 @@
 #include <cstring>
 #include "engine.hpp"
 #include "kernels.hpp"
+#include "wide.hpp"
 
 extern "C" {
 int mgbfs_generic_seed_i64_wide(uint32_t, const int64_t*, uint32_t, uint32_t, uint64_t*, uint64_t, uint64_t, uint32_t,
@@ -31,7 +32,7 @@ namespace mgbfs {
 
 namespace {
 constexpr uint64_t kHashSeed = 0x19f856a2ull;  // generic_run.rs:24 seeds the visited hash with this value
-constexpr uint32_t kMaxArena = 0x7ffffffeu;
+constexpr uint32_t kMaxArena = kGenericMaxArena;
 constexpr uint32_t kBatch = 1u << 20;
 
 #define MGBFS_ABI(call)                                                                      \
@@ -282,6 +283,11 @@ class GenericEngine final : public Engine {
 };
 
 Engine* make_generic_engine(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound) {
+  // States of one packed word (wide.hpp) keep their words instead of rows;
+  // the test flag forces the row table's equality path.
+  WideCode code;
+  if (!(o.flags & MGBFS_FLAG_TEST_COLLIDE_HASH) && make_wide(g, code, 63))
+    return make_generic_packed_engine(g, o, state_bound, code);
   return new GenericEngine(g, o, state_bound);
 }
 

@@ -43,19 +43,6 @@ struct NibbleAction {
   __device__ __forceinline__ uint32_t mask(uint32_t g) const { return gens.child_mask[g]; }
 };
 
-// Wide keys: the table through the constant address space, so that a
-// generator index that is uniform in the wave reads it with scalar loads.
-struct WideAction {
-  const WideTable* table;
-  uint32_t generators;
-  using ConstTable = const __attribute__((address_space(4))) WideTable*;
-  __device__ __forceinline__ uint32_t count() const { return generators; }
-  __device__ __forceinline__ uint64_t child(uint64_t key, uint32_t g) const {
-    return wide_child((ConstTable)table, key, g);
-  }
-  __device__ __forceinline__ uint32_t mask(uint32_t g) const { return ((ConstTable)table)->child_mask[g]; }
-};
-
 struct BlockLds {
   alignas(16) uint64_t table[kBlockSlots];
   uint32_t fresh;     // new states inserted

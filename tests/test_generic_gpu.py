@@ -7,6 +7,7 @@ each run with full 64-bit hashes and with every hash colliding (equality
 alone decides), plus the RESOURCE stop at a tiny capacity.
 """
 import math
+import random
 
 import pytest
 
@@ -95,3 +96,56 @@ def test_previous_layer_sample():
         run_layers(e)
         prev = sorted(map(tuple, e.sample(1, 1000)))
     assert prev == sorted(map(tuple, expected[-2]))
+
+
+# Graphs whose states fit one packed word: matrices, repeated or wide labels,
+# more positions than the nibble encoding has, directed and not.
+def directed(n, start, k, seed):
+    rng = random.Random(seed)
+    gens = []
+    for _ in range(k):
+        g = list(range(n))
+        rng.shuffle(g)
+        gens.append(g)
+    return GraphDefinition.permutation(gens, start)
+
+
+def sl2_directed(p):
+    return GraphDefinition.matrix(2, 2, [([1, 1, 0, 1], p), ([1, 0, 1, 1], p)], [1, 0, 0, 1])
+
+
+PACKED = {
+    "sl2_13_directed": lambda: sl2_directed(13),
+    "sl2_31_directed": lambda: sl2_directed(31),
+    "vectors_1009": lambda: GraphDefinition.matrix(2, 1, [([2, 1, 1, 1], 1009), ([1, 0, 1, 1], 1009)], [3, 1008]),
+    "labels9": lambda: directed(9, [0, 0, 1, 1, 2, 2, 3, 3, 300], 3, 1),
+    "two_labels24": lambda: directed(24, [-4] * 19 + [90] * 5, 2, 2),
+    "sixteen_generators": lambda: directed(10, [0, 0, 0, 1, 1, 2, 2, 3, 4, 5], 16, 3),
+    "one_state": lambda: directed(20, [7] * 20, 2, 4),
+}
+
+
+@pytest.mark.parametrize("name", list(PACKED))
+def test_packed_words_layer_sets_and_capacity(name):
+    g = PACKED[name]()
+    want = [sorted(map(tuple, x)) for x in O.c_exact_layers(g.to_dict(), 1 << 21)]
+    sizes = [len(x) for x in want]
+    total = sum(sizes)
+    with NativeEngine(g, backend="generic", capacity=total) as e:  # every row used
+        status, layers = run_layers(e)
+        assert status == 1 and layers == want
+        e.reset()
+        assert e.run() == 1 and e.layer_sizes() == sizes
+        assert sorted(map(tuple, e.sample(0, 1 << 20))) == want[-1]
+        if len(want) > 1:
+            assert sorted(map(tuple, e.sample(1, 1 << 20))) == want[-2]
+        info = e.info()
+        assert info["candidates"] == total * g.generator_count and info["history_layers"] == 0
+    for capacity in {total - 1, total // 2, 3} - {0}:  # the layer that does not fit stops the run
+        if capacity >= total:
+            continue
+        with NativeEngine(g, backend="generic", capacity=capacity) as e:
+            assert e.run() == 2
+            got = e.layer_sizes()
+            assert got == sizes[:len(got)] and sum(sizes[:len(got) + 1]) > capacity >= sum(got)
+            assert sorted(map(tuple, e.sample(0, 1 << 20))) == want[len(got) - 1]
