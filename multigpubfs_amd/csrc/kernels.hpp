@@ -63,9 +63,20 @@ enum LayerState : uint32_t {
 struct LayerRecord {
   uint64_t N, unique, ticks;  // ticks: wall_clock64() when the layer was counted
   uint64_t children;          // block_run: generated for this layer; owner layers: from it
-  uint32_t state, pad;
+  uint32_t state, pad;        // general path: the error word
   uint64_t seq;
+  uint64_t stamps[4];         // general path: LayerCounters.stamps
 };
+
+// Device words of a layer on the general path.
+struct LayerCounters {
+  unsigned long long unique;    // distinct children
+  uint32_t error, pad;
+  unsigned long long children;  // generated
+  unsigned long long spare;
+  unsigned long long stamps[4];  // wall_clock64() at the start of the layer, its partition, unique_diff and scan
+};
+static_assert(sizeof(LayerCounters) == 64, "one 64-byte line");
 
 // One-workgroup layers: everything fits one LDS table.
 constexpr uint32_t kBlockSlots = 16384;
@@ -152,8 +163,11 @@ hipError_t owner_export(const OwnerSlabs& cur, uint64_t* bank, uint32_t* off, co
                         uint64_t* prev_bank, uint32_t* prev_off, uint32_t owners, hipStream_t stream);
 
 uint64_t scan_workspace_words(uint64_t n);
-hipError_t exclusive_scan_u32(const uint32_t* in, uint64_t n, uint32_t* out, uint32_t* workspace,
-                              hipStream_t stream);
+// rec: report the layer of `counters` with the scan's total (see scan.hip).
+hipError_t exclusive_scan_u32(const uint32_t* in, uint64_t n, uint32_t* out, uint32_t* workspace, hipStream_t stream,
+                              LayerCounters* counters = nullptr, LayerRecord* rec = nullptr, uint64_t seq = 0);
+// One wall_clock64() reading as a record.
+hipError_t stamp_record(LayerRecord* rec, uint64_t seq, hipStream_t stream);
 hipError_t sorted_seed(uint64_t start_key, const SortedLayout& L, uint64_t* bank, uint32_t* off, uint32_t Ko,
                        hipStream_t stream);
 // Children of bank[0..F) routed by lane (sub-bucket >> K2) into slabs: slab
@@ -181,7 +195,7 @@ hipError_t sorted_expand_route_wide(const uint64_t* bank, uint64_t F, const Acti
 // zeroed by the caller).
 hipError_t sorted_partition(const uint64_t* in, const uint32_t* lcount, uint32_t lcap, uint32_t P, uint32_t nsub,
                             uint32_t K2, uint32_t* scount, uint32_t* error, uint64_t* out, uint64_t out_entries,
-                            hipStream_t stream);
+                            hipStream_t stream, unsigned long long* stamp = nullptr);
 // In-layer dedup of the sub-bucket slabs and difference against the
 // current bank and, when given, the previous one (banks partitioned into
 // nbo_c / nbo_p fine buckets); survivors are written back grouped by the
@@ -190,7 +204,8 @@ hipError_t sorted_unique_diff(uint64_t* cand, const uint32_t* scount, uint32_t n
                               const uint32_t* cur_off, uint32_t nbo_c, const uint64_t* prev, const uint32_t* prev_off,
                               uint32_t nbo_p, uint32_t fb, uint32_t* fine_counts, uint32_t* error,
                               unsigned long long* unique_total, unsigned long long* cand_total, uint32_t tagbits,
-                              bool merge, uint32_t grid_limit, hipStream_t stream);
+                              bool merge, uint32_t grid_limit, hipStream_t stream,
+                              unsigned long long* stamp = nullptr);
 // Writes nothing unless *error == 0 and the layer total off[nsub << fb]
 // fits bank_rows, so it may be queued before the host has read either.
 hipError_t sorted_compact(const uint64_t* cand, uint32_t nsub, uint32_t fb, const uint32_t* off, const uint32_t* error,
@@ -203,6 +218,6 @@ hipError_t sorted_capacity_check(const uint32_t* off, uint64_t n, uint64_t rows,
 hipError_t fill_u64(uint64_t* dst, uint64_t value, uint64_t count, hipStream_t stream);
 hipError_t fill_u32(uint32_t* dst, uint32_t value, uint64_t count, hipStream_t stream);
 hipError_t zero_u32x3(uint32_t* a, uint64_t na, uint32_t* b, uint64_t nb, uint32_t* c, uint64_t nc,
-                      hipStream_t stream);
+                      hipStream_t stream, unsigned long long* stamp = nullptr);
 
 }  // namespace mgbfs

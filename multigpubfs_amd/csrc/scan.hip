@@ -41,7 +41,9 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* w
 }
 
 __global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_t* __restrict__ in, uint64_t n,
-                                                                   uint32_t* __restrict__ block_sums) {
+                                                                   uint32_t* __restrict__ block_sums,
+                                                                   unsigned long long* stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
   __shared__ uint32_t wave_sums[kScanThreads / kWave];
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kScanTile;
   uint32_t s = 0;
@@ -56,7 +58,11 @@ __global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_
 }
 
 // Single block: exclusive scan of the block sums in place (any count).
-__global__ __launch_bounds__(kScanThreads) void scan_carry_kernel(uint32_t* __restrict__ sums, uint32_t count) {
+// With a record, the layer whose counts are scanned is reported: the total
+// is known here, before the offsets are written.
+__global__ __launch_bounds__(kScanThreads) void scan_carry_kernel(uint32_t* __restrict__ sums, uint32_t count,
+                                                                   const LayerCounters* counters, LayerRecord* rec,
+                                                                   uint64_t seq) {
   __shared__ uint32_t wave_sums[kScanThreads / kWave];
   uint32_t carry = 0;
   for (uint32_t base = 0; base < count; base += kScanThreads) {
@@ -67,7 +73,16 @@ __global__ __launch_bounds__(kScanThreads) void scan_carry_kernel(uint32_t* __re
     if (i < count) sums[i] = carry + ex;
     carry += total;
   }
-  if (threadIdx.x == 0) sums[count] = carry;
+  if (threadIdx.x != 0) return;
+  sums[count] = carry;
+  if (!rec) return;
+  rec->N = carry;
+  rec->unique = counters->unique;
+  rec->children = counters->children;
+  rec->state = counters->error;
+  rec->ticks = wall_clock64();
+  for (int k = 0; k < 4; ++k) rec->stamps[k] = counters->stamps[k];
+  __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ __launch_bounds__(kScanThreads) void scan_downsweep_kernel(const uint32_t* __restrict__ in, uint64_t n,
@@ -97,15 +112,15 @@ __global__ __launch_bounds__(kScanThreads) void scan_downsweep_kernel(const uint
 
 uint64_t scan_workspace_words(uint64_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
 
-hipError_t exclusive_scan_u32(const uint32_t* in, uint64_t n, uint32_t* out, uint32_t* workspace,
-                              hipStream_t stream) {
+hipError_t exclusive_scan_u32(const uint32_t* in, uint64_t n, uint32_t* out, uint32_t* workspace, hipStream_t stream,
+                              LayerCounters* counters, LayerRecord* rec, uint64_t seq) {
   if (n == 0) return hipErrorInvalidValue;
   const uint64_t blocks = (n + kScanTile - 1) / kScanTile;
   if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
   hipLaunchKernelGGL(scan_reduce_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kScanThreads), 0, stream, in, n,
-                     workspace);
+                     workspace, counters ? &counters->stamps[3] : nullptr);
   hipLaunchKernelGGL(scan_carry_kernel, dim3(1), dim3(kScanThreads), 0, stream, workspace,
-                     static_cast<uint32_t>(blocks));
+                     static_cast<uint32_t>(blocks), counters, rec, seq);
   hipLaunchKernelGGL(scan_downsweep_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kScanThreads), 0, stream, in, n,
                      workspace, out);
   return hipGetLastError();

@@ -49,9 +49,6 @@ class SortedEngine final : public Engine {
     if (!g.inverse_closed) throw std::runtime_error("SORTED_REQUIRES_INVERSE_CLOSED");
     MGBFS_HIP(hipSetDevice(device_));
     MGBFS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-    for (auto& e : ev_) MGBFS_HIP(hipEventCreate(&e));
-    for (auto& p : cev_)
-      for (auto& e : p) MGBFS_HIP(hipEventCreate(&e));
     budget_ = vram_budget(o);
     bound_ = state_space_bound(g);
     cap_limit_ = o.capacity ? o.capacity : ~0ull;
@@ -69,11 +66,9 @@ class SortedEngine final : public Engine {
     control_.allocate(kCtlOffset + sizeof(OwnerCtl) * kOwnerRing + 4 * kOwnerBuffers * kOwnersMax);
     fine_counts_.allocate(((1ull << kMaxBucketBits) + 1) * 4);
     for (int b = 0; b < 3; ++b) off_[b].allocate(((1ull << kMaxBucketBits) + 1) * 4);
-    // Pinned: the general path's readback words, then the layer records.
-    const size_t host_bytes = 64 + sizeof(LayerRecord) * (kBlockLayers + 1);
-    MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_), host_bytes, hipHostMallocDefault));
-    std::memset(host_, 0, host_bytes);
-    rec_ = reinterpret_cast<LayerRecord*>(host_ + 8);
+    const size_t rec_bytes = sizeof(LayerRecord) * (kBlockLayers + 1);
+    MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec_), rec_bytes, hipHostMallocDefault));
+    std::memset(rec_, 0, rec_bytes);
     int khz = 0;
     MGBFS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
     tick_seconds_ = khz > 0 ? 1e-3 / khz : 0.0;
@@ -88,12 +83,7 @@ class SortedEngine final : public Engine {
   ~SortedEngine() override {
     (void)hipSetDevice(device_);
     if (stream_) (void)hipStreamSynchronize(stream_);
-    if (host_) (void)hipHostFree(host_);
-    for (auto& e : ev_)
-      if (e) (void)hipEventDestroy(e);
-    for (auto& p : cev_)
-      for (auto& e : p)
-        if (e) (void)hipEventDestroy(e);
+    if (rec_) (void)hipHostFree(rec_);
     if (stream_) (void)hipStreamDestroy(stream_);
   }
 
@@ -108,7 +98,7 @@ class SortedEngine final : public Engine {
     nbo_[0] = 1;  // the start bank has one fine bucket
     block_rejected_ = owner_rejected_ = 0;
     start_bank();
-    cpending_[0] = cpending_[1] = false;
+    compacted_ = 0;
     layers.assign(1, 1);
     candidates = unique_candidates = 0;
     kernel_seconds = 0.0;
@@ -183,9 +173,11 @@ class SortedEngine final : public Engine {
       ensure_u32(scan_ws_, scan_workspace_words(1ull << kMaxBucketBits) + 16);
       const uint32_t fb = geo.fb, nbo = geo.nbo;
       // Counters (unique, error, candidates), sub-bucket and lane cursors.
+      // The kernels stamp their start times: eight timing events took 4.5 us
+      // each on the stream.
+      LayerCounters* counters = control_.as<LayerCounters>();
       MGBFS_HIP(zero_u32x3(reinterpret_cast<uint32_t*>(control_.as<uint64_t>()), 6, scount_.as<uint32_t>(), nsub,
-                           lcount_.as<uint32_t>(), K2 ? lslabs : 0, stream_));
-      MGBFS_HIP(hipEventRecord(ev_[0], stream_));
+                           lcount_.as<uint32_t>(), K2 ? lslabs : 0, stream_, &counters->stamps[0]));
       uint64_t* sub = sub_.as<uint64_t>();
       const uint32_t stride = K2 ? lcap : kSlabStride, full = K2 ? kErrLaneSlab : kErrBucketCap;
       uint32_t* cursors = K2 ? lcount_.as<uint32_t>() : scount_.as<uint32_t>();
@@ -198,38 +190,31 @@ class SortedEngine final : public Engine {
       else
         MGBFS_HIP(sorted_expand_route(bank_[cur_].as<uint64_t>(), F, gens_, layout_, masked, nsub, K2, NB1, P, lcap,
                                       stride, full, cursors, error_word(), routed_to, routed_entries, stream_));
-      MGBFS_HIP(hipEventRecord(ev_[1], stream_));
       if (K2)
         MGBFS_HIP(sorted_partition(lane_.as<uint64_t>(), lcount_.as<uint32_t>(), lcap, P, nsub, K2,
-                                   scount_.as<uint32_t>(), error_word(), sub, routed(sub_entries), stream_));
-      MGBFS_HIP(hipEventRecord(ev_[2], stream_));
+                                   scount_.as<uint32_t>(), error_word(), sub, routed(sub_entries), stream_,
+                                   &counters->stamps[1]));
       auto* control = reinterpret_cast<unsigned long long*>(control_.as<uint64_t>());
       MGBFS_HIP(sorted_unique_diff(
           sub, scount_.as<uint32_t>(), nsub, bank_[cur_].as<uint64_t>(), off_[cur_].as<uint32_t>(), nbo_[cur_],
           probe_prev ? bank_[prev_].as<uint64_t>() : nullptr, probe_prev ? off_[prev_].as<uint32_t>() : nullptr,
           probe_prev ? nbo_[prev_] : 0, fb, fine_counts_.as<uint32_t>(), error_word(), control, control + 2,
-          layout_.tagbits, layout_.prune != 0, unique_grid_, stream_));
-      MGBFS_HIP(hipEventRecord(ev_[4], stream_));
+          layout_.tagbits, layout_.prune != 0, unique_grid_, stream_, &counters->stamps[2]));
+      // The scan reports the layer (N, error word, counters) in pinned memory.
+      const uint64_t seq = seq_++;
       MGBFS_HIP(exclusive_scan_u32(fine_counts_.as<uint32_t>(), nbo, off_[nxt].as<uint32_t>(),
-                                   scan_ws_.as<uint32_t>(), stream_));
-      MGBFS_HIP(hipEventRecord(ev_[3], stream_));
-      // Readback: unique count, error word, candidate count, N (last offset).
-      MGBFS_HIP(hipMemcpyAsync(host_, control_.as<uint64_t>(), 24, hipMemcpyDeviceToHost, stream_));
-      MGBFS_HIP(hipMemcpyAsync(reinterpret_cast<uint32_t*>(host_ + 3), off_[nxt].as<uint32_t>() + nbo, 4,
-                               hipMemcpyDeviceToHost, stream_));
-      MGBFS_HIP(hipEventRecord(ev_[5], stream_));
+                                   scan_ws_.as<uint32_t>(), stream_, counters, rec_, seq));
       // The compaction is queued before the host has read N or the error
       // word; it writes nothing unless the layer is clean and fits the bank
       // as allocated now, and the host relaunches it after growing the bank.
-      // The host wakes on the readback alone, so its turnaround and the next
+      // The host wakes on the record alone, so its turnaround and the next
       // layer's launches overlap the compaction.
       const uint64_t early_rows = bank_cap_[nxt];
       if (early_rows) compact(sub, nsub, fb, nxt);
-      MGBFS_HIP(hipEventSynchronize(ev_[5]));
-      const uint32_t err = static_cast<uint32_t>(host_[1]);
-      const uint64_t C = host_[2];
-      const uint64_t N = static_cast<uint32_t>(host_[3]);
-      account(F, C, N, probe_prev ? count_[prev_] : 0, K2 != 0);
+      const LayerRecord rec = await(rec_[0], seq);
+      const uint32_t err = rec.state;
+      const uint64_t C = rec.children, N = rec.N;
+      account(rec, F, probe_prev ? count_[prev_] : 0, K2 != 0);
       if (err & kErrLaneSlab) {  // lane slab overflow: retry with twice the slack
         slack_ = slack_ ? 2 * slack_ : 1;
         ++retries;
@@ -245,7 +230,7 @@ class SortedEngine final : public Engine {
       if (err) return out_of_room(fatal, err);
       candidates += C;
       last_ratio_ = masked ? static_cast<double>(C) / static_cast<double>(F) : 0.0;
-      unique_candidates += host_[0];
+      unique_candidates += rec.unique;
       if (N == 0) {
         *next_count = 0;
         terminal = true;
@@ -311,7 +296,10 @@ class SortedEngine final : public Engine {
   uint64_t retry_count() const override { return retries; }
 
   void settle() override {
-    for (int s = 0; s < 2; ++s) read_compact(s);
+    if (!compacted_) return;
+    const uint64_t seq = seq_++;
+    MGBFS_HIP(stamp_record(rec_, seq, stream_));
+    end_compaction(await(rec_[0], seq).ticks);
   }
 
   double phase_seconds[kPhaseCount] = {};
@@ -400,6 +388,7 @@ class SortedEngine final : public Engine {
     for (uint32_t i = 0;; ++i) {
       const LayerRecord& rec = await(rec_[i], r.seq + i);
       if (i == 0) first = rec.ticks;
+      end_compaction(rec.ticks);
       const int s = take(rec, rec.children, rec.ticks - first);
       first = rec.ticks;
       if (s != kTakeNext) {
@@ -484,6 +473,7 @@ class SortedEngine final : public Engine {
           MGBFS_HIP(owner_report(ctl + most % kOwnerRing, rules, rec_ + most % kOwnerRing, seq + most, stream_));
       }
       const LayerRecord& rec = await(rec_[r % kOwnerRing], seq + r);
+      end_compaction(rec.ticks);
       if (r == 0) {
         s = rec.state == kLayerNext ? kTakeNext : kTakeRejected;
       } else {
@@ -538,16 +528,18 @@ class SortedEngine final : public Engine {
     return MGBFS_LAYER;  // a rejected layer after accepted ones is met again by the next call
   }
   // Waits for a record in pinned memory: 6 us after its kernel against 16
-  // for a copy and a stream wait.  The kernels always leave their records,
-  // so a long silence means a device error, which the stream wait reports.
+  // for a copy and a stream wait.  The kernels always leave their records;
+  // a stream that ends or fails without one is an error.
   const LayerRecord& await(const LayerRecord& rec, uint64_t seq) {
-    for (uint32_t spin = 0;; ++spin) {
-      if (__atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) == seq) return rec;
-      if (spin >= (1u << 20)) break;
+    auto there = [&] { return __atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) == seq; };
+    while (true) {
+      for (uint32_t spin = 0; spin < (1u << 18); ++spin)
+        if (there()) return rec;
+      const hipError_t e = hipStreamQuery(stream_);
+      if (e == hipErrorNotReady) continue;
+      MGBFS_HIP(e);
+      if (!there()) throw std::runtime_error("SORTED_LAYER_RECORD");
     }
-    MGBFS_HIP(hipStreamSynchronize(stream_));
-    if (__atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) != seq) throw std::runtime_error("SORTED_LAYER_RECORD");
-    return rec;
   }
   int free_bank(int cur, int prev) const {
     for (int b = 0; b < 3; ++b)
@@ -592,28 +584,19 @@ class SortedEngine final : public Engine {
     terminal = true;
     return MGBFS_RESOURCE;
   }
-  // Compactions run unwaited; each is bracketed by one of two event pairs,
-  // read (and charged to phase 3) when the pair is reused or on settle().
-  // A pair is reused two compactions later, after the host has waited on
-  // the stream past it (a later readback, or the sync before a bank grows),
-  // so that read does not block.
+  // A compaction runs unwaited: the time from the layer's record to the next
+  // stamp on the stream is charged to it (phase 3).
   void compact(uint64_t* sub, uint32_t nsub, uint32_t fb, int nxt) {
-    const int s = cslot_ ^= 1;
-    read_compact(s);
-    MGBFS_HIP(hipEventRecord(cev_[s][0], stream_));
     MGBFS_HIP(sorted_compact(sub, nsub, fb, off_[nxt].as<uint32_t>(), error_word(), bank_cap_[nxt],
                              bank_[nxt].as<uint64_t>(), stream_));
-    MGBFS_HIP(hipEventRecord(cev_[s][1], stream_));
-    cpending_[s] = true;
   }
-  void read_compact(int s) {
-    if (!cpending_[s]) return;
-    MGBFS_HIP(hipEventSynchronize(cev_[s][1]));
-    float ms = 0.f;
-    MGBFS_HIP(hipEventElapsedTime(&ms, cev_[s][0], cev_[s][1]));
-    phase_seconds[3] += ms * 1e-3;
-    kernel_seconds += ms * 1e-3;
-    cpending_[s] = false;
+  void end_compaction(uint64_t ticks) {
+    if (compacted_) {
+      const double s = static_cast<double>(ticks - compacted_) * tick_seconds_;
+      phase_seconds[3] += s;
+      kernel_seconds += s;
+    }
+    compacted_ = 0;
   }
   // Routing output size as passed to the kernels; the test flag reports an
   // oversized output so they take their 64-bit addressing path.
@@ -621,20 +604,20 @@ class SortedEngine final : public Engine {
     return (flags_ & MGBFS_FLAG_TEST_WIDE_ROUTING) ? ~0ull : entries;
   }
   int next_bank() const { return free_bank(cur_, prev_); }
-  // Phase times (events on the engine stream) and modelled streaming bytes
+  // Phase times (the kernels' start stamps) and modelled streaming bytes
   // (see the kernel file header).  Phase 2 is unique_diff alone; the fine
   // count scan is charged to phase 3 with the compaction it feeds.
-  void account(uint64_t F, uint64_t C, uint64_t N, uint64_t Fp, bool partitioned) {
-    float a = 0, b = 0, c = 0, d = 0;
-    MGBFS_HIP(hipEventElapsedTime(&a, ev_[0], ev_[1]));
-    MGBFS_HIP(hipEventElapsedTime(&b, ev_[1], ev_[2]));
-    MGBFS_HIP(hipEventElapsedTime(&c, ev_[2], ev_[4]));
-    MGBFS_HIP(hipEventElapsedTime(&d, ev_[4], ev_[3]));
-    phase_seconds[0] += a * 1e-3;
-    phase_seconds[1] += b * 1e-3;
-    phase_seconds[2] += c * 1e-3;
-    phase_seconds[3] += d * 1e-3;
-    kernel_seconds += (a + b + c + d) * 1e-3;
+  void account(const LayerRecord& rec, uint64_t F, uint64_t Fp, bool partitioned) {
+    const uint64_t C = rec.children, N = rec.N;
+    end_compaction(rec.stamps[0]);
+    const uint64_t routed = partitioned ? rec.stamps[1] : rec.stamps[2];
+    const uint64_t ticks[4] = {routed - rec.stamps[0], rec.stamps[2] - routed, rec.stamps[3] - rec.stamps[2],
+                               rec.ticks - rec.stamps[3]};
+    for (int p = 0; p < 4; ++p) {
+      phase_seconds[p] += static_cast<double>(ticks[p]) * tick_seconds_;
+      kernel_seconds += static_cast<double>(ticks[p]) * tick_seconds_;
+    }
+    compacted_ = rec.ticks;
     const uint64_t be = 8 * F + 8 * C, bp = partitioned ? 16 * C : 0, bu = 8 * C + 8 * F + 8 * Fp + 8 * N;
     phase_bytes[0] += be;
     phase_bytes[1] += bp;
@@ -706,17 +689,14 @@ class SortedEngine final : public Engine {
   uint64_t bank_cap_[3] = {0, 0, 0}, count_[3] = {0, 0, 0};
   uint32_t nbo_[3] = {0, 0, 0};  // fine buckets of each bank
   int cur_ = 0, prev_ = -1;
-  uint64_t* host_ = nullptr;
   DeviceBuffer owner_;               // owner layers' slab arrays
-  LayerRecord* rec_ = nullptr;       // pinned, after host_'s words
+  LayerRecord* rec_ = nullptr;       // pinned: what the kernels report of their layers
   uint64_t seq_ = 1, bound_ = 0;     // next unused record number; state-space bound (0 = unknown)
   double tick_seconds_ = 0.0;        // one wall_clock64() tick
   size_t block_rejected_ = 0;        // layers.size() when the one-workgroup kernel last refused a layer
   size_t owner_rejected_ = 0;        // the same of the owner layers
   bool general_only_ = false;
-  hipEvent_t ev_[6] = {}, cev_[2][2] = {};
-  bool cpending_[2] = {false, false};
-  int cslot_ = 0;
+  uint64_t compacted_ = 0;           // ticks of the record before a compaction not yet timed
 };
 
 Engine* make_sorted_engine(const Graph& g, const mgbfs_engine_options& o, const WideCode* wide) {

@@ -176,8 +176,9 @@ __global__ __launch_bounds__(kRouteThreads) void partition_scatter_kernel(const 
                                                                            uint32_t* __restrict__ scount,
                                                                            uint32_t* __restrict__ error,
                                                                            uint64_t* __restrict__ out,
-                                                                           uint32_t dump) {
+                                                                           uint32_t dump, unsigned long long* stamp) {
   __shared__ TileLds t;
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
   clear_tile_counters(t);
   __syncthreads();
   const uint64_t slab = blockIdx.x;
@@ -237,6 +238,7 @@ struct UniqueArgs {
   uint32_t merge;    // OR the back-edge masks of duplicates into the kept entry
   uint32_t fb, nbo_c, nbo_p, tagbits, buckets;  // buckets: sub-buckets of this layer
   uint64_t range_inv;                           // range_inverse(buckets)
+  unsigned long long* stamp;                    // receives the start time (null: none)
 };
 
 // Bank entry h: if its state is in the table, set `mark` in that slot's
@@ -388,6 +390,7 @@ template <bool kPrev>
 __global__ __launch_bounds__(kUniqueThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void unique_diff_kernel(
     UniqueArgs a) {
   __shared__ UniqueLds u;
+  if (a.stamp && blockIdx.x == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();
   const uint32_t fine_bits = a.fb, fine = 1u << fine_bits;
   const uint32_t nbo = a.buckets << fine_bits;  // fine buckets of the layer written
   // Fine bucket of a survivor of sub-bucket f, within f.  A layer whose
@@ -659,13 +662,13 @@ hipError_t sorted_expand_route(const uint64_t* bank, uint64_t F, const PackedGen
 
 hipError_t sorted_partition(const uint64_t* in, const uint32_t* lcount, uint32_t lcap, uint32_t P, uint32_t nsub,
                             uint32_t K2, uint32_t* scount, uint32_t* error, uint64_t* out, uint64_t out_entries,
-                            hipStream_t stream) {
+                            hipStream_t stream, unsigned long long* stamp) {
   if (K2 == 0 || K2 > kMaxPassBits || (nsub & ((1u << K2) - 1u)) || nsub == 0 || nsub > (1u << kMaxBucketBits) ||
       (nsub >> K2) > (1u << kMaxPassBits) || P == 0 || lcap == 0)
     return hipErrorInvalidValue;
   const uint32_t blocks = (nsub >> K2) * P;
   hipLaunchKernelGGL(partition_scatter_kernel, dim3(blocks), dim3(kRouteThreads), 0, stream, in, lcount, lcap, P, nsub,
-                     K2, scount, error, out, dump_index(out_entries));
+                     K2, scount, error, out, dump_index(out_entries), stamp);
   return hipGetLastError();
 }
 
@@ -673,7 +676,7 @@ hipError_t sorted_unique_diff(uint64_t* cand, const uint32_t* scount, uint32_t n
                               const uint32_t* cur_off, uint32_t nbo_c, const uint64_t* prev, const uint32_t* prev_off,
                               uint32_t nbo_p, uint32_t fb, uint32_t* fine_counts, uint32_t* error,
                               unsigned long long* unique_total, unsigned long long* cand_total, uint32_t tagbits,
-                              bool merge, uint32_t grid_limit, hipStream_t stream) {
+                              bool merge, uint32_t grid_limit, hipStream_t stream, unsigned long long* stamp) {
   if (nsub == 0 || !cur || !cur_off || fb > kMaxFineBits || (static_cast<uint64_t>(nsub) << fb) > (1ull << kMaxBucketBits) ||
       (cur && (nbo_c == 0 || nbo_c > (1u << kMaxBucketBits))) ||
       (prev && (nbo_p == 0 || nbo_p > (1u << kMaxBucketBits))) || grid_limit == 0)
@@ -684,7 +687,7 @@ hipError_t sorted_unique_diff(uint64_t* cand, const uint32_t* scount, uint32_t n
   // G <= tagbits - 2), so the mark bit tagbits-1 is free and a marked entry
   // never equals the all-ones empty marker.
   UniqueArgs a{cand, scount, cur, cur_off, prev, prev_off, fine_counts, error, unique_total, cand_total, tagmask,
-               1ull << (tagbits - 1), merge ? 1u : 0u, fb, nbo_c, nbo_p, tagbits, nsub, range_inverse(nsub)};
+               1ull << (tagbits - 1), merge ? 1u : 0u, fb, nbo_c, nbo_p, tagbits, nsub, range_inverse(nsub), stamp};
   const uint32_t grid = std::min<uint32_t>(nsub, grid_limit);
   if (prev)
     hipLaunchKernelGGL(unique_diff_kernel<true>, dim3(grid), dim3(kUniqueThreads), 0, stream, a);

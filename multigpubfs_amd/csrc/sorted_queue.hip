@@ -210,6 +210,12 @@ __global__ void sorted_start_kernel(uint64_t stored, uint64_t* bank, uint32_t* o
   if (threadIdx.x < 8) control[threadIdx.x] = 0;
 }
 
+__global__ void stamp_record_kernel(LayerRecord* rec, uint64_t seq) {
+  if (threadIdx.x != 0) return;
+  rec->ticks = wall_clock64();
+  __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------------ owner layers
 
 __global__ __launch_bounds__(kBlockThreads) void owner_begin_kernel(uint32_t* counts, uint32_t words, OwnerCtl* ctl,
@@ -561,6 +567,11 @@ hipError_t sorted_block_run(const BlockRun& run, const ActionRef& act, hipStream
 
 hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t* control, hipStream_t stream) {
   hipLaunchKernelGGL(sorted_start_kernel, dim3(1), dim3(64), 0, stream, stored, bank, off, control);
+  return hipGetLastError();
+}
+
+hipError_t stamp_record(LayerRecord* rec, uint64_t seq, hipStream_t stream) {
+  hipLaunchKernelGGL(stamp_record_kernel, dim3(1), dim3(64), 0, stream, rec, seq);
   return hipGetLastError();
 }
 
