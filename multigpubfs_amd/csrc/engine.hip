@@ -840,7 +840,7 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
 static Engine* create(const Graph& g, const mgbfs_engine_options& o) {
   switch (choose_backend(g, o.backend)) {
     case MGBFS_BACKEND_BITMAP:
-      return make_bitmap_engine(g, o);
+      return rank_bitmap_takes(g, o) ? make_rank_bitmap_engine(g, o) : make_bitmap_engine(g, o);
     case MGBFS_BACKEND_SORTED:
       return new HandoverEngine(g, o);
     case MGBFS_BACKEND_SEGMENTED: {

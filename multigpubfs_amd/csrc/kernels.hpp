@@ -146,6 +146,44 @@ struct OwnerLayer {
   uint64_t seq;
 };
 
+// Permutation bitmap by owners (rank_owner.hip).
+constexpr uint32_t kRankDegree = 12;
+
+struct RankPlan {
+  uint32_t degree, owners, magic;  // magic: floor(2^32 / owners)
+  uint32_t slice_words, list_cap;  // per owner: bitmap words (a multiple of 4), states
+};
+
+struct RankLayer {
+  RankPlan plan;
+  uint32_t claim;        // 0: send only (the layer is in the list already)
+  const uint32_t* in;    // messages of this layer: owners x in_cap
+  uint32_t* in_count;    // cleared
+  uint32_t in_cap;
+  uint32_t* out;         // messages of the next layer
+  uint32_t* out_count;
+  uint32_t out_cap, out_dump;  // out_dump: set by rank_layer
+  uint32_t* bitmap;      // owners x slice_words
+  uint32_t* list;        // owners x list_cap: states in discovery order
+  const uint32_t* ends_before;  // list ends per owner after the layer before
+  uint32_t* ends_now;           // and after this one
+  const OwnerCtl* before;
+  OwnerCtl *now, *after;
+  OwnerRules rules;
+  LayerRecord* rec;      // record of the layer before
+  uint64_t seq;
+};
+
+RankPlan rank_plan(uint32_t degree);
+hipError_t rank_seed(const RankPlan& p, uint64_t start_key, uint32_t* bitmap, uint32_t* list, uint32_t* ends,
+                     hipStream_t stream);
+hipError_t rank_layer(const RankLayer& a, const PackedGenerators& gens, hipStream_t stream);
+// Up to `limit` states of the layer [lo, hi) as packed keys.
+hipError_t rank_export(const RankPlan& p, const uint32_t* list, const uint32_t* lo, const uint32_t* hi, uint64_t limit,
+                       uint64_t* keys, hipStream_t stream);
+hipError_t rank_report(const OwnerCtl* ctl, const OwnerRules& rules, LayerRecord* rec, uint64_t seq,
+                       hipStream_t stream);
+
 hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t* control, hipStream_t stream);
 hipError_t sorted_block_run(const BlockRun& run, const ActionRef& act, hipStream_t stream);
 // Zeroes the owners' counts (`words` of them from `counts`) and the first

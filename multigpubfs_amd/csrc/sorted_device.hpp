@@ -124,10 +124,12 @@ struct RunCursors {
 // `between` runs after the tile is placed in LDS and before its write-out:
 // the caller issues the next tile's loads there (v is no longer read), so
 // they are in flight during the write-out.
-template <int PER, typename BucketFn, typename BaseFn, typename BetweenFn>
+// The output may be narrower than the tile's words (Out): their low part is
+// written.
+template <int PER, typename BucketFn, typename BaseFn, typename BetweenFn, typename Out>
 __device__ __forceinline__ void route_regs(TileLds& t, const uint64_t (&v)[PER], uint32_t valid,
                                            BucketFn bkt, const RunCursors& runs, BaseFn slab_base,
-                                           uint64_t* __restrict__ out, uint32_t dump, BetweenFn between) {
+                                           Out* __restrict__ out, uint32_t dump, BetweenFn between) {
   // No branches per element: an invalid element takes its rank from the
   // lane's spare counter and is parked in the lane's slot past the tile.
   const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -194,7 +196,7 @@ __device__ __forceinline__ void route_regs(TileLds& t, const uint64_t (&v)[PER],
 #pragma unroll
       for (int u = 0; u < kRound; ++u) {
         const uint32_t j = r + threadIdx.x + u * kRouteThreads;
-        if (j < ne) out[o[u] + j] = h[u];  // 32-bit index arithmetic, wraps as intended
+        if (j < ne) out[o[u] + j] = static_cast<Out>(h[u]);  // 32-bit index arithmetic, wraps as intended
       }
     }
   } else {
@@ -202,7 +204,7 @@ __device__ __forceinline__ void route_regs(TileLds& t, const uint64_t (&v)[PER],
       const uint64_t h = t.s[j];
       const uint32_t b = bkt(h);
       const uint32_t off = t.off[b];
-      if (off != kDropRun) out[slab_base(b) + off + (j - t.lstart[b])] = h;
+      if (off != kDropRun) out[slab_base(b) + off + (j - t.lstart[b])] = static_cast<Out>(h);
     }
   }
   // No barrier here: the next tile's placement and scan come after its

@@ -23,6 +23,7 @@
 #include <algorithm>
 #include "common.hpp"
 #include "kernels.hpp"
+#include "owner_device.hpp"
 #include "sorted_device.hpp"
 #include "wide.hpp"
 
@@ -32,16 +33,6 @@ namespace {
 
 constexpr int kBlockThreads = 1024;
 constexpr uint32_t kNoBank = 3;
-
-// Nibble-packed permutations: generators by value, shift groups.
-struct NibbleAction {
-  PackedGenerators gens;
-  __device__ __forceinline__ uint32_t count() const { return gens.count; }
-  __device__ __forceinline__ uint64_t child(uint64_t key, uint32_t g) const {
-    return apply_groups(key, gens, static_cast<int>(g));
-  }
-  __device__ __forceinline__ uint32_t mask(uint32_t g) const { return gens.child_mask[g]; }
-};
 
 struct BlockLds {
   alignas(16) uint64_t table[kBlockSlots];
@@ -227,25 +218,6 @@ __global__ __launch_bounds__(kBlockThreads) void owner_begin_kernel(uint32_t* co
     c.imported = threadIdx.x == 0;
     ctl[threadIdx.x] = c;
   }
-}
-
-// How a finished layer leaves the session; every workgroup of the next
-// launch comes to the same answer from the same totals.
-__device__ __forceinline__ uint32_t owner_state(const OwnerCtl& c, const OwnerRules& rules) {
-  const uint32_t N = static_cast<uint32_t>(c.counts), children = static_cast<uint32_t>(c.counts >> 32);
-  if (c.error || N > rules.rows) return kLayerRejected;
-  if (N == 0) return kLayerEmpty;
-  const bool few = children < rules.low && !c.imported;
-  return c.spill || few || children > rules.high ? kLayerStop : kLayerNext;
-}
-
-__device__ __forceinline__ void owner_publish(const OwnerCtl& c, uint32_t state, LayerRecord* rec, uint64_t seq) {
-  rec->N = static_cast<uint32_t>(c.counts);
-  rec->children = c.counts >> 32;
-  rec->unique = c.unique;
-  rec->ticks = wall_clock64();
-  rec->state = state;
-  __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // A routing tile holds kSendItems x 512 child slots, generator-major over P

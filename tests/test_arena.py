@@ -59,3 +59,17 @@ def test_wide_keys_match_plain_actions(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "wide keys ok" in out.stdout
+
+
+def test_owner_bitmap_ranks(tmp_path):
+    """Ranks, their inverse and their owners (multigpubfs_amd/csrc/rank_owner.hip)."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not installed")
+    exe = tmp_path / "rank_check"
+    subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-std=c++17", "-O1", "-I", str(ROOT / "multigpubfs_amd" / "csrc"),
+                    str(ROOT / "tests" / "native" / "rank_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "rank ok" in out.stdout

@@ -444,3 +444,30 @@ def test_bitmap_run_to_end_at_every_tile_depth(generators):
     with NativeEngine(GraphDefinition.permutation(gens, list(range(n))), backend="permutation_bitmap") as e:
         assert e.run() == 1
         assert e.layer_sizes() == ref
+
+
+# Degrees 3 to 12 run with every workgroup owning a slice of the bitmap
+# (rank_owner.hip), others and a set capacity over one shared bitmap: the
+# smallest groups, one generator, back edges named (up to 14 generators) and
+# not (15, 16), and so many generators that the messages of a layer do not fit
+# at first (degree 9: 5,076 and 5,654 per owner, up to 12,000 and 18,000 sent).
+@pytest.mark.parametrize("capacity", [0, math.factorial(9)], ids=["owned", "shared"])
+@pytest.mark.parametrize("n,count,closed", [(2, 1, True), (3, 2, False), (4, 1, False), (5, 2, True), (7, 15, False),
+                                            (8, 16, False), (9, 7, True), (9, 16, False)])
+def test_bitmap_layer_sets_and_samples_match_oracle(n, count, closed, capacity):
+    gens = random_generators(random.Random(100 * n + count), n, count, closed)
+    start = list(range(n))[::-1]
+    ref = O.packed_bfs(n, gens, start=start, keep_keys=True)
+    with NativeEngine(GraphDefinition.permutation(gens, start), backend="permutation_bitmap", capacity=capacity) as e:
+        sizes, keys = run_all_layers(e, keep_keys=True)
+        assert sizes == ref["layers"]
+        assert keys == [sorted(k) for k in ref["keys"]]
+        e.reset()
+        assert e.advance() == (0 if len(sizes) > 1 else 1)
+        if len(sizes) > 1:
+            assert e.run() == 1
+        assert e.layer_sizes() == ref["layers"]
+        assert e.info()["total_states"] == sum(sizes)
+        assert sorted(O.pack(r) for r in e.sample(0, 10**6)) == sorted(ref["keys"][-1])
+        if len(sizes) > 1:
+            assert sorted(O.pack(r) for r in e.sample(1, 10**6)) == sorted(ref["keys"][-2])
