@@ -152,13 +152,25 @@ constexpr uint32_t kRankDegree = 12;
 struct RankPlan {
   uint32_t degree, owners, magic;  // magic: floor(2^32 / owners)
   uint32_t slice_words, list_cap;  // per owner: bitmap words (a multiple of 4), states
+  uint32_t count_stride;           // words from one owner's message counter to the next
+};
+
+// Generators over byte permutations (rank_owner.hip: child_of), each with
+// the tag of the children it makes (0: no inverse among the generators).
+struct RankGenerator {
+  uint32_t low[3], high[3], tag, pad;
+};
+struct RankGenerators {
+  uint32_t count, tagged;  // tagged: how many have a tag
+  RankGenerator of[kMaxGenerators];
 };
 
 struct RankLayer {
   RankPlan plan;
+  uint32_t slots;        // children per state: generators, or one less when each state has a tag
   uint32_t claim;        // 0: send only (the layer is in the list already)
   const uint32_t* in;    // messages of this layer: owners x in_cap
-  uint32_t* in_count;    // cleared
+  uint32_t* in_count;    // cleared (count_stride words apart)
   uint32_t in_cap;
   uint32_t* out;         // messages of the next layer
   uint32_t* out_count;
@@ -177,7 +189,8 @@ struct RankLayer {
 RankPlan rank_plan(uint32_t degree);
 hipError_t rank_seed(const RankPlan& p, uint64_t start_key, uint32_t* bitmap, uint32_t* list, uint32_t* ends,
                      hipStream_t stream);
-hipError_t rank_layer(const RankLayer& a, const PackedGenerators& gens, hipStream_t stream);
+RankGenerators rank_generators(const PackedGenerators& gens);
+hipError_t rank_layer(const RankLayer& a, const RankGenerators& gens, hipStream_t stream);
 // Up to `limit` states of the layer [lo, hi) as packed keys.
 hipError_t rank_export(const RankPlan& p, const uint32_t* list, const uint32_t* lo, const uint32_t* hi, uint64_t limit,
                        uint64_t* keys, hipStream_t stream);

@@ -36,7 +36,7 @@ class RankBitmapEngine final : public Engine {
     bitmap_.allocate(W * plan_.slice_words * 4);
     list_.allocate(W * plan_.list_cap * 4);
     // Counts of both message buffers, then the list ends, then the controls.
-    words_.allocate((2 + kEnds) * W * 4 + 16 + sizeof(OwnerCtl) * (kRing + 1));
+    words_.allocate((2 * plan_.count_stride + kEnds) * W * 4 + 16 + sizeof(OwnerCtl) * (kRing + 1));
     keys_.allocate(kKeys * 8);
     MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec_), sizeof(LayerRecord) * kRing, hipHostMallocDefault));
     std::memset(rec_, 0, sizeof(LayerRecord) * kRing);
@@ -58,7 +58,7 @@ class RankBitmapEngine final : public Engine {
   void reset() override {
     MGBFS_HIP(hipSetDevice(device_));
     const uint64_t W = plan_.owners;
-    MGBFS_HIP(zero_u32x3(bitmap_.as<uint32_t>(), W * plan_.slice_words, words_.as<uint32_t>(), (2 + kEnds) * W, nullptr,
+    MGBFS_HIP(zero_u32x3(bitmap_.as<uint32_t>(), W * plan_.slice_words, words_.as<uint32_t>(), (2 * plan_.count_stride + kEnds) * W, nullptr,
                          0, stream_));
     MGBFS_HIP(rank_seed(plan_, start_key_, bitmap_.as<uint32_t>(), list_.as<uint32_t>(), ends(0), stream_));
     layers.assign(1, 1);
@@ -113,13 +113,14 @@ class RankBitmapEngine final : public Engine {
       const std::vector<int> inv = inverse_index(gens_);
       for (uint32_t a = 0; a < gens_.count; ++a) gens_.child_tag[a] = inv[a] >= 0 ? static_cast<uint8_t>(inv[a] + 1) : 0;
     }
+    rank_gens_ = rank_generators(gens_);
     history_layers = g.inverse_closed ? 3 : 0;
     start_key_ = g.start_key();
   }
-  uint32_t* counts(uint32_t parity) { return words_.as<uint32_t>() + parity * plan_.owners; }
-  uint32_t* ends(uint64_t layer) { return words_.as<uint32_t>() + (2 + layer % kEnds) * plan_.owners; }
+  uint32_t* counts(uint32_t parity) { return words_.as<uint32_t>() + parity * plan_.count_stride * plan_.owners; }
+  uint32_t* ends(uint64_t layer) { return words_.as<uint32_t>() + (2 * plan_.count_stride + layer % kEnds) * plan_.owners; }
   OwnerCtl* ctl(uint64_t layer) {
-    const uint64_t at = ((2 + kEnds) * 4ull * plan_.owners + 15) / 16 * 16;
+    const uint64_t at = ((2 * plan_.count_stride + kEnds) * 4ull * plan_.owners + 15) / 16 * 16;
     return reinterpret_cast<OwnerCtl*>(words_.as<char>() + at) + layer % kRing;
   }
   void ensure_messages(uint32_t cap) {
@@ -136,14 +137,15 @@ class RankBitmapEngine final : public Engine {
   // Layer d is in the list: sends its children.  Its control block is the
   // one the next layer's launch reads.
   void send(uint64_t d) {
-    MGBFS_HIP(owner_begin(counts(0), 2 * plan_.owners, ctl(d), static_cast<uint32_t>(layers.back()), stream_));
+    MGBFS_HIP(owner_begin(counts(0), 2 * plan_.count_stride * plan_.owners, ctl(d), static_cast<uint32_t>(layers.back()), stream_));
     MGBFS_HIP(fill_u32(reinterpret_cast<uint32_t*>(ctl(d + 1)), 0u, sizeof(OwnerCtl) / 4, stream_));
     parity_ = 0;
     RankLayer a = layer_args(d);
     a.claim = 0;
+    a.slots = gens_.count;  // the start has no tag
     a.out = messages_[0].as<uint32_t>();
     a.out_count = counts(0);
-    MGBFS_HIP(rank_layer(a, gens_, stream_));
+    MGBFS_HIP(rank_layer(a, rank_gens_, stream_));
     sent_ = true;
   }
   // Arguments of layer d's launch (buffers of the current parity).
@@ -151,6 +153,7 @@ class RankBitmapEngine final : public Engine {
     RankLayer a{};
     a.plan = plan_;
     a.claim = 1;
+    a.slots = rank_gens_.tagged == gens_.count && gens_.count > 1 ? gens_.count - 1 : gens_.count;
     a.in = messages_[parity_].as<uint32_t>();
     a.in_count = counts(parity_);
     a.in_cap = cap_;
@@ -193,7 +196,7 @@ class RankBitmapEngine final : public Engine {
     for (uint64_t d = d0;; ++d) {
       for (; queued < target && queued <= d + kAheadLayers; ++queued) {
         const RankLayer a = layer_args(queued + 1);
-        MGBFS_HIP(rank_layer(a, gens_, stream_));
+        MGBFS_HIP(rank_layer(a, rank_gens_, stream_));
         parity_ ^= 1u;
         if (queued + 1 == target)
           MGBFS_HIP(rank_report(ctl(target), a.rules, rec_ + target % kRing, base_ + target, stream_));
@@ -251,6 +254,7 @@ class RankBitmapEngine final : public Engine {
   uint32_t n_;
   RankPlan plan_;
   PackedGenerators gens_{};
+  RankGenerators rank_gens_{};
   uint64_t start_key_ = 0, budget_ = 0;
   DeviceBuffer bitmap_, list_, words_, keys_, messages_[2];
   uint32_t cap_ = 0, parity_ = 0;  // messages per owner; the buffer holding the current layer's children
