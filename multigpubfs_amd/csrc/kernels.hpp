@@ -105,6 +105,10 @@ struct BlockRun {
 // kSlabStride entries per owner.
 constexpr uint32_t kOwnersMax = 1024;
 constexpr uint32_t kOwnersSmall = 256;
+// Words from one owner's counter to the next (side by side,
+// the reservations of all owners queue on a few cache lines: S_10 sorted 747,
+// 723, 654, 641 us at 1, 8, 16, 32 words).
+constexpr uint32_t kCountStride = 16;
 constexpr uint32_t kOwnerMean = 4600;  // children per owner at most (a slab holds kUniqueCap)
 
 // Totals of one owner layer; zeroed two launches before its own.
@@ -125,7 +129,7 @@ struct OwnerRules {
 
 struct OwnerSlabs {
   uint64_t* data;   // owners x kSlabStride entries
-  uint32_t* count;  // entries per owner
+  uint32_t* count;  // entries per owner, kCountStride words apart
 };
 
 struct OwnerImport {

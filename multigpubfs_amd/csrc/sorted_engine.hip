@@ -63,7 +63,7 @@ class SortedEngine final : public Engine {
     // per CU, prefetching the next sub-bucket's bounds, measured slower
     // (127 and 122 vs 120 ms per S13 BFS).
     unique_grid_ = 1u << kMaxBucketBits;
-    control_.allocate(kCtlOffset + sizeof(OwnerCtl) * kOwnerRing + 4 * kOwnerBuffers * kOwnersMax);
+    control_.allocate(kCtlOffset + sizeof(OwnerCtl) * kOwnerRing + 4 * kOwnerBuffers * kOwnersMax * kCountStride);
     fine_counts_.allocate(((1ull << kMaxBucketBits) + 1) * 4);
     for (int b = 0; b < 3; ++b) off_[b].allocate(((1ull << kMaxBucketBits) + 1) * 4);
     const size_t rec_bytes = sizeof(LayerRecord) * (kBlockLayers + 1);
@@ -422,7 +422,7 @@ class SortedEngine final : public Engine {
     uint32_t* counts = reinterpret_cast<uint32_t*>(ctl + kOwnerRing);
     OwnerSlabs slab[kOwnerBuffers];  // candidates 0 and 1, layers 2 + bank index
     for (uint32_t k = 0; k < kOwnerBuffers; ++k)
-      slab[k] = OwnerSlabs{owner_.as<uint64_t>() + k * entries, counts + k * kOwnersMax};
+      slab[k] = OwnerSlabs{owner_.as<uint64_t>() + k * entries, counts + k * kOwnersMax * kCountStride};
     const bool probe_prev = prev_ >= 0 && !layout_.prune;
     // 1,024 owners take 28 us where 256 take 18 (12,000 children, S_11 with
     // ten generators), so a shrinking search changes over; a new session
@@ -431,7 +431,7 @@ class SortedEngine final : public Engine {
     const OwnerRules rules{owners, rows, low, owners * kOwnerMean};
     const uint64_t seq = seq_;
     seq_ += kBlockLayers + 2;
-    MGBFS_HIP(owner_begin(counts, kOwnerBuffers * kOwnersMax, ctl, static_cast<uint32_t>(F), stream_));
+    MGBFS_HIP(owner_begin(counts, kOwnerBuffers * kOwnersMax * kCountStride, ctl, static_cast<uint32_t>(F), stream_));
     OwnerImport im{};
     im.cur = bank_[cur_].as<uint64_t>();
     im.F = static_cast<uint32_t>(F);

@@ -211,7 +211,8 @@ __global__ void stamp_record_kernel(LayerRecord* rec, uint64_t seq) {
 
 __global__ __launch_bounds__(kBlockThreads) void owner_begin_kernel(uint32_t* counts, uint32_t words, OwnerCtl* ctl,
                                                                      uint32_t F) {
-  for (uint32_t i = threadIdx.x; i < words; i += kBlockThreads) counts[i] = 0;
+  for (uint32_t i = blockIdx.x * kBlockThreads + threadIdx.x; i < words; i += gridDim.x * kBlockThreads) counts[i] = 0;
+  if (blockIdx.x) return;
   if (threadIdx.x < 2) {
     OwnerCtl c{};
     c.counts = threadIdx.x == 0 ? F : 0u;
@@ -271,7 +272,7 @@ __device__ __forceinline__ uint32_t owner_send(TileLds& t, const uint64_t* paren
                                                const OwnerSlabs& out, uint32_t* spill) {
   return send_tile(
       t, parents, count, masked, act, L, [owners](uint64_t h) { return range_index(h, owners); },
-      RunCursors{out.count, 1, kUniqueCap, spill, 1u},
+      RunCursors{out.count, kCountStride, kUniqueCap, spill, 1u},
       [](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; }, out.data, owners * kSlabStride);
 }
 
@@ -327,7 +328,7 @@ __global__ __launch_bounds__(kRouteThreads) void owner_import_kernel(OwnerImport
       v[k] = i < n ? from[i] : 0;
       valid |= i < n ? 1u << k : 0u;
     }
-    const RunCursors runs{to.count, 1, kUniqueCap, &im.ctl->error, kErrBucketCap};
+    const RunCursors runs{to.count, kCountStride, kUniqueCap, &im.ctl->error, kErrBucketCap};
     auto slab_base = [](uint32_t b) { return static_cast<uint64_t>(b) * kSlabStride; };
     auto bkt = [owners](uint64_t h) { return range_index(h, owners); };
     route_regs(t, v, valid, bkt, runs, slab_base, to.data, owners * kSlabStride, [] {});
@@ -374,8 +375,8 @@ __global__ __launch_bounds__(kRouteThreads) void owner_layer_kernel(OwnerLayer a
   uint64_t* table = reinterpret_cast<uint64_t*>(lds);
   const uint32_t f = blockIdx.x;
   const OwnerCtl before = *a.before;
-  uint32_t c = a.in.count[f];
-  const uint32_t ncur = a.cur.count[f], nprev = a.prev.data ? a.prev.count[f] : 0u;
+  uint32_t c = a.in.count[f * kCountStride];
+  const uint32_t ncur = a.cur.count[f * kCountStride], nprev = a.prev.data ? a.prev.count[f * kCountStride] : 0u;
   const uint32_t state = owner_state(before, a.rules);
   const bool run = !before.halt && state == kLayerNext;
   if (f == 0 && threadIdx.x == 0) {
@@ -391,15 +392,15 @@ __global__ __launch_bounds__(kRouteThreads) void owner_layer_kernel(OwnerLayer a
   if (c > kUniqueCap) {  // the sender flagged it; this layer cannot be selected
     if (threadIdx.x == 0) {
       atomicOr(&a.now->error, kErrBucketCap);
-      a.next.count[f] = 0;
+      a.next.count[f * kCountStride] = 0;
     }
     c = 0;
   }
   if (c == 0) {
     __syncthreads();  // every thread has read the count
     if (threadIdx.x == 0) {
-      a.in.count[f] = 0;
-      a.next.count[f] = 0;
+      a.in.count[f * kCountStride] = 0;
+      a.next.count[f * kCountStride] = 0;
     }
     return;
   }
@@ -477,8 +478,8 @@ __global__ __launch_bounds__(kRouteThreads) void owner_layer_kernel(OwnerLayer a
   if (lane == kWave - 1 && mine) atomicAdd(&made, mine);
   __syncthreads();
   if (threadIdx.x == 0) {
-    a.in.count[f] = 0;
-    a.next.count[f] = N;
+    a.in.count[f * kCountStride] = 0;
+    a.next.count[f * kCountStride] = N;
     atomicAdd(&a.now->counts, static_cast<unsigned long long>(N) | (static_cast<unsigned long long>(made) << 32));
     atomicAdd(&a.now->unique, static_cast<unsigned long long>(occupied));
   }
@@ -501,14 +502,14 @@ __global__ __launch_bounds__(kRouteThreads) void owner_export_kernel(OwnerSlabs 
   uint64_t* to = second ? prev_bank : bank;
   uint32_t* offsets = second ? prev_off : off;
   uint32_t before = 0;
-  for (uint32_t j = threadIdx.x; j < f; j += kRouteThreads) before += s.count[j];
+  for (uint32_t j = threadIdx.x; j < f; j += kRouteThreads) before += s.count[j * kCountStride];
   before = wave_incl_scan(before);
   if ((threadIdx.x & (kWave - 1)) == kWave - 1) sums[threadIdx.x / kWave] = before;
   __syncthreads();
   before = 0;
 #pragma unroll
   for (uint32_t w = 0; w < kRouteThreads / kWave; ++w) before += sums[w];
-  const uint32_t n = s.count[f];
+  const uint32_t n = s.count[f * kCountStride];
   if (threadIdx.x == 0) {
     offsets[f] = before;
     if (f + 1 == owners) offsets[owners] = before + n;
@@ -548,7 +549,7 @@ hipError_t stamp_record(LayerRecord* rec, uint64_t seq, hipStream_t stream) {
 }
 
 hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream) {
-  hipLaunchKernelGGL(owner_begin_kernel, dim3(1), dim3(kBlockThreads), 0, stream, counts, words, ctl, F);
+  hipLaunchKernelGGL(owner_begin_kernel, dim3(std::min<uint32_t>(16, (words + 4 * kBlockThreads - 1) / (4 * kBlockThreads))), dim3(kBlockThreads), 0, stream, counts, words, ctl, F);
   return hipGetLastError();
 }
 
