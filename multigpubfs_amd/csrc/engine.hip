@@ -548,11 +548,15 @@ static uint32_t choose_backend(const Graph& g, uint32_t requested) {
 
 // The sorted backend, handing the run to the segmented backend when a
 // layer exceeds its limits (its last two layers become the segmented
-// backend's banks; the sorted engine and its memory are released).
+// backend's banks; the sorted engine and its memory are released).  Where
+// the library picks the backend, permutations of degree 8 to 12 run by
+// owners of the bitmap instead (rank_bitmap_for_auto), and what they report
+// is the bitmap backend's.
 class HandoverEngine final : public Engine {
  public:
   HandoverEngine(const Graph& g, const mgbfs_engine_options& o) : g_(g), o_(o) {
-    inner_.reset(make_sorted_engine(g, o));
+    by_owners_ = rank_bitmap_for_auto(g, o);
+    inner_.reset(by_owners_ ? make_rank_bitmap_engine(g, o) : make_sorted_engine(g, o));
     mirror();
   }
   int advance(uint64_t* next_count, uint32_t* fatal) override {
@@ -585,7 +589,18 @@ class HandoverEngine final : public Engine {
   }
   void rebind(const Graph& g) override {
     if (handovers_) throw std::runtime_error("ENGINE_REBIND_AFTER_HANDOVER");
-    inner_->rebind(g);
+    if (!by_owners_) {
+      inner_->rebind(g);
+    } else {
+      if (g.elements != g_.elements || !g.packable() || !g.inverse_closed) throw std::runtime_error("ENGINE_REBIND_SHAPE");
+      by_owners_ = rank_bitmap_for_auto(g, o_);
+      if (by_owners_) {
+        inner_->rebind(g);
+      } else {  // repeated labels: sorted, as any graph of the degree may be
+        std::unique_ptr<Engine> next(make_sorted_engine(g, o_));
+        inner_ = std::move(next);
+      }
+    }
     g_ = g;
     mirror();
   }
@@ -641,6 +656,7 @@ class HandoverEngine final : public Engine {
   std::unique_ptr<Engine> inner_;
   Carried carried_;
   uint32_t handovers_ = 0;
+  bool by_owners_ = false;
 };
 
 // The segmented backend on graphs whose states are one packed word

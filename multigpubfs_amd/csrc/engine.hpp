@@ -130,6 +130,7 @@ Engine* make_bitmap_engine(const Graph& g, const mgbfs_engine_options& o);
 // The bitmap backend by owners (rank_engine.hip) and what it takes: degree 3
 // to 12, no row capacity asked for, memory for its lists and messages.
 bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o);
+bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o);
 Engine* make_rank_bitmap_engine(const Graph& g, const mgbfs_engine_options& o);
 struct WideCode;
 // wide: packed code of a graph outside the nibble encoding (null: none).

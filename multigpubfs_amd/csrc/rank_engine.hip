@@ -28,7 +28,6 @@ class RankBitmapEngine final : public Engine {
     set_graph(g);
     MGBFS_HIP(hipSetDevice(device_));
     MGBFS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-    budget_ = vram_budget(o);
     int khz = 0;
     MGBFS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
     tick_seconds_ = khz > 0 ? 1e-3 / khz : 0.0;
@@ -40,6 +39,7 @@ class RankBitmapEngine final : public Engine {
     keys_.allocate(kKeys * 8);
     MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec_), sizeof(LayerRecord) * kRing, hipHostMallocDefault));
     std::memset(rec_, 0, sizeof(LayerRecord) * kRing);
+    ensure_messages(first_cap(plan_, g.generators));
     reset();
   }
   ~RankBitmapEngine() override {
@@ -49,10 +49,10 @@ class RankBitmapEngine final : public Engine {
     if (stream_) (void)hipStreamDestroy(stream_);
   }
 
-  // Device bytes of the bitmap, the list and the first message buffers.
-  static uint64_t bytes_for(const Graph& g) {
+  // Device bytes with message buffers that hold every layer.
+  static uint64_t most_bytes(const Graph& g) {
     const RankPlan p = rank_plan(g.elements);
-    return p.owners * (4ull * p.slice_words + 4ull * p.list_cap + 8ull * first_cap(p, g.generators)) + (1u << 20);
+    return p.owners * (4ull * p.slice_words + 4ull * p.list_cap + 8ull * last_cap(p, g.generators)) + (1u << 20);
   }
 
   void reset() override {
@@ -105,7 +105,12 @@ class RankBitmapEngine final : public Engine {
   // Messages per owner at first: a fifth of all children there can be (the
   // widest LRX layer sends 15% of them).
   static uint32_t first_cap(const RankPlan& p, uint32_t generators) {
-    return static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators / 5 + 1027) / 4 * 4);
+    return std::min(last_cap(p, generators),
+                    static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators / 5 + 1027) / 4 * 4));
+  }
+  // ... and at most: a state is a child of `generators` states.
+  static uint32_t last_cap(const RankPlan& p, uint32_t generators) {
+    return static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(p.list_cap) * generators + 3, 1u << 30) / 4 * 4);
   }
   void set_graph(const Graph& g) {
     gens_ = g.packed_generators();
@@ -126,8 +131,6 @@ class RankBitmapEngine final : public Engine {
   void ensure_messages(uint32_t cap) {
     if (cap <= cap_) return;
     const uint64_t entries = static_cast<uint64_t>(plan_.owners) * cap + kRouteDump;
-    if (device_bytes - messages_[0].bytes() - messages_[1].bytes() + 8 * entries > budget_)
-      throw std::runtime_error("BITMAP_VRAM_CAPACITY");
     MGBFS_HIP(hipStreamSynchronize(stream_));
     for (auto& m : messages_) m.release();
     for (auto& m : messages_) m.allocate(entries * 4);
@@ -179,8 +182,9 @@ class RankBitmapEngine final : public Engine {
     while (true) {
       const int s = session(target);
       if (s != kSendAgain) return s;
-      if (cap_ > (1u << 30)) throw std::runtime_error("BITMAP_VRAM_CAPACITY");
-      ensure_messages(2 * cap_);
+      const uint32_t last = last_cap(plan_, gens_.count);
+      if (cap_ >= last) throw std::runtime_error("BITMAP_MESSAGES");
+      ensure_messages(std::min(2 * cap_, last));
       if (layers.size() - 1 == target) return MGBFS_LAYER;  // its children are sent by the next call
     }
   }
@@ -255,7 +259,7 @@ class RankBitmapEngine final : public Engine {
   RankPlan plan_;
   PackedGenerators gens_{};
   RankGenerators rank_gens_{};
-  uint64_t start_key_ = 0, budget_ = 0;
+  uint64_t start_key_ = 0;
   DeviceBuffer bitmap_, list_, words_, keys_, messages_[2];
   uint32_t cap_ = 0, parity_ = 0;  // messages per owner; the buffer holding the current layer's children
   bool sent_ = false;              // ... which are complete
@@ -267,12 +271,28 @@ class RankBitmapEngine final : public Engine {
 // All degrees that ranks and slices are made for: faster from the smallest to
 // degree 12 (figures in rank_owner.hip).  A capacity bounds the rows of a
 // layer and a message buffer is not one, so a set capacity keeps the shared
-// bitmap; so does a budget that has no room for the messages to double
-// (degree 12: 4.3 GB and again as much).
+// bitmap; so does a budget that does not hold the messages of every layer
+// (degree 12 with three generators: 13.5 GB, of which 4.3 are used).
 bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o) {
   if (g.elements < 3 || g.elements > kRankDegree || o.capacity || g.generators > kMaxGenerators) return false;
   MGBFS_HIP(hipSetDevice(o.device));
-  return 2 * RankBitmapEngine::bytes_for(g) <= vram_budget(o);
+  return RankBitmapEngine::most_bytes(g) <= vram_budget(o);
+}
+
+// Inverse-closed graphs whose backend the library picks run by owners of the
+// bitmap from degree 8 on (sorted -> owners, warm: LRX 8 0.36 -> 0.23 ms, 9
+// 0.47 -> 0.31, 10 0.65 -> 0.48, 11 2.9 -> 1.3, 12 13.7 -> 10.5; Coxeter 11
+// 5.5 -> 3.0, 12 96 -> 33; four random generators with inverses, 11 4.9 ->
+// 1.8); below, the sorted backend's single workgroup does (LRX 7 0.145
+// against 0.162 ms, 4 0.036 against 0.054).
+// A set that is only declared closed keeps the sorted backend's retention.
+bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o) {
+  if (o.backend != MGBFS_BACKEND_AUTO || !g.inverse_closed || g.elements < 8 || !g.packable() || !g.distinct_perm() ||
+      (o.flags & ~MGBFS_FLAG_MAX_CAPACITY) || !rank_bitmap_takes(g, o))
+    return false;
+  for (int at : inverse_index(g.packed_generators()))
+    if (at < 0) return false;
+  return true;
 }
 
 Engine* make_rank_bitmap_engine(const Graph& g, const mgbfs_engine_options& o) { return new RankBitmapEngine(g, o); }

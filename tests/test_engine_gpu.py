@@ -471,3 +471,24 @@ def test_bitmap_layer_sets_and_samples_match_oracle(n, count, closed, capacity):
         assert sorted(O.pack(r) for r in e.sample(0, 10**6)) == sorted(ref["keys"][-1])
         if len(sizes) > 1:
             assert sorted(O.pack(r) for r in e.sample(1, 10**6)) == sorted(ref["keys"][-2])
+
+
+# Left to choose, the library runs inverse-closed permutations of degree 8 to
+# 12 by owners of the bitmap; a rebound engine still takes what the sorted
+# backend takes (repeated labels) and refuses what it refuses.
+@pytest.mark.parametrize("n,budget,name", [(7, 0, "sorted"), (8, 0, "permutation_bitmap"), (10, 0, "permutation_bitmap"),
+                                           (11, 1 << 30, "sorted")])
+def test_auto_backend_by_degree_and_budget(n, budget, name):
+    gens = O.lrx_generators(n)
+    with NativeEngine(lrx(n), vram_budget=budget) as e:
+        assert e.backend_name == NAMES[name]
+        assert e.run() == 1 and e.layer_sizes() == O.packed_bfs(n)["layers"]
+        e.rebind(GraphDefinition.permutation(gens[::-1], list(range(n))))
+        assert e.run() == 1 and e.layer_sizes() == O.packed_bfs(n)["layers"]
+        start = [0, 1] * (n // 2) + [2] * (n % 2)
+        graph = {"action": {"kind": "permutation", "degree": n, "generators": gens}, "start": start}
+        with pytest.raises(RuntimeError):
+            e.rebind(GraphDefinition.permutation([gens[0], gens[2]], list(range(n))))
+        e.rebind(GraphDefinition.permutation(gens, start))
+        assert e.run() == 1 and e.backend_name == NAMES["sorted"]
+        assert e.layer_sizes() == [len(x) for x in O.c_exact_layers(graph, math.factorial(n))]
