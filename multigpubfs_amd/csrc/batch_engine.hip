@@ -12,6 +12,7 @@
 #include "batch.hpp"
 #include "engine.hpp"
 #include "kernels.hpp"
+#include "rank_run.hpp"
 
 namespace mgbfs {
 
@@ -109,11 +110,28 @@ struct BatchPlan {
   uint32_t max_layers = kDefaultMaxLayers;
 };
 
+// A bitmap instance run by owners of the bitmap (rank_run.hpp) in its slot's
+// block, beside the graph that runs the others.  Large degrees only: their
+// layers fill the chip, and no claim is a global atomic (alone, LRX of
+// degree 12 33 -> 10.5 ms, 11 4.8 -> 1.3 ms).  Many smaller instances are
+// better off sharing launches: 256 random sets of degree 9 and 10 take 42 ms
+// in the graph and would take 55 ms one after the other.  (Twenty mixed jobs
+// of degree 8 to 12 and SL(2, Z_p): 94.5 -> 51.8 ms.)
+constexpr uint32_t kOwnedDegree = 11;
+
+struct OwnedInstance {
+  explicit OwnedInstance(uint32_t degree) : run(degree) {}
+  RankRun run;
+  bool started = false, outgrown = false;
+  uint32_t status = kInstActive, error = 0;
+};
+
 class BatchEngine {
  public:
   BatchEngine(const mgbfs_batch_options& o) : device_(o.device) {
     MGBFS_HIP(hipSetDevice(device_));
     MGBFS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+    MGBFS_HIP(hipStreamCreateWithFlags(&owned_stream_, hipStreamNonBlocking));
     slots_n_ = o.max_slots ? std::min(o.max_slots, kBatchMaxSlots) : 256;
     budget_ = o.vram_budget;
     if (!budget_) {
@@ -152,11 +170,13 @@ class BatchEngine {
     std::memset(host_inst_.data(), 0, sizeof(BatchInstance) * slots_n_);
     MGBFS_HIP(hipMemcpy(inst_.as<void>(), host_inst_.data(), sizeof(BatchInstance) * slots_n_, hipMemcpyHostToDevice));
     slots_.resize(slots_n_);
+    owned_.resize(slots_n_);
     capture();
   }
   ~BatchEngine() {
     (void)hipSetDevice(device_);
     if (stream_) (void)hipStreamSynchronize(stream_);
+    if (owned_stream_) (void)hipStreamSynchronize(owned_stream_);
     if (exec_) (void)hipGraphExecDestroy(exec_);
     if (graph_) (void)hipGraphDestroy(graph_);
     if (host_flag_) (void)hipHostFree(host_flag_);
@@ -167,6 +187,7 @@ class BatchEngine {
     slots_.clear();
     arena_.trim();
     if (stream_) (void)hipStreamDestroy(stream_);
+    if (owned_stream_) (void)hipStreamDestroy(owned_stream_);
   }
 
   // Planned footprint (the admission unit) and the visited-set choice.
@@ -261,11 +282,17 @@ class BatchEngine {
   // all), planned layer capacity and restarts after an outgrown layer.
   void instance_info(int32_t slot, uint32_t& visited, uint32_t& history, uint64_t& cap, uint32_t& restarts) const {
     check_slot(slot);
+    restarts = jobs_[slot].restarts;
+    if (owned_[slot]) {
+      visited = 1;
+      history = 0;
+      cap = state_space_bound(jobs_[slot].graph);
+      return;
+    }
     const BatchInstance& d = host_inst_[slot];
     visited = d.visited == kVisBitmap ? 1 : 2;
     history = d.rolling ? 3 : 0;
     cap = d.cap;
-    restarts = jobs_[slot].restarts;
   }
 
   // Lays out a slot's block (frontiers, layer sizes, visited set) from its
@@ -275,7 +302,50 @@ class BatchEngine {
     Slot& sl = slots_[slot];
     const uint64_t keys_bytes = arena_round(p.cap * 8), sizes_bytes = arena_round(8ull * p.max_layers);
     sl.block = arena_.take(2 * keys_bytes + sizes_bytes + p.visited_bytes, budget_);
-    char* base = sl.block.ptr;
+    sl.used = true;
+    sl.reported = false;
+    sl.planned = p.bytes;
+    used_ += p.bytes;
+    kinds_[slot] = g.kind;
+    rows_[slot] = g.rows;
+    cols_[slot] = g.cols;
+    if (!install_owned(slot, p)) install_shared(slot, p);
+  }
+
+  // The slot's block as bitmap, list, words and, with what is left, two
+  // message buffers of at least a message per state each; false where that
+  // does not fit or the graph is not for owners.
+  bool install_owned(int32_t slot, const BatchPlan& p) {
+    const Graph& g = jobs_[slot].graph;
+    if (p.visited != kVisBitmap || g.elements < kOwnedDegree || g.elements > kRankDegree) return false;
+    auto o = std::make_unique<OwnedInstance>(g.elements);
+    const RankPlan& rp = o->run.plan;
+    const Block& block = slots_[slot].block;
+    uint64_t at = 0;
+    auto part = [&](uint64_t bytes) {
+      const uint64_t start = at;
+      at += arena_round(bytes);
+      return reinterpret_cast<uint32_t*>(block.ptr + start);
+    };
+    RankMemory& m = o->run.memory;
+    m.bitmap = part(4ull * rp.owners * rp.slice_words);
+    m.list = part(4ull * rp.owners * rp.list_cap);
+    m.words = part(RankRun::words_bytes(rp));
+    const uint64_t least = 4 * (static_cast<uint64_t>(rp.owners) * rp.list_cap + kRouteDump) + 2 * kArenaAlign;
+    if (block.bytes < at + 2 * least) return false;
+    const uint64_t each = (block.bytes - at) / 2 / kArenaAlign * kArenaAlign;
+    m.cap = static_cast<uint32_t>(std::min<uint64_t>((each / 4 - kRouteDump) / rp.owners,
+                                                     RankRun::last_cap(rp, g.generators)) / 4 * 4);
+    for (uint32_t*& x : m.messages) x = part(each);
+    o->run.set_graph(g);
+    owned_[slot] = std::move(o);
+    return true;
+  }
+
+  void install_shared(int32_t slot, const BatchPlan& p) {
+    const Graph& g = jobs_[slot].graph;
+    const uint64_t keys_bytes = arena_round(p.cap * 8), sizes_bytes = arena_round(8ull * p.max_layers);
+    char* base = slots_[slot].block.ptr;
     BatchInstance& d = host_inst_[slot];
     std::memset(&d, 0, sizeof d);
     d.front = reinterpret_cast<uint64_t*>(base);
@@ -328,13 +398,6 @@ class BatchEngine {
     // by the next flush(), which the next step runs before its graph.
     pending_[slot] = kInstallSeed;
     pending_key_[slot] = start_key;
-    sl.used = true;
-    sl.reported = false;
-    sl.planned = p.bytes;
-    used_ += p.bytes;
-    kinds_[slot] = g.kind;
-    rows_[slot] = g.rows;
-    cols_[slot] = g.cols;
   }
 
   // Runs up to `layers` layers of every active instance; returns how many
@@ -344,14 +407,48 @@ class BatchEngine {
     const uint32_t launches = std::max<uint32_t>(1, (layers + layers_per_graph_ - 1) / layers_per_graph_);
     flush();
     for (uint32_t k = 0; k < launches; ++k) MGBFS_HIP(hipGraphLaunch(exec_, stream_));
+    for (uint32_t s = 0; s < slots_n_; ++s)
+      if (owned_[s] && (owned_[s]->status & kInstActive)) run_owned(s, launches * layers_per_graph_);
     refresh();
     uint32_t active = 0;
     for (uint32_t s = 0; s < slots_n_; ++s) {
       if (!slots_[s].used) continue;
+      if (owned_[s]) {
+        if (owned_[s]->status & kInstActive) ++active;
+        if (!owned_[s]->outgrown) continue;
+        const Job& job = jobs_[s];
+        owned_[s].reset();
+        install_shared(static_cast<int32_t>(s), plan_with(job.graph, job.visited, job.max_layers, false, 1));
+        continue;
+      }
       if (host_inst_[s].status & kInstDone) restart_if_outgrown(s);
       if ((host_inst_[s].status & kInstActive) || pending_[s] == kInstallSeed) ++active;
     }
     return active;
+  }
+
+  // Up to `most` layers of an owned instance.  One whose messages do not fit
+  // the block starts over in the graph, in the same block.
+  void run_owned(uint32_t s, uint32_t most) {
+    OwnedInstance& o = *owned_[s];
+    RankRun& run = o.run;
+    const uint32_t limit = jobs_[s].max_layers ? jobs_[s].max_layers : kDefaultMaxLayers;
+    if (!o.started) run.start(owned_stream_);
+    o.started = true;
+    // A layer past the last that is allowed is an error, and is not listed.
+    const uint64_t target = std::min<uint64_t>(run.layers.size() - 1 + most, limit);
+    const int r = run.run(target, records_, owned_stream_);
+    if (r == MGBFS_LAYER && run.layers.size() <= limit) return;
+    MGBFS_HIP(hipStreamSynchronize(owned_stream_));  // launches queued past the end
+    if (r == RankRun::kSendAgain && run.layers.size() <= limit) {
+      o.outgrown = true;  // step() moves it to the graph
+      return;
+    }
+    if (run.layers.size() > limit) {
+      run.layers.resize(limit);
+      o.error |= kErrCount;
+    }
+    o.status = kInstDone;
   }
 
   // A rolling instance whose layer outgrew its planned capacity (next
@@ -382,16 +479,27 @@ class BatchEngine {
   std::vector<int32_t> poll(uint32_t limit) {
     std::vector<int32_t> out;
     for (uint32_t s = 0; s < slots_n_ && out.size() < limit; ++s)
-      if (slots_[s].used && !slots_[s].reported && (host_inst_[s].status & kInstDone)) {
+      if (slots_[s].used && !slots_[s].reported &&
+          ((owned_[s] ? owned_[s]->status : host_inst_[s].status) & kInstDone)) {
         slots_[s].reported = true;
         out.push_back(static_cast<int32_t>(s));
       }
-    gather(out);
+    std::vector<int32_t> shared;
+    for (int32_t s : out)
+      if (!owned_[s]) shared.push_back(s);
+    gather(shared);
     return out;
   }
 
   void result(int32_t slot, std::vector<uint64_t>& sizes, uint32_t& status, uint32_t& error) {
     check_slot(slot);
+    if (owned_[slot]) {
+      const OwnedInstance& o = *owned_[slot];
+      sizes = o.started ? o.run.layers : std::vector<uint64_t>(1, 1);
+      status = o.status;
+      error = o.error;
+      return;
+    }
     const BatchInstance& d = host_inst_[slot];
     if (finished_[slot].ready) {
       sizes = finished_[slot].sizes;
@@ -406,6 +514,10 @@ class BatchEngine {
   // Current-layer states of a slot as int64 rows (at most limit).
   void sample(int32_t slot, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) {
     check_slot(slot);
+    if (owned_[slot]) {
+      sample_owned(slot, limit, rows, count);
+      return;
+    }
     const BatchInstance& d = host_inst_[slot];
     count = std::min<uint64_t>(limit, d.count);
     std::vector<uint64_t> keys(count);
@@ -423,11 +535,15 @@ class BatchEngine {
     check_slot(slot);
     MGBFS_HIP(hipSetDevice(device_));
     Slot& sl = slots_[slot];
-    BatchInstance& d = host_inst_[slot];
-    std::memset(&d, 0, sizeof d);
-    // The cleared descriptor is installed by the next flush, before any
-    // graph reads descriptors again, so the range can be reused at once.
-    pending_[slot] = kInstallOnly;
+    if (owned_[slot]) {
+      MGBFS_HIP(hipStreamSynchronize(owned_stream_));
+      owned_[slot].reset();  // its descriptor is clear
+    } else {
+      // The cleared descriptor is installed by the next flush, before any
+      // graph reads descriptors again, so the range can be reused at once.
+      std::memset(&host_inst_[slot], 0, sizeof(BatchInstance));
+      pending_[slot] = kInstallOnly;
+    }
     arena_.give(sl.block, budget_);
     used_ -= sl.planned;
     sl = Slot{};
@@ -440,6 +556,24 @@ class BatchEngine {
   uint32_t slots() const { return slots_n_; }
 
  private:
+  void sample_owned(int32_t slot, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) {
+    OwnedInstance& o = *owned_[slot];
+    if (!o.started) o.run.start(owned_stream_);
+    o.started = true;
+    count = std::min<uint64_t>(limit, o.run.layers.back());
+    std::vector<uint64_t> keys(count);
+    DeviceBuffer out;
+    if (count) {
+      out.allocate(8 * count);
+      o.run.export_layer(0, count, out.as<uint64_t>(), owned_stream_);
+      MGBFS_HIP(hipMemcpyAsync(keys.data(), out.as<void>(), 8 * count, hipMemcpyDeviceToHost, owned_stream_));
+      MGBFS_HIP(hipStreamSynchronize(owned_stream_));
+    }
+    const uint32_t n = o.run.plan.degree;
+    rows.assign(count * n, 0);
+    for (uint64_t r = 0; r < count; ++r)
+      for (uint32_t e = 0; e < n; ++e) rows[r * n + e] = static_cast<int64_t>((keys[r] >> (4 * e)) & 15u);
+  }
   void check_slot(int32_t slot) const {
     if (slot < 0 || static_cast<uint32_t>(slot) >= slots_n_ || !slots_[slot].used)
       throw std::runtime_error("BATCH_SLOT");
@@ -549,7 +683,9 @@ class BatchEngine {
   };
 
   int device_ = 0;
-  hipStream_t stream_ = nullptr;
+  hipStream_t stream_ = nullptr, owned_stream_ = nullptr;
+  RankRecords records_;
+  std::vector<std::unique_ptr<OwnedInstance>> owned_;  // per slot: null for instances in the graph
   uint32_t slots_n_ = 0, grid_ = 0, clear_grid_ = 0, layers_per_graph_ = kLayersPerGraph;
   uint32_t threads_ = 256, hash_load_pct_ = 50, layer_pct_ = 30, bitmap_bias_permille_ = 1000;
   uint32_t history_ = 0;

@@ -1,28 +1,158 @@
-// Host runtime of the permutation bitmap by owners (rank_owner.hip): the
-// bitmap backend for degrees 3 to 12 when no row capacity is asked for.
-// Layers are queued ahead of the host, which follows their records; a full
-// message slab stops the queue after its layer, and the host sends that
-// layer's children again with twice the room.
+// Host runtime of the permutation bitmap by owners (rank_owner.hip).
+// RankRun: one search in memory that its owner gives it; layers are queued
+// ahead of the host, which follows their records, and a full message slab
+// stops the queue after its layer.  RankBitmapEngine: the bitmap backend for
+// degrees 3 to 12 when no row capacity is asked for; after a full slab it
+// sends that layer's children again with twice the room.
 #include <algorithm>
 #include <cstring>
 #include <vector>
 #include "engine.hpp"
 #include "kernels.hpp"
+#include "rank_run.hpp"
 
 namespace mgbfs {
 
-namespace {
+// ------------------------------------------------------------ one search
 
-constexpr uint32_t kRing = 64;   // control blocks and records
-constexpr uint32_t kAheadLayers = 4;
-constexpr uint32_t kEnds = 4;    // list ends kept: of the last layers
-constexpr int kSendAgain = -1;
+RankRecords::RankRecords() {
+  MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec), sizeof(LayerRecord) * kRing, hipHostMallocDefault));
+  std::memset(rec, 0, sizeof(LayerRecord) * kRing);
+}
+RankRecords::~RankRecords() {
+  if (rec) (void)hipHostFree(rec);
+}
 
-}  // namespace
+uint64_t RankRun::words_bytes(const RankPlan& p) {
+  return (2 * p.count_stride + kEnds) * 4ull * p.owners + 16 + sizeof(OwnerCtl) * (RankRecords::kRing + 1);
+}
+
+uint32_t RankRun::first_cap(const RankPlan& p, uint32_t generators) {
+  return std::min(last_cap(p, generators),
+                  static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators / 5 + 1027) / 4 * 4));
+}
+uint32_t RankRun::last_cap(const RankPlan& p, uint32_t generators) {
+  return static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(p.list_cap) * generators + 3, 1u << 30) / 4 * 4);
+}
+
+void RankRun::set_graph(const Graph& g) {
+  PackedGenerators gens = g.packed_generators();
+  if (gens.count <= 14) {
+    const std::vector<int> inv = inverse_index(gens);
+    for (uint32_t a = 0; a < gens.count; ++a) gens.child_tag[a] = inv[a] >= 0 ? static_cast<uint8_t>(inv[a] + 1) : 0;
+  }
+  gens_ = rank_generators(gens);
+  start_key_ = g.start_key();
+}
+
+void RankRun::start(hipStream_t stream) {
+  const uint64_t W = plan.owners;
+  MGBFS_HIP(zero_u32x3(memory.bitmap, W * plan.slice_words, memory.words, (2 * plan.count_stride + kEnds) * W, nullptr, 0,
+                       stream));
+  MGBFS_HIP(rank_seed(plan, start_key_, memory.bitmap, memory.list, ends(0), stream));
+  layers.assign(1, 1);
+  sent_ = false;
+  seconds = 0.0;
+}
+
+OwnerCtl* RankRun::ctl(uint64_t layer) {
+  const uint64_t at = ((2 * plan.count_stride + kEnds) * 4ull * plan.owners + 15) / 16 * 16;
+  return reinterpret_cast<OwnerCtl*>(reinterpret_cast<char*>(memory.words) + at) + layer % RankRecords::kRing;
+}
+
+// Layer d is in the list: sends its children.  Its control block is the
+// one the next layer's launch reads.
+void RankRun::send(uint64_t d, hipStream_t stream) {
+  MGBFS_HIP(owner_begin(counts(0), 2 * plan.count_stride * plan.owners, ctl(d), static_cast<uint32_t>(layers.back()), stream));
+  MGBFS_HIP(fill_u32(reinterpret_cast<uint32_t*>(ctl(d + 1)), 0u, sizeof(OwnerCtl) / 4, stream));
+  parity_ = 0;
+  RankLayer a = layer_args(d, nullptr, 0);
+  a.claim = 0;
+  a.slots = gens_.count;  // the start has no tag
+  a.out = memory.messages[0];
+  a.out_count = counts(0);
+  MGBFS_HIP(rank_layer(a, gens_, stream));
+  sent_ = true;
+}
+
+// Arguments of layer d's launch (buffers of the current parity).
+RankLayer RankRun::layer_args(uint64_t d, LayerRecord* rec, uint64_t seq) {
+  RankLayer a{};
+  a.plan = plan;
+  a.claim = 1;
+  a.slots = gens_.tagged == gens_.count && gens_.count > 1 ? gens_.count - 1 : gens_.count;
+  a.in = memory.messages[parity_];
+  a.in_count = counts(parity_);
+  a.in_cap = memory.cap;
+  a.out = memory.messages[parity_ ^ 1u];
+  a.out_count = counts(parity_ ^ 1u);
+  a.out_cap = memory.cap;
+  a.bitmap = memory.bitmap;
+  a.list = memory.list;
+  a.ends_before = d ? ends(d - 1) : ends(kEnds - 1);  // zeros before the start layer
+  a.ends_now = ends(d);
+  a.before = d ? ctl(d - 1) : nullptr;
+  a.now = ctl(d);
+  a.after = ctl(d + 1);
+  a.rules = OwnerRules{plan.owners, ~0u, 0u, ~0u};
+  a.rec = rec;
+  a.seq = seq;
+  return a;
+}
+
+// The record of layer d, numbered base + d, is written by the launch of
+// layer d + 1, or by a report after the last.
+int RankRun::run(uint64_t target, RankRecords& records, hipStream_t stream) {
+  constexpr uint32_t kRing = RankRecords::kRing;
+  const uint64_t d0 = layers.size() - 1, base = records.base += 1ull << 32;
+  auto rec = [&](uint64_t d) { return records.rec + d % kRing; };
+  if (!sent_) send(d0, stream);
+  uint64_t queued = d0, ticks = 0;
+  for (uint64_t d = d0;; ++d) {
+    for (; queued < target && queued <= d + kAheadLayers; ++queued) {
+      const RankLayer a = layer_args(queued + 1, rec(queued), base + queued);
+      MGBFS_HIP(rank_layer(a, gens_, stream));
+      parity_ ^= 1u;
+      if (queued + 1 == target) MGBFS_HIP(rank_report(ctl(target), a.rules, rec(target), base + target, stream));
+    }
+    const LayerRecord& got = await(*rec(d), base + d, stream);
+    if (d != d0) {
+      seconds += static_cast<double>(got.ticks - ticks) * tick_seconds;
+      if (got.state == kLayerRejected) throw std::runtime_error("BITMAP_LAYER");
+      if (got.state == kLayerEmpty) return MGBFS_COMPLETE;
+      layers.push_back(got.N);
+    }
+    ticks = got.ticks;
+    if (got.state == kLayerStop) {
+      sent_ = false;
+      return kSendAgain;
+    }
+    if (d == target) return MGBFS_LAYER;
+  }
+}
+
+const LayerRecord& RankRun::await(const LayerRecord& rec, uint64_t seq, hipStream_t stream) {
+  auto there = [&] { return __atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) == seq; };
+  while (true) {
+    for (uint32_t spin = 0; spin < (1u << 18); ++spin)
+      if (there()) return rec;
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) continue;
+    MGBFS_HIP(e);
+    if (!there()) throw std::runtime_error("BITMAP_LAYER_RECORD");
+  }
+}
+
+void RankRun::export_layer(uint64_t back, uint64_t limit, uint64_t* keys, hipStream_t stream) {
+  const uint64_t d = layers.size() - 1 - back;
+  MGBFS_HIP(rank_export(plan, memory.list, d ? ends(d - 1) : ends(kEnds - 1), ends(d), limit, keys, stream));
+}
+
+// ------------------------------------------------------------ backend
 
 class RankBitmapEngine final : public Engine {
  public:
-  RankBitmapEngine(const Graph& g, const mgbfs_engine_options& o) : n_(g.elements), plan_(rank_plan(g.elements)) {
+  RankBitmapEngine(const Graph& g, const mgbfs_engine_options& o) : n_(g.elements), run_(g.elements) {
     device_ = o.device;
     backend = MGBFS_BACKEND_BITMAP;
     set_graph(g);
@@ -30,45 +160,39 @@ class RankBitmapEngine final : public Engine {
     MGBFS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     int khz = 0;
     MGBFS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
-    tick_seconds_ = khz > 0 ? 1e-3 / khz : 0.0;
-    const uint64_t W = plan_.owners;
-    bitmap_.allocate(W * plan_.slice_words * 4);
-    list_.allocate(W * plan_.list_cap * 4);
-    // Counts of both message buffers, then the list ends, then the controls.
-    words_.allocate((2 * plan_.count_stride + kEnds) * W * 4 + 16 + sizeof(OwnerCtl) * (kRing + 1));
+    run_.tick_seconds = khz > 0 ? 1e-3 / khz : 0.0;
+    const RankPlan& p = run_.plan;
+    bitmap_.allocate(4ull * p.owners * p.slice_words);
+    list_.allocate(4ull * p.owners * p.list_cap);
+    words_.allocate(RankRun::words_bytes(p));
     keys_.allocate(kKeys * 8);
-    MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec_), sizeof(LayerRecord) * kRing, hipHostMallocDefault));
-    std::memset(rec_, 0, sizeof(LayerRecord) * kRing);
-    ensure_messages(first_cap(plan_, g.generators));
+    run_.memory.bitmap = bitmap_.as<uint32_t>();
+    run_.memory.list = list_.as<uint32_t>();
+    run_.memory.words = words_.as<uint32_t>();
+    ensure_messages(RankRun::first_cap(p, g.generators));
     reset();
   }
   ~RankBitmapEngine() override {
     (void)hipSetDevice(device_);
     if (stream_) (void)hipStreamSynchronize(stream_);
-    if (rec_) (void)hipHostFree(rec_);
     if (stream_) (void)hipStreamDestroy(stream_);
   }
 
   // Device bytes with message buffers that hold every layer.
   static uint64_t most_bytes(const Graph& g) {
     const RankPlan p = rank_plan(g.elements);
-    return p.owners * (4ull * p.slice_words + 4ull * p.list_cap + 8ull * last_cap(p, g.generators)) + (1u << 20);
+    return p.owners * (4ull * p.slice_words + 4ull * p.list_cap + 8ull * RankRun::last_cap(p, g.generators)) + (1u << 20);
   }
 
   void reset() override {
     MGBFS_HIP(hipSetDevice(device_));
-    const uint64_t W = plan_.owners;
-    MGBFS_HIP(zero_u32x3(bitmap_.as<uint32_t>(), W * plan_.slice_words, words_.as<uint32_t>(), (2 * plan_.count_stride + kEnds) * W, nullptr,
-                         0, stream_));
-    MGBFS_HIP(rank_seed(plan_, start_key_, bitmap_.as<uint32_t>(), list_.as<uint32_t>(), ends(0), stream_));
-    layers.assign(1, 1);
-    sent_ = false;
+    run_.start(stream_);
+    layers = run_.layers;
     candidates = unique_candidates = 0;
     kernel_seconds = 0.0;
     launches = 0;
     streamed_bytes = 0;
     terminal = false;
-    update_bytes();
   }
 
   int advance(uint64_t* next_count, uint32_t* fatal) override {
@@ -86,6 +210,7 @@ class RankBitmapEngine final : public Engine {
   void rebind(const Graph& g) override {
     if (g.elements != n_ || !g.packable() || !g.distinct_perm()) throw std::runtime_error("ENGINE_REBIND_SHAPE");
     set_graph(g);
+    ensure_messages(RankRun::first_cap(run_.plan, g.generators));
     reset();
   }
   void layer_keys(std::vector<uint64_t>& out) override { export_layer(0, layers.back(), out); }
@@ -102,170 +227,65 @@ class RankBitmapEngine final : public Engine {
 
  private:
   static constexpr uint64_t kKeys = 1024;
-  // Messages per owner at first: a fifth of all children there can be (the
-  // widest LRX layer sends 15% of them).
-  static uint32_t first_cap(const RankPlan& p, uint32_t generators) {
-    return std::min(last_cap(p, generators),
-                    static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators / 5 + 1027) / 4 * 4));
-  }
-  // ... and at most: a state is a child of `generators` states.
-  static uint32_t last_cap(const RankPlan& p, uint32_t generators) {
-    return static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(p.list_cap) * generators + 3, 1u << 30) / 4 * 4);
-  }
   void set_graph(const Graph& g) {
-    gens_ = g.packed_generators();
-    if (gens_.count <= 14) {
-      const std::vector<int> inv = inverse_index(gens_);
-      for (uint32_t a = 0; a < gens_.count; ++a) gens_.child_tag[a] = inv[a] >= 0 ? static_cast<uint8_t>(inv[a] + 1) : 0;
-    }
-    rank_gens_ = rank_generators(gens_);
+    run_.set_graph(g);
     history_layers = g.inverse_closed ? 3 : 0;
-    start_key_ = g.start_key();
-  }
-  uint32_t* counts(uint32_t parity) { return words_.as<uint32_t>() + parity * plan_.count_stride * plan_.owners; }
-  uint32_t* ends(uint64_t layer) { return words_.as<uint32_t>() + (2 * plan_.count_stride + layer % kEnds) * plan_.owners; }
-  OwnerCtl* ctl(uint64_t layer) {
-    const uint64_t at = ((2 * plan_.count_stride + kEnds) * 4ull * plan_.owners + 15) / 16 * 16;
-    return reinterpret_cast<OwnerCtl*>(words_.as<char>() + at) + layer % kRing;
   }
   void ensure_messages(uint32_t cap) {
-    if (cap <= cap_) return;
-    const uint64_t entries = static_cast<uint64_t>(plan_.owners) * cap + kRouteDump;
-    MGBFS_HIP(hipStreamSynchronize(stream_));
-    for (auto& m : messages_) m.release();
-    for (auto& m : messages_) m.allocate(entries * 4);
-    cap_ = cap;
-    update_bytes();
-  }
-  // Layer d is in the list: sends its children.  Its control block is the
-  // one the next layer's launch reads.
-  void send(uint64_t d) {
-    MGBFS_HIP(owner_begin(counts(0), 2 * plan_.count_stride * plan_.owners, ctl(d), static_cast<uint32_t>(layers.back()), stream_));
-    MGBFS_HIP(fill_u32(reinterpret_cast<uint32_t*>(ctl(d + 1)), 0u, sizeof(OwnerCtl) / 4, stream_));
-    parity_ = 0;
-    RankLayer a = layer_args(d);
-    a.claim = 0;
-    a.slots = gens_.count;  // the start has no tag
-    a.out = messages_[0].as<uint32_t>();
-    a.out_count = counts(0);
-    MGBFS_HIP(rank_layer(a, rank_gens_, stream_));
-    sent_ = true;
-  }
-  // Arguments of layer d's launch (buffers of the current parity).
-  RankLayer layer_args(uint64_t d) {
-    RankLayer a{};
-    a.plan = plan_;
-    a.claim = 1;
-    a.slots = rank_gens_.tagged == gens_.count && gens_.count > 1 ? gens_.count - 1 : gens_.count;
-    a.in = messages_[parity_].as<uint32_t>();
-    a.in_count = counts(parity_);
-    a.in_cap = cap_;
-    a.out = messages_[parity_ ^ 1u].as<uint32_t>();
-    a.out_count = counts(parity_ ^ 1u);
-    a.out_cap = cap_;
-    a.bitmap = bitmap_.as<uint32_t>();
-    a.list = list_.as<uint32_t>();
-    a.ends_before = d ? ends(d - 1) : ends(kEnds - 1);  // zeros before the start layer
-    a.ends_now = ends(d);
-    a.before = d ? ctl(d - 1) : nullptr;
-    a.now = ctl(d);
-    a.after = ctl(d + 1);
-    a.rules = OwnerRules{plan_.owners, ~0u, 0u, ~0u};
-    a.rec = rec_ + (d ? d - 1 : 0) % kRing;
-    a.seq = base_ + (d ? d - 1 : 0);
-    return a;
+    if (cap > run_.memory.cap) {
+      const uint64_t entries = static_cast<uint64_t>(run_.plan.owners) * cap + kRouteDump;
+      MGBFS_HIP(hipStreamSynchronize(stream_));
+      run_.memory.cap = 0;
+      for (auto& m : messages_) m.release();
+      for (auto& m : messages_) m.allocate(entries * 4);
+      for (int i = 0; i < 2; ++i) run_.memory.messages[i] = messages_[i].as<uint32_t>();
+      run_.memory.cap = cap;
+    }
+    device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + keys_.bytes() + messages_[0].bytes() +
+                   messages_[1].bytes();
   }
   int run_layers(uint32_t most) {
     MGBFS_HIP(hipSetDevice(device_));
-    ensure_messages(first_cap(plan_, gens_.count));
     const uint64_t target = layers.size() - 1 + most;  // depth to reach
-    while (true) {
-      const int s = session(target);
-      if (s != kSendAgain) return s;
-      const uint32_t last = last_cap(plan_, gens_.count);
-      if (cap_ >= last) throw std::runtime_error("BITMAP_MESSAGES");
-      ensure_messages(std::min(2 * cap_, last));
-      if (layers.size() - 1 == target) return MGBFS_LAYER;  // its children are sent by the next call
-    }
-  }
-  // Layers up to depth `target`, or the end, or a layer whose children did
-  // not fit the message slabs (kSendAgain: whatever was queued after it did
-  // nothing).  The record of layer d, numbered base_ + d, is written by the
-  // launch of layer d + 1, or by a report after the last.
-  int session(uint64_t target) {
-    const uint64_t d0 = layers.size() - 1;
-    base_ += 1ull << 32;
-    if (!sent_) send(d0);
-    uint64_t queued = d0, ticks = 0;
-    for (uint64_t d = d0;; ++d) {
-      for (; queued < target && queued <= d + kAheadLayers; ++queued) {
-        const RankLayer a = layer_args(queued + 1);
-        MGBFS_HIP(rank_layer(a, rank_gens_, stream_));
-        parity_ ^= 1u;
-        if (queued + 1 == target)
-          MGBFS_HIP(rank_report(ctl(target), a.rules, rec_ + target % kRing, base_ + target, stream_));
+    int s = MGBFS_LAYER;
+    do {
+      s = run_.run(target, records_, stream_);
+      if (s == RankRun::kSendAgain) {
+        const uint32_t last = RankRun::last_cap(run_.plan, run_.generators());
+        if (run_.memory.cap >= last) throw std::runtime_error("BITMAP_MESSAGES");
+        ensure_messages(static_cast<uint32_t>(std::min<uint64_t>(2ull * run_.memory.cap, last)));
+        if (run_.layers.size() - 1 == target) s = MGBFS_LAYER;  // its children are sent by the next call
       }
-      const LayerRecord& rec = await(rec_[d % kRing], base_ + d);
-      if (d != d0) {
-        kernel_seconds += static_cast<double>(rec.ticks - ticks) * tick_seconds_;
-        candidates += layers.back() * gens_.count;
-        streamed_bytes += 8 * (layers.back() + rec.N);
-        ++launches;
-        if (rec.state == kLayerRejected) throw std::runtime_error("BITMAP_LAYER");
-        if (rec.state == kLayerEmpty) {
-          terminal = true;
-          return MGBFS_COMPLETE;
-        }
-        layers.push_back(rec.N);
-      }
-      ticks = rec.ticks;
-      if (rec.state == kLayerStop) {
-        sent_ = false;
-        return kSendAgain;
-      }
-      if (d == target) return MGBFS_LAYER;
+    } while (s == RankRun::kSendAgain);
+    const size_t before = layers.size();
+    layers = run_.layers;
+    kernel_seconds = run_.seconds;
+    terminal = s == MGBFS_COMPLETE;
+    // Every layer expanded by these launches, an empty one at the end too.
+    for (size_t d = before; d < layers.size() + (terminal ? 1 : 0); ++d) {
+      candidates += layers[d - 1] * run_.generators();
+      streamed_bytes += 8 * (layers[d - 1] + (d < layers.size() ? layers[d] : 0));
+      ++launches;
     }
-  }
-  const LayerRecord& await(const LayerRecord& rec, uint64_t seq) {
-    auto there = [&] { return __atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) == seq; };
-    while (true) {
-      for (uint32_t spin = 0; spin < (1u << 18); ++spin)
-        if (there()) return rec;
-      const hipError_t e = hipStreamQuery(stream_);
-      if (e == hipErrorNotReady) continue;
-      MGBFS_HIP(e);
-      if (!there()) throw std::runtime_error("BITMAP_LAYER_RECORD");
-    }
+    return s;
   }
   // States of the current layer (back = 0) or the one before.
   void export_layer(uint64_t back, uint64_t limit, std::vector<uint64_t>& out) {
     MGBFS_HIP(hipSetDevice(device_));
-    const uint64_t d = layers.size() - 1 - back;
     DeviceBuffer large;
     if (limit > kKeys) large.allocate(limit * 8);
     uint64_t* keys = limit > kKeys ? large.as<uint64_t>() : keys_.as<uint64_t>();
     out.resize(limit);
     if (!limit) return;
-    MGBFS_HIP(rank_export(plan_, list_.as<uint32_t>(), d ? ends(d - 1) : ends(kEnds - 1), ends(d), limit, keys, stream_));
+    run_.export_layer(back, limit, keys, stream_);
     MGBFS_HIP(hipMemcpyAsync(out.data(), keys, limit * 8, hipMemcpyDeviceToHost, stream_));
     MGBFS_HIP(hipStreamSynchronize(stream_));
   }
-  void update_bytes() {
-    device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + keys_.bytes() + messages_[0].bytes() +
-                   messages_[1].bytes();
-  }
 
   uint32_t n_;
-  RankPlan plan_;
-  PackedGenerators gens_{};
-  RankGenerators rank_gens_{};
-  uint64_t start_key_ = 0;
+  RankRun run_;
+  RankRecords records_;
   DeviceBuffer bitmap_, list_, words_, keys_, messages_[2];
-  uint32_t cap_ = 0, parity_ = 0;  // messages per owner; the buffer holding the current layer's children
-  bool sent_ = false;              // ... which are complete
-  uint64_t base_ = 0;
-  double tick_seconds_ = 0.0;
-  LayerRecord* rec_ = nullptr;     // pinned
 };
 
 // All degrees that ranks and slices are made for: faster from the smallest to

@@ -2,6 +2,7 @@
 oracle's (committed golden tables) and the one-at-a-time engine's."""
 import json
 import math
+import random
 from pathlib import Path
 
 import pytest
@@ -226,3 +227,34 @@ def test_batch_options_are_validated():
             BatchEngine(max_slots=2, **bad)
     with pytest.raises(ValueError):
         BatchEngine(max_slots=2, history="three")
+
+
+# Bitmap instances of degree 11 and 12 run by owners of the bitmap beside the
+# graph of the others: alone and in a mix, stopped at a layer limit (one short
+# of the search, its exact length), released half way, and with more children
+# in a layer (up to 10 per state of the group) than their messages hold, where they start over.
+def test_large_bitmap_instances_run_beside_the_graph():
+    n = 11
+    lrx_gens = O.lrx_generators(n)
+    rng = random.Random(8)
+    many = [rng.sample(range(n), n) for _ in range(14)]
+    ref, ref_many, small = O.packed_bfs(n)["layers"], O.packed_bfs(n, many)["layers"], O.packed_bfs(9)["layers"]
+    jobs = [(lrx_gens, n, 0), (O.lrx_generators(9), 9, 0), (lrx_gens, n, len(ref) - 1), (many, n, 0), (lrx_gens, n, len(ref))]
+    with BatchEngine(max_slots=8, vram_budget=16 << 30) as b:
+        half = b.admit(GraphDefinition.permutation(lrx_gens, list(range(n))))
+        b.step(8)
+        b.release(half)
+        slots = [b.admit(GraphDefinition.permutation(g, list(range(k))), max_layers=m) for g, k, m in jobs]
+        b.step(3)
+        assert b.result(slots[0])[0] == ref[:len(b.result(slots[0])[0])]
+        done = []
+        while len(done) < len(jobs):
+            b.step(4)
+            done += b.poll()
+        results = [b.result(s) for s in slots]
+        last = b.sample(slots[0], n)
+        infos = [b.instance_info(s) for s in slots]
+    assert [r[0] for r in results] == [ref, small, ref[:-1], ref_many, ref]
+    assert [bool(r[2]) for r in results] == [False, False, True, False, False]
+    assert len(last) == ref[-1] and all(sorted(row) == list(range(n)) for row in last)
+    assert all(i["visited"] == "bitmap" and i["restarts"] == 0 and i["history_layers"] == 0 for i in infos)
