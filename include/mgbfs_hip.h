@@ -338,6 +338,10 @@ int mgbfs_batch_usage(void* batch, uint64_t* used, uint64_t* budget, uint32_t* s
 int mgbfs_batch_instance_info(void* batch, int32_t slot, uint32_t* visited, uint32_t* history_layers,
                               uint64_t* layer_capacity, uint32_t* restarts);
 void mgbfs_batch_destroy(void* batch);
+/* Destroyed batches leave up to 16 GiB of device memory for the next ones of
+ * the process.  It counts as free in every budget of this library, and is
+ * given back when one of its allocations fails, or here. */
+void mgbfs_release_cached_memory(int32_t device);
 
 /* --------------------------------------------- generic SoA kernel ABI */
 /* Same signatures and argument meaning as the reference's libmgbfs_cuda

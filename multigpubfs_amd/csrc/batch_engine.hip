@@ -32,6 +32,7 @@ uint64_t next_pow2(uint64_t x) {
 // to the working set.  Chunks grow geometrically (kArenaFirst doubling to
 // kArenaMax) within the engine's budget; a chunk that is entirely free is
 // handed back to the device only when the arena holds more than the budget.
+// At the end they go to the process's cache, where the next arena looks first.
 constexpr uint64_t kArenaFirst = 1ull << 30;
 constexpr uint64_t kArenaMax = 32ull << 30;
 
@@ -43,6 +44,7 @@ struct Block {
 
 class DeviceArena {
  public:
+  explicit DeviceArena(int device) : device_(device) {}
   Block take(uint64_t bytes, uint64_t budget) {
     bytes = arena_round(bytes);
     for (uint32_t c = 0; c < chunks_.size(); ++c) {
@@ -56,9 +58,11 @@ class DeviceArena {
     uint32_t c = 0;
     while (c < chunks_.size() && chunks_[c].buf.bytes()) ++c;
     if (c == chunks_.size()) chunks_.emplace_back();
-    chunks_[c].buf.allocate(size);
+    chunks_[c].buf = device_cache_take(device_, bytes, std::max(size, budget - std::min(budget, reserved_)));
+    if (!chunks_[c].buf.bytes()) chunks_[c].buf.allocate(size);
+    size = chunks_[c].buf.bytes() / kArenaAlign * kArenaAlign;
     chunks_[c].ranges = RangeSet(size);
-    reserved_ += size;
+    reserved_ += chunks_[c].buf.bytes();
     next_ = std::min(2 * next_, kArenaMax);
     uint64_t off = 0;
     chunks_[c].ranges.take(bytes, &off);
@@ -75,13 +79,12 @@ class DeviceArena {
     }
     b = Block{};
   }
-  void trim() {
+  // The owner is done with all of it, and its streams are idle.
+  void close() {
     for (Chunk& ch : chunks_)
-      if (ch.buf.bytes() && ch.ranges.empty()) {
-        reserved_ -= ch.buf.bytes();
-        ch.buf.release();
-        ch.ranges = RangeSet();
-      }
+      if (ch.buf.bytes()) device_cache_give(device_, std::move(ch.buf));
+    chunks_.clear();
+    reserved_ = 0;
   }
   uint64_t reserved() const { return reserved_; }
 
@@ -90,6 +93,7 @@ class DeviceArena {
     DeviceBuffer buf;
     RangeSet ranges;
   };
+  int device_;
   std::vector<Chunk> chunks_;
   uint64_t reserved_ = 0, next_ = kArenaFirst;
 };
@@ -128,7 +132,7 @@ struct OwnedInstance {
 
 class BatchEngine {
  public:
-  BatchEngine(const mgbfs_batch_options& o) : device_(o.device) {
+  BatchEngine(const mgbfs_batch_options& o) : device_(o.device), arena_(o.device) {
     MGBFS_HIP(hipSetDevice(device_));
     MGBFS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     MGBFS_HIP(hipStreamCreateWithFlags(&owned_stream_, hipStreamNonBlocking));
@@ -137,6 +141,7 @@ class BatchEngine {
     if (!budget_) {
       size_t fr = 0, tot = 0;
       MGBFS_HIP(hipMemGetInfo(&fr, &tot));
+      fr += device_cache_bytes(device_);
       budget_ = fr > (4ull << 30) ? fr - (4ull << 30) : 0;
     }
     hipDeviceProp_t prop;
@@ -185,7 +190,7 @@ class BatchEngine {
     if (host_req_) (void)hipHostFree(host_req_);
     if (host_out_) (void)hipHostFree(host_out_);
     slots_.clear();
-    arena_.trim();
+    arena_.close();
     if (stream_) (void)hipStreamDestroy(stream_);
     if (owned_stream_) (void)hipStreamDestroy(owned_stream_);
   }

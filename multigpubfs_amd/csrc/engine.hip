@@ -88,6 +88,7 @@ uint64_t vram_budget(const mgbfs_engine_options& o) {
   if (o.vram_budget) return o.vram_budget;
   size_t fr = 0, tot = 0;
   MGBFS_HIP(hipMemGetInfo(&fr, &tot));
+  fr += device_cache_bytes(o.device);
   const uint64_t reserve = (o.flags & MGBFS_FLAG_MAX_CAPACITY) ? (256ull << 20) : (2ull << 30);
   return fr > reserve ? fr - reserve : 0;
 }

@@ -23,6 +23,8 @@ struct HipError : std::runtime_error {
   } while (0)
 
 // Owned device allocation (freed on destruction, on the owning device).
+bool device_cache_release(int device);  // device_cache.hip
+
 class DeviceBuffer {
  public:
   DeviceBuffer() = default;
@@ -34,7 +36,14 @@ class DeviceBuffer {
   void allocate(size_t bytes) {
     release();
     if (bytes == 0) bytes = 8;
-    MGBFS_HIP(hipMalloc(&ptr_, bytes));
+    hipError_t e = hipMalloc(&ptr_, bytes);
+    if (e == hipErrorOutOfMemory) {
+      int device = 0;
+      (void)hipGetLastError();
+      if (hipGetDevice(&device) == hipSuccess && device_cache_release(device)) e = hipMalloc(&ptr_, bytes);
+    }
+    if (e != hipSuccess) ptr_ = nullptr;
+    MGBFS_HIP(e);
     bytes_ = bytes;
   }
   void release() {
@@ -53,6 +62,14 @@ class DeviceBuffer {
   void* ptr_ = nullptr;
   size_t bytes_ = 0;
 };
+
+// Whole buffers kept between batch engines (device_cache.hip): the smallest
+// of least to most bytes (an empty buffer when none is kept); a buffer that
+// no stream uses any more; the bytes kept; all of them back to the device
+// (false: there were none).
+DeviceBuffer device_cache_take(int device, uint64_t least, uint64_t most);
+void device_cache_give(int device, DeviceBuffer&& buf);
+uint64_t device_cache_bytes(int device);
 
 // Host copy of the graph description (validated).
 struct Graph {

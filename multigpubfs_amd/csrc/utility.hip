@@ -1,6 +1,7 @@
 // Small device utilities: fills (used instead of hipMemsetAsync so that
 // layer loops stay capturable in hipGraphs) and device queries.
 #include "common.hpp"
+#include "engine.hpp"
 #include "kernels.hpp"
 #include "../../include/mgbfs_hip.h"
 
@@ -72,7 +73,7 @@ extern "C" int mgbfs_hip_device_info(int32_t device, uint32_t* compute_units, ui
   if (wave_size) *wave_size = static_cast<uint32_t>(prop.warpSize);
   if (lds_bytes) *lds_bytes = static_cast<uint32_t>(prop.sharedMemPerBlock);
   if (total_bytes) *total_bytes = tot;
-  if (free_bytes) *free_bytes = fr;
+  if (free_bytes) *free_bytes = fr + mgbfs::device_cache_bytes(device);
   return 0;
 }
 

@@ -239,7 +239,8 @@ def test_large_bitmap_instances_run_beside_the_graph():
     rng = random.Random(8)
     many = [rng.sample(range(n), n) for _ in range(14)]
     ref, ref_many, small = O.packed_bfs(n)["layers"], O.packed_bfs(n, many)["layers"], O.packed_bfs(9)["layers"]
-    jobs = [(lrx_gens, n, 0), (O.lrx_generators(9), 9, 0), (lrx_gens, n, len(ref) - 1), (many, n, 0), (lrx_gens, n, len(ref))]
+    jobs = [(lrx_gens, n, 0), (O.lrx_generators(9), 9, 0), (lrx_gens, n, len(ref) - 1), (many, n, 0),
+            (lrx_gens, n, len(ref))]
     with BatchEngine(max_slots=8, vram_budget=16 << 30) as b:
         half = b.admit(GraphDefinition.permutation(lrx_gens, list(range(n))))
         b.step(8)
@@ -258,3 +259,35 @@ def test_large_bitmap_instances_run_beside_the_graph():
     assert [bool(r[2]) for r in results] == [False, False, True, False, False]
     assert len(last) == ref[-1] and all(sorted(row) == list(range(n)) for row in last)
     assert all(i["visited"] == "bitmap" and i["restarts"] == 0 and i["history_layers"] == 0 for i in infos)
+
+
+# Arena chunks outlive their engine in a bounded cache: later engines (with
+# smaller, equal and larger needs, of two threads) find them with the contents
+# they were left with, and count them as free memory.
+def test_engines_reuse_kept_memory_exactly():
+    import threading
+    from multigpubfs_amd._native import load
+    inst = [x["graph"] for x in GOLDEN[:12]]
+    golden = [x["layer_sizes"] for x in GOLDEN[:12]]
+    assert run_batched(inst)[0] == golden
+    with BatchEngine(vram_budget=8 << 30) as b:
+        slot = b.admit(GraphDefinition.permutation(O.lrx_generators(11), list(range(11))), visited="hash")
+        b.run()
+        assert b.result(slot)[0] == O.packed_bfs(11)["layers"]
+    with BatchEngine() as b:
+        kept = b.usage()["budget"]
+    load().mgbfs_release_cached_memory(0)
+    with BatchEngine() as b:
+        assert abs(b.usage()["budget"] - kept) < 1 << 30
+    out = {}
+
+    def work(k, **options):
+        out[k] = [run_batched(inst[k::2], **options)[0] for _ in range(3)]
+
+    threads = [threading.Thread(target=work, args=(0,)),
+               threading.Thread(target=work, args=(1,), kwargs={"visited": "hash"})]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert out == {k: [golden[k::2]] * 3 for k in (0, 1)}
