@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include "common.hpp"
+#include "kernels.hpp"
 
 namespace mgbfs {
 
@@ -61,6 +62,39 @@ struct BatchInstance {
   // parent, already visited).  tag_shift 64 = no tags.
   uint8_t child_tag[kBatchMaxGens];
   uint32_t tag_shift;
+  // Bitmap by owners (rank_owner.hip; rank.owners 0: not): the bitmap is
+  // owners x slice_words, new states go to the owners' lists, children to
+  // their owners' messages.  A step claims the messages of the step before;
+  // where those were the last of their layer's, the claimed states are the
+  // next layer, else the layer goes on: an owner sends at most `chunk`
+  // states a step, so that the messages hold any layer's children.
+  RankPlan rank;
+  uint32_t slots;         // children per state: generators, or one less when all have tags
+  uint32_t chunk, message_cap, message_dump;
+  uint32_t unfinished;    // the layer's states were not all sent yet
+  uint32_t more;          // the same, of the step running
+  uint32_t parity;        // messages[parity] are the ones to claim
+  uint32_t* list;         // owners x list_cap
+  uint32_t* words;        // OwnedWords
+  uint32_t* messages[2];  // owners x message_cap, + kRouteDump
+  RankGenerator rank_gen[kBatchMaxGens];
+};
+
+// An owned instance's words: the message counters (count_stride apart, one
+// set per buffer), then per owner the list's length, the rows sent so far,
+// the layer's end, and the first row of the last four layers.
+struct OwnedWords {
+  uint32_t *count[2], *rows, *sent, *end, *first;
+  __host__ __device__ static uint64_t words(const RankPlan& p) { return (2ull * p.count_stride + 7) * p.owners; }
+  __host__ __device__ OwnedWords(uint32_t* w, const RankPlan& p) {
+    const uint64_t W = p.owners;
+    count[0] = w;
+    count[1] = count[0] + W * p.count_stride;
+    rows = count[1] + W * p.count_stride;
+    sent = rows + W;
+    end = sent + W;
+    first = end + W;
+  }
 };
 
 // Deferred descriptor upload: slot <- staged descriptor, then (seed != 0)
@@ -71,7 +105,9 @@ struct BatchInstall {
 };
 
 hipError_t batch_reset_flag(uint32_t* flag, hipStream_t stream);
-// prefix: 2 * (slots + 1) words (expansion tiles, then clear work items).
+// prefix: kBatchPrefixes * (slots + 1) words (expansion tiles, clear work
+// items, owners), then the owners' work counter.
+constexpr uint32_t kBatchPrefixes = 3;
 hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, hipStream_t stream);
 // threads: 128, 256 or 512 per workgroup; tile = 2 * threads parents.
 hipError_t batch_expand(BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t tile, uint32_t grid,
@@ -80,6 +116,12 @@ hipError_t batch_expand(BatchInstance* inst, uint32_t slots, const uint32_t* pre
 // (work items from the second half of batch_tiles' prefix).
 hipError_t batch_clear(const BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t grid,
                        hipStream_t stream);
+// A step of every owner of the owned instances; grid: at most two blocks
+// per CU run at once.
+hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, uint32_t grid, hipStream_t stream);
+// States of the current layer of an owned instance (a staged copy of its
+// descriptor), packed keys.
+hipError_t batch_owned_export(const BatchInstance& inst, uint64_t limit, uint64_t* keys, hipStream_t stream);
 hipError_t batch_finish(BatchInstance* inst, uint32_t slots, uint32_t* any_active, hipStream_t stream);
 hipError_t batch_gather_sizes(const BatchInstance* inst, const uint32_t* req, uint32_t n, uint64_t* out,
                               hipStream_t stream);

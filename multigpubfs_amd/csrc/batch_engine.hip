@@ -1,6 +1,6 @@
 // Host side of the batched multi-instance engine: slot admission with VRAM
 // planning, a pooled device allocator, and a hipGraph-captured layer loop
-// (reset flag, then K x [tiles, clear, expand, finish]) replayed until no instance
+// (reset flag, then K x [tiles, clear, expand, owned, finish]) replayed until no instance
 // is active.  Instances join and leave at layer boundaries, so the same
 // object serves both the fixed sweep and continuous-batching serving.
 #include <algorithm>
@@ -12,7 +12,6 @@
 #include "batch.hpp"
 #include "engine.hpp"
 #include "kernels.hpp"
-#include "rank_run.hpp"
 
 namespace mgbfs {
 
@@ -114,28 +113,31 @@ struct BatchPlan {
   uint32_t max_layers = kDefaultMaxLayers;
 };
 
-// A bitmap instance run by owners of the bitmap (rank_run.hpp) in its slot's
-// block, beside the graph that runs the others.  Large degrees only: their
-// layers fill the chip, and no claim is a global atomic (alone, LRX of
-// degree 12 33 -> 10.5 ms, 11 4.8 -> 1.3 ms).  Many smaller instances are
-// better off sharing launches: 256 random sets of degree 9 and 10 take 42 ms
-// in the graph and would take 55 ms one after the other.  (Twenty mixed jobs
-// of degree 8 to 12 and SL(2, Z_p): 94.5 -> 51.8 ms.)
-constexpr uint32_t kOwnedDegree = 11;
+// Bitmap instances of these degrees run by owners of the bitmap where their
+// slot's block holds it: no claim is a global atomic (27 G/s for the whole
+// chip), states take four bytes.  Sweeps of 16, 60, 256 random sets of degree
+// 9 and 10 went from 5.6, 13.5, 45 to 3.9, 7.9, 22.5 ms, 6, 12, 20 mixed jobs
+// of degree 8 to 12 and SL(2, Z_p) from 8.3, 41, 94 to 4.8, 19, 52 ms (of
+// which 20 are hash tables).  Below degree 9 an instance has too little work
+// to split.
+constexpr uint32_t kOwnedDegree = 9;
 
-struct OwnedInstance {
-  explicit OwnedInstance(uint32_t degree) : run(degree) {}
-  RankRun run;
-  bool started = false, outgrown = false;
-  uint32_t status = kInstActive, error = 0;
-};
+// Owners of an instance when `instances` run.  Alone a degree 9 or 10 search
+// has 251; many together have fewer, so that a step of small layers stays
+// near two owners a workgroup (16 instances: 251, 101 or 53 owners 6.0, 3.6,
+// 3.8 ms; 30: 101 or 53 5.8, 5.1 ms), but not below 53, where a tile's
+// children meet on too few counters (60 instances: 53 or 23 owners 7.8, 9.0
+// ms).  Degrees 11 and 12 keep their own number: their layers are large.
+uint32_t owners_for(uint32_t degree, uint32_t instances) {
+  if (degree >= 11) return rank_plan(degree).owners;
+  return 251 * instances <= 2048 ? 251 : (101 * instances <= 2048 ? 101 : 53);
+}
 
 class BatchEngine {
  public:
   BatchEngine(const mgbfs_batch_options& o) : device_(o.device), arena_(o.device) {
     MGBFS_HIP(hipSetDevice(device_));
     MGBFS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-    MGBFS_HIP(hipStreamCreateWithFlags(&owned_stream_, hipStreamNonBlocking));
     slots_n_ = o.max_slots ? std::min(o.max_slots, kBatchMaxSlots) : 256;
     budget_ = o.vram_budget;
     if (!budget_) {
@@ -148,6 +150,7 @@ class BatchEngine {
     MGBFS_HIP(hipGetDeviceProperties(&prop, device_));
     grid_ = o.grid ? o.grid : static_cast<uint32_t>(prop.multiProcessorCount) * 8;
     clear_grid_ = static_cast<uint32_t>(prop.multiProcessorCount);
+    owned_grid_ = static_cast<uint32_t>(prop.multiProcessorCount) * 2;
     layers_per_graph_ = o.layers_per_graph ? o.layers_per_graph : kLayersPerGraph;
     threads_ = o.threads ? o.threads : 256;
     if (threads_ != 128 && threads_ != 256 && threads_ != 512) throw std::runtime_error("BATCH_OPTION_THREADS");
@@ -159,7 +162,7 @@ class BatchEngine {
     if (layer_pct_ > 100) throw std::runtime_error("BATCH_OPTION_LAYER_PCT");
     bitmap_bias_permille_ = o.bitmap_bias_permille ? o.bitmap_bias_permille : 1000;
     inst_.allocate(sizeof(BatchInstance) * slots_n_);
-    prefix_.allocate(8 * (slots_n_ + 1));
+    prefix_.allocate(4 * (kBatchPrefixes * (slots_n_ + 1) + 1));
     flag_.allocate(64);
     MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_flag_), 64, hipHostMallocDefault));
     MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_mirror_), sizeof(BatchInstance) * slots_n_,
@@ -175,13 +178,12 @@ class BatchEngine {
     std::memset(host_inst_.data(), 0, sizeof(BatchInstance) * slots_n_);
     MGBFS_HIP(hipMemcpy(inst_.as<void>(), host_inst_.data(), sizeof(BatchInstance) * slots_n_, hipMemcpyHostToDevice));
     slots_.resize(slots_n_);
-    owned_.resize(slots_n_);
+    owned_wanted_.assign(slots_n_, 0);
     capture();
   }
   ~BatchEngine() {
     (void)hipSetDevice(device_);
     if (stream_) (void)hipStreamSynchronize(stream_);
-    if (owned_stream_) (void)hipStreamSynchronize(owned_stream_);
     if (exec_) (void)hipGraphExecDestroy(exec_);
     if (graph_) (void)hipGraphDestroy(graph_);
     if (host_flag_) (void)hipHostFree(host_flag_);
@@ -192,7 +194,6 @@ class BatchEngine {
     slots_.clear();
     arena_.close();
     if (stream_) (void)hipStreamDestroy(stream_);
-    if (owned_stream_) (void)hipStreamDestroy(owned_stream_);
   }
 
   // Planned footprint (the admission unit) and the visited-set choice.
@@ -287,17 +288,11 @@ class BatchEngine {
   // all), planned layer capacity and restarts after an outgrown layer.
   void instance_info(int32_t slot, uint32_t& visited, uint32_t& history, uint64_t& cap, uint32_t& restarts) const {
     check_slot(slot);
-    restarts = jobs_[slot].restarts;
-    if (owned_[slot]) {
-      visited = 1;
-      history = 0;
-      cap = state_space_bound(jobs_[slot].graph);
-      return;
-    }
     const BatchInstance& d = host_inst_[slot];
     visited = d.visited == kVisBitmap ? 1 : 2;
     history = d.rolling ? 3 : 0;
     cap = d.cap;
+    restarts = jobs_[slot].restarts;
   }
 
   // Lays out a slot's block (frontiers, layer sizes, visited set) from its
@@ -314,40 +309,10 @@ class BatchEngine {
     kinds_[slot] = g.kind;
     rows_[slot] = g.rows;
     cols_[slot] = g.cols;
-    if (!install_owned(slot, p)) install_shared(slot, p);
+    lay_out(slot, p);
   }
 
-  // The slot's block as bitmap, list, words and, with what is left, two
-  // message buffers of at least a message per state each; false where that
-  // does not fit or the graph is not for owners.
-  bool install_owned(int32_t slot, const BatchPlan& p) {
-    const Graph& g = jobs_[slot].graph;
-    if (p.visited != kVisBitmap || g.elements < kOwnedDegree || g.elements > kRankDegree) return false;
-    auto o = std::make_unique<OwnedInstance>(g.elements);
-    const RankPlan& rp = o->run.plan;
-    const Block& block = slots_[slot].block;
-    uint64_t at = 0;
-    auto part = [&](uint64_t bytes) {
-      const uint64_t start = at;
-      at += arena_round(bytes);
-      return reinterpret_cast<uint32_t*>(block.ptr + start);
-    };
-    RankMemory& m = o->run.memory;
-    m.bitmap = part(4ull * rp.owners * rp.slice_words);
-    m.list = part(4ull * rp.owners * rp.list_cap);
-    m.words = part(RankRun::words_bytes(rp));
-    const uint64_t least = 4 * (static_cast<uint64_t>(rp.owners) * rp.list_cap + kRouteDump) + 2 * kArenaAlign;
-    if (block.bytes < at + 2 * least) return false;
-    const uint64_t each = (block.bytes - at) / 2 / kArenaAlign * kArenaAlign;
-    m.cap = static_cast<uint32_t>(std::min<uint64_t>((each / 4 - kRouteDump) / rp.owners,
-                                                     RankRun::last_cap(rp, g.generators)) / 4 * 4);
-    for (uint32_t*& x : m.messages) x = part(each);
-    o->run.set_graph(g);
-    owned_[slot] = std::move(o);
-    return true;
-  }
-
-  void install_shared(int32_t slot, const BatchPlan& p) {
+  void lay_out(int32_t slot, const BatchPlan& p) {
     const Graph& g = jobs_[slot].graph;
     const uint64_t keys_bytes = arena_round(p.cap * 8), sizes_bytes = arena_round(8ull * p.max_layers);
     char* base = slots_[slot].block.ptr;
@@ -399,6 +364,8 @@ class BatchEngine {
           d.mat[k][e] = static_cast<int32_t>(g.matrices[static_cast<size_t>(k) * g.rows * g.rows + e]);
       for (uint32_t e = 0; e < g.elements; ++e) start_key |= static_cast<uint64_t>(g.start[e]) << (e * eb);
     }
+    const bool first_try = !jobs_[slot].shared;
+    owned_wanted_[slot] = p.visited == kVisBitmap && first_try && g.elements >= kOwnedDegree && g.elements <= kRankDegree;
     // The visited set is emptied, and the descriptor installed and seeded,
     // by the next flush(), which the next step runs before its graph.
     pending_[slot] = kInstallSeed;
@@ -412,48 +379,14 @@ class BatchEngine {
     const uint32_t launches = std::max<uint32_t>(1, (layers + layers_per_graph_ - 1) / layers_per_graph_);
     flush();
     for (uint32_t k = 0; k < launches; ++k) MGBFS_HIP(hipGraphLaunch(exec_, stream_));
-    for (uint32_t s = 0; s < slots_n_; ++s)
-      if (owned_[s] && (owned_[s]->status & kInstActive)) run_owned(s, launches * layers_per_graph_);
     refresh();
     uint32_t active = 0;
     for (uint32_t s = 0; s < slots_n_; ++s) {
       if (!slots_[s].used) continue;
-      if (owned_[s]) {
-        if (owned_[s]->status & kInstActive) ++active;
-        if (!owned_[s]->outgrown) continue;
-        const Job& job = jobs_[s];
-        owned_[s].reset();
-        install_shared(static_cast<int32_t>(s), plan_with(job.graph, job.visited, job.max_layers, false, 1));
-        continue;
-      }
       if (host_inst_[s].status & kInstDone) restart_if_outgrown(s);
       if ((host_inst_[s].status & kInstActive) || pending_[s] == kInstallSeed) ++active;
     }
     return active;
-  }
-
-  // Up to `most` layers of an owned instance.  One whose messages do not fit
-  // the block starts over in the graph, in the same block.
-  void run_owned(uint32_t s, uint32_t most) {
-    OwnedInstance& o = *owned_[s];
-    RankRun& run = o.run;
-    const uint32_t limit = jobs_[s].max_layers ? jobs_[s].max_layers : kDefaultMaxLayers;
-    if (!o.started) run.start(owned_stream_);
-    o.started = true;
-    // A layer past the last that is allowed is an error, and is not listed.
-    const uint64_t target = std::min<uint64_t>(run.layers.size() - 1 + most, limit);
-    const int r = run.run(target, records_, owned_stream_);
-    if (r == MGBFS_LAYER && run.layers.size() <= limit) return;
-    MGBFS_HIP(hipStreamSynchronize(owned_stream_));  // launches queued past the end
-    if (r == RankRun::kSendAgain && run.layers.size() <= limit) {
-      o.outgrown = true;  // step() moves it to the graph
-      return;
-    }
-    if (run.layers.size() > limit) {
-      run.layers.resize(limit);
-      o.error |= kErrCount;
-    }
-    o.status = kInstDone;
   }
 
   // A rolling instance whose layer outgrew its planned capacity (next
@@ -461,6 +394,14 @@ class BatchEngine {
   // state bound, when the budget allows; otherwise its error stands.
   void restart_if_outgrown(uint32_t s) {
     const BatchInstance& d = host_inst_[s];
+    if (d.rank.owners && (d.error & kErrFutureCap) && !slots_[s].reported) {
+      // An owner got more messages than its share with its reserve: once
+      // more over the shared bitmap, in the same block.
+      Job& job = jobs_[s];
+      job.shared = true;
+      lay_out(static_cast<int32_t>(s), plan_with(job.graph, job.visited, job.max_layers, false, 1));
+      return;
+    }
     if (!d.rolling || !(d.error & (kErrFutureCap | kErrTableFull)) || slots_[s].reported) return;
     Job& job = jobs_[s];
     if (d.cap >= state_space_bound(job.graph)) return;
@@ -484,27 +425,16 @@ class BatchEngine {
   std::vector<int32_t> poll(uint32_t limit) {
     std::vector<int32_t> out;
     for (uint32_t s = 0; s < slots_n_ && out.size() < limit; ++s)
-      if (slots_[s].used && !slots_[s].reported &&
-          ((owned_[s] ? owned_[s]->status : host_inst_[s].status) & kInstDone)) {
+      if (slots_[s].used && !slots_[s].reported && (host_inst_[s].status & kInstDone)) {
         slots_[s].reported = true;
         out.push_back(static_cast<int32_t>(s));
       }
-    std::vector<int32_t> shared;
-    for (int32_t s : out)
-      if (!owned_[s]) shared.push_back(s);
-    gather(shared);
+    gather(out);
     return out;
   }
 
   void result(int32_t slot, std::vector<uint64_t>& sizes, uint32_t& status, uint32_t& error) {
     check_slot(slot);
-    if (owned_[slot]) {
-      const OwnedInstance& o = *owned_[slot];
-      sizes = o.started ? o.run.layers : std::vector<uint64_t>(1, 1);
-      status = o.status;
-      error = o.error;
-      return;
-    }
     const BatchInstance& d = host_inst_[slot];
     if (finished_[slot].ready) {
       sizes = finished_[slot].sizes;
@@ -519,14 +449,18 @@ class BatchEngine {
   // Current-layer states of a slot as int64 rows (at most limit).
   void sample(int32_t slot, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) {
     check_slot(slot);
-    if (owned_[slot]) {
-      sample_owned(slot, limit, rows, count);
-      return;
-    }
     const BatchInstance& d = host_inst_[slot];
     count = std::min<uint64_t>(limit, d.count);
     std::vector<uint64_t> keys(count);
-    if (count) MGBFS_HIP(hipMemcpy(keys.data(), d.front, count * 8, hipMemcpyDeviceToHost));
+    if (count && d.rank.owners) {
+      DeviceBuffer out;
+      out.allocate(8 * count);
+      MGBFS_HIP(batch_owned_export(d, count, out.as<uint64_t>(), stream_));
+      MGBFS_HIP(hipStreamSynchronize(stream_));
+      MGBFS_HIP(hipMemcpy(keys.data(), out.as<void>(), count * 8, hipMemcpyDeviceToHost));
+    } else if (count) {
+      MGBFS_HIP(hipMemcpy(keys.data(), d.front, count * 8, hipMemcpyDeviceToHost));
+    }
     const uint32_t w = d.action == kActPerm ? d.degree : d.rows * d.cols;
     rows.assign(count * w, 0);
     for (uint64_t r = 0; r < count; ++r)
@@ -540,15 +474,11 @@ class BatchEngine {
     check_slot(slot);
     MGBFS_HIP(hipSetDevice(device_));
     Slot& sl = slots_[slot];
-    if (owned_[slot]) {
-      MGBFS_HIP(hipStreamSynchronize(owned_stream_));
-      owned_[slot].reset();  // its descriptor is clear
-    } else {
-      // The cleared descriptor is installed by the next flush, before any
-      // graph reads descriptors again, so the range can be reused at once.
-      std::memset(&host_inst_[slot], 0, sizeof(BatchInstance));
-      pending_[slot] = kInstallOnly;
-    }
+    BatchInstance& d = host_inst_[slot];
+    std::memset(&d, 0, sizeof d);
+    // The cleared descriptor is installed by the next flush, before any
+    // graph reads descriptors again, so the range can be reused at once.
+    pending_[slot] = kInstallOnly;
     arena_.give(sl.block, budget_);
     used_ -= sl.planned;
     sl = Slot{};
@@ -561,24 +491,6 @@ class BatchEngine {
   uint32_t slots() const { return slots_n_; }
 
  private:
-  void sample_owned(int32_t slot, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) {
-    OwnedInstance& o = *owned_[slot];
-    if (!o.started) o.run.start(owned_stream_);
-    o.started = true;
-    count = std::min<uint64_t>(limit, o.run.layers.back());
-    std::vector<uint64_t> keys(count);
-    DeviceBuffer out;
-    if (count) {
-      out.allocate(8 * count);
-      o.run.export_layer(0, count, out.as<uint64_t>(), owned_stream_);
-      MGBFS_HIP(hipMemcpyAsync(keys.data(), out.as<void>(), 8 * count, hipMemcpyDeviceToHost, owned_stream_));
-      MGBFS_HIP(hipStreamSynchronize(owned_stream_));
-    }
-    const uint32_t n = o.run.plan.degree;
-    rows.assign(count * n, 0);
-    for (uint64_t r = 0; r < count; ++r)
-      for (uint32_t e = 0; e < n; ++e) rows[r * n + e] = static_cast<int64_t>((keys[r] >> (4 * e)) & 15u);
-  }
   void check_slot(int32_t slot) const {
     if (slot < 0 || static_cast<uint32_t>(slot) >= slots_n_ || !slots_[slot].used)
       throw std::runtime_error("BATCH_SLOT");
@@ -587,17 +499,59 @@ class BatchEngine {
     BatchInstance* inst = inst_.as<BatchInstance>();
     uint32_t* prefix = prefix_.as<uint32_t>();
     uint32_t* flag = flag_.as<uint32_t>();
-    MGBFS_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
+    // Relaxed: thread-local capture still refuses the allocations and copies
+    // of other threads' engines, and fails with them.
+    MGBFS_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed));
     MGBFS_HIP(batch_reset_flag(flag, stream_));
     for (uint32_t k = 0; k < layers_per_graph_; ++k) {
       MGBFS_HIP(batch_tiles(inst, slots_n_, 2 * threads_, prefix, stream_));
       MGBFS_HIP(batch_clear(inst, slots_n_, prefix, clear_grid_, stream_));
       MGBFS_HIP(batch_expand(inst, slots_n_, prefix, 2 * threads_, grid_, threads_, stream_));
+      MGBFS_HIP(batch_owned(inst, slots_n_, prefix, owned_grid_, stream_));
       MGBFS_HIP(batch_finish(inst, slots_n_, flag, stream_));
     }
     MGBFS_HIP(hipStreamEndCapture(stream_, &graph_));
     MGBFS_HIP(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
   }
+  // The slot's block as bitmap and words (adjoining, emptied together as
+  // bitmap_bits), list, layer sizes and two message buffers.  Steps send so
+  // few states that an owner's share of their children leaves a third of its
+  // messages free.
+  void lay_out_owned(uint32_t slot, uint32_t running) {
+    const Graph& g = jobs_[slot].graph;
+    BatchInstance& d = host_inst_[slot];
+    const Block& block = slots_[slot].block;
+    const RankPlan p = rank_plan(g.elements, owners_for(g.elements, running));
+    uint64_t at = 0;
+    auto part = [&](uint64_t bytes) {
+      const uint64_t start = at;
+      at += arena_round(bytes);
+      return block.ptr + start;
+    };
+    const uint64_t bitmap_words = static_cast<uint64_t>(p.owners) * p.slice_words, words = OwnedWords::words(p);
+    uint32_t* bitmap = reinterpret_cast<uint32_t*>(part(4 * (bitmap_words + words)));
+    uint32_t* list = reinterpret_cast<uint32_t*>(part(4ull * p.owners * p.list_cap));
+    uint64_t* sizes = reinterpret_cast<uint64_t*>(part(8ull * d.max_layers));
+    if (block.bytes < at + 2 * kArenaAlign) return;
+    const uint64_t each = (block.bytes - at) / 2 / kArenaAlign * kArenaAlign;
+    if (each / 4 < kRouteDump + 64ull * p.owners) return;
+    const uint64_t cap = std::min<uint64_t>((each / 4 - kRouteDump) / p.owners, 1u << 28) / 4 * 4;
+    const RankGenerators gens = rank_generators(g.packed_generators(), d.child_tag);
+    d.slots = gens.tagged == gens.count && gens.count > 1 ? gens.count - 1 : gens.count;
+    if (cap < 3ull * d.slots) return;
+    d.rank = p;
+    d.chunk = static_cast<uint32_t>(cap * 2 / 3 / d.slots);
+    d.message_cap = static_cast<uint32_t>(cap);
+    d.message_dump = route_dump_index(cap * p.owners, kRouteDump);
+    d.bitmap = bitmap;
+    d.bitmap_bits = 32 * (bitmap_words + words);
+    d.words = bitmap + bitmap_words;
+    d.list = list;
+    d.layer_sizes = sizes;
+    for (uint32_t*& m : d.messages) m = reinterpret_cast<uint32_t*>(part(each));
+    std::memcpy(d.rank_gen, gens.of, sizeof d.rank_gen);
+  }
+
   // Installs every descriptor admitted or released since the last flush
   // (the latest content per slot) with one upload and two kernels: the
   // visited sets of the admitted ones are emptied, then the descriptors are
@@ -609,6 +563,13 @@ class BatchEngine {
     uint32_t n = 0;
     uint64_t clear_bytes = 0;  // largest visited set to empty
     BatchInstall* req = reinterpret_cast<BatchInstall*>(host_stage_ + slots_n_);
+    // How many instances run from here on decides how finely the new ones
+    // are split.
+    uint32_t running = 0;
+    for (uint32_t s = 0; s < slots_n_; ++s)
+      running += pending_[s] == kInstallSeed || (slots_[s].used && (host_inst_[s].status & kInstActive));
+    for (uint32_t s = 0; s < slots_n_; ++s)
+      if (pending_[s] == kInstallSeed && owned_wanted_[s]) lay_out_owned(s, running);
     for (uint32_t s = 0; s < slots_n_; ++s) {
       if (pending_[s] == kNothing) continue;
       const BatchInstance& d = host_inst_[s];
@@ -685,13 +646,13 @@ class BatchEngine {
   struct Job {
     Graph graph;
     uint32_t visited = 0, max_layers = 0, scale = 1, restarts = 0;
+    bool shared = false;  // not by owners (again)
   };
 
   int device_ = 0;
-  hipStream_t stream_ = nullptr, owned_stream_ = nullptr;
-  RankRecords records_;
-  std::vector<std::unique_ptr<OwnedInstance>> owned_;  // per slot: null for instances in the graph
-  uint32_t slots_n_ = 0, grid_ = 0, clear_grid_ = 0, layers_per_graph_ = kLayersPerGraph;
+  hipStream_t stream_ = nullptr;
+  std::vector<uint8_t> owned_wanted_;  // per slot: laid out for owners by the next flush, if its block holds that
+  uint32_t slots_n_ = 0, grid_ = 0, clear_grid_ = 0, owned_grid_ = 0, layers_per_graph_ = kLayersPerGraph;
   uint32_t threads_ = 256, hash_load_pct_ = 50, layer_pct_ = 30, bitmap_bias_permille_ = 1000;
   uint32_t history_ = 0;
   std::vector<Job> jobs_;

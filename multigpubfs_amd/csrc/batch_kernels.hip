@@ -1,5 +1,5 @@
 // Batched multi-instance BFS kernels.  One layer of every active instance
-// is four launches, all capturable in a hipGraph (no host readback, no
+// is five launches, all capturable in a hipGraph (no host readback, no
 // memset nodes):
 //   batch_tiles  : one block scans the per-instance tile counts
 //                  ceil(count / tile) of the active instances -> prefix,
@@ -13,11 +13,14 @@
 //                  instance's own visited set (Lehmer-rank bitmap or open
 //                  addressing hash with full-key equality) and new ones are
 //                  appended with one atomic per workgroup.
+//   batch_owned  : bitmap instances of some size run by owners of the bitmap
+//                  instead (rank_owner.hip), a workgroup an owner at a time.
 //   batch_finish : one thread per instance records the layer size, swaps the
 //                  frontier buffers and retires finished instances.
 #include <algorithm>
 #include "batch.hpp"
 #include "kernels.hpp"
+#include "rank_device.hpp"
 
 namespace mgbfs {
 
@@ -251,14 +254,18 @@ __global__ __launch_bounds__(1024) void batch_tiles_kernel(const BatchInstance* 
                                                            uint32_t* prefix) {
   __shared__ uint32_t wave_sums[1024 / kWave];
   const uint32_t i = threadIdx.x;
-  uint32_t v = 0, c = 0;
-  if (i < slots && (inst[i].status & kInstActive) && !inst[i].error) {
+  uint32_t v = 0, c = 0, o = 0;
+  if (i < slots && (inst[i].status & kInstActive) && !inst[i].error && inst[i].rank.owners) {
+    o = inst[i].rank.owners;
+  } else if (i < slots && (inst[i].status & kInstActive) && !inst[i].error) {
     v = static_cast<uint32_t>((inst[i].count + tile - 1) / tile);
     if (inst[i].rolling && inst[i].depth >= 2)
       c = static_cast<uint32_t>((inst[i].table_stride + kClearChunk - 1) / kClearChunk);
   }
   block_scan_out(v, slots, wave_sums, prefix);
   block_scan_out(c, slots, wave_sums, prefix + slots + 1);
+  block_scan_out(o, slots, wave_sums, prefix + 2 * (slots + 1));
+  if (i == 0) prefix[kBatchPrefixes * (slots + 1)] = 0;
 }
 
 // Eight waves per SIMD (64 VGPRs, no spills): the grid of 8 blocks per CU
@@ -377,6 +384,94 @@ __global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8
   }
 }
 
+// A step of one owner after the other (BatchInstance: `rank` and below).
+// Blocks take owners from a counter: an owner's work goes with its layer,
+// and instances of several sizes run together.  What bounds it and what it
+// measured: rank_owner.hip.
+__global__ __launch_bounds__(kRouteThreads)
+    __attribute__((amdgpu_waves_per_eu(4))) void batch_owned_kernel(BatchInstance* inst, uint32_t slots,
+                                                                    uint32_t* prefix) {
+  __shared__ alignas(16) char lds[sizeof(TileLds)];
+  __shared__ RankGenerator gen[kBatchMaxGens];
+  __shared__ uint32_t rows, task;
+  const uint32_t* opre = prefix + 2 * (slots + 1);
+  uint32_t* counter = prefix + kBatchPrefixes * (slots + 1);
+  const uint32_t total = opre[slots];
+  while (total) {
+    __syncthreads();  // the last owner's LDS is read
+    if (threadIdx.x == 0) task = atomicAdd(counter, 1u);
+    __syncthreads();
+    const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(task)));  // uniform
+    if (t >= total) return;
+    uint32_t lo = 0, hi = slots - 1;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi + 1) / 2;
+      if (opre[mid] <= t) lo = mid;
+      else hi = mid - 1;
+    }
+    lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lo)));
+    BatchInstance& s = inst[lo];
+    const uint32_t f = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t - opre[lo])));
+    const RankPlan p = s.rank;
+    const OwnedWords w(s.words, p);
+    const uint32_t parity = s.parity, depth = s.depth, cap = s.message_cap;
+    const bool unfinished = s.unfinished != 0;
+    uint32_t* list = s.list + static_cast<uint64_t>(f) * p.list_cap;
+    const uint32_t c = min(w.count[parity][f * p.count_stride], cap);
+    uint32_t first = w.sent[f], end = w.end[f];
+    if (threadIdx.x == 0) rows = w.rows[f];
+    for (uint32_t i = threadIdx.x; i < kBatchMaxGens * sizeof(RankGenerator) / 4; i += kRouteThreads)
+      reinterpret_cast<uint32_t*>(gen)[i] = reinterpret_cast<const uint32_t*>(s.rank_gen)[i];
+    __syncthreads();
+    if (c)
+      rank_claim(lds, &rows, p, s.bitmap + static_cast<uint64_t>(f) * p.slice_words,
+                 s.messages[parity] + static_cast<uint64_t>(f) * cap, c, list);
+    const uint32_t have = rows;
+    if (!unfinished) {  // the claimed states are the next layer
+      first = end;
+      end = have;
+    }
+    const uint32_t upto = end - first > s.chunk ? first + s.chunk : end;
+    if (threadIdx.x == 0) {
+      w.count[parity][f * p.count_stride] = 0;
+      w.rows[f] = have;
+      w.sent[f] = upto;
+      w.end[f] = end;
+      if (!unfinished) {
+        w.first[((depth + 1) & 3u) * p.owners + f] = first;
+        if (end != first) atomicAdd(&s.next_count, static_cast<unsigned long long>(end - first));
+      }
+      if (upto != end) atomicOr(&s.more, 1u);
+    }
+    if (upto != first) {
+      __syncthreads();  // the slice is stored, the list is in place
+      const RankOut o{s.messages[parity ^ 1u], w.count[parity ^ 1u], cap, s.message_dump, &s.error, kErrFutureCap,
+                      s.generators, s.slots};
+      (void)rank_send(lds, gen, p, f, list, first, upto, o);
+    }
+  }
+}
+
+__global__ __launch_bounds__(kRouteThreads) void batch_owned_export_kernel(RankPlan p, uint32_t* words, uint32_t depth,
+                                                                           const uint32_t* list, uint64_t limit,
+                                                                           uint64_t* keys) {
+  __shared__ uint32_t sums[kRouteThreads / kWave];
+  const OwnedWords w(words, p);
+  const uint32_t* lo = w.first + (depth & 3u) * p.owners;
+  const uint32_t f = blockIdx.x;
+  uint32_t before = 0;
+  for (uint32_t j = threadIdx.x; j < f; j += kRouteThreads) before += w.end[j] - lo[j];
+  before = wave_incl_scan(before);
+  if ((threadIdx.x & (kWave - 1)) == kWave - 1) sums[threadIdx.x / kWave] = before;
+  __syncthreads();
+  before = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kRouteThreads / kWave; ++k) before += sums[k];
+  const uint32_t* from = list + static_cast<uint64_t>(f) * p.list_cap + lo[f];
+  for (uint32_t i = threadIdx.x; i < w.end[f] - lo[f]; i += kRouteThreads)
+    if (before + i < limit) keys[before + i] = key_of(unrank((from[i] >> 4) * p.owners + f, p.degree));
+}
+
 __global__ void batch_finish_kernel(BatchInstance* inst, uint32_t slots, uint32_t* any_active) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= slots) return;
@@ -385,6 +480,16 @@ __global__ void batch_finish_kernel(BatchInstance* inst, uint32_t slots, uint32_
   if (s.error) {
     s.status = kInstDone;
     return;
+  }
+  if (s.rank.owners) {
+    const bool layer = !s.unfinished;
+    s.unfinished = s.more;
+    s.more = 0;
+    s.parity ^= 1u;
+    if (!layer) {
+      atomicOr(any_active, 1u);
+      return;
+    }
   }
   const uint64_t nc = s.next_count;
   if (nc == 0) {
@@ -416,7 +521,32 @@ __global__ void batch_gather_sizes_kernel(const BatchInstance* inst, const uint3
   }
 }
 
+// The start state in its owner's list and its children in the messages; the
+// bitmap and the words are zero.
+__device__ void seed_owned(BatchInstance& s, uint64_t start_key) {
+  const RankPlan p = s.rank;
+  const OwnedWords w(s.words, p);
+  const Bytes start = bytes_of(start_key);
+  const Place at = place_of(rank_of(start), p.owners, p.magic);
+  s.bitmap[static_cast<uint64_t>(at.owner) * p.slice_words + (at.position >> 5)] = 1u << (at.position & 31u);
+  s.list[static_cast<uint64_t>(at.owner) * p.list_cap] = at.position << 4;
+  w.rows[at.owner] = w.sent[at.owner] = w.end[at.owner] = 1;
+  for (uint32_t g = 0; g < s.generators; ++g) {
+    const Place to = place_of(rank_of(child_of(start, s.rank_gen[g])), p.owners, p.magic);
+    uint32_t& n = w.count[0][to.owner * p.count_stride];
+    if (n < s.message_cap)
+      s.messages[0][static_cast<uint64_t>(to.owner) * s.message_cap + n++] = (to.position << 4) | s.rank_gen[g].tag;
+  }
+  s.count = 1;
+  s.next_count = 0;
+  s.depth = s.parity = s.more = s.unfinished = 0;
+  s.layer_sizes[0] = 1;
+  s.error = 0;
+  s.status = kInstActive;
+}
+
 __device__ void seed_instance(BatchInstance& s, uint64_t start_key) {
+  if (s.rank.owners) return seed_owned(s, start_key);
   uint32_t err = 0;
   const bool claimed = s.visited == kVisHash && s.rolling ? table_claim(s.table, s.table_slots, start_key, err, s.table_slots)
                                                           : batch_claim(s, start_key, err);
@@ -505,6 +635,19 @@ hipError_t batch_clear(const BatchInstance* inst, uint32_t slots, const uint32_t
                        hipStream_t stream) {
   if (slots == 0 || slots > kBatchMaxSlots || grid == 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(batch_clear_kernel, dim3(grid), dim3(256), 0, stream, inst, slots, prefix + slots + 1);
+  return hipGetLastError();
+}
+
+hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, uint32_t grid, hipStream_t stream) {
+  if (slots == 0 || slots > kBatchMaxSlots || grid == 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(batch_owned_kernel, dim3(grid), dim3(kRouteThreads), 0, stream, inst, slots, prefix);
+  return hipGetLastError();
+}
+
+hipError_t batch_owned_export(const BatchInstance& s, uint64_t limit, uint64_t* keys, hipStream_t stream) {
+  if (!s.rank.owners) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(batch_owned_export_kernel, dim3(s.rank.owners), dim3(kRouteThreads), 0, stream, s.rank, s.words,
+                     s.depth, s.list, limit, keys);
   return hipGetLastError();
 }
 

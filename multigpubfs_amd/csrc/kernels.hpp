@@ -190,10 +190,11 @@ struct RankLayer {
   uint64_t seq;
 };
 
-RankPlan rank_plan(uint32_t degree);
+RankPlan rank_plan(uint32_t degree, uint32_t owners = 0);  // owners 0: those of a search alone
 hipError_t rank_seed(const RankPlan& p, uint64_t start_key, uint32_t* bitmap, uint32_t* list, uint32_t* ends,
                      hipStream_t stream);
-RankGenerators rank_generators(const PackedGenerators& gens);
+// tags: of the children each generator makes.
+RankGenerators rank_generators(const PackedGenerators& gens, const uint8_t* tags);
 hipError_t rank_layer(const RankLayer& a, const RankGenerators& gens, hipStream_t stream);
 // Up to `limit` states of the layer [lo, hi) as packed keys.
 hipError_t rank_export(const RankPlan& p, const uint32_t* list, const uint32_t* lo, const uint32_t* hi, uint64_t limit,

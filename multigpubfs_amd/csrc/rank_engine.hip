@@ -41,7 +41,7 @@ void RankRun::set_graph(const Graph& g) {
     const std::vector<int> inv = inverse_index(gens);
     for (uint32_t a = 0; a < gens.count; ++a) gens.child_tag[a] = inv[a] >= 0 ? static_cast<uint8_t>(inv[a] + 1) : 0;
   }
-  gens_ = rank_generators(gens);
+  gens_ = rank_generators(gens, gens.child_tag);
   start_key_ = g.start_key();
 }
 

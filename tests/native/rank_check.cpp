@@ -50,7 +50,7 @@ int main() {
       for (uint32_t i = 0; i < n; ++i) gens.src[g][i] = static_cast<uint8_t>(perm[i]);
       gens.child_tag[g] = static_cast<uint8_t>(g % 3);
     }
-    const RankGenerators by = rank_generators(gens);
+    const RankGenerators by = rank_generators(gens, gens.child_tag);
     if (by.count != gens.count || by.tagged != 10) return 7;
     for (uint32_t i = 0; i < 100000; ++i) {
       const uint32_t r = i < 50000 && i < total ? i : i == 60000 ? total - 1 : rng() % total;

@@ -229,11 +229,11 @@ def test_batch_options_are_validated():
         BatchEngine(max_slots=2, history="three")
 
 
-# Bitmap instances of degree 11 and 12 run by owners of the bitmap beside the
-# graph of the others: alone and in a mix, stopped at a layer limit (one short
-# of the search, its exact length), released half way, and with more children
-# in a layer (up to 10 per state of the group) than their messages hold, where they start over.
-def test_large_bitmap_instances_run_beside_the_graph():
+# Bitmap instances of degree 9 to 12 run by owners of the bitmap: alone and in
+# a mix, stopped at a layer limit (one short of the search, its exact length),
+# released half way, and with more children in a layer (up to 10 per state of
+# the group) than their messages hold at a time.
+def test_large_bitmap_instances_by_owners():
     n = 11
     lrx_gens = O.lrx_generators(n)
     rng = random.Random(8)
@@ -259,6 +259,31 @@ def test_large_bitmap_instances_run_beside_the_graph():
     assert [bool(r[2]) for r in results] == [False, False, True, False, False]
     assert len(last) == ref[-1] and all(sorted(row) == list(range(n)) for row in last)
     assert all(i["visited"] == "bitmap" and i["restarts"] == 0 and i["history_layers"] == 0 for i in infos)
+
+
+@pytest.mark.parametrize("n,count,closed,copies", [(8, 3, False, 1), (9, 1, True, 1), (9, 16, False, 1),
+                                                   (9, 14, False, 9), (10, 2, False, 1), (10, 5, True, 21)])
+def test_owned_instances_match_oracle_layer_by_layer(n, count, closed, copies):
+    # 1, 9 and 21 instances: 251, 101 and 53 owners (degree 8: none); back
+    # edges named (closed sets up to 14) or not; the current layer's states
+    # after every step, whole where the layer is small.
+    rng = random.Random(n * count)
+    gens = [rng.sample(range(n), n) for _ in range(count)]
+    if closed:
+        gens += [[g.index(i) for i in range(n)] for g in gens]
+    ref = O.packed_bfs(n, gens, keep_keys=True)
+    seen = 0
+    with BatchEngine(max_slots=32, layers_per_graph=1) as b:
+        slots = [b.admit(GraphDefinition.permutation(gens, list(range(n)))) for _ in range(copies)]
+        while b.step(1):
+            d = len(b.result(slots[-1])[0]) - 1
+            rows = [O.pack(r) for r in b.sample(slots[-1], n, 2000)]
+            assert len(rows) == min(2000, ref["layers"][d]) == len(set(rows))
+            assert set(rows) <= set(ref["keys"][d])
+            seen += 1
+        assert [b.result(s)[0] for s in slots] == [ref["layers"]] * copies
+        assert {O.pack(r) for r in b.sample(slots[0], n, 10**6)} == set(ref["keys"][-1])
+    assert seen >= len(ref["layers"]) - 1
 
 
 # Arena chunks outlive their engine in a bounded cache: later engines (with
