@@ -29,7 +29,7 @@ uint64_t RankRun::words_bytes(const RankPlan& p) {
 
 uint32_t RankRun::first_cap(const RankPlan& p, uint32_t generators) {
   return std::min(last_cap(p, generators),
-                  static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators / 5 + 1027) / 4 * 4));
+                  static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators * (p.degree <= 10 ? 2 : 1) / 5 + 1027) / 4 * 4));
 }
 uint32_t RankRun::last_cap(const RankPlan& p, uint32_t generators) {
   return static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(p.list_cap) * generators + 3, 1u << 30) / 4 * 4);

@@ -32,8 +32,10 @@ class RankRun {
   explicit RankRun(uint32_t degree) : plan(rank_plan(degree)) {}
   static uint64_t words_bytes(const RankPlan& p);
   // Messages per owner: at first a fifth of all children there can be (the
-  // widest LRX layer sends 15% of them), at most all of them (a state is a
-  // child of `generators` states).
+  // widest LRX layer sends 15% of them), two fifths up to degree 10, where
+  // memory is small (random sets' layers: engines created, run and dropped
+  // for sets of degree 9 and 10 1.85 -> 1.22 ms each, without the growing);
+  // at most all of them (a state is a child of `generators` states).
   static uint32_t first_cap(const RankPlan& p, uint32_t generators);
   static uint32_t last_cap(const RankPlan& p, uint32_t generators);
 
