@@ -121,7 +121,7 @@ typedef struct mgbfs_engine_info {
  * GenericDistributedMemoryPlan (crates/mgbfs-runtime/src/generic_memory.rs:
  * 36-49, generic_distributed_memory.rs:7-13) for the backend this library
  * would pick.  (An engine created with MGBFS_BACKEND_AUTO runs inverse-closed
- * permutations of degree 8 to 12 on the bitmap backend where its memory fits
+ * permutations of degree 3 to 12 on the bitmap backend where its memory fits
  * the budget and no capacity is set; their plan is the sorted backend's,
  * which takes them otherwise.)  With options->vram_budget = 0 the budget is the device's free
  * memory minus the 2 GiB (or 256 MiB, MGBFS_FLAG_MAX_CAPACITY) reserve. */

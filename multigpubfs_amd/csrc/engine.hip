@@ -550,7 +550,7 @@ static uint32_t choose_backend(const Graph& g, uint32_t requested) {
 // The sorted backend, handing the run to the segmented backend when a
 // layer exceeds its limits (its last two layers become the segmented
 // backend's banks; the sorted engine and its memory are released).  Where
-// the library picks the backend, permutations of degree 8 to 12 run by
+// the library picks the backend, permutations of degree 3 to 12 run by
 // owners of the bitmap instead (rank_bitmap_for_auto), and what they report
 // is the bitmap backend's.
 class HandoverEngine final : public Engine {

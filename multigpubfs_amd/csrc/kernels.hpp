@@ -190,12 +190,32 @@ struct RankLayer {
   uint64_t seq;
 };
 
-RankPlan rank_plan(uint32_t degree, uint32_t owners = 0);  // owners 0: those of a search alone
+// One owner (degrees up to kRankBlockDegree): layers [depth, target)
+// expanded in one launch by one workgroup.  sizes[i] (pinned, kRankBlockLayers)
+// is the size of layer depth + 1 + i, the last of them 0 when the search ended;
+// the record has their number in N and the start time in stamps[0].
+constexpr uint32_t kRankBlockDegree = 8;
+constexpr uint32_t kRankBlockLayers = 4096;
+
+struct RankBlock {
+  RankPlan plan;
+  uint32_t tagged;  // every state but the start has a tag
+  uint32_t* bitmap;
+  uint32_t* list;
+  uint32_t* ends;   // list end after layer d at ends[d % 4], 0 before layer 0
+  uint32_t depth, target;
+  uint32_t* sizes;
+  LayerRecord* rec;
+  uint64_t seq;
+};
+
+RankPlan rank_plan(uint32_t degree, uint32_t owners = 0);  // owners 0: those of a large search alone
 hipError_t rank_seed(const RankPlan& p, uint64_t start_key, uint32_t* bitmap, uint32_t* list, uint32_t* ends,
                      hipStream_t stream);
 // tags: of the children each generator makes.
 RankGenerators rank_generators(const PackedGenerators& gens, const uint8_t* tags);
 hipError_t rank_layer(const RankLayer& a, const RankGenerators& gens, hipStream_t stream);
+hipError_t rank_block(const RankBlock& a, const RankGenerators& gens, hipStream_t stream);
 // Up to `limit` states of the layer [lo, hi) as packed keys.
 hipError_t rank_export(const RankPlan& p, const uint32_t* list, const uint32_t* lo, const uint32_t* hi, uint64_t limit,
                        uint64_t* keys, hipStream_t stream);

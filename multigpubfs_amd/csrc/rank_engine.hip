@@ -16,7 +16,9 @@ namespace mgbfs {
 // ------------------------------------------------------------ one search
 
 RankRecords::RankRecords() {
-  MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec), sizeof(LayerRecord) * kRing, hipHostMallocDefault));
+  MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec), sizeof(LayerRecord) * kRing + 4 * kRankBlockLayers,
+                          hipHostMallocDefault));
+  sizes = reinterpret_cast<uint32_t*>(rec + kRing);
   std::memset(rec, 0, sizeof(LayerRecord) * kRing);
 }
 RankRecords::~RankRecords() {
@@ -28,20 +30,38 @@ uint64_t RankRun::words_bytes(const RankPlan& p) {
 }
 
 uint32_t RankRun::first_cap(const RankPlan& p, uint32_t generators) {
-  return std::min(last_cap(p, generators),
-                  static_cast<uint32_t>((static_cast<uint64_t>(p.list_cap) * generators * (p.degree <= 10 ? 2 : 1) / 5 + 1027) / 4 * 4));
+  if (p.owners == 1) return 0;
+  const uint64_t fifth = static_cast<uint64_t>(p.list_cap) * generators / 5;
+  return std::min(last_cap(p, generators), static_cast<uint32_t>((fifth * (p.degree <= 10 ? 2 : 1) + 1027) / 4 * 4));
 }
 uint32_t RankRun::last_cap(const RankPlan& p, uint32_t generators) {
   return static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(p.list_cap) * generators + 3, 1u << 30) / 4 * 4);
 }
 
-void RankRun::set_graph(const Graph& g) {
+static RankGenerators generators_of(const Graph& g) {
   PackedGenerators gens = g.packed_generators();
   if (gens.count <= 14) {
     const std::vector<int> inv = inverse_index(gens);
     for (uint32_t a = 0; a < gens.count; ++a) gens.child_tag[a] = inv[a] >= 0 ? static_cast<uint8_t>(inv[a] + 1) : 0;
   }
-  gens_ = rank_generators(gens, gens.child_tag);
+  return rank_generators(gens, gens.child_tag);
+}
+
+// Children per state but the start: where all have a tag, not the one back.
+static uint32_t slots_of(const RankGenerators& gens) {
+  return gens.tagged == gens.count && gens.count > 1 ? gens.count - 1 : gens.count;
+}
+
+// A child takes the one workgroup 1.4 ns, a layer over 251 owners 8 us: LRX 8
+// (81 thousand children, 29 layers) 120 against 228 us, but seven children a
+// state in 10 layers 221 against 90.  Degree 7 stays below the line with any
+// generators.
+uint32_t RankRun::owners_for(const Graph& g) {
+  return g.elements <= kRankBlockDegree && factorial_u64(g.elements) * slots_of(generators_of(g)) <= 100000 ? 1 : 0;
+}
+
+void RankRun::set_graph(const Graph& g) {
+  gens_ = generators_of(g);
   start_key_ = g.start_key();
 }
 
@@ -80,7 +100,7 @@ RankLayer RankRun::layer_args(uint64_t d, LayerRecord* rec, uint64_t seq) {
   RankLayer a{};
   a.plan = plan;
   a.claim = 1;
-  a.slots = gens_.tagged == gens_.count && gens_.count > 1 ? gens_.count - 1 : gens_.count;
+  a.slots = slots_of(gens_);
   a.in = memory.messages[parity_];
   a.in_count = counts(parity_);
   a.in_cap = memory.cap;
@@ -103,6 +123,7 @@ RankLayer RankRun::layer_args(uint64_t d, LayerRecord* rec, uint64_t seq) {
 // The record of layer d, numbered base + d, is written by the launch of
 // layer d + 1, or by a report after the last.
 int RankRun::run(uint64_t target, RankRecords& records, hipStream_t stream) {
+  if (plan.owners == 1) return run_block(target, records, stream);
   constexpr uint32_t kRing = RankRecords::kRing;
   const uint64_t d0 = layers.size() - 1, base = records.base += 1ull << 32;
   auto rec = [&](uint64_t d) { return records.rec + d % kRing; };
@@ -131,6 +152,32 @@ int RankRun::run(uint64_t target, RankRecords& records, hipStream_t stream) {
   }
 }
 
+// As run(), by one workgroup.
+int RankRun::run_block(uint64_t target, RankRecords& records, hipStream_t stream) {
+  while (layers.size() - 1 < target) {
+    const uint64_t depth = layers.size() - 1, seq = records.base += 1ull << 32;
+    RankBlock a{};
+    a.plan = plan;
+    a.tagged = slots_of(gens_) != gens_.count;
+    a.bitmap = memory.bitmap;
+    a.list = memory.list;
+    a.ends = ends(0);
+    a.depth = static_cast<uint32_t>(depth);
+    a.target = static_cast<uint32_t>(std::min<uint64_t>(target, depth + kRankBlockLayers));
+    a.sizes = records.sizes;
+    a.rec = records.rec;
+    a.seq = seq;
+    MGBFS_HIP(rank_block(a, gens_, stream));
+    const LayerRecord& got = await(*records.rec, seq, stream);
+    seconds += static_cast<double>(got.ticks - got.stamps[0]) * tick_seconds;
+    for (uint64_t i = 0; i < got.N; ++i) {
+      if (records.sizes[i] == 0) return MGBFS_COMPLETE;
+      layers.push_back(records.sizes[i]);
+    }
+  }
+  return MGBFS_LAYER;
+}
+
 const LayerRecord& RankRun::await(const LayerRecord& rec, uint64_t seq, hipStream_t stream) {
   auto there = [&] { return __atomic_load_n(&rec.seq, __ATOMIC_ACQUIRE) == seq; };
   while (true) {
@@ -152,7 +199,7 @@ void RankRun::export_layer(uint64_t back, uint64_t limit, uint64_t* keys, hipStr
 
 class RankBitmapEngine final : public Engine {
  public:
-  RankBitmapEngine(const Graph& g, const mgbfs_engine_options& o) : n_(g.elements), run_(g.elements) {
+  RankBitmapEngine(const Graph& g, const mgbfs_engine_options& o) : n_(g.elements), run_(g) {
     device_ = o.device;
     backend = MGBFS_BACKEND_BITMAP;
     set_graph(g);
@@ -300,14 +347,13 @@ bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o) {
 }
 
 // Inverse-closed graphs whose backend the library picks run by owners of the
-// bitmap from degree 8 on (sorted -> owners, warm: LRX 8 0.36 -> 0.23 ms, 9
-// 0.47 -> 0.31, 10 0.65 -> 0.48, 11 2.9 -> 1.3, 12 13.7 -> 10.5; Coxeter 11
-// 5.5 -> 3.0, 12 96 -> 33; four random generators with inverses, 11 4.9 ->
-// 1.8); below, the sorted backend's single workgroup does (LRX 7 0.145
-// against 0.162 ms, 4 0.036 against 0.054).
+// bitmap (sorted -> owners, warm: LRX 4 0.037 -> 0.014 ms, 7 0.145 -> 0.038,
+// 8 0.36 -> 0.12, 9 0.42 -> 0.31, 10 0.65 -> 0.48, 11 2.5 -> 1.3, 12 13.5 ->
+// 10.5; Coxeter 6 0.11 -> 0.02, 11 5.5 -> 3.0, 12 96 -> 33; four random
+// generators with inverses, 11 5.1 -> 1.9).
 // A set that is only declared closed keeps the sorted backend's retention.
 bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o) {
-  if (o.backend != MGBFS_BACKEND_AUTO || !g.inverse_closed || g.elements < 8 || !g.packable() || !g.distinct_perm() ||
+  if (o.backend != MGBFS_BACKEND_AUTO || !g.inverse_closed || !g.packable() || !g.distinct_perm() ||
       (o.flags & ~MGBFS_FLAG_MAX_CAPACITY) || !rank_bitmap_takes(g, o))
     return false;
   for (int at : inverse_index(g.packed_generators()))

@@ -20,7 +20,7 @@
 //
 // Whole LRX searches, one shared bitmap -> owners: degree 12 33.0 -> 10.6
 // ms, 11 4.77 -> 1.32 ms, 10 2.04 -> 0.48 ms, 9 1.44 -> 0.31 ms, 8 0.77 ->
-// 0.23 ms, 3 0.16 -> 0.03 ms; [L, X] of degree 10 3.41 -> 0.65 ms.  S_11's
+// 0.23 ms (less by one workgroup, below); [L, X] of degree 10 3.41 -> 0.65 ms.  S_11's
 // widest layer (3.05 M states, 6.1 M messages) takes 61 us, 445 VALU
 // instructions a state: half of the wave cycles wait at the routing's
 // barriers, global traffic (30 MB of messages and states, 10 MB of slices)
@@ -34,6 +34,9 @@
 namespace mgbfs {
 
 namespace {
+
+constexpr uint32_t kBlockRunThreads = 1024;
+constexpr uint32_t kBlockRunWords = 1264;  // 8! bits, rounded up
 
 __global__ void rank_seed_kernel(RankPlan p, uint64_t start_key, uint32_t* bitmap, uint32_t* list, uint32_t* ends) {
   if (threadIdx.x != 0) return;
@@ -97,6 +100,79 @@ __global__ __launch_bounds__(kRouteThreads)
   }
 }
 
+// Small searches by one workgroup: the bitmap (5 KB at degree 8) in LDS, no
+// messages, layer after layer in one launch.  Threads take children one each
+// while a layer has at most one for every thread, and parents otherwise
+// (rebuilt once).  251 owners -> one workgroup, whole searches: LRX 4 54 -> 14
+// us, 7 162 -> 38, 8 228 -> 120 (29 layers of 4 us: two dependent LDS steps,
+// the list's round trip through L2 and 1.4 parents a thread).
+__global__ __launch_bounds__(kBlockRunThreads) void rank_block_kernel(RankBlock a, RankGenerators gens) {
+  __shared__ alignas(16) uint32_t bits[kBlockRunWords];
+  __shared__ RankGenerator gen[kMaxGenerators];
+  __shared__ uint32_t rows;
+  const RankPlan p = a.plan;
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const unsigned long long began = wall_clock64();
+  for (uint32_t i = threadIdx.x; i < p.slice_words; i += kBlockRunThreads) bits[i] = a.bitmap[i];
+  for (uint32_t i = threadIdx.x; i < kMaxGenerators * sizeof(RankGenerator) / 4; i += kBlockRunThreads)
+    reinterpret_cast<uint32_t*>(gen)[i] = reinterpret_cast<const uint32_t*>(gens.of)[i];
+  uint32_t start = a.depth ? a.ends[(a.depth - 1) & 3u] : 0u, end = a.ends[a.depth & 3u];
+  if (threadIdx.x == 0) rows = end;
+  __syncthreads();
+  // Claims a child and appends it (whole waves come here).
+  auto claim = [&](bool valid, const Bytes& parent, uint32_t g) {
+    const RankGenerator& by = gen[g];
+    const uint32_t r = rank_of(child_of(parent, by)), bit = 1u << (r & 31u);
+    const bool fresh = valid && !(atomicOr(&bits[r >> 5], bit) & bit);
+    const uint64_t b = __ballot(fresh);
+    uint32_t at = 0;
+    if (lane == 0 && b) at = atomicAdd(&rows, static_cast<uint32_t>(__popcll(b)));
+    at = __shfl(at, 0, kWave) + static_cast<uint32_t>(__popcll(b & ((1ull << lane) - 1)));
+    if (fresh) a.list[at] = (r << 4) | by.tag;
+  };
+  uint32_t d = a.depth, run = 0;
+  while (d < a.target) {
+    const bool all = d == 0 || !a.tagged;
+    const uint32_t S = all ? gens.count : gens.count - 1, n = end - start;
+    if (n * S <= kBlockRunThreads) {
+      if (threadIdx.x / kWave * kWave < n * S) {
+        const uint32_t i = min(threadIdx.x, n * S - 1), at = i / S, j = i - at * S;
+        const uint32_t m = a.list[start + at], tag = m & 15u;
+        const uint32_t g = all ? j : j + (j + 1 >= tag ? 1u : 0u);
+        claim(threadIdx.x < n * S && !(all && g + 1 == tag), unrank(m >> 4, p.degree), g);
+      }
+    } else {
+      for (uint32_t i = threadIdx.x; i / kWave * kWave < n; i += kBlockRunThreads) {
+        const uint32_t m = a.list[start + min(i, n - 1)], tag = m & 15u;
+        const Bytes parent = unrank(m >> 4, p.degree);
+        for (uint32_t j = 0; j < S; ++j) {
+          const uint32_t g = all ? j : j + (j + 1 >= tag ? 1u : 0u);
+          claim(i < n && !(all && g + 1 == tag), parent, g);
+        }
+      }
+    }
+    __syncthreads();
+    start = end;
+    end = rows;
+    ++d;
+    if (threadIdx.x == 0) {
+      a.ends[d & 3u] = end;
+      a.sizes[run] = end - start;
+    }
+    ++run;
+    if (end == start) break;
+    __syncthreads();  // everyone has read the list's length
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < p.slice_words; i += kBlockRunThreads) a.bitmap[i] = bits[i];
+  if (threadIdx.x == 0) {
+    a.rec->N = run;
+    a.rec->stamps[0] = began;
+    a.rec->ticks = wall_clock64();
+    __hip_atomic_store(&a.rec->seq, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // States [first, last) of a layer, as packed keys in any order: owner f's
 // part of the layer is list rows [lo[f], hi[f]).
 __global__ __launch_bounds__(kRouteThreads) void rank_export_kernel(RankPlan p, const uint32_t* list,
@@ -143,6 +219,16 @@ hipError_t rank_layer(const RankLayer& a, const RankGenerators& gens, hipStream_
   return hipGetLastError();
 }
 
+hipError_t rank_block(const RankBlock& a, const RankGenerators& gens, hipStream_t stream) {
+  const RankPlan& p = a.plan;
+  if (p.owners != 1 || p.degree < 3 || p.degree > kRankBlockDegree || p.slice_words > kBlockRunWords ||
+      gens.count == 0 || gens.count > kMaxGenerators || a.target <= a.depth || a.target - a.depth > kRankBlockLayers ||
+      (a.tagged && gens.count < 2))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rank_block_kernel, dim3(1), dim3(kBlockRunThreads), 0, stream, a, gens);
+  return hipGetLastError();
+}
+
 hipError_t rank_export(const RankPlan& p, const uint32_t* list, const uint32_t* lo, const uint32_t* hi, uint64_t limit,
                        uint64_t* keys, hipStream_t stream) {
   hipLaunchKernelGGL(rank_export_kernel, dim3(p.owners), dim3(kRouteThreads), 0, stream, p, list, lo, hi, limit, keys);
@@ -183,7 +269,7 @@ RankPlan rank_plan(uint32_t degree, uint32_t owners) {
   // 1.34, 12 10.83 / 10.57 / 11.11 / 11.22, where tiles are many and the
   // lines touched count).
   p.count_stride = degree <= 10 ? 32 : (degree == 11 ? 16 : 8);
-  p.magic = static_cast<uint32_t>((1ull << 32) / p.owners);
+  p.magic = p.owners == 1 ? ~0u : static_cast<uint32_t>((1ull << 32) / p.owners);
   const uint64_t positions = (factorial_u64(degree) + p.owners - 1) / p.owners;
   p.slice_words = static_cast<uint32_t>((positions + 127) / 128 * 4);
   p.list_cap = static_cast<uint32_t>(positions);

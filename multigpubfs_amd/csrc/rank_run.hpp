@@ -15,6 +15,7 @@ struct RankRecords {
   RankRecords(const RankRecords&) = delete;
   RankRecords& operator=(const RankRecords&) = delete;
   LayerRecord* rec = nullptr;
+  uint32_t* sizes = nullptr;  // kRankBlockLayers, of a run in one launch
   uint64_t base = 0;  // number of a run's layer 0
 };
 
@@ -29,9 +30,11 @@ struct RankMemory {
 class RankRun {
  public:
   static constexpr int kSendAgain = -1;
-  explicit RankRun(uint32_t degree) : plan(rank_plan(degree)) {}
+  explicit RankRun(const Graph& g) : plan(rank_plan(g.elements, owners_for(g))) {}
+  // 1: one workgroup runs the search.  0: the owners of its degree.
+  static uint32_t owners_for(const Graph& g);
   static uint64_t words_bytes(const RankPlan& p);
-  // Messages per owner: at first a fifth of all children there can be (the
+  // Messages per owner (one owner: none): at first a fifth of all children there can be (the
   // widest LRX layer sends 15% of them), two fifths up to degree 10, where
   // memory is small (random sets' layers: engines created, run and dropped
   // for sets of degree 9 and 10 1.85 -> 1.22 ms each, without the growing);
@@ -61,6 +64,7 @@ class RankRun {
   uint32_t* counts(uint32_t parity) { return memory.words + parity * plan.count_stride * plan.owners; }
   uint32_t* ends(uint64_t layer) { return memory.words + (2 * plan.count_stride + layer % kEnds) * plan.owners; }
   OwnerCtl* ctl(uint64_t layer);
+  int run_block(uint64_t target, RankRecords& records, hipStream_t stream);
   void send(uint64_t d, hipStream_t stream);
   RankLayer layer_args(uint64_t d, LayerRecord* rec, uint64_t seq);
   const LayerRecord& await(const LayerRecord& rec, uint64_t seq, hipStream_t stream);
