@@ -16,9 +16,10 @@ namespace mgbfs {
 // ------------------------------------------------------------ one search
 
 RankRecords::RankRecords() {
-  MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec), sizeof(LayerRecord) * kRing + 4 * kRankBlockLayers,
+  MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec), sizeof(LayerRecord) * kRing + 8 * kKeys + 4 * kRankBlockLayers,
                           hipHostMallocDefault));
-  sizes = reinterpret_cast<uint32_t*>(rec + kRing);
+  keys = reinterpret_cast<uint64_t*>(rec + kRing);
+  sizes = reinterpret_cast<uint32_t*>(keys + kKeys);
   std::memset(rec, 0, sizeof(LayerRecord) * kRing);
 }
 RankRecords::~RankRecords() {
@@ -212,7 +213,6 @@ class RankBitmapEngine final : public Engine {
     bitmap_.allocate(4ull * p.owners * p.slice_words);
     list_.allocate(4ull * p.owners * p.list_cap);
     words_.allocate(RankRun::words_bytes(p));
-    keys_.allocate(kKeys * 8);
     run_.memory.bitmap = bitmap_.as<uint32_t>();
     run_.memory.list = list_.as<uint32_t>();
     run_.memory.words = words_.as<uint32_t>();
@@ -273,7 +273,6 @@ class RankBitmapEngine final : public Engine {
   const char* name() const override { return "PERMUTATION_BITMAP_LEHMER"; }
 
  private:
-  static constexpr uint64_t kKeys = 1024;
   void set_graph(const Graph& g) {
     run_.set_graph(g);
     history_layers = g.inverse_closed ? 3 : 0;
@@ -288,7 +287,7 @@ class RankBitmapEngine final : public Engine {
       for (int i = 0; i < 2; ++i) run_.memory.messages[i] = messages_[i].as<uint32_t>();
       run_.memory.cap = cap;
     }
-    device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + keys_.bytes() + messages_[0].bytes() +
+    device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + messages_[0].bytes() +
                    messages_[1].bytes();
   }
   int run_layers(uint32_t most) {
@@ -319,20 +318,25 @@ class RankBitmapEngine final : public Engine {
   // States of the current layer (back = 0) or the one before.
   void export_layer(uint64_t back, uint64_t limit, std::vector<uint64_t>& out) {
     MGBFS_HIP(hipSetDevice(device_));
-    DeviceBuffer large;
-    if (limit > kKeys) large.allocate(limit * 8);
-    uint64_t* keys = limit > kKeys ? large.as<uint64_t>() : keys_.as<uint64_t>();
     out.resize(limit);
     if (!limit) return;
-    run_.export_layer(back, limit, keys, stream_);
-    MGBFS_HIP(hipMemcpyAsync(out.data(), keys, limit * 8, hipMemcpyDeviceToHost, stream_));
+    if (limit <= RankRecords::kKeys) {  // written to pinned memory by the kernel
+      run_.export_layer(back, limit, records_.keys, stream_);
+      MGBFS_HIP(hipStreamSynchronize(stream_));
+      std::copy(records_.keys, records_.keys + limit, out.begin());
+      return;
+    }
+    DeviceBuffer keys;
+    keys.allocate(limit * 8);
+    run_.export_layer(back, limit, keys.as<uint64_t>(), stream_);
+    MGBFS_HIP(hipMemcpyAsync(out.data(), keys.as<void>(), limit * 8, hipMemcpyDeviceToHost, stream_));
     MGBFS_HIP(hipStreamSynchronize(stream_));
   }
 
   uint32_t n_;
   RankRun run_;
   RankRecords records_;
-  DeviceBuffer bitmap_, list_, words_, keys_, messages_[2];
+  DeviceBuffer bitmap_, list_, words_, messages_[2];
 };
 
 // All degrees that ranks and slices are made for: faster from the smallest to

@@ -15,6 +15,8 @@ struct RankRecords {
   RankRecords(const RankRecords&) = delete;
   RankRecords& operator=(const RankRecords&) = delete;
   LayerRecord* rec = nullptr;
+  static constexpr uint64_t kKeys = 1024;
+  uint64_t* keys = nullptr;   // kKeys, of a small sample
   uint32_t* sizes = nullptr;  // kRankBlockLayers, of a run in one launch
   uint64_t base = 0;  // number of a run's layer 0
 };
