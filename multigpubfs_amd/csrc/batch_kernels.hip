@@ -452,15 +452,19 @@ __global__ __launch_bounds__(kRouteThreads)
   }
 }
 
+// States of layer `depth`.  rejected: the search stopped at its layer limit,
+// so the last step has claimed the layer after it too; its first rows are the
+// end of this one.
 __global__ __launch_bounds__(kRouteThreads) void batch_owned_export_kernel(RankPlan p, uint32_t* words, uint32_t depth,
-                                                                           const uint32_t* list, uint64_t limit,
-                                                                           uint64_t* keys) {
+                                                                           uint32_t rejected, const uint32_t* list,
+                                                                           uint64_t limit, uint64_t* keys) {
   __shared__ uint32_t sums[kRouteThreads / kWave];
   const OwnedWords w(words, p);
   const uint32_t* lo = w.first + (depth & 3u) * p.owners;
+  const uint32_t* hi = rejected ? w.first + ((depth + 1) & 3u) * p.owners : w.end;
   const uint32_t f = blockIdx.x;
   uint32_t before = 0;
-  for (uint32_t j = threadIdx.x; j < f; j += kRouteThreads) before += w.end[j] - lo[j];
+  for (uint32_t j = threadIdx.x; j < f; j += kRouteThreads) before += hi[j] - lo[j];
   before = wave_incl_scan(before);
   if ((threadIdx.x & (kWave - 1)) == kWave - 1) sums[threadIdx.x / kWave] = before;
   __syncthreads();
@@ -468,7 +472,7 @@ __global__ __launch_bounds__(kRouteThreads) void batch_owned_export_kernel(RankP
 #pragma unroll
   for (uint32_t k = 0; k < kRouteThreads / kWave; ++k) before += sums[k];
   const uint32_t* from = list + static_cast<uint64_t>(f) * p.list_cap + lo[f];
-  for (uint32_t i = threadIdx.x; i < w.end[f] - lo[f]; i += kRouteThreads)
+  for (uint32_t i = threadIdx.x; i < hi[f] - lo[f]; i += kRouteThreads)
     if (before + i < limit) keys[before + i] = key_of(unrank((from[i] >> 4) * p.owners + f, p.degree));
 }
 
@@ -647,7 +651,7 @@ hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, ui
 hipError_t batch_owned_export(const BatchInstance& s, uint64_t limit, uint64_t* keys, hipStream_t stream) {
   if (!s.rank.owners) return hipErrorInvalidValue;
   hipLaunchKernelGGL(batch_owned_export_kernel, dim3(s.rank.owners), dim3(kRouteThreads), 0, stream, s.rank, s.words,
-                     s.depth, s.list, limit, keys);
+                     s.depth, (s.error & kErrCount) ? 1u : 0u, s.list, limit, keys);
   return hipGetLastError();
 }
 

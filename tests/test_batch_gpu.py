@@ -316,3 +316,20 @@ def test_engines_reuse_kept_memory_exactly():
     for t in threads:
         t.join()
     assert out == {k: [golden[k::2]] * 3 for k in (0, 1)}
+
+
+@pytest.mark.parametrize("n,layers,copies", [(8, 9, 1), (9, 12, 1), (10, 3, 1), (10, 14, 1), (10, 14, 9), (10, 14, 21),
+                                             (11, 13, 1)])
+def test_sample_of_an_instance_stopped_at_its_layer_limit(n, layers, copies):
+    # The step that meets the limit has found the next layer already: the
+    # sample still holds the last layer of the result, and only it.
+    gens = O.lrx_generators(n)
+    ref = O.packed_bfs(n, gens, keep_keys=True)
+    with BatchEngine(max_slots=32, vram_budget=8 << 30) as b:
+        slots = [b.admit(GraphDefinition.permutation(gens, list(range(n))), max_layers=layers) for _ in range(copies)]
+        b.run()
+        for s in slots:
+            sizes, _, error = b.result(s)
+            assert error and sizes == ref["layers"][:layers]
+            rows = [O.pack(r) for r in b.sample(s, n, 10**7)]
+            assert sorted(rows) == sorted(ref["keys"][layers - 1])
