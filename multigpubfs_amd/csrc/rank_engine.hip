@@ -216,8 +216,8 @@ class RankBitmapEngine final : public Engine {
     run_.memory.bitmap = bitmap_.as<uint32_t>();
     run_.memory.list = list_.as<uint32_t>();
     run_.memory.words = words_.as<uint32_t>();
-    ensure_messages(RankRun::first_cap(p, g.generators));
     reset();
+    ensure_messages(wanted_);
   }
   ~RankBitmapEngine() override {
     (void)hipSetDevice(device_);
@@ -234,6 +234,7 @@ class RankBitmapEngine final : public Engine {
   void reset() override {
     MGBFS_HIP(hipSetDevice(device_));
     run_.start(stream_);
+    wanted_ = std::max(run_.memory.cap, RankRun::first_cap(run_.plan, run_.generators()));
     layers = run_.layers;
     candidates = unique_candidates = 0;
     kernel_seconds = 0.0;
@@ -256,8 +257,8 @@ class RankBitmapEngine final : public Engine {
   }
   void rebind(const Graph& g) override {
     if (g.elements != n_ || !g.packable() || !g.distinct_perm()) throw std::runtime_error("ENGINE_REBIND_SHAPE");
-    set_graph(g);
     ensure_messages(RankRun::first_cap(run_.plan, g.generators));
+    set_graph(g);
     reset();
   }
   void layer_keys(std::vector<uint64_t>& out) override { export_layer(0, layers.back(), out); }
@@ -277,43 +278,52 @@ class RankBitmapEngine final : public Engine {
     run_.set_graph(g);
     history_layers = g.inverse_closed ? 3 : 0;
   }
+  void update_bytes() {
+    device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + messages_[0].bytes() + messages_[1].bytes();
+  }
+  // Message buffers of `cap` entries per owner.  The old ones go first (two
+  // pairs of the worst case need not fit), so they are out of the run's reach
+  // before they are freed: when the new ones cannot be had, the run has none,
+  // and its next call asks again.
   void ensure_messages(uint32_t cap) {
     if (cap > run_.memory.cap) {
       const uint64_t entries = static_cast<uint64_t>(run_.plan.owners) * cap + kRouteDump;
       MGBFS_HIP(hipStreamSynchronize(stream_));
-      run_.memory.cap = 0;
+      run_.drop_messages();
       for (auto& m : messages_) m.release();
+      update_bytes();
       for (auto& m : messages_) m.allocate(entries * 4);
       for (int i = 0; i < 2; ++i) run_.memory.messages[i] = messages_[i].as<uint32_t>();
       run_.memory.cap = cap;
     }
-    device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + messages_[0].bytes() +
-                   messages_[1].bytes();
+    update_bytes();
   }
   int run_layers(uint32_t most) {
     MGBFS_HIP(hipSetDevice(device_));
     const uint64_t target = layers.size() - 1 + most;  // depth to reach
-    int s = MGBFS_LAYER;
-    do {
-      s = run_.run(target, records_, stream_);
-      if (s == RankRun::kSendAgain) {
-        const uint32_t last = RankRun::last_cap(run_.plan, run_.generators());
-        if (run_.memory.cap >= last) throw std::runtime_error("BITMAP_MESSAGES");
-        ensure_messages(static_cast<uint32_t>(std::min<uint64_t>(2ull * run_.memory.cap, last)));
-        if (run_.layers.size() - 1 == target) s = MGBFS_LAYER;  // its children are sent by the next call
-      }
-    } while (s == RankRun::kSendAgain);
+    while (true) {
+      ensure_messages(wanted_);
+      const int s = run_.run(target, records_, stream_);
+      take_layers(s == MGBFS_COMPLETE);
+      if (s != RankRun::kSendAgain) return s;
+      const uint32_t last = RankRun::last_cap(run_.plan, run_.generators());
+      if (run_.memory.cap >= last) throw std::runtime_error("BITMAP_MESSAGES");
+      wanted_ = static_cast<uint32_t>(std::min<uint64_t>(2ull * run_.memory.cap, last));
+      if (layers.size() - 1 == target) return MGBFS_LAYER;  // its children are sent by the next call
+    }
+  }
+  // The run's new layers: every layer expanded by its launches, an empty one
+  // at the end too.
+  void take_layers(bool complete) {
     const size_t before = layers.size();
     layers = run_.layers;
     kernel_seconds = run_.seconds;
-    terminal = s == MGBFS_COMPLETE;
-    // Every layer expanded by these launches, an empty one at the end too.
+    terminal = complete;
     for (size_t d = before; d < layers.size() + (terminal ? 1 : 0); ++d) {
       candidates += layers[d - 1] * run_.generators();
       streamed_bytes += 8 * (layers[d - 1] + (d < layers.size() ? layers[d] : 0));
       ++launches;
     }
-    return s;
   }
   // States of the current layer (back = 0) or the one before.
   void export_layer(uint64_t back, uint64_t limit, std::vector<uint64_t>& out) {
@@ -337,6 +347,7 @@ class RankBitmapEngine final : public Engine {
   RankRun run_;
   RankRecords records_;
   DeviceBuffer bitmap_, list_, words_, messages_[2];
+  uint32_t wanted_ = 0;  // messages per owner that the next layers need
 };
 
 // All degrees that ranks and slices are made for: faster from the smallest to

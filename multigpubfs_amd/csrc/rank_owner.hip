@@ -211,7 +211,8 @@ hipError_t rank_layer(const RankLayer& a, const RankGenerators& gens, hipStream_
   const RankPlan& p = a.plan;
   if (p.owners == 0 || p.owners > kOwnersMax || p.degree < 3 || p.degree > kRankDegree || gens.count == 0 ||
       gens.count > kMaxGenerators || a.slots == 0 || a.slots > gens.count || a.slots + 1 < gens.count ||
-      p.slice_words % 4 || p.slice_words * 4ull > sizeof(TileLds) || a.out_cap % 4 || a.in_cap % 4)
+      p.slice_words % 4 || p.slice_words * 4ull > sizeof(TileLds) || !a.out || a.out_cap == 0 || a.out_cap % 4 ||
+      (a.claim && (!a.in || a.in_cap == 0)) || a.in_cap % 4)
     return hipErrorInvalidValue;
   RankLayer b = a;
   b.out_dump = route_dump_index(static_cast<uint64_t>(p.owners) * a.out_cap, kTile);

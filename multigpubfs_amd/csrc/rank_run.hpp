@@ -46,6 +46,12 @@ class RankRun {
 
   void set_graph(const Graph& g);
   void start(hipStream_t stream);
+  // The message buffers go: children sent to them are sent again.
+  void drop_messages() {
+    memory.cap = 0;
+    memory.messages[0] = memory.messages[1] = nullptr;
+    sent_ = false;
+  }
   // Layers up to depth `target`: MGBFS_LAYER there, MGBFS_COMPLETE after the
   // last, kSendAgain when the children of the last layer did not fit the
   // messages (they are sent anew by the next run).  Launches queued past the
