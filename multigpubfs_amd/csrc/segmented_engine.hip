@@ -327,7 +327,9 @@ class SegmentedEngine final : public Engine {
       if (!fits((want - bank.capacity) * elements_ * sizeof(S))) return false;
     }
     MGBFS_HIP(hipStreamSynchronize(stream_));
+    bank.capacity = 0;  // nothing to be used if the allocation throws
     bank.arena.release();
+    update_bytes();
     bank.arena.allocate(want * elements_ * sizeof(S));
     bank.capacity = want;
     update_bytes();

@@ -76,7 +76,6 @@ class SortedEngine final : public Engine {
     general_only_ = flags_ & (MGBFS_FLAG_TEST_COARSE_BUCKETS | MGBFS_FLAG_TEST_TIGHT_SLABS |
                               MGBFS_FLAG_TEST_WIDE_ROUTING | MGBFS_FLAG_TEST_SORTED_CAP);
     update_bytes();
-    if (!grow_bank(0, 1024)) throw std::runtime_error("SORTED_VRAM_CAPACITY");
     reset();
   }
 
@@ -89,6 +88,7 @@ class SortedEngine final : public Engine {
 
   void reset() override {
     MGBFS_HIP(hipSetDevice(device_));
+    if (!grow_bank(0, 1024)) throw std::runtime_error("SORTED_VRAM_CAPACITY");
     cur_ = 0;
     prev_ = -1;
     slack_ = (flags_ & MGBFS_FLAG_TEST_TIGHT_SLABS) ? 0 : 1;
@@ -331,6 +331,7 @@ class SortedEngine final : public Engine {
   // Entries of one slab array (with the routing dump area).
   static constexpr uint64_t owner_entries(uint32_t owners) { return owners * static_cast<uint64_t>(kSlabStride) + kRouteDump; }
   void start_bank() {
+    if (!bank_cap_[0]) throw std::runtime_error("SORTED_VRAM_CAPACITY");  // lost to a growth that failed
     MGBFS_HIP(sorted_start(keymix(start_key_, layout_.km) << layout_.tagbits, bank_[0].as<uint64_t>(),
                            off_[0].as<uint32_t>(), control_.as<uint64_t>(), stream_));
   }
@@ -632,18 +633,24 @@ class SortedEngine final : public Engine {
     }
   }
   // Lane slabs (entries) and sub-bucket slabs (entries); grown, never shrunk.
+  // A buffer goes before its successor is allocated, so its size is 0 until
+  // that is there: a growth that throws leaves nothing to be used.
   bool ensure_slabs(uint64_t lane_entries, uint64_t sub_entries) {
     if (lane_cap_ >= lane_entries && sub_cap_ >= sub_entries) return true;
     uint64_t lane = std::max(lane_cap_, lane_entries), sub = std::max(sub_cap_, sub_entries);
     if (!fits((lane - lane_cap_ + sub - sub_cap_) * 8)) return false;
     MGBFS_HIP(hipStreamSynchronize(stream_));
     if (lane > lane_cap_) {
+      lane_cap_ = 0;
       lane_.release();
+      update_bytes();
       lane_.allocate(lane * 8);
       lane_cap_ = lane;
     }
     if (sub > sub_cap_) {
+      sub_cap_ = 0;
       sub_.release();
+      update_bytes();
       sub_.allocate(sub * 8);
       sub_cap_ = sub;
     }
@@ -656,7 +663,9 @@ class SortedEngine final : public Engine {
     if (!fits((want - bank_cap_[b]) * 8)) want = rows;
     if (!fits((want - bank_cap_[b]) * 8)) return false;
     MGBFS_HIP(hipStreamSynchronize(stream_));
+    bank_cap_[b] = 0;
     bank_[b].release();
+    update_bytes();
     bank_[b].allocate(want * 8);
     bank_cap_[b] = want;
     update_bytes();

@@ -16,6 +16,7 @@ struct Device {
   std::map<char*, size_t> live;  // device allocations
   size_t used = 0, limit = ~static_cast<size_t>(0);
   int current = 0, launches = 0;
+  long room = -1;  // allocations that still succeed (-1: all)
 };
 inline Device& dev() {
   static Device d;
@@ -48,7 +49,8 @@ extern "C" {
 hipError_t hipMalloc(void** p, size_t bytes) {
   fake::Device& d = fake::dev();
   *p = nullptr;
-  if (d.used + bytes > d.limit) return hipErrorOutOfMemory;
+  if (d.used + bytes > d.limit || d.room == 0) return hipErrorOutOfMemory;
+  if (d.room > 0) --d.room;
   *p = std::calloc(1, bytes);
   d.live[static_cast<char*>(*p)] = bytes;
   d.used += bytes;
