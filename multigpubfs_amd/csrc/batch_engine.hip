@@ -300,8 +300,7 @@ class BatchEngine {
   void install(int32_t slot, const BatchPlan& p) {
     const Graph& g = jobs_[slot].graph;
     Slot& sl = slots_[slot];
-    const uint64_t keys_bytes = arena_round(p.cap * 8), sizes_bytes = arena_round(8ull * p.max_layers);
-    sl.block = arena_.take(2 * keys_bytes + sizes_bytes + p.visited_bytes, budget_);
+    sl.block = arena_.take(block_bytes(p), budget_);
     sl.used = true;
     sl.reported = false;
     sl.planned = p.bytes;
@@ -310,6 +309,10 @@ class BatchEngine {
     rows_[slot] = g.rows;
     cols_[slot] = g.cols;
     lay_out(slot, p);
+  }
+
+  static uint64_t block_bytes(const BatchPlan& p) {
+    return 2 * arena_round(p.cap * 8) + arena_round(8ull * p.max_layers) + p.visited_bytes;
   }
 
   void lay_out(int32_t slot, const BatchPlan& p) {
@@ -396,10 +399,15 @@ class BatchEngine {
     const BatchInstance& d = host_inst_[s];
     if (d.rank.owners && (d.error & kErrFutureCap) && !slots_[s].reported) {
       // An owner got more messages than its share with its reserve: once
-      // more over the shared bitmap, in the same block.
+      // more over the shared bitmap, which the block was planned for.  (An
+      // automatic choice made anew, without rolling tables to compare with,
+      // may be a hash table, which the block need not hold.)
       Job& job = jobs_[s];
+      const BatchPlan p = plan_with(job.graph, 1, job.max_layers, false, 1);
+      if (block_bytes(p) > slots_[s].block.bytes) return;
       job.shared = true;
-      lay_out(static_cast<int32_t>(s), plan_with(job.graph, job.visited, job.max_layers, false, 1));
+      ++job.restarts;
+      lay_out(static_cast<int32_t>(s), p);
       return;
     }
     if (!d.rolling || !(d.error & (kErrFutureCap | kErrTableFull)) || slots_[s].reported) return;

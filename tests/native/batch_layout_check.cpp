@@ -1,0 +1,142 @@
+// Host check of the batch engine's layouts (batch_engine.hip) on a HIP
+// runtime in host memory: where an instance's parts lie, alone and after the
+// restart that follows a full message slab, under every choice of history,
+// layer share and bitmap bias.  The kernels only set what the check asks for.
+#include <vector>
+#include "fake_hip.hpp"
+#include "device_cache.hip"
+#include "engine.hip"
+#include "batch_engine.hip"
+#define rank_seed device_rank_seed
+#define rank_layer device_rank_layer
+#define rank_block device_rank_block
+#define rank_export device_rank_export
+#define rank_report device_rank_report
+#include "rank_owner.hip"
+
+using fake::holds;
+using fake::require;
+using namespace mgbfs;
+
+static BatchInstance* inst;  // the device's
+static uint32_t overflow;    // owned instances' next step ends in this error
+static uint32_t slots;
+
+extern "C" hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) {
+  for (uint32_t i = 0; i < slots; ++i)
+    if (inst[i].status & kInstActive) {
+      inst[i].error = inst[i].rank.owners ? overflow : 0;
+      inst[i].status = kInstDone;
+    }
+  return fake::launch(s);
+}
+
+namespace mgbfs {
+hipError_t batch_reset_flag(uint32_t*, hipStream_t) { return hipSuccess; }
+hipError_t batch_tiles(BatchInstance*, uint32_t, uint32_t, uint32_t*, hipStream_t) { return hipSuccess; }
+hipError_t batch_clear(const BatchInstance*, uint32_t, const uint32_t*, uint32_t, hipStream_t) { return hipSuccess; }
+hipError_t batch_expand(BatchInstance*, uint32_t, const uint32_t*, uint32_t, uint32_t, uint32_t, hipStream_t) {
+  return hipSuccess;
+}
+hipError_t batch_owned(BatchInstance*, uint32_t, uint32_t*, uint32_t, hipStream_t) { return hipSuccess; }
+hipError_t batch_finish(BatchInstance*, uint32_t, uint32_t*, hipStream_t) { return hipSuccess; }
+hipError_t batch_clear_visited(const BatchInstance*, const BatchInstall*, uint32_t, uint64_t, hipStream_t s) {
+  return fake::launch(s);
+}
+hipError_t batch_install(BatchInstance* to, const BatchInstance* staged, const BatchInstall* req, uint32_t n,
+                         hipStream_t s) {
+  inst = to;
+  for (uint32_t q = 0; q < n; ++q) {
+    to[req[q].slot] = staged[q];
+    if (req[q].seed) to[req[q].slot].status = kInstActive;
+  }
+  return fake::launch(s);
+}
+hipError_t batch_gather_sizes(const BatchInstance*, const uint32_t*, uint32_t, uint64_t*, hipStream_t s) {
+  return fake::launch(s);
+}
+}  // namespace mgbfs
+
+struct Range {
+  char *from, *to;
+};
+static Range range(const void* p, uint64_t bytes) {
+  char* at = static_cast<char*>(const_cast<void*>(p));
+  return Range{at, at + bytes};
+}
+
+// Everything the kernels may touch of an instance.
+static std::vector<Range> parts(const BatchInstance& d) {
+  std::vector<Range> r{range(d.layer_sizes, 8ull * d.max_layers)};
+  if (d.rank.owners) {
+    const RankPlan& p = d.rank;
+    r.push_back(range(d.bitmap, 4ull * p.owners * p.slice_words));
+    r.push_back(range(d.words, 4 * OwnedWords::words(p)));
+    r.push_back(range(d.list, 4ull * p.owners * p.list_cap));
+    for (uint32_t* m : d.messages) r.push_back(range(m, 4 * (static_cast<uint64_t>(p.owners) * d.message_cap + kRouteDump)));
+    return r;
+  }
+  r.push_back(range(d.front, 8 * d.cap));
+  r.push_back(range(d.next, 8 * d.cap));
+  if (d.visited == kVisBitmap) r.push_back(range(d.bitmap, (d.bitmap_bits + 31) / 32 * 4));
+  else r.push_back(range(d.table, (d.rolling ? 3 : 1) * 8ull * d.table_slots));
+  return r;
+}
+
+int main() {
+  uint32_t owned = 0, restarted = 0;
+  for (uint32_t n : {9u, 10u, 11u})
+    for (uint32_t history : {0u, 1u, 2u})
+      for (uint32_t pct : {1u, 30u, 100u})
+        for (uint32_t bias : {1u, 3u, 5u, 8u, 20u, 1000u})
+          for (uint64_t expected : {0ull, 20000ull, 120000ull, 200000ull}) {
+            Graph g;
+            g.elements = n;
+            g.generators = 3;
+            g.inverse_closed = true;
+            g.expected_states = expected;
+            for (uint32_t i = 0; i < n; ++i) g.perms.push_back((i + 1) % n);
+            for (uint32_t i = 0; i < n; ++i) g.perms.push_back((i + n - 1) % n);
+            for (uint32_t i = 0; i < n; ++i) g.perms.push_back(i < 2 ? 1 - i : i);
+            for (uint32_t i = 0; i < n; ++i) g.start.push_back(i);
+            mgbfs_batch_options o{};
+            slots = o.max_slots = 3;
+            o.vram_budget = 24ull << 30;
+            o.history = history;
+            o.layer_pct = pct;
+            o.bitmap_bias_permille = bias;
+            BatchEngine b(o);
+            int32_t s[3];
+            for (int32_t& k : s) require(b.admit(g, 0, 40, &k) == 0, "three instances admitted");
+            auto apart = [&] {
+              std::vector<Range> all;
+              for (uint32_t i = 0; i < 3; ++i)
+                for (const Range& r : parts(inst[i])) all.push_back(r);
+              std::sort(all.begin(), all.end(), [](const Range& x, const Range& y) { return x.from < y.from; });
+              for (size_t i = 0; i < all.size(); ++i) {
+                require(holds(all[i].from, all[i].to - all[i].from), "a part inside the arena");
+                require(i == 0 || all[i - 1].to <= all[i].from, "parts that do not overlap");
+              }
+            };
+            overflow = kErrFutureCap;
+            b.step(1);
+            apart();
+            const bool by_owners = inst[0].rank.owners != 0;
+            owned += by_owners;
+            overflow = 0;
+            b.step(1);
+            apart();
+            uint32_t visited = 0, layers = 0, restarts = 0;
+            uint64_t cap = 0;
+            for (int32_t k : s) {
+              b.instance_info(k, visited, layers, cap, restarts);
+              require(!by_owners || (visited == 1 && !inst[k].rank.owners && !inst[k].error && restarts == 1),
+                      "an overflow starts over on the shared bitmap");
+              restarted += restarts;
+            }
+          }
+  require(owned > 20 && restarted == 3 * owned, "instances by owners among them");
+  mgbfs_release_cached_memory(0);
+  std::printf("batch layout ok\n");
+  return 0;
+}

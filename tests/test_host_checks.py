@@ -8,7 +8,8 @@ from pathlib import Path
 import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
-CHECKS = {"rank_memory_check": "rank memory ok", "sorted_memory_check": "sorted memory ok"}
+CHECKS = {"rank_memory_check": "rank memory ok", "sorted_memory_check": "sorted memory ok",
+          "batch_layout_check": "batch layout ok"}
 
 
 @pytest.mark.parametrize("name", list(CHECKS))
