@@ -675,21 +675,17 @@ class PackedSegmentedEngine final : public Engine {
     mirror();
   }
   int advance(uint64_t* next_count, uint32_t* fatal) override {
+    if (terminal) throw std::runtime_error("ENGINE_TERMINAL");
     int s = inner_->advance(next_count, fatal);
-    if (s == kAdvanceHandover) {
-      go_on_segmented();
-      s = inner_->advance(next_count, fatal);
-    }
+    if (s == kAdvanceHandover) s = go_on_segmented() ? inner_->advance(next_count, fatal) : stop(fatal);
     complete_ = s == MGBFS_COMPLETE;
     mirror();
     return s;
   }
   int run_to_end() override {
+    uint32_t fatal = 0;
     int s = inner_->run_to_end();
-    if (s == kAdvanceHandover) {
-      go_on_segmented();
-      s = inner_->run_to_end();
-    }
+    if (s == kAdvanceHandover) s = go_on_segmented() ? inner_->run_to_end() : stop(&fatal);
     complete_ = s == MGBFS_COMPLETE;
     mirror();
     return s;
@@ -704,7 +700,7 @@ class PackedSegmentedEngine final : public Engine {
       seconds_ = 0.0;
       launches_ = streamed_ = 0;
     }
-    complete_ = false;
+    complete_ = stopped_ = false;
     mirror();
   }
   void layer_keys(std::vector<uint64_t>& out) override {
@@ -729,15 +725,36 @@ class PackedSegmentedEngine final : public Engine {
   }
 
  private:
-  void go_on_segmented() {
+  // The last two layers into segmented tables, beside the banks that hold
+  // them: a given budget holds both until the banks are freed.  False: they
+  // do not fit.
+  bool go_on_segmented() {
     PackedHandover h;
     if (!inner_->handover(h)) throw std::runtime_error("ENGINE_HANDOVER");
+    mgbfs_engine_options o = o_;
+    if (o.vram_budget) {
+      if (o.vram_budget <= h.held) return false;
+      o.vram_budget -= h.held;
+    }
+    std::unique_ptr<Engine> next;
+    try {
+      next.reset(make_segmented_from_packed(g_, o, state_space_bound(g_), h));
+    } catch (const AdoptCapacity&) {
+      return false;
+    }
     seconds_ = inner_->kernel_seconds;
     launches_ = inner_->launches;
     streamed_ = inner_->streamed_bytes;
-    std::unique_ptr<Engine> next(make_segmented_from_packed(g_, o_, state_space_bound(g_), h));
     inner_ = std::move(next);
+    inner_->memory_returned(h.held);
     packed_ = false;
+    return true;
+  }
+  // The layers found stay, as the packed ones, and so do their samples.
+  int stop(uint32_t* fatal) {
+    *fatal = kErrVisitedCap;
+    stopped_ = true;
+    return MGBFS_RESOURCE;
   }
   // Every layer but the current one has been expanded, the last one too
   // once the search is complete.
@@ -751,13 +768,14 @@ class PackedSegmentedEngine final : public Engine {
     kernel_seconds = inner_->kernel_seconds + seconds_;
     launches = inner_->launches + launches_;
     streamed_bytes = inner_->streamed_bytes + streamed_;
-    terminal = inner_->terminal;
+    terminal = stopped_ || inner_->terminal;
   }
   Graph g_;
   mgbfs_engine_options o_;
   WideCode code_;
   std::unique_ptr<Engine> inner_;
   bool packed_ = false, complete_ = false;
+  bool stopped_ = false;  // neither form has room for the next layer
   double seconds_ = 0.0;  // of the packed part of a run that went on segmented
   uint64_t launches_ = 0, streamed_ = 0;
 };

@@ -110,6 +110,8 @@ class Engine {
   // Sorted backend: describes its last two layers after advance() returned
   // kAdvanceHandover (its limits are exceeded) and frees its scratch.
   virtual bool handover(struct PackedHandover&) { return false; }
+  // The engine that handed its layers to this one has freed `bytes`.
+  virtual void memory_returned(uint64_t bytes) { (void)bytes; }
   virtual void layer_keys(std::vector<uint64_t>& out) = 0;
   virtual void sample(uint32_t which, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) = 0;
   virtual const char* name() const = 0;
@@ -166,6 +168,11 @@ struct PackedHandover {
   uint32_t tagbits = 0;
   const WideCode* wide = nullptr;  // null: nibble keys
   std::vector<uint64_t> layers;
+  uint64_t held = 0;  // device bytes of the sorted engine while its layers are taken over
+};
+// The two layers do not fit beside the sorted engine.
+struct AdoptCapacity : std::runtime_error {
+  AdoptCapacity() : std::runtime_error("SEGMENTED_ADOPT_CAPACITY") {}
 };
 Engine* make_segmented_from_packed(const Graph& g, const mgbfs_engine_options& o, uint64_t state_bound,
                                    const PackedHandover& h);

@@ -147,6 +147,8 @@ class SegmentedEngine final : public Engine {
     reset_counters();
   }
 
+  void memory_returned(uint64_t bytes) override { budget_ += bytes; }
+
   int advance(uint64_t* next_count, uint32_t* fatal) override {
     if (terminal) throw std::runtime_error("ENGINE_TERMINAL");
     MGBFS_HIP(hipSetDevice(device_));
@@ -382,12 +384,12 @@ class SegmentedEngine final : public Engine {
     return true;
   }
   void adopt_bank(int b, const uint64_t* vals, uint64_t count, const PackedHandover& h, const DeviceBuffer& labels) {
-    if (!ensure_arena(b, count)) throw std::runtime_error("SEGMENTED_ADOPT_CAPACITY");
+    if (!ensure_arena(b, count)) throw AdoptCapacity();
     MGBFS_HIP(segmented_adopt_packed<S>(vals, count, h.km, h.tagbits, elements_, h.wide ? h.wide->table.bits : 4,
                                         labels.bytes() ? labels.as<int64_t>() : nullptr,
                                         banks_[b].arena.template as<S>(), banks_[b].capacity, stream_));
     banks_[b].used = static_cast<uint32_t>(count);
-    if (!add_segment(b, count)) throw std::runtime_error("SEGMENTED_ADOPT_CAPACITY");
+    if (!add_segment(b, count)) throw AdoptCapacity();
     seed_rows(b, 0, static_cast<uint32_t>(count));
   }
   hipError_t launch(int target, uint64_t begin, uint32_t count) {

@@ -267,6 +267,9 @@ class SortedEngine final : public Engine {
     sub_.release();
     owner_.release();
     lane_cap_ = sub_cap_ = 0;
+    const int spare = next_bank();
+    bank_cap_[spare] = 0;
+    bank_[spare].release();
     h.wide = wide_.get();
     h.cur = bank_[cur_].as<uint64_t>();
     h.cur_count = count_[cur_];
@@ -276,6 +279,7 @@ class SortedEngine final : public Engine {
     h.tagbits = layout_.tagbits;
     h.layers = layers;
     update_bytes();
+    h.held = device_bytes;
     return true;
   }
 

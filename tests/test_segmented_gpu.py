@@ -264,3 +264,31 @@ def test_wide_keys_hand_over_to_segmented_tables(name):
                 assert e.layer_sizes() == want and sorted(map(tuple, e.sample(0, 1000))) == last
                 assert e.info()["candidates"] == 4 * sum(want)
                 e.reset()
+
+
+@pytest.mark.parametrize("step", [False, True])
+def test_wide_keys_out_of_memory_stop_with_their_layers(step):
+    # SL(2, Z_431), 80 million states, in 1.2 GB: the packed layers run out of
+    # room, and the last two as tables do not fit beside them.
+    p, budget = 431, 1184 << 20
+    g = sl2(p)
+    with NativeEngine(g, backend="segmented") as e:
+        assert e.run() == 1
+        full = e.layer_sizes()
+    assert sum(full) == p * (p * p - 1)
+    with NativeEngine(g, backend="segmented", vram_budget=budget) as e:
+        for _ in range(2):
+            status = 0
+            while step and status == 0:
+                status = e.advance()
+            assert (status if step else e.run()) == 2
+            assert e.fatal or not step
+            sizes = e.layer_sizes()
+            assert 8 < len(sizes) < len(full) and sizes == full[:len(sizes)]
+            for which in (0, 1):
+                rows = e.sample(which, 1000)
+                assert len({tuple(r) for r in rows}) == 1000
+                assert all((r[0] * r[3] - r[1] * r[2]) % p == 1 and 0 <= min(r) and max(r) < p for r in rows)
+            info = e.info()
+            assert info["device_bytes"] <= budget and info["candidates"] == 4 * sum(sizes[:-1])
+            e.reset()
