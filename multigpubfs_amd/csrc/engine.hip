@@ -123,10 +123,8 @@ class BitmapEngine final : public Engine {
     marks_.allocate((kAhead + 2) * 8);
     MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_ctl_), 64, hipHostMallocDefault));
     MGBFS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_marks_), (kAhead + 2) * 8, hipHostMallocDefault));
-    cap_limit_ = o.capacity ? o.capacity : domain_;
-    // Frontier buffers grow on demand up to what the budget admits.
-    const uint64_t frontier_budget = (budget_ - bitmap_bytes) / 2 / 8;
-    cap_limit_ = std::min(cap_limit_, frontier_budget);
+    capacity_ = o.capacity ? o.capacity : domain_;
+    set_limit();  // frontier buffers grow on demand up to it
     if (cap_limit_ == 0) throw std::runtime_error("BITMAP_VRAM_CAPACITY");
     grow(front_, front_cap_, std::min<uint64_t>(cap_limit_, 1u << 16));
     grow(next_, next_cap_, std::min<uint64_t>(cap_limit_, 1u << 16));
@@ -335,8 +333,15 @@ class BitmapEngine final : public Engine {
     count = keys.size();
   }
   const char* name() const override { return "PERMUTATION_BITMAP_LEHMER"; }
+  void memory_returned(uint64_t bytes) override {
+    budget_ += bytes;
+    set_limit();
+  }
 
  private:
+  // Rows of a layer: the caller's capacity, and what two frontier buffers
+  // beside the bitmap may hold.
+  void set_limit() { cap_limit_ = std::min(capacity_, (budget_ - bitmap_.bytes()) / 2 / 8); }
   uint32_t* error_word() { return reinterpret_cast<uint32_t*>(control_.as<uint64_t>() + 1); }
   // Generator table, parent-edge tags (nibble 15, when the state uses at
   // most 15 nibbles) and start state of a graph.
@@ -412,7 +417,7 @@ class BitmapEngine final : public Engine {
   static constexpr uint64_t kAheadStates = 1ull << 27;
   PackedGenerators gens_;
   uint32_t n_;
-  uint64_t domain_ = 0, budget_ = 0, cap_limit_ = 0;
+  uint64_t domain_ = 0, budget_ = 0, capacity_ = 0, cap_limit_ = 0;
   DeviceBuffer bitmap_, front_, next_, control_, stash_, marks_;
   uint64_t front_cap_ = 0, next_cap_ = 0, count_ = 0, prev_count_ = 0, stash_count_ = 0, start_key_ = 0,
            key_mask_ = ~0ull;
@@ -552,12 +557,13 @@ static uint32_t choose_backend(const Graph& g, uint32_t requested) {
 // backend's banks; the sorted engine and its memory are released).  Where
 // the library picks the backend, permutations of degree 3 to 12 run by
 // owners of the bitmap instead (rank_bitmap_for_auto), and what they report
-// is the bitmap backend's.
+// is the bitmap backend's.  The bitmap backend by name is here too while it
+// runs by owners: a rebound graph may need the shared bitmap.
 class HandoverEngine final : public Engine {
  public:
   HandoverEngine(const Graph& g, const mgbfs_engine_options& o) : g_(g), o_(o) {
-    by_owners_ = rank_bitmap_for_auto(g, o);
-    inner_.reset(by_owners_ ? make_rank_bitmap_engine(g, o) : make_sorted_engine(g, o));
+    by_owners_ = owners_take(g, 0);
+    inner_.reset(by_owners_ ? make_rank_bitmap_engine(g, o) : make_other(g));
     mirror();
   }
   int advance(uint64_t* next_count, uint32_t* fatal) override {
@@ -588,18 +594,25 @@ class HandoverEngine final : public Engine {
     }
     mirror();
   }
+  // What this engine holds counts as free for the choice, which is taken
+  // anew: it is kept, or makes room for the other form.  That is made first,
+  // so that a failure leaves the old graph running.
   void rebind(const Graph& g) override {
     if (handovers_) throw std::runtime_error("ENGINE_REBIND_AFTER_HANDOVER");
     if (!by_owners_) {
       inner_->rebind(g);
     } else {
-      if (g.elements != g_.elements || !g.packable() || !g.inverse_closed) throw std::runtime_error("ENGINE_REBIND_SHAPE");
-      by_owners_ = rank_bitmap_for_auto(g, o_);
-      if (by_owners_) {
+      const bool named = o_.backend == MGBFS_BACKEND_BITMAP;
+      if (g.elements != g_.elements || !g.packable() || (named ? !g.distinct_perm() : !g.inverse_closed))
+        throw std::runtime_error("ENGINE_REBIND_SHAPE");
+      const uint64_t held = inner_->device_bytes;
+      if (owners_take(g, held)) {
         inner_->rebind(g);
-      } else {  // repeated labels: sorted, as any graph of the degree may be
-        std::unique_ptr<Engine> next(make_sorted_engine(g, o_));
+      } else {  // repeated labels, or more generators than there is memory for
+        std::unique_ptr<Engine> next(make_other(g));
         inner_ = std::move(next);
+        if (!o_.vram_budget) inner_->memory_returned(held);
+        by_owners_ = false;
       }
     }
     g_ = g;
@@ -626,6 +639,12 @@ class HandoverEngine final : public Engine {
     uint64_t candidates = 0, unique = 0, launches = 0, streamed = 0;
     double seconds = 0.0;
   };
+  bool owners_take(const Graph& g, uint64_t held) const {
+    return o_.backend == MGBFS_BACKEND_BITMAP ? rank_bitmap_takes(g, o_, held) : rank_bitmap_for_auto(g, o_, held);
+  }
+  Engine* make_other(const Graph& g) const {
+    return o_.backend == MGBFS_BACKEND_BITMAP ? make_bitmap_engine(g, o_) : make_sorted_engine(g, o_);
+  }
   void hand_over() {
     PackedHandover h;
     if (!inner_->handover(h)) throw std::runtime_error("ENGINE_HANDOVER");
@@ -875,7 +894,8 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
 static Engine* create(const Graph& g, const mgbfs_engine_options& o) {
   switch (choose_backend(g, o.backend)) {
     case MGBFS_BACKEND_BITMAP:
-      return rank_bitmap_takes(g, o) ? make_rank_bitmap_engine(g, o) : make_bitmap_engine(g, o);
+      if (rank_bitmap_takes(g, o)) return new HandoverEngine(g, o);
+      return make_bitmap_engine(g, o);
     case MGBFS_BACKEND_SORTED:
       return new HandoverEngine(g, o);
     case MGBFS_BACKEND_SEGMENTED: {

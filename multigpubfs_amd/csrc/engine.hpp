@@ -110,7 +110,7 @@ class Engine {
   // Sorted backend: describes its last two layers after advance() returned
   // kAdvanceHandover (its limits are exceeded) and frees its scratch.
   virtual bool handover(struct PackedHandover&) { return false; }
-  // The engine that handed its layers to this one has freed `bytes`.
+  // The engine in whose place this one came has freed `bytes`.
   virtual void memory_returned(uint64_t bytes) { (void)bytes; }
   virtual void layer_keys(std::vector<uint64_t>& out) = 0;
   virtual void sample(uint32_t which, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) = 0;
@@ -147,9 +147,10 @@ constexpr int kAdvanceHandover = 3;
 
 Engine* make_bitmap_engine(const Graph& g, const mgbfs_engine_options& o);
 // The bitmap backend by owners (rank_engine.hip) and what it takes: degree 3
-// to 12, no row capacity asked for, memory for its lists and messages.
-bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o);
-bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o);
+// to 12, no row capacity asked for, memory for its lists and messages (`held`
+// bytes of it held by the engine that would be rebound).
+bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o, uint64_t held = 0);
+bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o, uint64_t held = 0);
 Engine* make_rank_bitmap_engine(const Graph& g, const mgbfs_engine_options& o);
 struct WideCode;
 // wide: packed code of a graph outside the nibble encoding (null: none).

@@ -209,13 +209,7 @@ class RankBitmapEngine final : public Engine {
     int khz = 0;
     MGBFS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
     run_.tick_seconds = khz > 0 ? 1e-3 / khz : 0.0;
-    const RankPlan& p = run_.plan;
-    bitmap_.allocate(4ull * p.owners * p.slice_words);
-    list_.allocate(4ull * p.owners * p.list_cap);
-    words_.allocate(RankRun::words_bytes(p));
-    run_.memory.bitmap = bitmap_.as<uint32_t>();
-    run_.memory.list = list_.as<uint32_t>();
-    run_.memory.words = words_.as<uint32_t>();
+    take_plan(run_.plan);
     reset();
     ensure_messages(wanted_);
   }
@@ -257,9 +251,12 @@ class RankBitmapEngine final : public Engine {
   }
   void rebind(const Graph& g) override {
     if (g.elements != n_ || !g.packable() || !g.distinct_perm()) throw std::runtime_error("ENGINE_REBIND_SHAPE");
-    ensure_messages(RankRun::first_cap(run_.plan, g.generators));
+    const RankPlan p = rank_plan(n_, RankRun::owners_for(g));
+    if (p.owners != run_.plan.owners) take_plan(p);
+    else ensure_messages(RankRun::first_cap(p, g.generators));  // or the old graph stays
     set_graph(g);
     reset();
+    ensure_messages(wanted_);
   }
   void layer_keys(std::vector<uint64_t>& out) override { export_layer(0, layers.back(), out); }
   void sample(uint32_t which, uint64_t limit, std::vector<int64_t>& rows, uint64_t& count) override {
@@ -277,6 +274,24 @@ class RankBitmapEngine final : public Engine {
   void set_graph(const Graph& g) {
     run_.set_graph(g);
     history_layers = g.inverse_closed ? 3 : 0;
+  }
+  // Bitmap, lists and words of a plan, for a reset.  The old ones go when all
+  // are there (plans change at the smallest degrees only).
+  void take_plan(const RankPlan& p) {
+    DeviceBuffer bitmap, list, words;
+    bitmap.allocate(4ull * p.owners * p.slice_words);
+    list.allocate(4ull * p.owners * p.list_cap);
+    words.allocate(RankRun::words_bytes(p));
+    MGBFS_HIP(hipStreamSynchronize(stream_));
+    run_.drop_messages();
+    for (auto& m : messages_) m.release();
+    bitmap_ = std::move(bitmap);
+    list_ = std::move(list);
+    words_ = std::move(words);
+    run_.plan = p;
+    run_.memory.bitmap = bitmap_.as<uint32_t>();
+    run_.memory.list = list_.as<uint32_t>();
+    run_.memory.words = words_.as<uint32_t>();
   }
   void update_bytes() {
     device_bytes = bitmap_.bytes() + list_.bytes() + words_.bytes() + messages_[0].bytes() + messages_[1].bytes();
@@ -355,10 +370,10 @@ class RankBitmapEngine final : public Engine {
 // layer and a message buffer is not one, so a set capacity keeps the shared
 // bitmap; so does a budget that does not hold the messages of every layer
 // (degree 12 with three generators: 13.5 GB, of which 4.3 are used).
-bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o) {
+bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o, uint64_t held) {
   if (g.elements < 3 || g.elements > kRankDegree || o.capacity || g.generators > kMaxGenerators) return false;
-  MGBFS_HIP(hipSetDevice(o.device));
-  return RankBitmapEngine::most_bytes(g) <= vram_budget(o);
+  if (!o.vram_budget) MGBFS_HIP(hipSetDevice(o.device));
+  return RankBitmapEngine::most_bytes(g) <= vram_budget(o) + (o.vram_budget ? 0 : held);
 }
 
 // Inverse-closed graphs whose backend the library picks run by owners of the
@@ -367,9 +382,9 @@ bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o) {
 // 10.5; Coxeter 6 0.11 -> 0.02, 11 5.5 -> 3.0, 12 96 -> 33; four random
 // generators with inverses, 11 5.1 -> 1.9).
 // A set that is only declared closed keeps the sorted backend's retention.
-bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o) {
+bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o, uint64_t held) {
   if (o.backend != MGBFS_BACKEND_AUTO || !g.inverse_closed || !g.packable() || !g.distinct_perm() ||
-      (o.flags & ~MGBFS_FLAG_MAX_CAPACITY) || !rank_bitmap_takes(g, o))
+      (o.flags & ~MGBFS_FLAG_MAX_CAPACITY) || !rank_bitmap_takes(g, o, held))
     return false;
   for (int at : inverse_index(g.packed_generators()))
     if (at < 0) return false;

@@ -61,7 +61,7 @@ class RankRun {
   void export_layer(uint64_t back, uint64_t limit, uint64_t* keys, hipStream_t stream);
   uint32_t generators() const { return gens_.count; }
 
-  const RankPlan plan;
+  RankPlan plan;
   RankMemory memory{};
   std::vector<uint64_t> layers;
   double seconds = 0.0, tick_seconds = 0.0;  // between the records of layers run

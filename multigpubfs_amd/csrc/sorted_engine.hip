@@ -306,6 +306,8 @@ class SortedEngine final : public Engine {
     end_compaction(await(rec_[0], seq).ticks);
   }
 
+  void memory_returned(uint64_t bytes) override { budget_ += bytes; }
+
   double phase_seconds[kPhaseCount] = {};
   uint64_t phase_bytes[kPhaseCount] = {};
   uint64_t retries = 0;
