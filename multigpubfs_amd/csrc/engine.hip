@@ -552,6 +552,27 @@ static uint32_t choose_backend(const Graph& g, uint32_t requested) {
   }
 }
 
+// In the place of an engine whose successor could not be made: every call is
+// refused until a reset makes one.
+class LostEngine final : public Engine {
+ public:
+  explicit LostEngine(const Engine& e) : name_(e.name()) {
+    backend = e.backend;
+    history_layers = e.history_layers;
+    state_bytes = e.state_bytes;
+    layers.assign(1, 1);
+  }
+  int advance(uint64_t*, uint32_t*) override { return lost(); }
+  void reset() override { lost(); }
+  void layer_keys(std::vector<uint64_t>&) override { lost(); }
+  void sample(uint32_t, uint64_t, std::vector<int64_t>&, uint64_t&) override { lost(); }
+  const char* name() const override { return name_; }
+
+ private:
+  [[noreturn]] static int lost() { throw std::runtime_error("ENGINE_RESET_FAILED"); }
+  const char* name_;
+};
+
 // The sorted backend, handing the run to the segmented backend when a
 // layer exceeds its limits (its last two layers become the segmented
 // backend's banks; the sorted engine and its memory are released).  Where
@@ -586,7 +607,7 @@ class HandoverEngine final : public Engine {
   }
   void reset() override {
     if (handovers_) {
-      inner_.reset();
+      inner_.reset(new LostEngine(*this));
       inner_.reset(make_sorted_engine(g_, o_));
       carried_ = {};
     } else {
@@ -713,7 +734,7 @@ class PackedSegmentedEngine final : public Engine {
     if (packed_) {
       inner_->reset();
     } else {
-      inner_.reset();
+      inner_.reset(new LostEngine(*this));
       inner_.reset(make_sorted_engine(g_, o_, &code_));
       packed_ = true;
       seconds_ = 0.0;

@@ -155,6 +155,27 @@ int main() {
     e->run_to_end();
     require(block_runs == 2, "and back");
   }
+  // A reset that cannot make its engine refuses calls, and the next one tries
+  // again.
+  o.backend = MGBFS_BACKEND_SORTED;
+  {
+    const Graph g = graph_of(13, swaps(13, 12), true);
+    std::unique_ptr<Engine> e(create(g, o));
+    uint64_t n = 0;
+    uint32_t fatal = 0;
+    hand_over = 1;
+    require(e->advance(&n, &fatal) == MGBFS_COMPLETE && e->backend == MGBFS_BACKEND_SEGMENTED, "a hand-over");
+    refuse_other = 1;
+    require(throws([&] { e->reset(); }) && throws([&] { e->advance(&n, &fatal); }), "calls are refused");
+    std::vector<int64_t> rows;
+    require(throws([&] { e->sample(0, 1, rows, n); }) && e->name() != nullptr, "samples too");
+    mgbfs_engine_info info{};
+    e->settle();
+    e->fill_info(info);
+    refuse_other = 0;
+    e->reset();
+    require(e->advance(&n, &fatal) == MGBFS_COMPLETE && e->backend == MGBFS_BACKEND_SORTED, "until one succeeds");
+  }
   std::printf("rebind ok\n");
   return 0;
 }
