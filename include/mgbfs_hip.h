@@ -282,7 +282,7 @@ int mgbfs_sorted_unpack(uint32_t degree, const uint64_t* values, uint64_t count,
 
 /* ------------------------------------------------- batched instances */
 /* Many independent BFS instances advanced together, one layer of every
- * active instance per step, by a hipGraph-captured layer loop; instances are
+ * active instance per step, by a layer loop in a hipGraph; instances are
  * admitted and released at layer boundaries (continuous batching).  The
  * reference has no batched kernel (its nearest relative is the sequential
  * resident worker of crates/mgbfs-runtime/src/generic_session.rs:6-71 and
@@ -294,7 +294,7 @@ typedef struct mgbfs_batch_options {
   int32_t device;
   uint32_t max_slots;        /* <= 1024 (0 = 256)                              */
   uint64_t vram_budget;      /* bytes for admitted jobs (0 = free - 4 GiB)      */
-  uint32_t layers_per_graph; /* layers captured per hipGraph launch (0 = 4)     */
+  uint32_t layers_per_graph; /* layers per hipGraph launch (0 = 4)     */
   uint32_t grid;             /* persistent expand grid (0 = 8 x CUs)            */
   uint32_t threads;          /* expand workgroup: 128, 256 or 512 (0 = 256)     */
   uint32_t hash_load_pct;    /* hash tables filled to at most this % (0 = 50)   */

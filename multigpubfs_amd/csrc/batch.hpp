@@ -104,25 +104,33 @@ struct BatchInstall {
   uint64_t start_key;
 };
 
-hipError_t batch_reset_flag(uint32_t* flag, hipStream_t stream);
+// The layer loop is a graph of kernels, each after the one before.  It is
+// built node by node: while a stream is captured, in any mode, the runtime
+// refuses the copies of other threads' engines (and of whatever else runs in
+// the process), and the capture fails with them.
+struct GraphChain {
+  hipGraph_t graph = nullptr;
+  hipGraphNode_t last = nullptr;
+};
+hipError_t batch_reset_flag(uint32_t* flag, GraphChain& chain);
 // prefix: kBatchPrefixes * (slots + 1) words (expansion tiles, clear work
 // items, owners), then the owners' work counter.
 constexpr uint32_t kBatchPrefixes = 3;
-hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, hipStream_t stream);
+hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, GraphChain& chain);
 // threads: 128, 256 or 512 per workgroup; tile = 2 * threads parents.
 hipError_t batch_expand(BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t tile, uint32_t grid,
-                        uint32_t threads, hipStream_t stream);
+                        uint32_t threads, GraphChain& chain);
 // Clears the table the next layer of every active rolling instance claims in
 // (work items from the second half of batch_tiles' prefix).
 hipError_t batch_clear(const BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t grid,
-                       hipStream_t stream);
+                       GraphChain& chain);
 // A step of every owner of the owned instances; grid: at most two blocks
 // per CU run at once.
-hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, uint32_t grid, hipStream_t stream);
+hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, uint32_t grid, GraphChain& chain);
 // States of the current layer of an owned instance (a staged copy of its
 // descriptor), packed keys.
 hipError_t batch_owned_export(const BatchInstance& inst, uint64_t limit, uint64_t* keys, hipStream_t stream);
-hipError_t batch_finish(BatchInstance* inst, uint32_t slots, uint32_t* any_active, hipStream_t stream);
+hipError_t batch_finish(BatchInstance* inst, uint32_t slots, uint32_t* any_active, GraphChain& chain);
 hipError_t batch_gather_sizes(const BatchInstance* inst, const uint32_t* req, uint32_t n, uint64_t* out,
                               hipStream_t stream);
 // Empties the visited set of every seeding request's staged descriptor

@@ -1,5 +1,5 @@
 // Host side of the batched multi-instance engine: slot admission with VRAM
-// planning, a pooled device allocator, and a hipGraph-captured layer loop
+// planning, a pooled device allocator, and a layer loop in a hipGraph
 // (reset flag, then K x [tiles, clear, expand, owned, finish]) replayed until no instance
 // is active.  Instances join and leave at layer boundaries, so the same
 // object serves both the fixed sweep and continuous-batching serving.
@@ -179,7 +179,7 @@ class BatchEngine {
     MGBFS_HIP(hipMemcpy(inst_.as<void>(), host_inst_.data(), sizeof(BatchInstance) * slots_n_, hipMemcpyHostToDevice));
     slots_.resize(slots_n_);
     owned_wanted_.assign(slots_n_, 0);
-    capture();
+    build_graph();
   }
   ~BatchEngine() {
     (void)hipSetDevice(device_);
@@ -503,22 +503,20 @@ class BatchEngine {
     if (slot < 0 || static_cast<uint32_t>(slot) >= slots_n_ || !slots_[slot].used)
       throw std::runtime_error("BATCH_SLOT");
   }
-  void capture() {
+  void build_graph() {
     BatchInstance* inst = inst_.as<BatchInstance>();
     uint32_t* prefix = prefix_.as<uint32_t>();
     uint32_t* flag = flag_.as<uint32_t>();
-    // Relaxed: thread-local capture still refuses the allocations and copies
-    // of other threads' engines, and fails with them.
-    MGBFS_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed));
-    MGBFS_HIP(batch_reset_flag(flag, stream_));
+    MGBFS_HIP(hipGraphCreate(&graph_, 0));
+    GraphChain chain{graph_};
+    MGBFS_HIP(batch_reset_flag(flag, chain));
     for (uint32_t k = 0; k < layers_per_graph_; ++k) {
-      MGBFS_HIP(batch_tiles(inst, slots_n_, 2 * threads_, prefix, stream_));
-      MGBFS_HIP(batch_clear(inst, slots_n_, prefix, clear_grid_, stream_));
-      MGBFS_HIP(batch_expand(inst, slots_n_, prefix, 2 * threads_, grid_, threads_, stream_));
-      MGBFS_HIP(batch_owned(inst, slots_n_, prefix, owned_grid_, stream_));
-      MGBFS_HIP(batch_finish(inst, slots_n_, flag, stream_));
+      MGBFS_HIP(batch_tiles(inst, slots_n_, 2 * threads_, prefix, chain));
+      MGBFS_HIP(batch_clear(inst, slots_n_, prefix, clear_grid_, chain));
+      MGBFS_HIP(batch_expand(inst, slots_n_, prefix, 2 * threads_, grid_, threads_, chain));
+      MGBFS_HIP(batch_owned(inst, slots_n_, prefix, owned_grid_, chain));
+      MGBFS_HIP(batch_finish(inst, slots_n_, flag, chain));
     }
-    MGBFS_HIP(hipStreamEndCapture(stream_, &graph_));
     MGBFS_HIP(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
   }
   // The slot's block as bitmap and words (adjoining, emptied together as

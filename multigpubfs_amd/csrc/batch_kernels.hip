@@ -1,5 +1,5 @@
 // Batched multi-instance BFS kernels.  One layer of every active instance
-// is five launches, all capturable in a hipGraph (no host readback, no
+// is five launches, all kernels of a hipGraph (no host readback, no
 // memset nodes):
 //   batch_tiles  : one block scans the per-instance tile counts
 //                  ceil(count / tile) of the active instances -> prefix,
@@ -18,6 +18,8 @@
 //   batch_finish : one thread per instance records the layer size, swaps the
 //                  frontier buffers and retires finished instances.
 #include <algorithm>
+#include <tuple>
+#include <type_traits>
 #include "batch.hpp"
 #include "kernels.hpp"
 #include "rank_device.hpp"
@@ -605,47 +607,56 @@ __global__ void batch_install_kernel(BatchInstance* inst, const BatchInstance* s
 
 }  // namespace
 
-hipError_t batch_reset_flag(uint32_t* flag, hipStream_t stream) {
-  hipLaunchKernelGGL(batch_reset_flag_kernel, dim3(1), dim3(64), 0, stream, flag);
-  return hipGetLastError();
+// A kernel after the chain's last one; its arguments are copied here.
+template <typename... P, typename... A>
+static hipError_t add_kernel(GraphChain& chain, void (*kernel)(P...), uint32_t grid, uint32_t block, A... args) {
+  std::tuple<std::remove_const_t<P>...> values(args...);
+  void* params[sizeof...(P)];
+  std::apply([&](auto&... v) { uint32_t k = 0; ((params[k++] = const_cast<void*>(static_cast<const void*>(&v))), ...); }, values);
+  hipKernelNodeParams node{};
+  node.func = reinterpret_cast<void*>(kernel);
+  node.gridDim = dim3(grid);
+  node.blockDim = dim3(block);
+  node.kernelParams = params;
+  hipGraphNode_t added = nullptr;
+  const hipError_t e = hipGraphAddKernelNode(&added, chain.graph, chain.last ? &chain.last : nullptr, chain.last ? 1 : 0, &node);
+  if (e == hipSuccess) chain.last = added;
+  return e;
 }
 
-hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, hipStream_t stream) {
+hipError_t batch_reset_flag(uint32_t* flag, GraphChain& chain) {
+  return add_kernel(chain, batch_reset_flag_kernel, 1, 64, flag);
+}
+
+hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, GraphChain& chain) {
   if (slots == 0 || slots > kBatchMaxSlots || tile == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(batch_tiles_kernel, dim3(1), dim3(1024), 0, stream, inst, slots, tile, prefix);
-  return hipGetLastError();
+  return add_kernel(chain, batch_tiles_kernel, 1, 1024, inst, slots, tile, prefix);
 }
 
 hipError_t batch_expand(BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t tile, uint32_t grid,
-                        uint32_t threads, hipStream_t stream) {
+                        uint32_t threads, GraphChain& chain) {
   if (slots == 0 || slots > kBatchMaxSlots || tile != threads * kBatchItems || grid == 0) return hipErrorInvalidValue;
   switch (threads) {
     case 128:
-      hipLaunchKernelGGL(batch_expand_kernel<128>, dim3(grid), dim3(128), 0, stream, inst, slots, prefix, tile);
-      break;
+      return add_kernel(chain, batch_expand_kernel<128>, grid, 128, inst, slots, prefix, tile);
     case 256:
-      hipLaunchKernelGGL(batch_expand_kernel<256>, dim3(grid), dim3(256), 0, stream, inst, slots, prefix, tile);
-      break;
+      return add_kernel(chain, batch_expand_kernel<256>, grid, 256, inst, slots, prefix, tile);
     case 512:
-      hipLaunchKernelGGL(batch_expand_kernel<512>, dim3(grid), dim3(512), 0, stream, inst, slots, prefix, tile);
-      break;
+      return add_kernel(chain, batch_expand_kernel<512>, grid, 512, inst, slots, prefix, tile);
     default:
       return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 hipError_t batch_clear(const BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t grid,
-                       hipStream_t stream) {
+                       GraphChain& chain) {
   if (slots == 0 || slots > kBatchMaxSlots || grid == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(batch_clear_kernel, dim3(grid), dim3(256), 0, stream, inst, slots, prefix + slots + 1);
-  return hipGetLastError();
+  return add_kernel(chain, batch_clear_kernel, grid, 256, inst, slots, prefix + slots + 1);
 }
 
-hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, uint32_t grid, hipStream_t stream) {
+hipError_t batch_owned(BatchInstance* inst, uint32_t slots, uint32_t* prefix, uint32_t grid, GraphChain& chain) {
   if (slots == 0 || slots > kBatchMaxSlots || grid == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(batch_owned_kernel, dim3(grid), dim3(kRouteThreads), 0, stream, inst, slots, prefix);
-  return hipGetLastError();
+  return add_kernel(chain, batch_owned_kernel, grid, kRouteThreads, inst, slots, prefix);
 }
 
 hipError_t batch_owned_export(const BatchInstance& s, uint64_t limit, uint64_t* keys, hipStream_t stream) {
@@ -655,9 +666,8 @@ hipError_t batch_owned_export(const BatchInstance& s, uint64_t limit, uint64_t* 
   return hipGetLastError();
 }
 
-hipError_t batch_finish(BatchInstance* inst, uint32_t slots, uint32_t* any_active, hipStream_t stream) {
-  hipLaunchKernelGGL(batch_finish_kernel, dim3((slots + 255) / 256), dim3(256), 0, stream, inst, slots, any_active);
-  return hipGetLastError();
+hipError_t batch_finish(BatchInstance* inst, uint32_t slots, uint32_t* any_active, GraphChain& chain) {
+  return add_kernel(chain, batch_finish_kernel, (slots + 255) / 256, 256, inst, slots, any_active);
 }
 
 hipError_t batch_gather_sizes(const BatchInstance* inst, const uint32_t* req, uint32_t n, uint64_t* out,

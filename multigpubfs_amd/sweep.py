@@ -7,7 +7,7 @@ in {9, 10}, k uniform in 2..5 generators, each a uniform random permutation
 inverse-closed), odd ones do not (directed, full visited history).
 
 `run_batched` advances all instances together through the batch engine
-(hipGraph-captured layer loop); `run_sequential` runs the same instances one
+(layer loop in a hipGraph); `run_sequential` runs the same instances one
 at a time through the plain single-instance engine.  Both return per-instance
 layer tables, which must be identical.  Every leg validates its instances
 and builds their library descriptors before its clock starts, so the timed

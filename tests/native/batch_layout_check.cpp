@@ -32,14 +32,14 @@ extern "C" hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) {
 }
 
 namespace mgbfs {
-hipError_t batch_reset_flag(uint32_t*, hipStream_t) { return hipSuccess; }
-hipError_t batch_tiles(BatchInstance*, uint32_t, uint32_t, uint32_t*, hipStream_t) { return hipSuccess; }
-hipError_t batch_clear(const BatchInstance*, uint32_t, const uint32_t*, uint32_t, hipStream_t) { return hipSuccess; }
-hipError_t batch_expand(BatchInstance*, uint32_t, const uint32_t*, uint32_t, uint32_t, uint32_t, hipStream_t) {
+hipError_t batch_reset_flag(uint32_t*, GraphChain&) { return hipSuccess; }
+hipError_t batch_tiles(BatchInstance*, uint32_t, uint32_t, uint32_t*, GraphChain&) { return hipSuccess; }
+hipError_t batch_clear(const BatchInstance*, uint32_t, const uint32_t*, uint32_t, GraphChain&) { return hipSuccess; }
+hipError_t batch_expand(BatchInstance*, uint32_t, const uint32_t*, uint32_t, uint32_t, uint32_t, GraphChain&) {
   return hipSuccess;
 }
-hipError_t batch_owned(BatchInstance*, uint32_t, uint32_t*, uint32_t, hipStream_t) { return hipSuccess; }
-hipError_t batch_finish(BatchInstance*, uint32_t, uint32_t*, hipStream_t) { return hipSuccess; }
+hipError_t batch_owned(BatchInstance*, uint32_t, uint32_t*, uint32_t, GraphChain&) { return hipSuccess; }
+hipError_t batch_finish(BatchInstance*, uint32_t, uint32_t*, GraphChain&) { return hipSuccess; }
 hipError_t batch_clear_visited(const BatchInstance*, const BatchInstall*, uint32_t, uint64_t, hipStream_t s) {
   return fake::launch(s);
 }

@@ -333,3 +333,33 @@ def test_sample_of_an_instance_stopped_at_its_layer_limit(n, layers, copies):
             assert error and sizes == ref["layers"][:layers]
             rows = [O.pack(r) for r in b.sample(s, n, 10**7)]
             assert sorted(rows) == sorted(ref["keys"][layers - 1])
+
+
+def test_engines_made_beside_other_threads_copies():
+    # Batch engines come and go in one thread while another's engines upload
+    # their generators and read their states back.
+    import threading
+    stop, errors, made = threading.Event(), [], [0, 0]
+
+    def others():
+        try:
+            while not stop.is_set():
+                with NativeEngine(sl2(13), backend="segmented", flags=128) as e:
+                    assert e.run() == 1 and len(e.sample(0, 1000)) == e.layer_sizes()[-1]
+                made[1] += 1
+        except Exception as exc:
+            errors.append(exc)
+
+    thread = threading.Thread(target=others)
+    thread.start()
+    try:
+        for _ in range(60):
+            with BatchEngine(max_slots=2) as b:
+                slot = b.admit(sl2(11))
+                b.run()
+                assert sum(b.result(slot)[0]) == 11 * 120
+            made[0] += 1
+    finally:
+        stop.set()
+        thread.join()
+    assert not errors and made[0] == 60 and made[1] > 5
