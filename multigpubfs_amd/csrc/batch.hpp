@@ -116,7 +116,10 @@ hipError_t batch_reset_flag(uint32_t* flag, GraphChain& chain);
 // prefix: kBatchPrefixes * (slots + 1) words (expansion tiles, clear work
 // items, owners), then the owners' work counter.
 constexpr uint32_t kBatchPrefixes = 3;
-hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, GraphChain& chain);
+// forms: of the instances that the step runs.
+constexpr uint32_t kBatchShared = 1, kBatchOwned = 2, kBatchForms = 4;
+hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, uint32_t forms,
+                       GraphChain& chain);
 // threads: 128, 256 or 512 per workgroup; tile = 2 * threads parents.
 hipError_t batch_expand(BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t tile, uint32_t grid,
                         uint32_t threads, GraphChain& chain);

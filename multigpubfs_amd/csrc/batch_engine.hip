@@ -1,7 +1,7 @@
 // Host side of the batched multi-instance engine: slot admission with VRAM
 // planning, a pooled device allocator, and a layer loop in a hipGraph
-// (reset flag, then K x [tiles, clear, expand, owned, finish]) replayed until no instance
-// is active.  Instances join and leave at layer boundaries, so the same
+// (reset flag, then K x [tiles, clear, expand, owned, finish], of which a step
+// takes what its instances need) replayed until no instance is active.  Instances join and leave at layer boundaries, so the same
 // object serves both the fixed sweep and continuous-batching serving.
 #include <algorithm>
 #include <cstring>
@@ -179,13 +179,15 @@ class BatchEngine {
     MGBFS_HIP(hipMemcpy(inst_.as<void>(), host_inst_.data(), sizeof(BatchInstance) * slots_n_, hipMemcpyHostToDevice));
     slots_.resize(slots_n_);
     owned_wanted_.assign(slots_n_, 0);
-    build_graph();
+    (void)graph_for(kBatchShared);
   }
   ~BatchEngine() {
     (void)hipSetDevice(device_);
     if (stream_) (void)hipStreamSynchronize(stream_);
-    if (exec_) (void)hipGraphExecDestroy(exec_);
-    if (graph_) (void)hipGraphDestroy(graph_);
+    for (hipGraphExec_t e : exec_)
+      if (e) (void)hipGraphExecDestroy(e);
+    for (hipGraph_t g : graph_)
+      if (g) (void)hipGraphDestroy(g);
     if (host_flag_) (void)hipHostFree(host_flag_);
     if (host_mirror_) (void)hipHostFree(host_mirror_);
     if (host_stage_) (void)hipHostFree(host_stage_);
@@ -380,8 +382,8 @@ class BatchEngine {
   uint32_t step(uint32_t layers) {
     MGBFS_HIP(hipSetDevice(device_));
     const uint32_t launches = std::max<uint32_t>(1, (layers + layers_per_graph_ - 1) / layers_per_graph_);
-    flush();
-    for (uint32_t k = 0; k < launches; ++k) MGBFS_HIP(hipGraphLaunch(exec_, stream_));
+    const hipGraphExec_t exec = graph_for(flush());
+    for (uint32_t k = 0; k < launches; ++k) MGBFS_HIP(hipGraphLaunch(exec, stream_));
     refresh();
     uint32_t active = 0;
     for (uint32_t s = 0; s < slots_n_; ++s) {
@@ -503,21 +505,31 @@ class BatchEngine {
     if (slot < 0 || static_cast<uint32_t>(slot) >= slots_n_ || !slots_[slot].used)
       throw std::runtime_error("BATCH_SLOT");
   }
-  void build_graph() {
+  // The layer loop for the given forms of instances.  A launch that finds
+  // nothing to do still takes 3 us a layer, so a step without instances by
+  // owners leaves their kernel out, one with no others leaves out theirs.
+  hipGraphExec_t graph_for(uint32_t forms) {
+    if (exec_[forms]) return exec_[forms];
     BatchInstance* inst = inst_.as<BatchInstance>();
     uint32_t* prefix = prefix_.as<uint32_t>();
     uint32_t* flag = flag_.as<uint32_t>();
-    MGBFS_HIP(hipGraphCreate(&graph_, 0));
-    GraphChain chain{graph_};
+    MGBFS_HIP(hipSetDevice(device_));
+    if (graph_[forms]) MGBFS_HIP(hipGraphDestroy(graph_[forms]));  // left by a failure
+    graph_[forms] = nullptr;
+    MGBFS_HIP(hipGraphCreate(&graph_[forms], 0));
+    GraphChain chain{graph_[forms]};
     MGBFS_HIP(batch_reset_flag(flag, chain));
     for (uint32_t k = 0; k < layers_per_graph_; ++k) {
-      MGBFS_HIP(batch_tiles(inst, slots_n_, 2 * threads_, prefix, chain));
-      MGBFS_HIP(batch_clear(inst, slots_n_, prefix, clear_grid_, chain));
-      MGBFS_HIP(batch_expand(inst, slots_n_, prefix, 2 * threads_, grid_, threads_, chain));
-      MGBFS_HIP(batch_owned(inst, slots_n_, prefix, owned_grid_, chain));
+      MGBFS_HIP(batch_tiles(inst, slots_n_, 2 * threads_, prefix, forms, chain));
+      if (forms & kBatchShared) {
+        MGBFS_HIP(batch_clear(inst, slots_n_, prefix, clear_grid_, chain));
+        MGBFS_HIP(batch_expand(inst, slots_n_, prefix, 2 * threads_, grid_, threads_, chain));
+      }
+      if (forms & kBatchOwned) MGBFS_HIP(batch_owned(inst, slots_n_, prefix, owned_grid_, chain));
       MGBFS_HIP(batch_finish(inst, slots_n_, flag, chain));
     }
-    MGBFS_HIP(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
+    MGBFS_HIP(hipGraphInstantiate(&exec_[forms], graph_[forms], nullptr, nullptr, 0));
+    return exec_[forms];
   }
   // The slot's block as bitmap and words (adjoining, emptied together as
   // bitmap_bits), list, layer sizes and two message buffers.  Steps send so
@@ -564,18 +576,25 @@ class BatchEngine {
   // installed and seeded.  Only the latest descriptor of a slot is staged,
   // so memory an instance released before the flush is cleared, if reused,
   // only as its new owner's visited set.  The pinned staging area is reused
-  // only after refresh() has waited.
-  void flush() {
+  // only after refresh() has waited.  Returns the forms of the instances
+  // that run from here on.
+  uint32_t flush() {
     uint32_t n = 0;
     uint64_t clear_bytes = 0;  // largest visited set to empty
     BatchInstall* req = reinterpret_cast<BatchInstall*>(host_stage_ + slots_n_);
     // How many instances run from here on decides how finely the new ones
     // are split.
-    uint32_t running = 0;
-    for (uint32_t s = 0; s < slots_n_; ++s)
-      running += pending_[s] == kInstallSeed || (slots_[s].used && (host_inst_[s].status & kInstActive));
-    for (uint32_t s = 0; s < slots_n_; ++s)
+    uint32_t running = 0, forms = 0;
+    auto runs = [&](uint32_t s) {
+      return pending_[s] == kInstallSeed || (slots_[s].used && (host_inst_[s].status & kInstActive));
+    };
+    for (uint32_t s = 0; s < slots_n_; ++s) running += runs(s);
+    for (uint32_t s = 0; s < slots_n_; ++s) {
+      if (!runs(s)) continue;
       if (pending_[s] == kInstallSeed && owned_wanted_[s]) lay_out_owned(s, running);
+      forms |= host_inst_[s].rank.owners ? kBatchOwned : kBatchShared;
+    }
+    if (!forms) forms = kBatchShared;
     for (uint32_t s = 0; s < slots_n_; ++s) {
       if (pending_[s] == kNothing) continue;
       const BatchInstance& d = host_inst_[s];
@@ -588,13 +607,14 @@ class BatchEngine {
       pending_[s] = kNothing;
       ++n;
     }
-    if (n == 0) return;
+    if (n == 0) return forms;
     const size_t bytes = sizeof(BatchInstance) * slots_n_ + sizeof(BatchInstall) * n;
     MGBFS_HIP(hipMemcpyAsync(stage_.as<void>(), host_stage_, bytes, hipMemcpyHostToDevice, stream_));
     const BatchInstance* staged = stage_.as<BatchInstance>();
     const BatchInstall* reqs = reinterpret_cast<const BatchInstall*>(staged + slots_n_);
     MGBFS_HIP(batch_clear_visited(staged, reqs, n, clear_bytes, stream_));
     MGBFS_HIP(batch_install(inst_.as<BatchInstance>(), staged, reqs, n, stream_));
+    return forms;
   }
   void refresh() {
     MGBFS_HIP(hipMemcpyAsync(host_mirror_, inst_.as<void>(), sizeof(BatchInstance) * slots_n_, hipMemcpyDeviceToHost,
@@ -657,7 +677,7 @@ class BatchEngine {
 
   int device_ = 0;
   hipStream_t stream_ = nullptr;
-  std::vector<uint8_t> owned_wanted_;  // per slot: laid out for owners by the next flush, if its block holds that
+  std::vector<uint8_t> owned_wanted_;  // per slot: may be laid out for owners by the next flush, if its block holds that
   uint32_t slots_n_ = 0, grid_ = 0, clear_grid_ = 0, owned_grid_ = 0, layers_per_graph_ = kLayersPerGraph;
   uint32_t threads_ = 256, hash_load_pct_ = 50, layer_pct_ = 30, bitmap_bias_permille_ = 1000;
   uint32_t history_ = 0;
@@ -680,8 +700,8 @@ class BatchEngine {
   std::vector<Slot> slots_;
   std::map<int32_t, uint32_t> kinds_, rows_, cols_;
   DeviceArena arena_;
-  hipGraph_t graph_ = nullptr;
-  hipGraphExec_t exec_ = nullptr;
+  hipGraph_t graph_[kBatchForms] = {};  // by the forms of instances they run
+  hipGraphExec_t exec_[kBatchForms] = {};
 };
 
 Graph intake_graph(const mgbfs_graph_desc* d);

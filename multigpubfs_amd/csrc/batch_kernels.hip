@@ -1,5 +1,5 @@
 // Batched multi-instance BFS kernels.  One layer of every active instance
-// is five launches, all kernels of a hipGraph (no host readback, no
+// is at most five launches, all kernels of a hipGraph (no host readback, no
 // memset nodes):
 //   batch_tiles  : one block scans the per-instance tile counts
 //                  ceil(count / tile) of the active instances -> prefix,
@@ -253,7 +253,7 @@ __device__ __forceinline__ void block_scan_out(uint32_t v, uint32_t slots, uint3
 // 1 ..]: clear chunks (kClearChunk slots) of the table each active rolling
 // instance claims its next layer in (table (depth + 1) % 3, from depth 2).
 __global__ __launch_bounds__(1024) void batch_tiles_kernel(const BatchInstance* inst, uint32_t slots, uint32_t tile,
-                                                           uint32_t* prefix) {
+                                                           uint32_t* prefix, uint32_t forms) {
   __shared__ uint32_t wave_sums[1024 / kWave];
   const uint32_t i = threadIdx.x;
   uint32_t v = 0, c = 0, o = 0;
@@ -264,10 +264,14 @@ __global__ __launch_bounds__(1024) void batch_tiles_kernel(const BatchInstance* 
     if (inst[i].rolling && inst[i].depth >= 2)
       c = static_cast<uint32_t>((inst[i].table_stride + kClearChunk - 1) / kClearChunk);
   }
-  block_scan_out(v, slots, wave_sums, prefix);
-  block_scan_out(c, slots, wave_sums, prefix + slots + 1);
-  block_scan_out(o, slots, wave_sums, prefix + 2 * (slots + 1));
-  if (i == 0) prefix[kBatchPrefixes * (slots + 1)] = 0;
+  if (forms & kBatchShared) {
+    block_scan_out(v, slots, wave_sums, prefix);
+    block_scan_out(c, slots, wave_sums, prefix + slots + 1);
+  }
+  if (forms & kBatchOwned) {
+    block_scan_out(o, slots, wave_sums, prefix + 2 * (slots + 1));
+    if (i == 0) prefix[kBatchPrefixes * (slots + 1)] = 0;
+  }
 }
 
 // Eight waves per SIMD (64 VGPRs, no spills): the grid of 8 blocks per CU
@@ -628,9 +632,10 @@ hipError_t batch_reset_flag(uint32_t* flag, GraphChain& chain) {
   return add_kernel(chain, batch_reset_flag_kernel, 1, 64, flag);
 }
 
-hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, GraphChain& chain) {
-  if (slots == 0 || slots > kBatchMaxSlots || tile == 0) return hipErrorInvalidValue;
-  return add_kernel(chain, batch_tiles_kernel, 1, 1024, inst, slots, tile, prefix);
+hipError_t batch_tiles(BatchInstance* inst, uint32_t slots, uint32_t tile, uint32_t* prefix, uint32_t forms,
+                       GraphChain& chain) {
+  if (slots == 0 || slots > kBatchMaxSlots || tile == 0 || forms == 0 || forms >= kBatchForms) return hipErrorInvalidValue;
+  return add_kernel(chain, batch_tiles_kernel, 1, 1024, inst, slots, tile, prefix, forms);
 }
 
 hipError_t batch_expand(BatchInstance* inst, uint32_t slots, const uint32_t* prefix, uint32_t tile, uint32_t grid,

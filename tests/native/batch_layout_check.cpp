@@ -21,6 +21,7 @@ using namespace mgbfs;
 static BatchInstance* inst;  // the device's
 static uint32_t overflow;    // owned instances' next step ends in this error
 static uint32_t slots;
+static uint32_t owned_nodes, shared_nodes;  // expansion kernels in the graphs built
 
 extern "C" hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) {
   for (uint32_t i = 0; i < slots; ++i)
@@ -33,12 +34,16 @@ extern "C" hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) {
 
 namespace mgbfs {
 hipError_t batch_reset_flag(uint32_t*, GraphChain&) { return hipSuccess; }
-hipError_t batch_tiles(BatchInstance*, uint32_t, uint32_t, uint32_t*, GraphChain&) { return hipSuccess; }
+hipError_t batch_tiles(BatchInstance*, uint32_t, uint32_t, uint32_t*, uint32_t, GraphChain&) { return hipSuccess; }
 hipError_t batch_clear(const BatchInstance*, uint32_t, const uint32_t*, uint32_t, GraphChain&) { return hipSuccess; }
 hipError_t batch_expand(BatchInstance*, uint32_t, const uint32_t*, uint32_t, uint32_t, uint32_t, GraphChain&) {
+  ++shared_nodes;
   return hipSuccess;
 }
-hipError_t batch_owned(BatchInstance*, uint32_t, uint32_t*, uint32_t, GraphChain&) { return hipSuccess; }
+hipError_t batch_owned(BatchInstance*, uint32_t, uint32_t*, uint32_t, GraphChain&) {
+  ++owned_nodes;
+  return hipSuccess;
+}
 hipError_t batch_finish(BatchInstance*, uint32_t, uint32_t*, GraphChain&) { return hipSuccess; }
 hipError_t batch_clear_visited(const BatchInstance*, const BatchInstall*, uint32_t, uint64_t, hipStream_t s) {
   return fake::launch(s);
@@ -84,6 +89,42 @@ static std::vector<Range> parts(const BatchInstance& d) {
 }
 
 int main() {
+  // Steps take the kernels that their instances need: degree 8, then 11, then
+  // both.
+  {
+    auto rotations = [](uint32_t n) {
+      Graph g;
+      g.elements = n;
+      g.generators = 2;
+      for (uint32_t i = 0; i < n; ++i) g.perms.push_back((i + 1) % n);
+      for (uint32_t i = 0; i < n; ++i) g.perms.push_back(i < 2 ? 1 - i : i);
+      for (uint32_t i = 0; i < n; ++i) g.start.push_back(i);
+      return g;
+    };
+    mgbfs_batch_options o{};
+    slots = o.max_slots = 2;
+    o.vram_budget = 4ull << 30;
+    o.layers_per_graph = 4;
+    BatchEngine b(o);
+    int32_t s = 0;
+    b.admit(rotations(8), 1, 0, &s);
+    b.step(1);
+    require(shared_nodes == 4 && owned_nodes == 0, "a step without instances by owners");
+    b.admit(rotations(11), 1, 0, &s);
+    b.step(1);
+    require(shared_nodes == 4 && owned_nodes == 4, "a step of instances by owners alone");
+    b.release(0);
+    b.release(1);
+    b.admit(rotations(8), 1, 0, &s);
+    b.admit(rotations(11), 1, 0, &s);
+    b.step(1);
+    require(shared_nodes == 8 && owned_nodes == 8, "a step of both");
+    b.release(0);
+    b.release(1);
+    b.admit(rotations(11), 1, 0, &s);
+    b.step(1);
+    require(shared_nodes == 8 && owned_nodes == 8, "graphs are built once");
+  }
   uint32_t owned = 0, restarted = 0;
   for (uint32_t n : {9u, 10u, 11u})
     for (uint32_t history : {0u, 1u, 2u})
