@@ -113,24 +113,59 @@ struct BatchPlan {
   uint32_t max_layers = kDefaultMaxLayers;
 };
 
-// Bitmap instances of these degrees run by owners of the bitmap where their
-// slot's block holds it: no claim is a global atomic (27 G/s for the whole
-// chip), states take four bytes.  Sweeps of 16, 60, 256 random sets of degree
-// 9 and 10 went from 5.6, 13.5, 45 to 3.9, 7.9, 22.5 ms, 6, 12, 20 mixed jobs
-// of degree 8 to 12 and SL(2, Z_p) from 8.3, 41, 94 to 4.8, 19, 52 ms (of
-// which 20 are hash tables).  Below degree 9 an instance has too little work
-// to split.
+// Bitmap instances of degree 9 to 12 whose generators reach the whole group
+// (reaches_whole_group) may run by owners of the bitmap: no claim is a global
+// atomic (27 G/s for the whole chip), states take four bytes.  What it costs
+// is a launch a layer when other instances run too, and a step of every owner
+// however few its states: eight rotation subgroups of S_12, twelve states
+// each, took 2.9 ms against 0.37.  So it is for what a step's instances are
+// together (times by owners over the shared bitmap's: LRX sets, then two
+// random generators, five with inverses, sixteen).
+//
+// Degree 11 and 12 always: one S_11 0.55, 0.61, 0.63, 0.69, S_12 0.44, 0.38,
+// 0.59, 0.40; one S_11 beside 32 S_8 0.67, 0.64, 0.70, 0.75.
+//
+// Degree 10 beside such (one S_10 with S_11 0.65, 0.52, 0.63, 0.67), or eight
+// and more (beside 8 S_8 0.70, 0.73, 0.70, 0.80), or alone (0.85, 0.77, 0.89,
+// 1.00), or four and more with at most twice as many of degree 9 (four each
+// 0.90, 0.71, 0.68, 0.77) and as many others (0.86, 0.74, 0.72, 0.83).  Not one
+// beside S_8 (1.19, 1.14, 1.17, 1.26), nor
+// one beside three S_9 (0.93, 0.81, 0.97, 1.12), two beside six (0.87, 0.70,
+// 1.04, 1.21).
+//
+// Degree 9 never by itself (two 1.06, 1.08, 1.20, 1.47; 200 of them 2.31,
+// 1.78, 1.12, 1.25), but with the others while it is not the most of them, as
+// a step then has one form (8 S_10 and 8 S_9: 0.72, 0.65, 0.66, 0.75 against
+// 0.80, 0.72, 0.81, 0.86 with degree 9 on the shared bitmap; 8 and 64: 1.50,
+// 1.21, 0.86, 0.93 against 0.87, 0.86, 0.88, 0.95; S_11 and 4 S_9: 0.77, 0.61,
+// 0.66, 0.71 against 0.73, 0.61, 0.72, 0.76).
 constexpr uint32_t kOwnedDegree = 9;
 
-// Owners of an instance when `instances` run.  Alone a degree 9 or 10 search
-// has 251; many together have fewer, so that a step of small layers stays
-// near two owners a workgroup (16 instances: 251, 101 or 53 owners 6.0, 3.6,
-// 3.8 ms; 30: 101 or 53 5.8, 5.1 ms), but not below 53, where a tile's
-// children meet on too few counters (60 instances: 53 or 23 owners 7.8, 9.0
-// ms).  Degrees 11 and 12 keep their own number: their layers are large.
-uint32_t owners_for(uint32_t degree, uint32_t instances) {
+// Instances of a step that may run by owners, by degree, and the others.
+struct OwnedChoice {
+  uint32_t large = 0, tens = 0, nines = 0, others = 0;
+  void count(uint32_t degree) { ++(degree >= 11 ? large : (degree == 10 ? tens : nines)); }
+  bool ten() const {
+    return large || tens >= 8 || (tens >= 4 && nines <= 2 * tens && others <= tens) || (nines == 0 && others == 0);
+  }
+  bool nine() const { return (large || (tens && ten())) && nines <= 2 * tens + 4 * large; }
+  bool takes(uint32_t degree) const { return degree >= 11 || (degree == 10 ? ten() : nine()); }
+  // Instances by owners that share the workgroups, one of degree 9 (a tenth of
+  // the states) for a quarter.
+  uint32_t together() const { return large + (ten() ? tens : 0) + (nine() ? (nines + 3) / 4 : 0); }
+};
+
+// Owners of an instance when `together` run by owners: at degree 9 and 10 so
+// many that a step's owners are about one a workgroup (S_10 LRX sets, milliseconds by
+// 251, 151, 101, 53 owners: one 1.24, 1.21, 1.24, 1.39; three 2.55, 1.49,
+// 1.50, 1.50; four 2.83, 2.11, 1.56, 1.54; eight 5.52, 3.45, 2.63, 1.84; with
+// sixteen generators 1.41, 1.37, 1.71, 2.59; 2.34, 1.84, 2.29, 2.66; 2.82,
+// 2.40, 2.35, 2.68; 5.19, 3.92, 4.16, 3.87), but not below 53, where a tile's
+// children meet on too few counters.  Degrees 11 and 12 keep their own number:
+// their layers are large.
+uint32_t owners_for(uint32_t degree, uint32_t together) {
   if (degree >= 11) return rank_plan(degree).owners;
-  return 251 * instances <= 2048 ? 251 : (101 * instances <= 2048 ? 101 : 53);
+  return together <= 3 ? 151 : (together <= 6 ? 101 : 53);
 }
 
 class BatchEngine {
@@ -370,7 +405,8 @@ class BatchEngine {
       for (uint32_t e = 0; e < g.elements; ++e) start_key |= static_cast<uint64_t>(g.start[e]) << (e * eb);
     }
     const bool first_try = !jobs_[slot].shared;
-    owned_wanted_[slot] = p.visited == kVisBitmap && first_try && g.elements >= kOwnedDegree && g.elements <= kRankDegree;
+    owned_wanted_[slot] = p.visited == kVisBitmap && first_try && g.elements >= kOwnedDegree &&
+                          g.elements <= kRankDegree && reaches_whole_group(g);
     // The visited set is emptied, and the descriptor installed and seeded,
     // by the next flush(), which the next step runs before its graph.
     pending_[slot] = kInstallSeed;
@@ -535,11 +571,11 @@ class BatchEngine {
   // bitmap_bits), list, layer sizes and two message buffers.  Steps send so
   // few states that an owner's share of their children leaves a third of its
   // messages free.
-  void lay_out_owned(uint32_t slot, uint32_t running) {
+  void lay_out_owned(uint32_t slot, uint32_t together) {
     const Graph& g = jobs_[slot].graph;
     BatchInstance& d = host_inst_[slot];
     const Block& block = slots_[slot].block;
-    const RankPlan p = rank_plan(g.elements, owners_for(g.elements, running));
+    const RankPlan p = rank_plan(g.elements, owners_for(g.elements, together));
     uint64_t at = 0;
     auto part = [&](uint64_t bytes) {
       const uint64_t start = at;
@@ -582,16 +618,22 @@ class BatchEngine {
     uint32_t n = 0;
     uint64_t clear_bytes = 0;  // largest visited set to empty
     BatchInstall* req = reinterpret_cast<BatchInstall*>(host_stage_ + slots_n_);
-    // How many instances run from here on decides how finely the new ones
-    // are split.
-    uint32_t running = 0, forms = 0;
+    // What runs from here on decides the form of the new instances, and how
+    // finely they are split.
+    uint32_t forms = 0;
+    OwnedChoice choice;
     auto runs = [&](uint32_t s) {
       return pending_[s] == kInstallSeed || (slots_[s].used && (host_inst_[s].status & kInstActive));
     };
-    for (uint32_t s = 0; s < slots_n_; ++s) running += runs(s);
+    auto may = [&](uint32_t s) { return pending_[s] == kInstallSeed ? owned_wanted_[s] : host_inst_[s].rank.owners; };
     for (uint32_t s = 0; s < slots_n_; ++s) {
       if (!runs(s)) continue;
-      if (pending_[s] == kInstallSeed && owned_wanted_[s]) lay_out_owned(s, running);
+      if (may(s)) choice.count(host_inst_[s].degree);
+      else ++choice.others;
+    }
+    for (uint32_t s = 0; s < slots_n_; ++s) {
+      if (!runs(s)) continue;
+      if (pending_[s] == kInstallSeed && owned_wanted_[s] && choice.takes(host_inst_[s].degree)) lay_out_owned(s, choice.together());
       forms |= host_inst_[s].rank.owners ? kBatchOwned : kBatchShared;
     }
     if (!forms) forms = kBatchShared;

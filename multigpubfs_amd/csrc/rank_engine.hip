@@ -196,6 +196,56 @@ void RankRun::export_layer(uint64_t back, uint64_t limit, uint64_t* keys, hipStr
   MGBFS_HIP(rank_export(plan, memory.list, d ? ends(d - 1) : ends(kEnds - 1), ends(d), limit, keys, stream));
 }
 
+// ------------------------------------------------------------ groups
+
+// A transitive group with a p-cycle, p prime and more than half the degree, is
+// primitive (no block of a system can be moved within p points without
+// meeting itself), and a primitive group with a p-cycle, p <= degree - 3,
+// holds the alternating group (Jordan).  An element has a p-cycle when a
+// power of it is one; in the whole group one in p has.  So: transitivity, then
+// random products of the generators (each of a few kept ones multiplied by
+// another) until one shows it.
+bool reaches_whole_group(const Graph& g) {
+  const uint32_t n = g.elements, G = g.generators;
+  uint32_t p = 0;
+  for (uint32_t q : {5u, 7u})
+    if (2 * q > n && q + 3 <= n) p = q;
+  if (g.kind != 0 || n > kRankDegree || !p || !G) return false;
+  uint32_t reached = 1;
+  for (uint32_t before = 0; before != reached;) {
+    before = reached;
+    for (uint32_t k = 0; k < G; ++k)
+      for (uint32_t i = 0; i < n; ++i)
+        if ((reached >> i) & 1u) reached |= 1u << g.perms[k * n + i];
+  }
+  if (reached != (1u << n) - 1) return false;
+  bool commute = true;  // a transitive commutative group has n elements
+  for (uint32_t a = 0; a < G; ++a)
+    for (uint32_t b = 0; b < a && commute; ++b)
+      for (uint32_t i = 0; i < n && commute; ++i)
+        commute = g.perms[a * n + g.perms[b * n + i]] == g.perms[b * n + g.perms[a * n + i]];
+  if (commute) return false;
+  constexpr uint32_t kKept = 8, kWarm = 32, kTries = 64;
+  uint8_t kept[kKept][kRankDegree];
+  for (uint32_t k = 0; k < kKept; ++k)
+    for (uint32_t i = 0; i < n; ++i) kept[k][i] = static_cast<uint8_t>(g.perms[(k % G) * n + i]);
+  uint32_t random = 1;
+  for (uint32_t t = 0; t < kWarm + kTries; ++t) {
+    random = random * 1664525u + 1013904223u;
+    const uint32_t a = random >> 29, b = (a + 1 + ((random >> 16) % (kKept - 1))) % kKept;
+    uint8_t product[kRankDegree];
+    for (uint32_t i = 0; i < n; ++i) product[i] = kept[a][kept[b][i]];
+    for (uint32_t i = 0; i < n; ++i) kept[a][i] = product[i];
+    if (t < kWarm) continue;
+    for (uint32_t i = 0, seen = 0; i < n; ++i) {
+      uint32_t length = 0;
+      for (uint32_t j = i; !((seen >> j) & 1u); j = product[j], ++length) seen |= 1u << j;
+      if (length == p) return true;
+    }
+  }
+  return false;
+}
+
 // ------------------------------------------------------------ backend
 
 class RankBitmapEngine final : public Engine {

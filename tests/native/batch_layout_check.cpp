@@ -3,19 +3,10 @@
 // restart that follows a full message slab, under every choice of history,
 // layer share and bitmap bias.  The kernels only set what the check asks for.
 #include <vector>
-#include "fake_hip.hpp"
-#include "device_cache.hip"
-#include "engine.hip"
+#include "rank_on_host.hpp"
 #include "batch_engine.hip"
-#define rank_seed device_rank_seed
-#define rank_layer device_rank_layer
-#define rank_block device_rank_block
-#define rank_export device_rank_export
-#define rank_report device_rank_report
-#include "rank_owner.hip"
 
 using fake::holds;
-using fake::require;
 using namespace mgbfs;
 
 static BatchInstance* inst;  // the device's
@@ -88,7 +79,27 @@ static std::vector<Range> parts(const BatchInstance& d) {
   return r;
 }
 
+// Which degrees of a step's instances go by owners.
+static bool takes(uint32_t degree, uint32_t large, uint32_t tens, uint32_t nines, uint32_t others) {
+  OwnedChoice c;
+  c.large = large;
+  c.tens = tens;
+  c.nines = nines;
+  c.others = others;
+  return c.takes(degree);
+}
+
 int main() {
+  require(takes(12, 1, 0, 0, 5) && takes(11, 1, 1, 9, 9), "degree 11 and 12 always");
+  require(takes(10, 0, 1, 0, 0) && takes(10, 0, 7, 0, 0) && takes(10, 1, 1, 0, 9) && takes(10, 0, 8, 99, 9) &&
+              takes(10, 0, 4, 8, 4),
+          "degree 10 alone, beside larger ones or many together");
+  require(!takes(10, 0, 1, 0, 1) && !takes(10, 0, 3, 1, 0) && !takes(10, 0, 4, 9, 0) && !takes(10, 0, 7, 0, 8) &&
+              !takes(10, 0, 3, 0, 1),
+          "not few of degree 10 beside others");
+  require(takes(9, 0, 4, 8, 0) && takes(9, 0, 8, 16, 9) && takes(9, 1, 0, 4, 9) && !takes(9, 0, 8, 17, 0) &&
+              !takes(9, 0, 0, 200, 0) && !takes(9, 0, 0, 1, 0) && !takes(9, 1, 0, 5, 0) && !takes(9, 0, 3, 1, 0),
+          "degree 9 beside enough larger ones");
   // Steps take the kernels that their instances need: degree 8, then 11, then
   // both.
   {

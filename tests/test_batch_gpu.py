@@ -335,6 +335,59 @@ def test_sample_of_an_instance_stopped_at_its_layer_limit(n, layers, copies):
             assert sorted(rows) == sorted(ref["keys"][layers - 1])
 
 
+# A step of the batch runs one form of instances or both, by what is there:
+# degree 10 alone (151, 101, 53 owners for 1, 4 and 21), degree 9 beside it or
+# beside degree 11, eight of degree 10 beside smaller ones, and sets that stay
+# on the shared bitmap; smaller searches join when some layers are done.
+@pytest.mark.parametrize("jobs", [{10: 1}, {10: 4}, {10: 21}, {10: 4, 9: 8}, {11: 1, 9: 4, 8: 2}, {10: 8, 8: 3}, {9: 3},
+                                  {10: 1, 8: 1}], ids=str)
+def test_forms_of_a_step_match_oracle(jobs):
+    rng = random.Random(5)
+    sets = {}
+    for n in {*jobs, 8}:
+        gens = [[(i + 1) % n for i in range(n)], rng.sample(range(n), n), rng.sample(range(n), n)]
+        sets[n] = gens, O.packed_bfs(n, gens, keep_keys=n <= 10)
+    late = [GraphDefinition.permutation(sets[8][0], list(range(8))), sl2(11), GOLDEN[0]["graph"]]
+    with BatchEngine(max_slots=32, layers_per_graph=1, vram_budget=16 << 30) as b:
+        slots = [(n, b.admit(GraphDefinition.permutation(sets[n][0], list(range(n)))))
+                 for n, count in jobs.items() for _ in range(count)]
+        watched = {n: s for n, s in slots}
+        steps = 0
+        while b.step(1):
+            steps += 1
+            for n, s in watched.items():
+                sizes, ref = b.result(s)[0], sets[n][1]
+                assert sizes == ref["layers"][:len(sizes)]
+                if n <= 10:
+                    rows = [O.pack(r) for r in b.sample(s, n, 500)]
+                    assert len(set(rows)) == min(500, sizes[-1]) and set(rows) <= set(ref["keys"][len(sizes) - 1])
+            if steps == 3:
+                late = [b.admit(g) for g in late]
+        for n, s in slots:
+            sizes, _, error = b.result(s)
+            assert not error and sizes == sets[n][1]["layers"]
+        assert b.result(late[0])[0] == sets[8][1]["layers"]
+        assert sum(b.result(late[1])[0]) == 11 * 120 and b.result(late[2])[0] == GOLDEN[0]["layer_sizes"]
+
+
+@pytest.mark.parametrize("copies,bound", [(1, 919200), (4, 916600), (21, 914200)])
+def test_overflowing_messages_start_over_on_the_shared_bitmap(copies, bound):
+    # A declared state bound far below n! leaves an owner room for some 70
+    # messages at a time, of which a step uses two thirds on average: now and then one gets more.
+    n = 10
+    gens = O.lrx_generators(n)
+    ref = O.packed_bfs(n, gens, keep_keys=True)
+    graph = GraphDefinition.permutation(gens, list(range(n)), expected_max_unique_states=bound)
+    with BatchEngine(max_slots=32, vram_budget=8 << 30) as b:
+        slots = [b.admit(graph, visited="bitmap") for _ in range(copies)]
+        b.run()
+        for s in slots:
+            sizes, _, error = b.result(s)
+            assert not error and sizes == ref["layers"]
+            assert sorted(O.pack(r) for r in b.sample(s, n, 10**6)) == sorted(ref["keys"][-1])
+        assert any(b.instance_info(s)["restarts"] for s in slots)
+
+
 def test_engines_made_beside_other_threads_copies():
     # Batch engines come and go in one thread while another's engines upload
     # their generators and read their states back.

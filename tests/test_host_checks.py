@@ -9,7 +9,8 @@ import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
 CHECKS = {"rank_memory_check": "rank memory ok", "sorted_memory_check": "sorted memory ok",
-          "batch_layout_check": "batch layout ok", "rebind_check": "rebind ok"}
+          "batch_layout_check": "batch layout ok", "rebind_check": "rebind ok",
+          "group_check": "groups ok"}
 
 
 @pytest.mark.parametrize("name", list(CHECKS))
