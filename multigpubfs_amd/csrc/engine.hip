@@ -914,9 +914,12 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
 
 static Engine* create(const Graph& g, const mgbfs_engine_options& o) {
   switch (choose_backend(g, o.backend)) {
-    case MGBFS_BACKEND_BITMAP:
-      if (rank_bitmap_takes(g, o)) return new HandoverEngine(g, o);
-      return make_bitmap_engine(g, o);
+    case MGBFS_BACKEND_BITMAP: {
+      if (!rank_bitmap_takes(g, o)) return make_bitmap_engine(g, o);
+      mgbfs_engine_options named = o;  // AUTO chooses it for directed sets
+      named.backend = MGBFS_BACKEND_BITMAP;
+      return new HandoverEngine(g, named);
+    }
     case MGBFS_BACKEND_SORTED:
       return new HandoverEngine(g, o);
     case MGBFS_BACKEND_SEGMENTED: {

@@ -123,6 +123,16 @@ int main() {
     require(e->layers.size() == 1 && !e->terminal, "at its start");
     d.limit = ~static_cast<size_t>(0);
   }
+  // AUTO takes directed sets to the bitmap too, rebound as by name.
+  {
+    const Graph one = graph_of(9, {{1, 2, 3, 4, 5, 6, 7, 8, 0}, swaps(9, 1)[0]}, false);
+    o.backend = MGBFS_BACKEND_AUTO;
+    std::unique_ptr<Engine> e(create(one, o));
+    require(e->backend == MGBFS_BACKEND_BITMAP && e->run_to_end() == MGBFS_COMPLETE && e->layers == plain(one),
+            "a directed set by owners");
+    e->rebind(graph_of(9, swaps(9, 3), false));
+    require(e->run_to_end() == MGBFS_COMPLETE && e->layers == plain(graph_of(9, swaps(9, 3), false)), "and rebound");
+  }
   // A given budget bounds a rebound engine by name too.
   o.backend = MGBFS_BACKEND_BITMAP;
   o.vram_budget = 64ull << 20;

@@ -492,3 +492,20 @@ def test_auto_backend_by_degree_and_budget(n, budget, name):
         e.rebind(GraphDefinition.permutation(gens, start))
         assert e.run() == 1 and e.backend_name == NAMES["sorted"]
         assert e.layer_sizes() == [len(x) for x in O.c_exact_layers(graph, math.factorial(n))]
+
+
+@pytest.mark.parametrize("n", [2, 3, 8, 10, 13])
+def test_auto_runs_directed_sets_on_the_bitmap(n):
+    gens = [O.lrx_generators(n)[0], O.lrx_generators(n)[2]] if n > 2 else [[1, 0]]
+    if n == 13:  # a small orbit over a 778 MB bitmap
+        gens = [[1, 2, 0] + list(range(3, 13)), list(range(9)) + [10, 11, 12, 9]]
+    with NativeEngine(GraphDefinition.permutation(gens, list(range(n)))) as e:
+        assert e.backend_name == NAMES["permutation_bitmap" if n > 2 else "sorted"]
+        assert e.run() == 1
+        sizes = e.layer_sizes()
+        if n <= 10:
+            assert sizes == O.packed_bfs(n, gens)["layers"]
+            e.rebind(GraphDefinition.permutation([gens[-1], gens[0]], list(range(n))))
+            assert e.run() == 1 and e.layer_sizes() == sizes
+        else:
+            assert sum(sizes) == 12
