@@ -320,19 +320,35 @@ class SortedEngine final : public Engine {
   }
 
  private:
-  // Bank rows for the layers run ahead, so that they need no growth: as many
-  // as the state space has, at most kAheadRows.  Called with the start layer
-  // current, which is written again as bank 0 may have moved.  Without the
-  // memory for it (an eighth of the budget at most, so that larger layers
-  // find theirs) the layers take the general path.
-  void reserve_banks() {
-    const uint64_t rows =
-        std::max<uint64_t>(2 * kBlockParents, std::min({bound_ ? bound_ : kAheadRows, cap_limit_, kAheadRows}));
-    if (bank_cap_[0] >= rows && bank_cap_[1] >= rows && bank_cap_[2] >= rows) return;
-    if (8 * (3 * rows + kOwnerBuffers * owner_entries(kOwnersSmall)) > budget_ / 8) return;
-    const bool grown = grow_bank(0, rows);
-    start_bank();
-    if (grown && grow_bank(1, rows)) grow_bank(2, rows);
+  // Bank rows for the layers run ahead, so that they need no growth: what one
+  // workgroup's table holds at the start; with the first owner layer as many
+  // as the state space has, at most kAheadRows (a search that stays small
+  // never pays for three 32 MB banks: rotations of 15 created and run 1.9 ms
+  // with them from the start, 0.3 without).  Without the memory for it (an
+  // eighth of the budget at most, so that larger layers find theirs) the
+  // layers take the general path.
+  void reserve_banks(uint64_t rows, uint64_t beside) {
+    if (8 * (3 * rows + beside) > budget_ / 8) return;
+    for (int b = 0; b < 3; ++b)
+      if (!widen_bank(b, rows)) return;
+  }
+  uint64_t owner_rows() const {
+    return std::max<uint64_t>(2 * kBlockParents, std::min({bound_ ? bound_ : kAheadRows, cap_limit_, kAheadRows}));
+  }
+  // grow_bank() with the layer in it kept.
+  bool widen_bank(int b, uint64_t rows) {
+    if (bank_cap_[b] >= rows) return true;
+    if (!fits(rows * 8)) return false;
+    DeviceBuffer fresh;
+    fresh.allocate(rows * 8);
+    if ((b == cur_ || b == prev_) && count_[b])
+      MGBFS_HIP(hipMemcpyAsync(fresh.as<uint64_t>(), bank_[b].as<uint64_t>(), count_[b] * 8, hipMemcpyDeviceToDevice,
+                               stream_));
+    MGBFS_HIP(hipStreamSynchronize(stream_));
+    bank_[b] = std::move(fresh);
+    bank_cap_[b] = rows;
+    update_bytes();
+    return true;
   }
   // Entries of one slab array (with the routing dump area).
   static constexpr uint64_t owner_entries(uint32_t owners) { return owners * static_cast<uint64_t>(kSlabStride) + kRouteDump; }
@@ -350,7 +366,7 @@ class SortedEngine final : public Engine {
   // is one for the general path (too large, or rejected on the device).
   int run_ahead(uint32_t max_layers) {
     if (general_only_) return kAheadNone;
-    if (layers.size() == 1) reserve_banks();
+    if (layers.size() == 1) reserve_banks(kBlockSlots, 0);
     const uint64_t F = count_[cur_], rows = bank_rows();
     const bool probe_prev = prev_ >= 0 && !layout_.prune;
     const uint64_t Fp = prev_ >= 0 ? count_[prev_] : 0;
@@ -359,8 +375,8 @@ class SortedEngine final : public Engine {
       const int s = run_block(max_layers, static_cast<uint32_t>(rows));
       if (s != kAheadNone) return s;
     }
-    if (F > rows || F * gens_.count > 0x7fffffffull || owner_rejected_ == layers.size()) return kAheadNone;
-    return run_owner(max_layers, static_cast<uint32_t>(rows));
+    if (F * gens_.count > 0x7fffffffull || owner_rejected_ == layers.size()) return kAheadNone;
+    return run_owner(max_layers);
   }
 
   // Children expected of the current layer (see advance_general): the last
@@ -412,10 +428,13 @@ class SortedEngine final : public Engine {
   // A session of owner layers: each is one launch, which also reports the
   // layer before it; the host stays kOwnerAhead launches ahead.  256 owners
   // (one workgroup per CU) while the children fit their slabs, else 1,024.
-  int run_owner(uint32_t max_layers, uint32_t rows) {
+  int run_owner(uint32_t max_layers) {
     const uint64_t F = count_[cur_], guess = children_guess(F);
     const uint32_t owners = guess <= kOwnersSmall * kOwnerMean / 2 ? kOwnersSmall : kOwnersMax;
     if (guess > static_cast<uint64_t>(owners) * kOwnerMean) return kAheadNone;
+    reserve_banks(owner_rows(), kOwnerBuffers * owner_entries(kOwnersSmall));
+    if (F > bank_rows()) return kAheadNone;
+    const uint32_t rows = static_cast<uint32_t>(bank_rows());
     const uint64_t entries = owner_entries(owners);
     if (owner_.bytes() < kOwnerBuffers * entries * 8) {
       if (kOwnerBuffers * entries * 8 > budget_ / 8 || !fits(kOwnerBuffers * entries * 8 - owner_.bytes()))

@@ -172,6 +172,12 @@ int main() {
         }
         require(k > 4, "allocations to fail");
       }
+  // A search that stays within one workgroup keeps small banks.
+  script = {1, 2, 2, 2, 1, 0};
+  o.flags = 0;
+  engine.reset(make_sorted_engine(g, o));
+  const uint64_t made = engine->device_bytes;
+  require(engine->run_to_end() == MGBFS_COMPLETE && engine->device_bytes - made < (1u << 20), "small banks");
   engine.reset();
   std::printf("sorted memory ok\n");
   return 0;
