@@ -419,9 +419,14 @@ class RankBitmapEngine final : public Engine {
 // degree 12 (figures in rank_owner.hip).  A capacity bounds the rows of a
 // layer and a message buffer is not one, so a set capacity keeps the shared
 // bitmap; so does a budget that does not hold the messages of every layer
-// (degree 12 with three generators: 13.5 GB, of which 4.3 are used).
+// (degree 12 with three generators: 13.5 GB, of which 4.3 are used).  The
+// buffers are made for the whole group, 0.3 GB at degree 11 and 4.3 at 12, so
+// generators that are not seen to reach it keep the other form there (two
+// swaps of S_12, four states: 76 to 140 ms to create, run and drop an engine
+// in a process that has used some memory, against 1.7).
 bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o, uint64_t held) {
   if (g.elements < 3 || g.elements > kRankDegree || o.capacity || g.generators > kMaxGenerators) return false;
+  if (g.elements >= 11 && !reaches_whole_group(g)) return false;
   if (!o.vram_budget) MGBFS_HIP(hipSetDevice(o.device));
   return RankBitmapEngine::most_bytes(g) <= vram_budget(o) + (o.vram_budget ? 0 : held);
 }

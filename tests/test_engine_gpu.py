@@ -509,3 +509,25 @@ def test_auto_runs_directed_sets_on_the_bitmap(n):
             assert e.run() == 1 and e.layer_sizes() == sizes
         else:
             assert sum(sizes) == 12
+
+
+@pytest.mark.parametrize("backend", ["auto", "permutation_bitmap"])
+@pytest.mark.parametrize("n", [11, 12])
+def test_small_groups_of_large_degree_take_little_memory(n, backend):
+    # Two swaps, and rotations: 4 and n states.  The library's choice is the
+    # sorted backend, by name the bitmap takes what its shared form takes.
+    rot = O.lrx_generators(n)[:2]
+    for gens, states in (([[1, 0] + list(range(2, n)), [0, 1, 3, 2] + list(range(4, n))], 4), (rot, n)):
+        with NativeEngine(GraphDefinition.permutation(gens, list(range(n))), backend=backend) as e:
+            assert e.backend_name == NAMES["sorted" if backend == "auto" else backend]
+            assert e.run() == 1 and sum(e.layer_sizes()) == states
+            held = e.info()["device_bytes"]
+            if backend == "auto":
+                assert held < 128 << 20
+            else:
+                with NativeEngine(GraphDefinition.permutation(gens, list(range(n))), backend=backend,
+                                  capacity=math.factorial(n)) as shared:
+                    assert shared.run() == 1 and held == shared.info()["device_bytes"]
+            if n == 11:
+                e.rebind(lrx(n))
+                assert e.run() == 1 and e.layer_sizes() == O.packed_bfs(n)["layers"]
