@@ -506,6 +506,11 @@ __global__ void batch_finish_kernel(BatchInstance* inst, uint32_t slots, uint32_
     s.status = kInstDone;
     return;
   }
+  if (s.rank.owners && nc > s.cap) {  // a layer beyond the state bound, which the lists have room for
+    s.error |= kErrFutureCap;
+    s.status = kInstDone;
+    return;
+  }
   if (s.depth + 1 >= s.max_layers) {
     s.error |= kErrCount;
     s.status = kInstDone;

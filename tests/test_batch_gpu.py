@@ -416,3 +416,21 @@ def test_engines_made_beside_other_threads_copies():
         stop.set()
         thread.join()
     assert not errors and made[0] == 60 and made[1] > 5
+
+
+@pytest.mark.parametrize("n", [8, 10])
+def test_layer_beyond_the_declared_bound_is_an_error(n):
+    # Sixteen generators: the widest layer holds more states than the graph
+    # declares in all, by owners (degree 10) as over the shared bitmap.
+    rng = random.Random(n)
+    gens = [rng.sample(range(n), n) for _ in range(16)]
+    ref = O.packed_bfs(n, gens)["layers"]
+    bound = {8: 5000, 10: 1_000_000}[n]
+    assert max(ref) > bound
+    with BatchEngine(max_slots=2) as b:
+        graph = GraphDefinition.permutation(gens, list(range(n)), expected_max_unique_states=bound)
+        slot, free = b.admit(graph, visited="bitmap"), b.admit(GraphDefinition.permutation(gens, list(range(n))))
+        b.run()
+        sizes, _, error = b.result(slot)
+        assert error and sizes == ref[:len(sizes)] and max(sizes) <= bound
+        assert b.result(free)[0] == ref and not b.result(free)[2]
