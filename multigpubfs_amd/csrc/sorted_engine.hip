@@ -52,6 +52,9 @@ class SortedEngine final : public Engine {
     budget_ = vram_budget(o);
     bound_ = state_space_bound(g);
     cap_limit_ = o.capacity ? o.capacity : ~0ull;
+    // The segmented tables hold no layer beyond the state bound (and a quarter,
+    // by which their arenas grow): such a layer goes there and ends the run.
+    if (wide_ && bound_) cap_limit_ = std::min(cap_limit_, bound_ + bound_ / 4);
     flags_ = o.flags;
     // Stored-value layout and parent-edge tags.
     const uint32_t key_bits = wide_ ? std::max(32u, wide_->key_bits()) : sorted_key_bits(n_);
@@ -357,9 +360,9 @@ class SortedEngine final : public Engine {
     MGBFS_HIP(sorted_start(keymix(start_key_, layout_.km) << layout_.tagbits, bank_[0].as<uint64_t>(),
                            off_[0].as<uint32_t>(), control_.as<uint64_t>(), stream_));
   }
-  uint64_t bank_rows() const {
-    return std::min({bank_cap_[0], bank_cap_[1], bank_cap_[2], cap_limit_, static_cast<uint64_t>(0xfffffff0u)});
-  }
+  uint64_t bank_room() const { return std::min({bank_cap_[0], bank_cap_[1], bank_cap_[2]}); }
+  // Rows that a layer run ahead may have.
+  uint64_t bank_rows() const { return std::min({bank_room(), cap_limit_, static_cast<uint64_t>(0xfffffff0u)}); }
 
   // Runs up to max_layers layers in the one-workgroup kernel or as owner
   // layers, whichever the current layer's size asks for; kAheadNone when it
@@ -370,7 +373,7 @@ class SortedEngine final : public Engine {
     const uint64_t F = count_[cur_], rows = bank_rows();
     const bool probe_prev = prev_ >= 0 && !layout_.prune;
     const uint64_t Fp = prev_ >= 0 ? count_[prev_] : 0;
-    if (F <= kBlockParents && (!probe_prev || Fp <= kBlockParents) && rows >= 2 * kBlockParents &&
+    if (F <= kBlockParents && (!probe_prev || Fp <= kBlockParents) && bank_room() >= 2 * kBlockParents &&
         children_guess(F) <= kBlockChildren && block_rejected_ != layers.size()) {
       const int s = run_block(max_layers, static_cast<uint32_t>(rows));
       if (s != kAheadNone) return s;

@@ -292,3 +292,22 @@ def test_wide_keys_out_of_memory_stop_with_their_layers(step):
             info = e.info()
             assert info["device_bytes"] <= budget and info["candidates"] == 4 * sum(sizes[:-1])
             e.reset()
+
+
+@pytest.mark.parametrize("name,bound", [("sl2", 2000), ("ring", 300)])
+def test_layer_beyond_the_declared_bound_stops_the_run(name, bound):
+    # Layers of up to 7,030 and 829 states, declared to be fewer in all.
+    if name == "sl2":
+        full = sl2(31)
+        g = GraphDefinition({**full.to_dict(), "expected_max_unique_states": bound})
+    else:
+        full = GraphDefinition.permutation(O.lrx_generators(18), [0] * 12 + [1] * 6)
+        g = GraphDefinition.permutation(O.lrx_generators(18), [0] * 12 + [1] * 6, expected_max_unique_states=bound)
+    want = [len(x) for x in oracle_layers(full, 1 << 20)]
+    assert max(want) > 1.25 * bound
+    with NativeEngine(g, backend="segmented") as e:
+        for _ in range(2):
+            assert e.run() == 2
+            sizes = e.layer_sizes()
+            assert sizes == want[:len(sizes)] and max(sizes) <= 1.25 * bound and len(sizes) > 3
+            e.reset()
