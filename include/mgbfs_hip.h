@@ -109,7 +109,8 @@ typedef struct mgbfs_engine_info {
   uint64_t device_bytes;   /* device memory held by the engine               */
   uint64_t peak_layer;     /* largest layer so far                           */
   uint64_t candidates;     /* generated children so far (edges expanded)     */
-  uint64_t unique_candidates; /* distinct children after in-layer dedup     */
+  uint64_t unique_candidates; /* distinct children after in-layer dedup (0 on
+                                 the bitmap and generic backends)             */
   double kernel_seconds;   /* summed device time of the hot kernels          */
   uint64_t kernel_launches;   /* launches of the hot kernels                 */
   uint64_t algorithmic_bytes; /* modelled streaming HBM bytes of those kernels */
@@ -154,14 +155,15 @@ int mgbfs_engine_create(const mgbfs_graph_desc* graph, const mgbfs_engine_option
 int mgbfs_engine_advance(void* engine, uint64_t* next_count, uint32_t* fatal);
 /* Runs advance() until completion, a resource stop, max_layers layers or
  * max_seconds (0 = unlimited).  Returns the last advance() status.  With
- * neither limit the permutation-bitmap backend may queue several layers per
- * host wait (same layers, same final state). */
+ * neither limit a backend may queue several layers per host wait (same
+ * layers, same final state). */
 int mgbfs_engine_run(void* engine, uint32_t max_layers, double max_seconds);
 int mgbfs_engine_query(void* engine, mgbfs_engine_info* info);
 /* Per-phase device seconds and modelled streaming HBM bytes of the hot
  * kernels, summed over the layers run so far.  Sorted backend phases:
- * 0 expand+route, 1 partition, 2 unique+difference, 3 compaction.
- * Bitmap backend: phase 0 is the fused expand kernel. */
+ * 0 expand+route, and whole layers where one kernel runs them (small and
+ * medium ones), 1 partition, 2 unique+difference, 3 compaction.  Other
+ * backends: phase 0 is all of it. */
 int mgbfs_engine_phases(void* engine, double* seconds, uint64_t* bytes, uint32_t count);
 /* Clears the visited state and re-seeds the start state, keeping every
  * allocation (repeat runs of the same graph, e.g. timing loops). */

@@ -65,7 +65,8 @@ struct LayerRecord {
   uint64_t children;          // block_run: generated for this layer; owner layers: from it
   uint32_t state, pad;        // general path: the error word
   uint64_t seq;
-  uint64_t stamps[4];         // general path: LayerCounters.stamps
+  uint64_t stamps[4];         // general path: LayerCounters.stamps; else [0]: when the launch (the session) began
+  uint64_t compacted;         // LayerCounters.compacted
 };
 
 // Device words of a layer on the general path.
@@ -73,7 +74,7 @@ struct LayerCounters {
   unsigned long long unique;    // distinct children
   uint32_t error, pad;
   unsigned long long children;  // generated
-  unsigned long long spare;
+  unsigned long long compacted;  // wall_clock64() at the end of the last compaction
   unsigned long long stamps[4];  // wall_clock64() at the start of the layer, its partition, unique_diff and scan
 };
 static_assert(sizeof(LayerCounters) == 64, "one 64-byte line");
@@ -98,6 +99,7 @@ struct BlockRun {
   uint32_t rows;             // rows every bank holds (and the caller's layer capacity)
   LayerRecord* rec;          // pinned: one record per layer run
   uint64_t seq;              // rec[i].seq = seq + i
+  const LayerCounters* counters;
 };
 
 // Owner layers: `owners` sub-buckets (equal ranges of the top 32 bits), one
@@ -225,8 +227,10 @@ hipError_t rank_report(const OwnerCtl* ctl, const OwnerRules& rules, LayerRecord
 hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t* control, hipStream_t stream);
 hipError_t sorted_block_run(const BlockRun& run, const ActionRef& act, hipStream_t stream);
 // Zeroes the owners' counts (`words` of them from `counts`) and the first
-// control blocks; ctl[0] becomes the imported layer's, of F states.
-hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream);
+// control blocks; ctl[0] becomes the imported layer's, of F states.  rec: the
+// record that the first layer will leave gets the time.
+hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream,
+                       LayerRecord* rec = nullptr, const LayerCounters* counters = nullptr);
 hipError_t owner_import(const OwnerImport& im, const ActionRef& act, const SortedLayout& L, uint32_t owners,
                         hipStream_t stream);
 hipError_t owner_layer(const OwnerLayer& a, const ActionRef& act, const SortedLayout& L, hipStream_t stream);
@@ -242,8 +246,8 @@ uint64_t scan_workspace_words(uint64_t n);
 // rec: report the layer of `counters` with the scan's total (see scan.hip).
 hipError_t exclusive_scan_u32(const uint32_t* in, uint64_t n, uint32_t* out, uint32_t* workspace, hipStream_t stream,
                               LayerCounters* counters = nullptr, LayerRecord* rec = nullptr, uint64_t seq = 0);
-// One wall_clock64() reading as a record.
-hipError_t stamp_record(LayerRecord* rec, uint64_t seq, hipStream_t stream);
+// A record of nothing but the counters' `compacted`.
+hipError_t stamp_record(LayerRecord* rec, const LayerCounters* counters, uint64_t seq, hipStream_t stream);
 hipError_t sorted_seed(uint64_t start_key, const SortedLayout& L, uint64_t* bank, uint32_t* off, uint32_t Ko,
                        hipStream_t stream);
 // Children of bank[0..F) routed by lane (sub-bucket >> K2) into slabs: slab
@@ -283,9 +287,10 @@ hipError_t sorted_unique_diff(uint64_t* cand, const uint32_t* scount, uint32_t n
                               bool merge, uint32_t grid_limit, hipStream_t stream,
                               unsigned long long* stamp = nullptr);
 // Writes nothing unless *error == 0 and the layer total off[nsub << fb]
-// fits bank_rows, so it may be queued before the host has read either.
+// fits bank_rows, so it may be queued before the host has read either.  done
+// (null: none) is raised to the time of its end.
 hipError_t sorted_compact(const uint64_t* cand, uint32_t nsub, uint32_t fb, const uint32_t* off, const uint32_t* error,
-                          uint64_t bank_rows, uint64_t* bank, hipStream_t stream);
+                          uint64_t bank_rows, uint64_t* bank, hipStream_t stream, unsigned long long* done = nullptr);
 
 // Sets kErrFutureCap in *error when off[n] > rows.
 hipError_t sorted_capacity_check(const uint32_t* off, uint64_t n, uint64_t rows, uint32_t* error,

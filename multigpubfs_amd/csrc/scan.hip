@@ -82,6 +82,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_carry_kernel(uint32_t* __re
   rec->state = counters->error;
   rec->ticks = wall_clock64();
   for (int k = 0; k < 4; ++k) rec->stamps[k] = counters->stamps[k];
+  rec->compacted = counters->compacted;
   __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

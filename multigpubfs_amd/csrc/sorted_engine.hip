@@ -25,9 +25,9 @@ namespace mgbfs {
 
 namespace {
 
-// Phases: expand, partition, unique, compact of the general path; layers run
-// ahead of the host (sorted_queue.hip) count as a whole.
-constexpr uint32_t kPhaseCount = 5;
+// Phases: expand, partition, unique, compact.  Layers run ahead of the host
+// (sorted_queue.hip) are one kernel each and count in the first.
+constexpr uint32_t kPhaseCount = 4;
 constexpr size_t kCtlOffset = 64;       // in control_: the owner layers' control ring, then their slab counts
 constexpr uint32_t kOwnerRing = 64;     // owner layers' control blocks and records
 constexpr uint32_t kOwnerAhead = 3;     // layers queued beyond the one whose record the host waits for
@@ -178,9 +178,8 @@ class SortedEngine final : public Engine {
       // Counters (unique, error, candidates), sub-bucket and lane cursors.
       // The kernels stamp their start times: eight timing events took 4.5 us
       // each on the stream.
-      LayerCounters* counters = control_.as<LayerCounters>();
       MGBFS_HIP(zero_u32x3(reinterpret_cast<uint32_t*>(control_.as<uint64_t>()), 6, scount_.as<uint32_t>(), nsub,
-                           lcount_.as<uint32_t>(), K2 ? lslabs : 0, stream_, &counters->stamps[0]));
+                           lcount_.as<uint32_t>(), K2 ? lslabs : 0, stream_, &counters()->stamps[0]));
       uint64_t* sub = sub_.as<uint64_t>();
       const uint32_t stride = K2 ? lcap : kSlabStride, full = K2 ? kErrLaneSlab : kErrBucketCap;
       uint32_t* cursors = K2 ? lcount_.as<uint32_t>() : scount_.as<uint32_t>();
@@ -196,17 +195,17 @@ class SortedEngine final : public Engine {
       if (K2)
         MGBFS_HIP(sorted_partition(lane_.as<uint64_t>(), lcount_.as<uint32_t>(), lcap, P, nsub, K2,
                                    scount_.as<uint32_t>(), error_word(), sub, routed(sub_entries), stream_,
-                                   &counters->stamps[1]));
+                                   &counters()->stamps[1]));
       auto* control = reinterpret_cast<unsigned long long*>(control_.as<uint64_t>());
       MGBFS_HIP(sorted_unique_diff(
           sub, scount_.as<uint32_t>(), nsub, bank_[cur_].as<uint64_t>(), off_[cur_].as<uint32_t>(), nbo_[cur_],
           probe_prev ? bank_[prev_].as<uint64_t>() : nullptr, probe_prev ? off_[prev_].as<uint32_t>() : nullptr,
           probe_prev ? nbo_[prev_] : 0, fb, fine_counts_.as<uint32_t>(), error_word(), control, control + 2,
-          layout_.tagbits, layout_.prune != 0, unique_grid_, stream_, &counters->stamps[2]));
+          layout_.tagbits, layout_.prune != 0, unique_grid_, stream_, &counters()->stamps[2]));
       // The scan reports the layer (N, error word, counters) in pinned memory.
       const uint64_t seq = seq_++;
       MGBFS_HIP(exclusive_scan_u32(fine_counts_.as<uint32_t>(), nbo, off_[nxt].as<uint32_t>(),
-                                   scan_ws_.as<uint32_t>(), stream_, counters, rec_, seq));
+                                   scan_ws_.as<uint32_t>(), stream_, counters(), rec_, seq));
       // The compaction is queued before the host has read N or the error
       // word; it writes nothing unless the layer is clean and fits the bank
       // as allocated now, and the host relaunches it after growing the bank.
@@ -305,8 +304,8 @@ class SortedEngine final : public Engine {
   void settle() override {
     if (!compacted_) return;
     const uint64_t seq = seq_++;
-    MGBFS_HIP(stamp_record(rec_, seq, stream_));
-    end_compaction(await(rec_[0], seq).ticks);
+    MGBFS_HIP(stamp_record(rec_, counters(), seq, stream_));
+    end_compaction(await(rec_[0], seq));
   }
 
   void memory_returned(uint64_t bytes) override { budget_ += bytes; }
@@ -408,13 +407,16 @@ class SortedEngine final : public Engine {
     r.rows = rows;
     r.rec = rec_;
     r.seq = seq_;
+    r.counters = counters();
     seq_ += kBlockLayers + 2;
     MGBFS_HIP(sorted_block_run(r, action(), stream_));
     uint64_t first = 0;
     for (uint32_t i = 0;; ++i) {
       const LayerRecord& rec = await(rec_[i], r.seq + i);
-      if (i == 0) first = rec.ticks;
-      end_compaction(rec.ticks);
+      if (i == 0) {
+        first = rec.stamps[0];
+        end_compaction(rec);
+      }
       const int s = take(rec, rec.children, rec.ticks - first);
       first = rec.ticks;
       if (s != kTakeNext) {
@@ -460,7 +462,8 @@ class SortedEngine final : public Engine {
     const OwnerRules rules{owners, rows, low, owners * kOwnerMean};
     const uint64_t seq = seq_;
     seq_ += kBlockLayers + 2;
-    MGBFS_HIP(owner_begin(counts, kOwnerBuffers * kOwnersMax * kCountStride, ctl, static_cast<uint32_t>(F), stream_));
+    MGBFS_HIP(owner_begin(counts, kOwnerBuffers * kOwnersMax * kCountStride, ctl, static_cast<uint32_t>(F), stream_,
+                          rec_, counters()));
     OwnerImport im{};
     im.cur = bank_[cur_].as<uint64_t>();
     im.F = static_cast<uint32_t>(F);
@@ -502,8 +505,9 @@ class SortedEngine final : public Engine {
           MGBFS_HIP(owner_report(ctl + most % kOwnerRing, rules, rec_ + most % kOwnerRing, seq + most, stream_));
       }
       const LayerRecord& rec = await(rec_[r % kOwnerRing], seq + r);
-      end_compaction(rec.ticks);
       if (r == 0) {
+        end_compaction(rec);
+        charge(0, rec.ticks - rec.stamps[0]);  // the import
         s = rec.state == kLayerNext ? kTakeNext : kTakeRejected;
       } else {
         s = take(rec, children, rec.ticks - ticks);
@@ -526,9 +530,7 @@ class SortedEngine final : public Engine {
   // A layer's record into the engine's state and counters; C: children
   // generated for it.
   int take(const LayerRecord& rec, uint64_t C, uint64_t ticks) {
-    const double seconds = static_cast<double>(ticks) * tick_seconds_;
-    phase_seconds[4] += seconds;
-    kernel_seconds += seconds;
+    charge(0, ticks);
     if (rec.state == kLayerRejected) return kTakeRejected;
     const uint64_t F = count_[cur_];
     const bool masked = layout_.prune && layers.size() > 1;
@@ -536,7 +538,7 @@ class SortedEngine final : public Engine {
     unique_candidates += rec.unique;
     last_ratio_ = masked ? static_cast<double>(C) / static_cast<double>(F) : 0.0;
     const uint64_t bytes = 16 * F + 16 * C + 8 * rec.N;
-    phase_bytes[4] += bytes;
+    phase_bytes[0] += bytes;
     streamed_bytes += bytes;
     ++launches;
     if (rec.state == kLayerEmpty) return kTakeEmpty;
@@ -613,18 +615,20 @@ class SortedEngine final : public Engine {
     terminal = true;
     return MGBFS_RESOURCE;
   }
-  // A compaction runs unwaited: the time from the layer's record to the next
-  // stamp on the stream is charged to it (phase 3).
+  LayerCounters* counters() { return control_.as<LayerCounters>(); }
+  void charge(uint32_t phase, uint64_t ticks) {
+    const double s = static_cast<double>(ticks) * tick_seconds_;
+    phase_seconds[phase] += s;
+    kernel_seconds += s;
+  }
+  // A compaction runs unwaited; the next record tells when it ended.  (Not
+  // when something else began: the host may have been away in between.)
   void compact(uint64_t* sub, uint32_t nsub, uint32_t fb, int nxt) {
     MGBFS_HIP(sorted_compact(sub, nsub, fb, off_[nxt].as<uint32_t>(), error_word(), bank_cap_[nxt],
-                             bank_[nxt].as<uint64_t>(), stream_));
+                             bank_[nxt].as<uint64_t>(), stream_, &counters()->compacted));
   }
-  void end_compaction(uint64_t ticks) {
-    if (compacted_) {
-      const double s = static_cast<double>(ticks - compacted_) * tick_seconds_;
-      phase_seconds[3] += s;
-      kernel_seconds += s;
-    }
+  void end_compaction(const LayerRecord& rec) {
+    if (compacted_ && rec.compacted > compacted_) charge(3, rec.compacted - compacted_);
     compacted_ = 0;
   }
   // Routing output size as passed to the kernels; the test flag reports an
@@ -638,14 +642,11 @@ class SortedEngine final : public Engine {
   // count scan is charged to phase 3 with the compaction it feeds.
   void account(const LayerRecord& rec, uint64_t F, uint64_t Fp, bool partitioned) {
     const uint64_t C = rec.children, N = rec.N;
-    end_compaction(rec.stamps[0]);
+    end_compaction(rec);
     const uint64_t routed = partitioned ? rec.stamps[1] : rec.stamps[2];
     const uint64_t ticks[4] = {routed - rec.stamps[0], rec.stamps[2] - routed, rec.stamps[3] - rec.stamps[2],
                                rec.ticks - rec.stamps[3]};
-    for (int p = 0; p < 4; ++p) {
-      phase_seconds[p] += static_cast<double>(ticks[p]) * tick_seconds_;
-      kernel_seconds += static_cast<double>(ticks[p]) * tick_seconds_;
-    }
+    for (int p = 0; p < 4; ++p) charge(p, ticks[p]);
     compacted_ = rec.ticks;
     const uint64_t be = 8 * F + 8 * C, bp = partitioned ? 16 * C : 0, bu = 8 * C + 8 * F + 8 * Fp + 8 * N;
     phase_bytes[0] += be;

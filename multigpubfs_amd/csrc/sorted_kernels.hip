@@ -582,13 +582,16 @@ __global__ __launch_bounds__(kUniqueThreads) __attribute__((amdgpu_waves_per_eu(
 __global__ __launch_bounds__(kRouteThreads) void compact_kernel(const uint64_t* __restrict__ cand, uint32_t nsub,
                                                                 uint32_t fb, const uint32_t* __restrict__ off,
                                                                 const uint32_t* __restrict__ error,
-                                                                uint64_t bank_rows, uint64_t* __restrict__ bank) {
+                                                                uint64_t bank_rows, uint64_t* __restrict__ bank,
+                                                                unsigned long long* done) {
   if (*error != 0 || off[static_cast<uint64_t>(nsub) << fb] > bank_rows) return;
   const uint32_t f = blockIdx.x;
   const uint64_t s = static_cast<uint64_t>(f) * kSlabStride;
   const uint32_t sh = fb;
   const uint64_t lo = off[static_cast<uint64_t>(f) << sh], hi = off[static_cast<uint64_t>(f + 1) << sh];
   for (uint64_t i = threadIdx.x; i < hi - lo; i += kRouteThreads) bank[lo + i] = cand[s + i];
+  // Blocks start in order: the last ones to end are among the last ones.
+  if (done && threadIdx.x == 0 && f + 1024 >= nsub) atomicMax(done, static_cast<unsigned long long>(wall_clock64()));
 }
 
 // Start layer: bank[0] = mix(start); offsets over 2^Ko fine buckets.
@@ -697,9 +700,9 @@ hipError_t sorted_unique_diff(uint64_t* cand, const uint32_t* scount, uint32_t n
 }
 
 hipError_t sorted_compact(const uint64_t* cand, uint32_t nsub, uint32_t fb, const uint32_t* off, const uint32_t* error,
-                          uint64_t bank_rows, uint64_t* bank, hipStream_t stream) {
+                          uint64_t bank_rows, uint64_t* bank, hipStream_t stream, unsigned long long* done) {
   hipLaunchKernelGGL(compact_kernel, dim3(nsub), dim3(kRouteThreads), 0, stream, cand, nsub, fb, off, error,
-                     bank_rows, bank);
+                     bank_rows, bank, done);
   return hipGetLastError();
 }
 

@@ -88,6 +88,10 @@ __global__ __launch_bounds__(kBlockThreads) void block_run_kernel(BlockRun r, Ac
   auto bank_of = [&](uint32_t b) { return b == 0 ? b0 : (b == 1 ? b1 : b2); };
   uint32_t cur = r.cur, prev = r.prev, F = r.F, Fp = r.prev_count, done = 0;
   LayerRecord* rec = r.rec;
+  if (threadIdx.x == 0) {
+    rec->stamps[0] = wall_clock64();
+    rec->compacted = r.counters->compacted;
+  }
   while (true) {
     const bool masked = L.prune && r.depth + done > 0;
     const uint64_t* from = bank_of(cur);
@@ -201,18 +205,23 @@ __global__ void sorted_start_kernel(uint64_t stored, uint64_t* bank, uint32_t* o
   if (threadIdx.x < 8) control[threadIdx.x] = 0;
 }
 
-__global__ void stamp_record_kernel(LayerRecord* rec, uint64_t seq) {
+__global__ void stamp_record_kernel(LayerRecord* rec, const LayerCounters* counters, uint64_t seq) {
   if (threadIdx.x != 0) return;
-  rec->ticks = wall_clock64();
+  rec->compacted = counters->compacted;
   __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ------------------------------------------------------------ owner layers
 
 __global__ __launch_bounds__(kBlockThreads) void owner_begin_kernel(uint32_t* counts, uint32_t words, OwnerCtl* ctl,
-                                                                     uint32_t F) {
+                                                                     uint32_t F, LayerRecord* rec,
+                                                                     const LayerCounters* counters) {
   for (uint32_t i = blockIdx.x * kBlockThreads + threadIdx.x; i < words; i += gridDim.x * kBlockThreads) counts[i] = 0;
   if (blockIdx.x) return;
+  if (rec && threadIdx.x == 0) {
+    rec->stamps[0] = wall_clock64();
+    rec->compacted = counters->compacted;
+  }
   if (threadIdx.x < 2) {
     OwnerCtl c{};
     c.counts = threadIdx.x == 0 ? F : 0u;
@@ -530,7 +539,7 @@ static hipError_t with_action(const ActionRef& act, F f) {
 }
 
 hipError_t sorted_block_run(const BlockRun& run, const ActionRef& act, hipStream_t stream) {
-  if (run.cur > 2 || run.prev > kNoBank || run.prev == run.cur || run.F == 0 || run.max_layers == 0 || !run.rec ||
+  if (run.cur > 2 || run.prev > kNoBank || run.prev == run.cur || run.F == 0 || run.max_layers == 0 || !run.rec || !run.counters ||
       run.F > kBlockParents || (run.prev < kNoBank && !run.L.prune && run.prev_count > kBlockParents))
     return hipErrorInvalidValue;
   return with_action(act, [&](auto a) {
@@ -543,13 +552,15 @@ hipError_t sorted_start(uint64_t stored, uint64_t* bank, uint32_t* off, uint64_t
   return hipGetLastError();
 }
 
-hipError_t stamp_record(LayerRecord* rec, uint64_t seq, hipStream_t stream) {
-  hipLaunchKernelGGL(stamp_record_kernel, dim3(1), dim3(64), 0, stream, rec, seq);
+hipError_t stamp_record(LayerRecord* rec, const LayerCounters* counters, uint64_t seq, hipStream_t stream) {
+  hipLaunchKernelGGL(stamp_record_kernel, dim3(1), dim3(64), 0, stream, rec, counters, seq);
   return hipGetLastError();
 }
 
-hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream) {
-  hipLaunchKernelGGL(owner_begin_kernel, dim3(std::min<uint32_t>(16, (words + 4 * kBlockThreads - 1) / (4 * kBlockThreads))), dim3(kBlockThreads), 0, stream, counts, words, ctl, F);
+hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t stream,
+                       LayerRecord* rec, const LayerCounters* counters) {
+  const uint32_t blocks = std::min<uint32_t>(16, (words + 4 * kBlockThreads - 1) / (4 * kBlockThreads));
+  hipLaunchKernelGGL(owner_begin_kernel, dim3(blocks), dim3(kBlockThreads), 0, stream, counts, words, ctl, F, rec, counters);
   return hipGetLastError();
 }
 

@@ -35,7 +35,8 @@ hipError_t zero_u32x3(uint32_t* a, uint64_t na, uint32_t* b, uint64_t nb, uint32
   std::fill(b, b + nb, 0u);
   return fake::launch(s);
 }
-hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t s) {
+hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t F, hipStream_t s, LayerRecord*,
+                       const LayerCounters*) {
   std::fill(counts, counts + words, 0u);
   ctl[0] = ctl[1] = OwnerCtl{};
   ctl[0].counts = F;

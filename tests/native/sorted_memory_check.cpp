@@ -36,7 +36,8 @@ hipError_t sorted_block_run(const BlockRun& r, const ActionRef&, hipStream_t s) 
   r.rec->seq = r.seq;
   return fake::launch(s);
 }
-hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t, hipStream_t s) {
+hipError_t owner_begin(uint32_t* counts, uint32_t words, OwnerCtl* ctl, uint32_t, hipStream_t s, LayerRecord*,
+                       const LayerCounters*) {
   require(holds(counts, 4ull * words) && holds(ctl, sizeof *ctl), "owners' counts");
   queued = 0;
   return fake::launch(s);
@@ -104,11 +105,11 @@ hipError_t exclusive_scan_u32(const uint32_t*, uint64_t n, uint32_t* out, uint32
   return fake::launch(s);
 }
 hipError_t sorted_compact(const uint64_t* cand, uint32_t nsub, uint32_t, const uint32_t*, const uint32_t*,
-                          uint64_t bank_rows, uint64_t* bank, hipStream_t s) {
+                          uint64_t bank_rows, uint64_t* bank, hipStream_t s, unsigned long long*) {
   require(holds(cand, 8ull * nsub * kSlabStride) && holds(bank, 8 * bank_rows), "a compaction");
   return fake::launch(s);
 }
-hipError_t stamp_record(LayerRecord* rec, uint64_t seq, hipStream_t s) {
+hipError_t stamp_record(LayerRecord* rec, const LayerCounters*, uint64_t seq, hipStream_t s) {
   rec->seq = seq;
   return fake::launch(s);
 }

@@ -531,3 +531,33 @@ def test_small_groups_of_large_degree_take_little_memory(n, backend):
             if n == 11:
                 e.rebind(lrx(n))
                 assert e.run() == 1 and e.layer_sizes() == O.packed_bfs(n)["layers"]
+
+
+@pytest.mark.parametrize("name", ["lrx8", "lrx9", "coxeter8_unmasked", "labels15"])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_sorted_phases_cover_the_run(name, stepwise):
+    make, flags = RUN_AHEAD[name]
+    with NativeEngine(GraphDefinition.permutation(*make()), backend="sorted", flags=flags) as e:
+        while stepwise and e.advance() == 0:
+            pass
+        assert e.status == 1 if stepwise else e.run() == 1
+        info, phases = e.info(), e.phases()
+    assert len(phases) == 4 and all(s >= 0 for s, _ in phases)
+    assert info["kernel_seconds"] > 0
+    assert math.isclose(sum(s for s, _ in phases), info["kernel_seconds"], rel_tol=1e-9)
+    assert sum(b for _, b in phases) == info["algorithmic_bytes"] > 0
+
+
+@pytest.mark.parametrize("flags", [0, 4], ids=["run_ahead", "general"])
+def test_kernel_seconds_leave_out_the_host(flags):
+    # The host sleeps between the layers (0.9 s in all); the kernels take some
+    # milliseconds, as when nothing waits.
+    import time
+    with NativeEngine(lrx(10), backend="sorted", flags=flags) as e:
+        assert e.run() == 1
+        together = e.info()["kernel_seconds"]
+        e.reset()
+        while e.advance() == 0:
+            time.sleep(0.02)
+        apart = e.info()["kernel_seconds"]
+    assert 0 < together < 0.1 and together / 8 < apart < 0.1
