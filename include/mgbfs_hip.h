@@ -121,10 +121,11 @@ typedef struct mgbfs_engine_info {
  * admission figures of the reference's GenericMemoryPlan /
  * GenericDistributedMemoryPlan (crates/mgbfs-runtime/src/generic_memory.rs:
  * 36-49, generic_distributed_memory.rs:7-13) for the backend this library
- * would pick.  (An engine created with MGBFS_BACKEND_AUTO runs inverse-closed
- * permutations of degree 3 to 12 on the bitmap backend where its memory fits
- * the budget and no capacity is set; their plan is the sorted backend's,
- * which takes them otherwise.)  With options->vram_budget = 0 the budget is the device's free
+ * would pick.  (With MGBFS_BACKEND_AUTO the plan of inverse-closed
+ * permutations is the sorted backend's, which ranks, whose layers have a
+ * capacity, run.  An engine without one may take the bitmap up to degree 12;
+ * its plan is the one of the backend that mgbfs_engine_info names.)  With
+ * options->vram_budget = 0 the budget is the device's free
  * memory minus the 2 GiB (or 256 MiB, MGBFS_FLAG_MAX_CAPACITY) reserve. */
 typedef struct mgbfs_engine_plan_info {
   uint32_t backend;          /* MGBFS_BACKEND_* chosen                               */

@@ -827,7 +827,7 @@ static bool packed_segmented(const Graph& g, const mgbfs_engine_options& o, Wide
   if (!g.inverse_closed || o.capacity ||
       (o.flags & (MGBFS_FLAG_TEST_COLLIDE_HASH | MGBFS_FLAG_TEST_TINY_SEGMENTS)) || !make_wide(g, code, 60))
     return false;
-  MGBFS_HIP(hipSetDevice(o.device));
+  if (!o.vram_budget) MGBFS_HIP(hipSetDevice(o.device));
   return vram_budget(o) >= (1ull << 30);
 }
 
@@ -835,11 +835,20 @@ static bool packed_segmented(const Graph& g, const mgbfs_engine_options& o, Wide
 // banks grown by a quarter, plus per child (G-1 with back-edge masks, else
 // G) a sub-bucket slab entry (8 B at the mean fill of 5000 of 5120) and an
 // owner-lane slab entry with its slack (10 B).
-static uint64_t sorted_bytes_per_state(const Graph& g) {
+static uint32_t sorted_children(const Graph& g, uint32_t key_bits) {
   const uint32_t G = g.generators;
-  const bool masks = G + 2 <= 64 - 4 * g.elements;
-  const uint32_t children = masks && G > 1 ? G - 1 : G;
-  return 30 + 18ull * children;
+  return G + 2 <= 64 - key_bits && G > 1 ? G - 1 : G;
+}
+static uint64_t sorted_bytes_per_state(uint32_t children) { return 30 + 18ull * children; }
+// Its fixed buffers, and the owners' slabs of layers run ahead (as
+// SortedEngine::run_owner takes them) for layers of up to `capacity` states.
+constexpr uint64_t kSortedFixed = 5 * ((1ull << 20) + 1) * 4 + (1ull << 20);
+static uint64_t sorted_slab_bytes(uint64_t capacity, uint32_t children, uint64_t budget) {
+  const auto slabs = [](uint64_t owners) { return 5 * 8 * (owners * kSlabStride + kRouteDump); };
+  const uint64_t most = capacity > (1ull << 40) ? ~0ull : capacity * children;
+  if (most <= kBlockChildren) return 0;
+  const uint64_t want = slabs(most <= kOwnersSmall * kOwnerMean / 2 ? kOwnersSmall : kOwnersMax);
+  return want <= budget / 8 ? want : std::min(slabs(kOwnersSmall), budget / 8);
 }
 
 mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o) {
@@ -852,7 +861,8 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
   const uint64_t G = g.generators;
   switch (p.backend) {
     case MGBFS_BACKEND_BITMAP: {
-      // BitmapEngine: n!-bit bitmap plus two frontier arrays of capacity rows.
+      // BitmapEngine: n!-bit bitmap plus two frontier arrays of capacity rows;
+      // by owners: lists of the whole group and the messages of any layer.
       const uint64_t domain = factorial_u64(g.elements);
       const uint64_t bitmap = (domain + 31) / 32 * 4;
       if (bitmap + 64 * 1024 > p.budget_bytes) throw std::runtime_error("BITMAP_VRAM_CAPACITY");
@@ -862,11 +872,15 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
       p.batch = p.capacity;
       p.table_slots = domain;
       p.device_bytes = bitmap + 16 * p.capacity + 8000 + 64;
+      if (rank_bitmap_takes(g, o)) {
+        p.capacity = p.batch = domain;
+        p.device_bytes = rank_bitmap_bytes(g);
+      }
       break;
     }
     case MGBFS_BACKEND_SORTED: {
-      const uint64_t per = sorted_bytes_per_state(g);
-      const uint64_t fixed = 5 * ((1ull << 20) + 1) * 4 + (1ull << 20);
+      const uint32_t children = sorted_children(g, 4 * g.elements);
+      const uint64_t per = sorted_bytes_per_state(children), fixed = kSortedFixed;
       if (fixed + per > p.budget_bytes) throw std::runtime_error("SORTED_VRAM_CAPACITY");
       uint64_t cap = (p.budget_bytes - fixed) / per;
       if (p.state_bound) cap = std::min(cap, p.state_bound);
@@ -877,7 +891,7 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
       p.capacity = cap;
       p.batch = cap;
       p.table_slots = 0;
-      p.device_bytes = fixed + per * cap;
+      p.device_bytes = std::min(p.budget_bytes, fixed + per * cap + sorted_slab_bytes(cap, children, p.budget_bytes));
       break;
     }
     case MGBFS_BACKEND_SEGMENTED: {
@@ -895,6 +909,14 @@ mgbfs_engine_plan_info plan_engine(const Graph& g, const mgbfs_engine_options& o
       p.batch = std::max<uint64_t>(1, std::min<uint64_t>(cap, (1ull << 22) / G));
       p.table_slots = 2 * cap;
       p.device_bytes = (g.inverse_closed ? 3 : 1) * per * cap;
+      // States of one word run in the sorted backend's banks first.
+      WideCode code;
+      if (packed_segmented(g, o, code)) {
+        const uint32_t children = sorted_children(g, std::max(32u, code.key_bits()));
+        const uint64_t packed = kSortedFixed + sorted_bytes_per_state(children) * cap +
+                                sorted_slab_bytes(cap, children, p.budget_bytes);
+        p.device_bytes = std::max(p.device_bytes, std::min(p.budget_bytes, packed));
+      }
       break;
     }
     default: {

@@ -151,6 +151,8 @@ Engine* make_bitmap_engine(const Graph& g, const mgbfs_engine_options& o);
 // bytes of it held by the engine that would be rebound).
 bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o, uint64_t held = 0);
 bool rank_bitmap_for_auto(const Graph& g, const mgbfs_engine_options& o, uint64_t held = 0);
+// Device bytes of its engine at most.
+uint64_t rank_bitmap_bytes(const Graph& g);
 // True: the permutations generate at least the alternating group of their
 // degree (5 to 12).  False: not, or not seen in a few tries.
 bool reaches_whole_group(const Graph& g);

@@ -441,8 +441,18 @@ BfsOutcome run_bfs(const GraphDoc& graph, const BfsRequest& req, EngineCache* ca
     if (cache) {
       cache->engine = engine;
       cache->key = key;
-      cache->plan = r.plan;
     }
+    // "auto" may take another backend for one device than the plan's, which
+    // is the one that ranks run: the report's plan is of the engine there is.
+    mgbfs_engine_info made{};
+    if (mgbfs_engine_query(engine, &made) == 0 && made.backend != r.plan.backend) {
+      mgbfs_engine_options named = opts;
+      named.backend = made.backend;
+      named.vram_budget = r.plan.budget_bytes;  // as it was before the engine's own memory
+      mgbfs_engine_plan_info plan{};
+      if (mgbfs_engine_plan(&desc, &named, &plan, err, sizeof err) == 0) r.plan = plan;
+    }
+    if (cache) cache->plan = r.plan;
   }
   if (cache) r.plan = cache->plan;
   r.setup_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - setup0).count();

@@ -269,12 +269,6 @@ class RankBitmapEngine final : public Engine {
     if (stream_) (void)hipStreamDestroy(stream_);
   }
 
-  // Device bytes with message buffers that hold every layer.
-  static uint64_t most_bytes(const Graph& g) {
-    const RankPlan p = rank_plan(g.elements);
-    return p.owners * (4ull * p.slice_words + 4ull * p.list_cap + 8ull * RankRun::last_cap(p, g.generators)) + (1u << 20);
-  }
-
   void reset() override {
     MGBFS_HIP(hipSetDevice(device_));
     run_.start(stream_);
@@ -415,6 +409,12 @@ class RankBitmapEngine final : public Engine {
   uint32_t wanted_ = 0;  // messages per owner that the next layers need
 };
 
+uint64_t rank_bitmap_bytes(const Graph& g) {
+  const RankPlan p = rank_plan(g.elements, RankRun::owners_for(g));
+  const uint64_t messages = p.owners == 1 ? 0 : p.owners * static_cast<uint64_t>(RankRun::last_cap(p, g.generators)) + kRouteDump;
+  return p.owners * (4ull * p.slice_words + 4ull * p.list_cap) + RankRun::words_bytes(p) + 2 * 4 * messages;
+}
+
 // All degrees that ranks and slices are made for: faster from the smallest to
 // degree 12 (figures in rank_owner.hip).  A capacity bounds the rows of a
 // layer and a message buffer is not one, so a set capacity keeps the shared
@@ -428,7 +428,7 @@ bool rank_bitmap_takes(const Graph& g, const mgbfs_engine_options& o, uint64_t h
   if (g.elements < 3 || g.elements > kRankDegree || o.capacity || g.generators > kMaxGenerators) return false;
   if (g.elements >= 11 && !reaches_whole_group(g)) return false;
   if (!o.vram_budget) MGBFS_HIP(hipSetDevice(o.device));
-  return RankBitmapEngine::most_bytes(g) <= vram_budget(o) + (o.vram_budget ? 0 : held);
+  return rank_bitmap_bytes(g) <= vram_budget(o) + (o.vram_budget ? 0 : held);
 }
 
 // Inverse-closed graphs whose backend the library picks run by owners of the

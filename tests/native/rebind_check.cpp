@@ -133,6 +133,17 @@ int main() {
     e->rebind(graph_of(9, swaps(9, 3), false));
     require(e->run_to_end() == MGBFS_COMPLETE && e->layers == plain(graph_of(9, swaps(9, 3), false)), "and rebound");
   }
+  // The plan by name holds what its engine comes to take.
+  for (uint32_t n : {3u, 7u, 8u, 9u})
+    for (uint32_t count : {1u, 2u, 16u}) {
+      o.backend = MGBFS_BACKEND_BITMAP;
+      o.vram_budget = 0;
+      const Graph g = graph_of(n, swaps(n, std::min(count, n == 3 ? 3u : 16u)), true);
+      const mgbfs_engine_plan_info p = plan_engine(g, o);
+      std::unique_ptr<Engine> e(create(g, o));
+      e->run_to_end();
+      require(p.backend == e->backend && e->device_bytes <= p.device_bytes, "no more than planned");
+    }
   // A given budget bounds a rebound engine by name too.
   o.backend = MGBFS_BACKEND_BITMAP;
   o.vram_budget = 64ull << 20;

@@ -259,3 +259,18 @@ def test_graph_rank_refuses_worlds_above_one(tmp_path):
     (tmp_path / "launch.json").write_text(json.dumps(launch))
     proc = mgbfs("graph-rank", path, tmp_path / "launch.json", "0", tmp_path / "id", tmp_path / "r1", "0", check=False)
     assert error_code(proc) == "GRAPH_LAUNCH_IDENTITY_OR_GEOMETRY"
+
+
+@pytest.mark.parametrize("graph,backend", [(lrx(8), "permutation_bitmap"), (lrx(10), "permutation_bitmap"),
+                                           (GraphDefinition.permutation(O.lrx_generators(13), [0] * 6 + [1] * 7), "sorted"),
+                                           (GraphDefinition.permutation(O.lrx_generators(15), [0] * 5 + [1] * 5 + [2] * 5), "sorted"),
+                                           (sl2(13), "segmented"), (sl2(101), "segmented"),
+                                           (GraphDefinition.permutation(O.lrx_generators(22), [0] * 11 + [1] * 11), "segmented"),
+                                           (directed_graph(), "permutation_bitmap")],
+                         ids=["lrx8", "lrx10", "labels13", "labels15", "sl2_13", "sl2_101", "ring22", "directed7"])
+def test_report_plan_is_of_the_engine_that_ran(tmp_path, graph, backend):
+    report = run_graph(graph, tmp_path / "out", device=0)
+    assert report["status"] == "COMPLETE"
+    assert report["plan"]["backend"] == backend
+    assert 0 < report["arena_bytes"] <= report["plan"]["device_bytes"]
+    assert report["capacity"] == report["plan"]["capacity"] >= max(report["layer_sizes"])
