@@ -499,6 +499,7 @@ class BatchEngine {
     count = std::min<uint64_t>(limit, d.count);
     std::vector<uint64_t> keys(count);
     if (count && d.rank.owners) {
+      MGBFS_HIP(hipSetDevice(device_));
       DeviceBuffer out;
       out.allocate(8 * count);
       MGBFS_HIP(batch_owned_export(d, count, out.as<uint64_t>(), stream_));
@@ -668,6 +669,7 @@ class BatchEngine {
   // kernel and one download, then a single wait.
   void gather(const std::vector<int32_t>& done) {
     if (done.empty()) return;
+    MGBFS_HIP(hipSetDevice(device_));
     uint64_t total = 0;
     for (int32_t slot : done) total += host_inst_[slot].depth + 1ull;
     if (total > 0xffffffffull) throw std::runtime_error("BATCH_GATHER_SIZE");

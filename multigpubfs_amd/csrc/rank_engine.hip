@@ -295,6 +295,7 @@ class RankBitmapEngine final : public Engine {
   }
   void rebind(const Graph& g) override {
     if (g.elements != n_ || !g.packable() || !g.distinct_perm()) throw std::runtime_error("ENGINE_REBIND_SHAPE");
+    MGBFS_HIP(hipSetDevice(device_));
     const RankPlan p = rank_plan(n_, RankRun::owners_for(g));
     if (p.owners != run_.plan.owners) take_plan(p);
     else ensure_messages(RankRun::first_cap(p, g.generators));  // or the old graph stays

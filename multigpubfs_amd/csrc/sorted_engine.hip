@@ -303,6 +303,7 @@ class SortedEngine final : public Engine {
 
   void settle() override {
     if (!compacted_) return;
+    MGBFS_HIP(hipSetDevice(device_));
     const uint64_t seq = seq_++;
     MGBFS_HIP(stamp_record(rec_, counters(), seq, stream_));
     end_compaction(await(rec_[0], seq));

@@ -48,6 +48,10 @@ hipError_t batch_install(BatchInstance* to, const BatchInstance* staged, const B
   }
   return fake::launch(s);
 }
+hipError_t batch_owned_export(const BatchInstance&, uint64_t, uint64_t* keys, hipStream_t s) {
+  require(holds(keys, 8), "a sample");
+  return fake::launch(s);
+}
 hipError_t batch_gather_sizes(const BatchInstance*, const uint32_t*, uint32_t, uint64_t*, hipStream_t s) {
   return fake::launch(s);
 }
@@ -135,6 +139,43 @@ int main() {
     b.admit(rotations(11), 1, 0, &s);
     b.step(1);
     require(shared_nodes == 8 && owned_nodes == 8, "graphs are built once");
+  }
+  // Calls from a thread whose current device is another.
+  {
+    Graph g;
+    g.elements = 11;
+    g.generators = 2;
+    for (uint32_t i = 0; i < 11; ++i) g.perms.push_back((i + 1) % 11);
+    for (uint32_t i = 0; i < 11; ++i) g.perms.push_back(i < 2 ? 1 - i : i);
+    for (uint32_t i = 0; i < 11; ++i) g.start.push_back(i);
+    mgbfs_release_cached_memory(0);
+    mgbfs_batch_options o{};
+    slots = o.max_slots = 2;
+    o.vram_budget = 4ull << 30;
+    o.device = 1;
+    fake::Device& d = fake::dev();
+    {
+      BatchEngine b(o);
+      int32_t s = 0;
+      d.current = 0;
+      b.admit(g, 1, 0, &s);
+      d.current = 0;
+      b.step(1);
+      require(inst[s].rank.owners != 0, "an instance by owners");
+      inst[s].count = 1;
+      b.step(1);
+      std::vector<int64_t> rows;
+      uint64_t n = 0;
+      d.current = 0;
+      b.sample(s, 1, rows, n);
+      d.current = 0;
+      require(n == 1 && b.poll(2).size() == 1, "a sample and the end");
+      d.current = 0;
+      b.release(s);
+      require(fake::all_on(1), "memory on the engine's device");
+    }
+    mgbfs_release_cached_memory(1);
+    d.current = 0;
   }
   uint32_t owned = 0, restarted = 0;
   for (uint32_t n : {9u, 10u, 11u})

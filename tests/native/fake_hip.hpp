@@ -14,6 +14,7 @@ namespace fake {
 
 struct Device {
   std::map<char*, size_t> live;  // device allocations
+  std::map<char*, int> home;     // and their devices
   size_t used = 0, limit = ~static_cast<size_t>(0);
   int current = 0, launches = 0;
   long room = -1;  // allocations that still succeed (-1: all)
@@ -43,6 +44,13 @@ struct Stream {
   int device;
 };
 
+// Is all memory on this device?
+inline bool all_on(int device) {
+  for (const auto& h : dev().home)
+    if (h.second != device) return false;
+  return true;
+}
+
 }  // namespace fake
 
 extern "C" {
@@ -53,6 +61,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   if (d.room > 0) --d.room;
   *p = std::calloc(1, bytes);
   d.live[static_cast<char*>(*p)] = bytes;
+  d.home[static_cast<char*>(*p)] = d.current;
   d.used += bytes;
   return hipSuccess;
 }
@@ -63,6 +72,7 @@ hipError_t hipFree(void* p) {
   fake::require(it != d.live.end(), "hipFree of what is not allocated");
   std::memset(p, 0xdd, std::min<size_t>(it->second, 1 << 20));
   d.used -= it->second;
+  d.home.erase(it->first);
   d.live.erase(it);
   std::free(p);
   return hipSuccess;

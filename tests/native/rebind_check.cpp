@@ -161,6 +161,32 @@ int main() {
             }),
             "repeated labels are refused as before");
   }
+  // An engine's calls from a thread whose current device is another.
+  for (uint32_t kind : {0u, static_cast<uint32_t>(MGBFS_BACKEND_BITMAP)}) {
+    o = mgbfs_engine_options{};
+    o.backend = kind;
+    o.device = 1;
+    const Graph two = graph_of(9, swaps(9, 8), true), more = graph_of(9, swaps(9, 16), true);
+    std::unique_ptr<Engine> e(create(two, o));
+    uint64_t n = 0;
+    std::vector<int64_t> rows;
+    d.current = 0;
+    e->rebind(more);
+    d.current = 0;
+    require(e->run_to_end() == MGBFS_COMPLETE, "a run");
+    d.current = 0;
+    e->reset();
+    for (uint32_t fatal, k = 0; k < 6; ++k) {
+      d.current = 0;
+      e->advance(&n, &fatal);
+    }
+    d.current = 0;
+    e->settle();
+    e->sample(0, 4000, rows, n);
+    require(n > 1024 && fake::all_on(1), "memory on the engine's device");
+    d.current = 0;
+  }
+  o = mgbfs_engine_options{};
   // One workgroup or many, by the rebound graph's children.
   o.vram_budget = 0;
   for (uint32_t kind : {0u, static_cast<uint32_t>(MGBFS_BACKEND_BITMAP)}) {

@@ -100,6 +100,7 @@ hipError_t exclusive_scan_u32(const uint32_t*, uint64_t n, uint32_t* out, uint32
   require(holds(out, 4 * (n + 1)) && holds(workspace, 4 * scan_workspace_words(n)), "a scan");
   rec->N = next_size();
   rec->children = 2 * engine->layers.back();
+  rec->ticks = 1;
   rec->state = 0;
   rec->seq = seq;
   return fake::launch(s);
@@ -179,6 +180,26 @@ int main() {
   engine.reset(make_sorted_engine(g, o));
   const uint64_t made = engine->device_bytes;
   require(engine->run_to_end() == MGBFS_COMPLETE && engine->device_bytes - made < (1u << 20), "small banks");
+  // Calls from a thread whose current device is another.
+  for (uint32_t flags : {0u, static_cast<uint32_t>(MGBFS_FLAG_TEST_TIGHT_SLABS)}) {
+    script = sizes;
+    o.flags = flags;
+    o.device = 1;
+    engine.reset(make_sorted_engine(g, o));
+    while (!engine->terminal) {
+      uint64_t n = 0;
+      uint32_t fatal = 0;
+      d.current = 0;
+      engine->advance(&n, &fatal);
+      d.current = 0;
+      engine->settle();
+      std::vector<int64_t> rows;
+      d.current = 0;
+      engine->sample(0, 1, rows, n);
+    }
+    require(engine->layers == want && fake::all_on(1), "memory on the engine's device");
+    d.current = 0;
+  }
   engine.reset();
   std::printf("sorted memory ok\n");
   return 0;
