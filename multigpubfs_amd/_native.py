@@ -228,6 +228,16 @@ def device_info(device: int = 0) -> dict:
                 free_bytes=fr.value)
 
 
+def release_cached_memory(device: int = 0) -> None:
+    """Give back the device memory (up to 16 GiB) that closed batch engines of
+    this process left for the next ones.  device_info() and this library's
+    budgets count it as free; other allocators of the process do not."""
+    lib = load()
+    lib.mgbfs_release_cached_memory.argtypes = [C.c_int32]
+    lib.mgbfs_release_cached_memory.restype = None
+    lib.mgbfs_release_cached_memory(device)
+
+
 HISTORY = {"auto": 0, "full": 1, "rolling": 2}
 
 

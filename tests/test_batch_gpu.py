@@ -434,3 +434,20 @@ def test_layer_beyond_the_declared_bound_is_an_error(n):
         sizes, _, error = b.result(slot)
         assert error and sizes == ref[:len(sizes)] and max(sizes) <= bound
         assert b.result(free)[0] == ref and not b.result(free)[2]
+
+
+def test_kept_memory_is_given_back_on_request():
+    import ctypes
+    from hip_memory import hip
+    from multigpubfs_amd import device_info, release_cached_memory
+
+    def kept():  # counted as free beyond what the device has
+        now, total = ctypes.c_size_t(), ctypes.c_size_t()
+        counted = device_info()["free_bytes"]
+        assert hip().hipMemGetInfo(ctypes.byref(now), ctypes.byref(total)) == 0
+        return counted - now.value
+
+    run_batched([x["graph"] for x in GOLDEN[:4]])
+    assert 1 << 30 <= kept() <= 16 << 30  # a chunk at least
+    release_cached_memory()
+    assert kept() == 0
