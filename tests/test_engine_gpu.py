@@ -561,3 +561,22 @@ def test_kernel_seconds_leave_out_the_host(flags):
             time.sleep(0.02)
         apart = e.info()["kernel_seconds"]
     assert 0 < together < 0.1 and together / 8 < apart < 0.1
+
+
+@pytest.mark.parametrize("generators", ["lrx", "directed", "random"])
+def test_shared_bitmap_run_to_end_at_every_tile_depth(generators):
+    # A capacity keeps the shared bitmap, whose queued layers give a thread one
+    # parent up to 524,288 parents and more beyond, up to what its generator
+    # count allows (directed: 12, LRX: 8, random: 3).
+    n = 11
+    rng = random.Random(2)
+    gens = {"lrx": O.lrx_generators(n), "directed": [O.lrx_generators(n)[0], O.lrx_generators(n)[2]],
+            "random": [rng.sample(range(n), n) for _ in range(8)]}[generators]
+    ref = O.packed_bfs(n, gens)["layers"]
+    assert max(ref) > 2 * 524288
+    with NativeEngine(GraphDefinition.permutation(gens, list(range(n))), backend="permutation_bitmap",
+                      capacity=math.factorial(n)) as e:
+        for _ in range(2):
+            assert e.run() == 1 and e.layer_sizes() == ref
+            e.reset()
+            assert e.advance() == 0

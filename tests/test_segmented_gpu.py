@@ -311,3 +311,24 @@ def test_layer_beyond_the_declared_bound_stops_the_run(name, bound):
             sizes = e.layer_sizes()
             assert sizes == want[:len(sizes)] and max(sizes) <= 1.25 * bound and len(sizes) > 3
             e.reset()
+
+
+@pytest.mark.parametrize("labels", [(7, 200), (-5, 70000)], ids=["bytes", "int64"])
+def test_wide_keys_hand_their_labels_over(labels):
+    # Sixteen generators over two labels on 24 places (2.7 million states):
+    # layers beyond the lowered limit of 2^18 children go on in the tables.
+    g = GraphDefinition.permutation(random_closed(24, 8, 9), [labels[0]] * 12 + [labels[1]] * 12)
+    seen = {}
+    for flags in (0, 128, SORTED_CAP):  # packed, the tables alone, handed over
+        with NativeEngine(g, backend="segmented", flags=flags) as e:
+            assert e.run() == 1
+            info = e.info()
+            last = sorted(map(tuple, e.sample(0, 1 << 22)))
+            seen[flags] = [e.layer_sizes(), last, info["candidates"]]
+            assert sum(e.layer_sizes()) == math.comb(24, 12) and len(last) == e.layer_sizes()[-1]
+            e.reset()
+            while sum(e.layer_sizes()) < 200_000:  # after the hand-over: the first 16 places of each state
+                assert e.advance() == 0
+            assert {v for which in (0, 1) for r in e.sample(which, 1000) for v in r} == set(labels)
+            seen[flags].append(sorted(e.layer_keys()))
+    assert seen[128] == seen[0] == seen[SORTED_CAP]
