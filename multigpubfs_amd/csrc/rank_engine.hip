@@ -396,10 +396,17 @@ class RankBitmapEngine final : public Engine {
       std::copy(records_.keys, records_.keys + limit, out.begin());
       return;
     }
+    // Through the idle message buffer where it holds them: a layer that was
+    // found is also read where no more device memory is left.
+    uint64_t room = 0;
+    uint64_t* to = run_.spare(&room);
     DeviceBuffer keys;
-    keys.allocate(limit * 8);
-    run_.export_layer(back, limit, keys.as<uint64_t>(), stream_);
-    MGBFS_HIP(hipMemcpyAsync(out.data(), keys.as<void>(), limit * 8, hipMemcpyDeviceToHost, stream_));
+    if (limit > room) {
+      keys.allocate(limit * 8);
+      to = keys.as<uint64_t>();
+    }
+    run_.export_layer(back, limit, to, stream_);
+    MGBFS_HIP(hipMemcpyAsync(out.data(), to, limit * 8, hipMemcpyDeviceToHost, stream_));
     MGBFS_HIP(hipStreamSynchronize(stream_));
   }
 

@@ -59,6 +59,11 @@ class RankRun {
   int run(uint64_t target, RankRecords& records, hipStream_t stream);
   // States of the current layer (back = 0) or the one before, as packed keys.
   void export_layer(uint64_t back, uint64_t limit, uint64_t* keys, hipStream_t stream);
+  // The message buffer that holds nothing between runs, as room for keys.
+  uint64_t* spare(uint64_t* keys) const {
+    *keys = memory.cap ? (static_cast<uint64_t>(plan.owners) * memory.cap + kRouteDump) / 2 : 0;
+    return reinterpret_cast<uint64_t*>(memory.messages[parity_ ^ 1u]);
+  }
   uint32_t generators() const { return gens_.count; }
 
   RankPlan plan;

@@ -67,6 +67,15 @@ int main() {
     require(search() == MGBFS_COMPLETE && e->layers == want, "the search completes when there is room");
     d.limit = d.used;
     e->reset();
+    // Whole layers are read back without more memory and without harm.
+    for (uint64_t count = 0, k = 0; k < 5; ++k) {
+      uint32_t fatal = 0;
+      std::vector<uint64_t> keys;
+      require(e->advance(&count, &fatal) == MGBFS_LAYER, "a layer");
+      e->layer_keys(keys);
+      std::sort(keys.begin(), keys.end());
+      require(keys.size() == e->layers.back() && std::unique(keys.begin(), keys.end()) == keys.end(), "its states");
+    }
     require(search() == MGBFS_COMPLETE && e->layers == want, "and again without more");
     // A rebind that needs larger buffers than there is room for leaves the
     // old graph in place.
