@@ -12,6 +12,7 @@ using namespace mgbfs;
 static BatchInstance* inst;  // the device's
 static uint32_t overflow;    // owned instances' next step ends in this error
 static uint32_t slots;
+static uint32_t exports;                    // samples of instances by owners
 static uint32_t owned_nodes, shared_nodes;  // expansion kernels in the graphs built
 
 extern "C" hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) {
@@ -49,7 +50,8 @@ hipError_t batch_install(BatchInstance* to, const BatchInstance* staged, const B
   return fake::launch(s);
 }
 hipError_t batch_owned_export(const BatchInstance&, uint64_t, uint64_t* keys, hipStream_t s) {
-  require(holds(keys, 8), "a sample");
+  ++exports;
+  keys[0] = 0;
   return fake::launch(s);
 }
 hipError_t batch_gather_sizes(const BatchInstance*, const uint32_t*, uint32_t, uint64_t*, hipStream_t s) {
@@ -167,9 +169,12 @@ int main() {
       std::vector<int64_t> rows;
       uint64_t n = 0;
       d.current = 0;
+      const size_t held = d.used;
+      d.limit = held;  // small samples need no device memory
       b.sample(s, 1, rows, n);
+      d.limit = ~static_cast<size_t>(0);
       d.current = 0;
-      require(n == 1 && b.poll(2).size() == 1, "a sample and the end");
+      require(exports == 1 && n == 1 && b.poll(2).size() == 1, "a sample and the end");
       d.current = 0;
       b.release(s);
       require(fake::all_on(1), "memory on the engine's device");
