@@ -1,8 +1,9 @@
 // Host side of the batched multi-instance engine: slot admission with VRAM
 // planning, a pooled device allocator, and a layer loop in a hipGraph
 // (reset flag, then K x [tiles, clear, expand, owned, finish], of which a step
-// takes what its instances need) replayed until no instance is active.  Instances join and leave at layer boundaries, so the same
-// object serves both the fixed sweep and continuous-batching serving.
+// takes what its instances need) replayed until no instance is active.
+// Instances join and leave at layer boundaries, so the same object serves both
+// the fixed sweep and continuous-batching serving.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -129,9 +130,8 @@ struct BatchPlan {
 // and more (beside 8 S_8 0.70, 0.73, 0.70, 0.80), or alone (0.85, 0.77, 0.89,
 // 1.00), or four and more with at most twice as many of degree 9 (four each
 // 0.90, 0.71, 0.68, 0.77) and as many others (0.86, 0.74, 0.72, 0.83).  Not one
-// beside S_8 (1.19, 1.14, 1.17, 1.26), nor
-// one beside three S_9 (0.93, 0.81, 0.97, 1.12), two beside six (0.87, 0.70,
-// 1.04, 1.21).
+// beside S_8 (1.19, 1.14, 1.17, 1.26), nor one beside three S_9 (0.93, 0.81,
+// 0.97, 1.12), two beside six (0.87, 0.70, 1.04, 1.21).
 //
 // Degree 9 never by itself (two 1.06, 1.08, 1.20, 1.47; 200 of them 2.31,
 // 1.78, 1.12, 1.25), but with the others while it is not the most of them, as
@@ -156,13 +156,13 @@ struct OwnedChoice {
 };
 
 // Owners of an instance when `together` run by owners: at degree 9 and 10 so
-// many that a step's owners are about one a workgroup (S_10 LRX sets, milliseconds by
-// 251, 151, 101, 53 owners: one 1.24, 1.21, 1.24, 1.39; three 2.55, 1.49,
-// 1.50, 1.50; four 2.83, 2.11, 1.56, 1.54; eight 5.52, 3.45, 2.63, 1.84; with
-// sixteen generators 1.41, 1.37, 1.71, 2.59; 2.34, 1.84, 2.29, 2.66; 2.82,
-// 2.40, 2.35, 2.68; 5.19, 3.92, 4.16, 3.87), but not below 53, where a tile's
-// children meet on too few counters.  Degrees 11 and 12 keep their own number:
-// their layers are large.
+// many that a step's owners are about one a workgroup (S_10 LRX sets, in
+// milliseconds by 251, 151, 101, 53 owners: one 1.24, 1.21, 1.24, 1.39; three
+// 2.55, 1.49, 1.50, 1.50; four 2.83, 2.11, 1.56, 1.54; eight 5.52, 3.45, 2.63,
+// 1.84; with sixteen generators 1.41, 1.37, 1.71, 2.59; 2.34, 1.84, 2.29, 2.66;
+// 2.82, 2.40, 2.35, 2.68; 5.19, 3.92, 4.16, 3.87), but not below 53, where a
+// tile's children meet on too few counters.  Degrees 11 and 12 keep their own
+// number: their layers are large.
 uint32_t owners_for(uint32_t degree, uint32_t together) {
   if (degree >= 11) return rank_plan(degree).owners;
   return together <= 3 ? 151 : (together <= 6 ? 101 : 53);
@@ -641,7 +641,8 @@ class BatchEngine {
     }
     for (uint32_t s = 0; s < slots_n_; ++s) {
       if (!runs(s)) continue;
-      if (pending_[s] == kInstallSeed && owned_wanted_[s] && choice.takes(host_inst_[s].degree)) lay_out_owned(s, choice.together());
+      if (pending_[s] == kInstallSeed && owned_wanted_[s] && choice.takes(host_inst_[s].degree))
+        lay_out_owned(s, choice.together());
       forms |= host_inst_[s].rank.owners ? kBatchOwned : kBatchShared;
     }
     if (!forms) forms = kBatchShared;
@@ -728,7 +729,7 @@ class BatchEngine {
 
   int device_ = 0;
   hipStream_t stream_ = nullptr;
-  std::vector<uint8_t> owned_wanted_;  // per slot: may be laid out for owners by the next flush, if its block holds that
+  std::vector<uint8_t> owned_wanted_;  // per slot: may be laid out for owners by flush(), if its block holds that
   uint32_t slots_n_ = 0, grid_ = 0, clear_grid_ = 0, owned_grid_ = 0, layers_per_graph_ = kLayersPerGraph;
   uint32_t threads_ = 256, hash_load_pct_ = 50, layer_pct_ = 30, bitmap_bias_permille_ = 1000;
   uint32_t history_ = 0;

@@ -231,10 +231,11 @@ class BitmapEngine final : public Engine {
 
   // Runs to the end with up to kAhead layers queued per host wait, when
   // both frontier buffers can hold every state not yet reached (so no layer
-  // can outgrow them, and none is chunked): each layer reads its size and
-  // counter base from marks_ (the running counter before and after the
-  // layer that produced it) and a one-thread kernel records the counter
-  // after it.  Otherwise, and for bigger state spaces, one layer per wait.
+  // can outgrow them, and none is chunked): each layer reads its size from
+  // marks_, where the layer before it counted its states, and counts the next
+  // one's beside it.  Otherwise, and for bigger state spaces, one layer per
+  // wait.  Reached at degree <= 11 with a capacity that holds every unreached
+  // state; without one those degrees run by owners (rank_engine.hip).
   int run_to_end() override {
     if (terminal) return MGBFS_LAYER;
     const uint64_t remaining = domain_ - total();
